@@ -745,8 +745,10 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     }
     // a column-major or pre-scaled X is restaged row-major first (the
     // reference converts a non-row-major input, sparse_matrix.cpp:720-736)
-    if ((xcol || pre) && spm->ncols) {
-        const size_t xb = spm->ncols * (size_t)k * es;
+    // X has orig's columns as rows: a gather-order image counts its hot
+    // columns on top of them
+    if ((xcol || pre) && orig->ncols) {
+        const size_t xb = orig->ncols * (size_t)k * es;
         if (xb > ctx->xstage.bytes) {
             if (ctx->xstage.ptr) FMX_HIP(ctx, hipFree(ctx->xstage.ptr));
             ctx->xstage.ptr = nullptr;
@@ -754,7 +756,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
             FMX_HIP(ctx, hipMalloc(&ctx->xstage.ptr, xb));
             ctx->xstage.bytes = xb;
         }
-        st = stage_dense_rows(ctx, dtype, spm->ncols, k, X, ldx, xcol, pre, ctx->xstage.ptr, s);
+        st = stage_dense_rows(ctx, dtype, orig->ncols, k, X, ldx, xcol, pre, ctx->xstage.ptr, s);
         if (st) return st;
         X = ctx->xstage.ptr;
         ldx = k;

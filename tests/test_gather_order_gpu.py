@@ -84,3 +84,24 @@ def test_gather_order_weighted_streamed_layouts(fmx, orc, rmat16, forced):
     res.multiply_scaled_async(Xt, Ys, post=post)
     want = orc.spmm(img, X.astype(np.float64)) * post.cpu().numpy()[:, None]
     assert rel(Ys.cpu().numpy(), want) <= 2.0 ** -24 + 1e-15
+
+
+@pytest.mark.parametrize("n,k,col", [(65536, 8, True), (65536, 16, False), (50001, 3, True)])
+def test_gather_order_restages_x_rows_only(fmx, orc, rmat16, forced, n, k, col):
+    """A column-major or pre-scaled X is restaged with as many rows as X has;
+    the image's extra (hot) columns have no rows of their own in X or in the
+    scales, which end with their allocations here."""
+    import torch
+    src, dst = (v[(rmat16[0] < n) & (rmat16[1] < n)] for v in rmat16)
+    img = orc.build_2d(src, dst, n=n, log2h=6, log2w=15)
+    spm = fmx.SparseMatrix.upload(img.data, img.offs)
+    assert spm.info.hot_columns > 0
+    rng = np.random.default_rng(n + k)
+    X = rng.random((n, k)).astype(np.float32)
+    pre, post = rng.random(n) + 0.5, rng.random(n) + 0.5
+    Xt = dev(X.T).t() if col else dev(X)
+    Y = torch.empty((n, k), dtype=torch.float32, device="cuda")
+    spm.multiply_scaled_async(Xt, Y, pre=dev(pre), post=dev(post))
+    staged = (X.astype(np.float64) * pre[:, None]).astype(np.float32).astype(np.float64)
+    want = orc.spmm(img, staged) * post[:, None]
+    assert rel(Y.cpu().numpy(), want) <= 2.0 ** -24 + 1e-15
