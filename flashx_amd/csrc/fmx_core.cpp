@@ -16,8 +16,7 @@ namespace fmx {
 
 Plan::~Plan()
 {
-    if (d_items) (void)hipFree(d_items);
-    if (d_splits) (void)hipFree(d_splits);
+    if (d_items) (void)hipFree(d_items);  // d_splits lies behind them
 }
 
 Scratch::~Scratch()
@@ -234,36 +233,6 @@ uint32_t band_rows(const fmx_spm *spm, int k, int s)
     return (uint32_t)std::min<uint64_t>(hs, spm->H);
 }
 
-// The directory entries of one block row at a time: from the host copy, or
-// (an image built on the device keeps its directory in HBM only) copied
-// from HBM when a plan first needs them, which is only for the block rows
-// whose bands are split.
-class DirRows {
-public:
-    DirRows(fmx_ctx *ctx, const fmx_spm *s) : ctx_(ctx), s_(s) {}
-    // entries brow_dir[br] .. brow_dir[br + 1] - 1, or null after a failed copy
-    const uint2 *row(uint64_t br)
-    {
-        const uint32_t lo = s_->brow_dir[br], hi = s_->brow_dir[br + 1];
-        if (!s_->dir.empty()) return s_->dir.data() + lo;
-        auto it = cache_.find(br);
-        if (it != cache_.end()) return it->second.data();
-        std::vector<uint2> &v = cache_[br];
-        v.resize(hi - lo);
-        if (hipMemcpy(v.data(), s_->d_dir + lo, (size_t)(hi - lo) * sizeof(uint2), hipMemcpyDeviceToHost) !=
-            hipSuccess) {
-            (void)hip_fail(ctx_, hipGetLastError(), "directory copy");
-            return nullptr;
-        }
-        return v.data();
-    }
-
-private:
-    fmx_ctx *ctx_;
-    const fmx_spm *s_;
-    std::map<uint64_t, std::vector<uint2>> cache_;
-};
-
 // The last tile of block row br (entries d, local indices 0..n-1) starting
 // at or before word p, as a directory index.
 static uint32_t tile_at(const fmx_spm *s, uint64_t br, const uint2 *d, uint32_t p)
@@ -276,8 +245,7 @@ static uint32_t tile_at(const fmx_spm *s, uint64_t br, const uint2 *d, uint32_t 
 
 // Tile-relative row in force at word `p` of the block row whose first word
 // is `base` in a host image (kNone if `p` is a row-part or COO header);
-// plan_carries computes the same on the device for an image without a host
-// copy.
+// plan_cuts finds the same on the device for an image without a host copy.
 static uint32_t carry_at(const fmx_spm *s, uint64_t base, uint32_t p)
 {
     const uint16_t *w = reinterpret_cast<const uint16_t *>(s->host_image()) + base;
@@ -308,21 +276,27 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
         }
     }
     // Work cap: a band whose stream exceeds it is split into near-equal word
-    // ranges reduced in order afterwards (power-law hub rows).
+    // ranges reduced in order afterwards (power-law hub rows).  A matrix with
+    // words to spare for every wave the chip holds caps at 8192 (or four mean
+    // bands).  A smaller one would end on the few waves that walk the hub
+    // bands' chunks one after the other, so its cap is its share of 16 waves
+    // per CU, at least two chunks: R-MAT scale 16, FP64 k = 8, 73 us uncapped,
+    // 25 at 1024 words, 26 at 512, 31 at 2048; 260,000 vertices, k = 20, four
+    // NMF sweeps 4.6 ms, 2.5 at 2048, 2.7 at 1024, 3.0 at 4096; scale 20
+    // weighted 485 us at 8192, 491 at 4096, 515 at 2048.
     uint64_t avg = bands.empty() ? 0 : total / bands.size();
-    uint64_t cap = std::max<uint64_t>(8192, 4 * avg);
+    const uint64_t share = total / ((uint64_t)ctx->num_cus * 16);
+    uint64_t cap = std::min(std::max<uint64_t>(8192, 4 * avg), std::max<uint64_t>(1024, share));
     const char *e = getenv("FMX_ITEM_CAP");
     if (e) cap = std::max<uint64_t>(64, strtoull(e, nullptr, 10));
     if (ordered) cap = UINT64_MAX;  // one item per band: its rows are summed in stream order
 
     std::vector<Split> splits;
     uint32_t nslots = 0;
-    // carries of binary split items, resolved after the loop: item index,
-    // block row's first word, cut word
-    std::vector<size_t> carry_item;
-    std::vector<uint64_t> carry_base;
-    std::vector<uint32_t> carry_word;
-    DirRows dir_rows(ctx, s);
+    // An image built on the device keeps its words and its directory in HBM
+    // only: the ranges of split bands leave the host as plain fractions of
+    // their block row, and a kernel moves them to where an item may start.
+    const bool dev_cuts = s->dir.empty();
     for (const Band &b : bands) {
         uint32_t pieces = (uint32_t)(b.words / cap + (b.words % cap != 0));
         if (pieces < 1) pieces = 1;
@@ -343,26 +317,27 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
             plan->items.push_back(t);
             continue;
         }
-        std::vector<uint32_t> cut(pieces + 1), dirs(pieces + 1), carries(pieces + 1);
+        std::vector<uint32_t> cut(pieces + 1), dirs(pieces + 1, base.dir_end), carries(pieces + 1, kNone);
         cut[0] = 0;
         dirs[0] = s->brow_dir[b.br];
-        carries[0] = kNone;
-        const uint2 *d = dir_rows.row(b.br);
-        if (!d) return FMX_EHIP;
+        const uint2 *d = dev_cuts ? nullptr : s->dir.data() + s->brow_dir[b.br];
         for (uint32_t i = 1; i < pieces; i++) {
             uint32_t p = (uint32_t)((uint64_t)b.words * i / pieces);
-            if (p <= cut[i - 1]) p = cut[i - 1] + 1;
-            const uint32_t t = tile_at(s, b.br, d, p);
-            const uint32_t tx = d[t - s->brow_dir[b.br]].x;
-            if (s->esz) {
-                // weighted: cut at the tile start at or before p, so no row
-                // and no value position is carried into a piece
-                p = std::max(tx, cut[i - 1]);
-            } else if (p < tx + 8) {
-                p = tx + 8;  // out of the tile header
+            dirs[i] = s->brow_dir[b.br];
+            if (!dev_cuts) {
+                if (p <= cut[i - 1]) p = cut[i - 1] + 1;
+                const uint32_t t = tile_at(s, b.br, d, p);
+                const uint32_t tx = d[t - s->brow_dir[b.br]].x;
+                if (s->esz) {
+                    // weighted: cut at the tile start at or before p, so no row
+                    // and no value position is carried into a piece
+                    p = std::max(tx, cut[i - 1]);
+                } else {
+                    if (p < tx + 8) p = tx + 8;  // out of the tile header
+                    carries[i] = carry_at(s, (uint64_t)s->offs[b.br] / 2, p);
+                }
+                dirs[i] = t;
             }
-            dirs[i] = t;
-            carries[i] = kNone;  // binary: resolved below
             cut[i] = p;
         }
         cut[pieces] = b.words;
@@ -378,25 +353,9 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
             t.dir_begin = dirs[i];
             t.carry = carries[i];
             t.slot = nslots++;
-            if (i > 0 && !s->esz) {
-                carry_item.push_back(plan->items.size());
-                carry_base.push_back((uint64_t)s->offs[b.br] / 2);
-                carry_word.push_back(cut[i]);
-            }
             plan->items.push_back(t);
         }
         splits.push_back(sp);
-    }
-    if (!carry_item.empty()) {
-        std::vector<uint32_t> c;
-        if (s->host_bytes()) {
-            c.resize(carry_item.size());
-            for (size_t j = 0; j < c.size(); j++) c[j] = carry_at(s, carry_base[j], carry_word[j]);
-        } else {
-            fmx_status st = plan_carries(ctx, s, carry_base, carry_word, c);
-            if (st) return st;
-        }
-        for (size_t j = 0; j < c.size(); j++) plan->items[carry_item[j]].carry = c[j];
     }
     // Longest items first, so the hardware dispatcher approximates LPT.
     std::stable_sort(plan->items.begin(), plan->items.end(),
@@ -432,16 +391,15 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     // The kernel trusts these invariants; check them before anything runs.
     for (const Item &t : plan->items) {
         // the first tile of the item starts at or before the item: the block
-        // row's first tile at word 0, or the tile a cut fell in
+        // row's first tile at word 0, or the tile a cut fell in (plan_cuts
+        // finds and checks that one for an image in HBM only)
         const uint64_t br = (((uint64_t)t.row0_hi << 32) | t.row0_lo) / s->H;
         bool first_ok = br < s->nbr;
-        if (first_ok && t.begin == 0) {
+        if (first_ok && (t.begin == 0 || dev_cuts)) {
             first_ok = t.dir_begin == s->brow_dir[br];
         } else if (first_ok) {
-            const uint2 *d = dir_rows.row(br);
-            if (!d) return FMX_EHIP;
             first_ok = t.dir_begin >= s->brow_dir[br] && t.dir_begin < s->brow_dir[br + 1] &&
-                       d[t.dir_begin - s->brow_dir[br]].x <= t.begin;
+                       s->dir[t.dir_begin].x <= t.begin;
         }
         const bool ok = first_ok && t.nwords >= 1 && t.dir_begin < t.dir_end && t.dir_end <= s->ntiles &&
                         t.rot_begin >= t.begin &&
@@ -477,12 +435,34 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     plan->nslots = nslots;
     plan->nsplits = (uint32_t)splits.size();
     if (plan->nitems) {
-        FMX_HIP(ctx, hipMalloc(&plan->d_items, plan->nitems * sizeof(Item)));
-        FMX_HIP(ctx, hipMemcpy(plan->d_items, plan->items.data(), plan->nitems * sizeof(Item), hipMemcpyHostToDevice));
-    }
-    if (plan->nsplits) {
-        FMX_HIP(ctx, hipMalloc(&plan->d_splits, plan->nsplits * sizeof(Split)));
-        FMX_HIP(ctx, hipMemcpy(plan->d_splits, splits.data(), plan->nsplits * sizeof(Split), hipMemcpyHostToDevice));
+        // items and splits in one allocation and one copy, through the
+        // context's pinned buffer where they fit (a pageable copy of 64 KB
+        // takes 35 us, a pinned one 12)
+        const size_t ib = plan->nitems * sizeof(Item), all = ib + plan->nsplits * sizeof(Split);
+        FMX_HIP(ctx, hipMalloc(&plan->d_items, all));
+        plan->d_splits = (Split *)((char *)plan->d_items + ib);
+        std::vector<char> host;
+        char *src = (char *)ctx->pinned + kPinnedStage;
+        if (all > kPinnedBytes - kPinnedStage) {
+            host.resize(all);
+            src = host.data();
+        }
+        if (dev_cuts)  // plan_cuts takes a split item's block-row length from here
+            for (Item &t : plan->items)
+                if (t.slot != kNone) {
+                    const uint64_t br = (((uint64_t)t.row0_hi << 32) | t.row0_lo) / s->H;
+                    t.rot_begin = (uint32_t)((s->offs[br + 1] - s->offs[br]) / 2);
+                }
+        memcpy(src, plan->items.data(), ib);
+        if (plan->nsplits) memcpy(src + ib, splits.data(), all - ib);
+        FMX_HIP(ctx, hipMemcpyAsync(plan->d_items, src, all, hipMemcpyHostToDevice, ctx->stream));
+        const bool moved = dev_cuts && nslots;
+        fmx_status st = moved ? plan_cuts(ctx, s, plan->d_items, plan->nitems) : FMX_OK;
+        // the copy reads host memory, and the items may be used on any stream
+        FMX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (st) return st;
+        if (moved && *(volatile uint32_t *)((char *)ctx->pinned + kPinnedFlag))
+            return fail(ctx, FMX_EINVAL, "internal error: inconsistent SpMM work item");
     }
     *out = plan.get();
     s->plans[key] = std::move(plan);
@@ -849,9 +829,15 @@ fmx_status fmx_ctx_create(int device, fmx_ctx **out)
     c->num_cus = prop.multiProcessorCount;
     c->lds_per_block = prop.sharedMemPerBlock;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return FMX_EHIP;
+    if (hipHostMalloc(&c->pinned, kPinnedBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipStreamDestroy(c->stream);
+        return FMX_ENOMEM;
+    }
+    memset(c->pinned, 0, kPinnedBytes);
     // the fixed scratch of fmx_gram_noalloc, looked up with the device current
     if (noalloc_scratch_lookup(c.get()) != FMX_OK) {
         (void)hipStreamDestroy(c->stream);
+        (void)hipHostFree(c->pinned);
         return FMX_EHIP;
     }
     *out = c.release();
@@ -867,6 +853,7 @@ fmx_status fmx_ctx_destroy(fmx_ctx *ctx)
         (void)hipStreamDestroy(ctx->stream);
     }
     if (ctx->ws) (void)hipFree(ctx->ws);
+    if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     delete ctx;
     return FMX_OK;
 }

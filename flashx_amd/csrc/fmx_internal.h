@@ -62,12 +62,16 @@ struct Plan {
     uint32_t nslots = 0;
     uint32_t nsplits = 0;
     Item *d_items = nullptr;
-    Split *d_splits = nullptr;
-    std::vector<Item> items;    // host copy (tests / diagnostics)
+    Split *d_splits = nullptr;  // in d_items' allocation
+    std::vector<Item> items;    // as built on the host (plan_cuts moves split ones on the device)
     // streamed matrices: the items of chunk c are [chunk_items[c], chunk_items[c+1])
     std::vector<uint32_t> chunk_items;
     ~Plan();
 };
+
+// The context's pinned host memory: counts that a kernel writes and the host
+// reads, a kernel's error flag, and a staging area for small uploads.
+constexpr size_t kPinnedCounts = 0, kPinnedFlag = 4096, kPinnedStage = 8192, kPinnedBytes = 8192 + (256 << 10);
 
 struct Scratch {
     void *ptr = nullptr;
@@ -89,6 +93,7 @@ struct fmx_ctx {
     fmx::Scratch xhot;         // grow-only: the hot rows of X, densely (gather-order images)
     void *noalloc_ws = nullptr;  // this device's copy of the fixed scratch (fmx_gram_noalloc)
     size_t noalloc_bytes = 0;
+    void *pinned = nullptr;      // pinned host memory (kPinned*)
 };
 
 struct fmx_spm {
@@ -170,11 +175,12 @@ fmx_status gather_order_lists(fmx_ctx *ctx, const fmx_spm *src, uint64_t ncols, 
 // (image_dev.hip).
 fmx_status decode_lists(fmx_ctx *ctx, const fmx_spm *src, uint32_t *rows, uint32_t *cols, void *vals,
                         uint32_t *uses);
-// carry[i]: the row in force at word p[i] of the block row whose first word
-// is base[i] (an absolute word index into the image in HBM), kNone at a
-// header word; p[i] lies past its tile's header (image_dev.hip).
-fmx_status plan_carries(fmx_ctx *ctx, const fmx_spm *s, const std::vector<uint64_t> &base,
-                        const std::vector<uint32_t> &p, std::vector<uint32_t> &carry);
+// The split items among the n device items of an image built on the device:
+// their ranges' ends move out of tile headers (binary) or back to a tile
+// start (weighted), and dir_begin, carry and the rotation fields are filled
+// in (image_dev.hip).  Sets the flag in ctx->pinned if an item is
+// inconsistent; on ctx->stream, not synchronised.
+fmx_status plan_cuts(fmx_ctx *ctx, const fmx_spm *s, Item *items, uint32_t n);
 fmx_status finish_streamed(fmx_ctx *ctx, fmx_spm *s, uint64_t chunk_bytes, bool whole_file);
 // The chunks, staging buffers and directory of an analysed streamed image
 // (or of its re-cut work image), without a gather-order image.

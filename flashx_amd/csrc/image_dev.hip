@@ -23,10 +23,10 @@
 //                 the wanted share (or the uses reach 0) is nhot;
 //   relabel       new ids, then every column of the list.
 //
-// plan_carries: for a word position inside a block row, the row of the SCSR
-// row part in force there (the word is a column index) or none (it is a
-// header), which a work item that starts there carries in (one wave per
-// position, searching back 64 words at a time).
+// plan_cuts: the split items of a work plan, whose ranges come as fractions
+// of their block row, moved to where an item may start (one wave per item:
+// a binary search of the directory, then a search back for the row in
+// force, 64 words at a time).
 #include "devprim.h"
 
 namespace fmx {
@@ -130,37 +130,71 @@ __global__ void __launch_bounds__(kT) relabel(uint32_t *cols, uint64_t nnz, cons
         cols[e] = newid[cols[e]];
 }
 
-// carry[i] for word p[i] of the block row starting at word base[i] (p[i]
-// lies past its tile's 8-word header): kNone if the word is a header (row
-// part or COO entry), else the row of the nearest row-part header before it.
-// One wave per cut: the lanes read 64 words back at a time and a ballot
-// finds the nearest header (a hub row's part can be thousands of words long;
-// the word after the tile header always has the header bit, so the search
-// ends inside the tile).
-__global__ void __launch_bounds__(kT) carries(const uint16_t *img, const uint64_t *base, const uint32_t *p,
-                                              uint64_t n, uint32_t *carry)
+// The last tile of the block row whose entries are dir[lo, hi) that starts at
+// or before word p (the first starts at word 0).
+__device__ __forceinline__ uint32_t tile_before(const uint2 *dir, uint32_t lo, uint32_t hi, uint32_t p)
+{
+    while (hi - lo > 1) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if (dir[mid].x <= p) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Split items (slot != kNone) of a plan: item words [begin, begin + nwords)
+// of a block row of rot_begin words, dir_begin its first directory entry.
+// Both ends move the same way, so neighbouring items still meet: out of the
+// header of the tile they fall in (binary), or back to its start (weighted;
+// a range inside one tile then becomes empty and its partial zero).  The row
+// in force at a binary item's first word, kNone if that word is a header
+// (row part or COO entry), is that of the nearest header before it: the
+// lanes read 64 words back at a time and a ballot finds it (a hub row's part
+// can be thousands of words long; the word behind the tile header always has
+// the header bit, so the search ends inside the tile).
+__global__ void __launch_bounds__(kT) fix_items(const uint16_t *img, const uint2 *dir, Item *items, uint32_t n,
+                                                int weighted, uint32_t *bad)
 {
     const int lane = threadIdx.x & 63;
-    const uint64_t nw = ((uint64_t)gridDim.x * kT) >> 6;
-    for (uint64_t i = (blockIdx.x * (uint64_t)kT + threadIdx.x) >> 6; i < n; i += nw) {
-        const uint16_t *w = img + base[i];
-        const int64_t q = p[i];
-        if (w[q] & 0x8000u) {
-            if (lane == 0) carry[i] = kNone;
-            continue;
+    const uint32_t i = blockIdx.x * (kT / 64) + (threadIdx.x >> 6);
+    if (i >= n) return;
+    const Item t = items[i];
+    if (t.slot == kNone) return;
+    const uint32_t words = t.rot_begin, d0 = t.dir_begin, d1 = t.dir_end;
+    uint32_t end[2], tile = d0;
+    for (int e = 0; e < 2; e++) {
+        uint32_t p = e ? t.begin + t.nwords : t.begin;
+        if (p != 0 && p < words) {
+            const uint32_t at = tile_before(dir, d0, d1, p), x = dir[at].x;
+            p = weighted ? x : max(p, x + 8);
+            if (e == 0) tile = at;
         }
-        for (int64_t hi = q - 1;; hi -= 64) {
-            const int64_t at = hi - lane;
-            const uint32_t v = at >= 0 ? w[at] : 0x8000u;
-            const uint64_t m = __ballot((v & 0x8000u) != 0);
-            if (m) {
-                const int l0 = __ffsll((unsigned long long)m) - 1;  // nearest to q
-                const uint32_t head = __shfl(v, l0, 64);
-                if (lane == 0) carry[i] = head & 0x7FFFu;
-                break;
+        end[e] = p;
+    }
+    uint32_t carry = kNone;
+    if (!weighted && end[0] != 0) {
+        const uint16_t *w = img + t.brow_word;
+        const int64_t q = end[0];
+        if (!(w[q] & 0x8000u)) {
+            for (int64_t hi = q - 1;; hi -= 64) {
+                const int64_t at = hi - lane;
+                const uint32_t v = at >= 0 ? w[at] : 0x8000u;
+                const uint64_t m = __ballot((v & 0x8000u) != 0);
+                if (m) {
+                    const int l0 = __ffsll((unsigned long long)m) - 1;  // nearest to q
+                    carry = __shfl(v, l0, 64) & 0x7FFFu;
+                    break;
+                }
             }
         }
     }
+    if (lane) return;
+    if (end[0] > end[1] || end[1] > words || d0 >= d1 || dir[tile].x > end[0]) *bad = 1;
+    Item *o = items + i;
+    o->begin = o->rot_begin = end[0];
+    o->nwords = end[1] - end[0];
+    o->dir_begin = o->rot_dir = tile;
+    o->carry = carry;
 }
 
 uint32_t grid_for(fmx_ctx *ctx, uint64_t n)
@@ -247,26 +281,14 @@ fmx_status gather_order_lists(fmx_ctx *ctx, const fmx_spm *src, uint64_t ncols, 
     return FMX_OK;
 }
 
-fmx_status plan_carries(fmx_ctx *ctx, const fmx_spm *s, const std::vector<uint64_t> &base,
-                        const std::vector<uint32_t> &p, std::vector<uint32_t> &carry)
+fmx_status plan_cuts(fmx_ctx *ctx, const fmx_spm *s, Item *items, uint32_t n)
 {
-    const uint64_t n = p.size();
-    carry.assign(n, kNone);
-    if (!n) return FMX_OK;
     if (!s->d_image) return fail(ctx, FMX_EINVAL, "internal error: the image is not in HBM");
-    hipStream_t st = ctx->stream;
-    DevBuf<uint64_t> db;
-    DevBuf<uint32_t> dp, dc;
-    FMX_HIP(ctx, db.alloc(n));
-    FMX_HIP(ctx, dp.alloc(n));
-    FMX_HIP(ctx, dc.alloc(n));
-    FMX_HIP(ctx, hipMemcpyAsync(db.p, base.data(), n * sizeof(uint64_t), hipMemcpyHostToDevice, st));
-    FMX_HIP(ctx, hipMemcpyAsync(dp.p, p.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(carries, dim3(grid_for(ctx, n * 64)), dim3(kT), 0, st, (const uint16_t *)s->d_image, db.p, dp.p, n,
-                       dc.p);
+    uint32_t *bad = (uint32_t *)((char *)ctx->pinned + kPinnedFlag);
+    *(volatile uint32_t *)bad = 0;
+    hipLaunchKernelGGL(fix_items, dim3((n + kT / 64 - 1) / (kT / 64)), dim3(kT), 0, ctx->stream,
+                       (const uint16_t *)s->d_image, s->d_dir, items, n, s->esz ? 1 : 0, bad);
     FMX_HIP(ctx, hipGetLastError());
-    FMX_HIP(ctx, hipMemcpyAsync(carry.data(), dc.p, n * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    FMX_HIP(ctx, hipStreamSynchronize(st));
     return FMX_OK;
 }
 

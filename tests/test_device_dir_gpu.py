@@ -87,3 +87,27 @@ def test_device_directory_weighted(fmx, orc, monkeypatch, lh):
             a.multiply_async(X, ya, seq=seq)
             b.multiply_async(X, yb, seq=seq)
             assert torch.equal(ya, yb), (k, seq)
+
+
+@pytest.mark.parametrize("n,lh,weighted", [(300, 5, False), (20011, 6, True), (20011, 15, False), (1 << 15, 7, True)])
+def test_small_matrix_splits_by_its_share(fmx, n, lh, weighted):
+    """The default work cap of a small matrix (1024 words): two hub rows of
+    most columns, spread over their tiles, are cut several times, at word
+    positions that the device moves as the host does."""
+    rng = np.random.default_rng(n + lh)
+    hub = np.arange(n, dtype=np.int32)
+    src = np.concatenate([np.full(n, 7, np.int32), np.full(n, n - 2, np.int32), rng.integers(0, n, 4 * n)]).astype(np.int32)
+    dst = np.concatenate([hub, hub, rng.integers(0, n, 4 * n)]).astype(np.int32)
+    if weighted:
+        vals = rng.integers(1, 9, src.size).astype(np.float32)
+        a = fmx.SparseMatrix.build_weighted(dev(src), dev(dst), dev(vals), n=n, log2_h=lh, log2_w=10)
+    else:
+        a = fmx.SparseMatrix.build(dev(src), dev(dst), n=n, log2_h=lh, log2_w=10)
+    b, _ = host_route(fmx, a)
+    for k in (1, 8, 10):
+        X = dev(rng.integers(-9, 10, (n, k)).astype(np.float32))
+        ya, yb = a.multiply(X), b.multiply(X)
+        assert np.array_equal(ya.cpu().numpy(), yb.cpu().numpy()), k
+        if not weighted:  # row 7 meets every column but its own
+            want = X.double().sum(0) - X[7].double()
+            assert np.array_equal(ya[7].double().cpu().numpy(), want.cpu().numpy())
