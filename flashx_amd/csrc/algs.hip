@@ -4,7 +4,7 @@
 // device, FP32 as the reference computes it:
 //   out_deg = max(A * 1, 1)                       (get_out_degree, :49-60, :83)
 //   pr = 1/n                                      (mat_init_operate, :31-43)
-//   repeat: in = pr / out_deg; pr1 = in * out_deg (:101-105)
+//   repeat: in = pr / out_deg; pr1 = in * out_deg (:101-105; pr_init, pr_step)
 //           out = A^T * in                        (:110, the SpMM kernel, k = 1)
 //           pr2 = d * out + (1 - d) / n           (:118-119)
 //           converged = #{|pr1 - pr2| < 0.001/n}  (:97, :120-124); pr = pr2
@@ -12,6 +12,7 @@
 // The element-wise steps use explicitly rounded operations, so that no
 // multiply-add is contracted and each step rounds as the reference's does;
 // only the SpMV sum differs (FP64 accumulation, rounded once).
+#include <algorithm>
 #include <vector>
 
 #include "dense.h"
@@ -34,36 +35,44 @@ __global__ void __launch_bounds__(kT) pr_fill(float *x, uint64_t n, float v)
     for (uint64_t i = blockIdx.x * (uint64_t)kT + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kT) x[i] = v;
 }
 
-__global__ void __launch_bounds__(kT) pr_init(float *deg, float *pr, uint64_t n, float p0)
+__global__ void __launch_bounds__(kT) pr_init(float *deg, float *pr, float *in, uint64_t n, float p0)
 {
     for (uint64_t i = blockIdx.x * (uint64_t)kT + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kT) {
-        deg[i] = deg[i] > 1.0f ? deg[i] : 1.0f;
+        const float d = deg[i] > 1.0f ? deg[i] : 1.0f;
+        deg[i] = d;
         pr[i] = p0;
+        in[i] = __fdiv_rn(p0, d);
     }
 }
 
-__global__ void __launch_bounds__(kT) pr_prepare(const float *pr, const float *deg, float *in, float *pr1,
-                                                 uint64_t n, unsigned long long *conv)
+// One iteration's element-wise steps behind its SpMV, and the next SpMV's
+// operand: pr1 is recomputed from this iteration's operand instead of being
+// stored, so a vertex costs three loads and two stores.  Each block writes
+// its count of converged vertices to counts (host memory that the device
+// sees), which the host adds up: one atomic counter for all waves made this
+// the longest kernel of an iteration (2^20 vertices: 93 us, the atomics
+// queueing on one word; 7 us like this).
+__global__ void __launch_bounds__(kT) pr_step(const float *out, const float *deg, float *pr, float *in, uint64_t n,
+                                              float damping, float add, float eps, uint32_t *counts)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *conv = 0;  // the counter of this iteration
+    __shared__ uint32_t wave[kT / 64];
+    uint32_t c = 0;
     for (uint64_t i = blockIdx.x * (uint64_t)kT + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kT) {
-        const float v = __fdiv_rn(pr[i], deg[i]);
-        in[i] = v;
-        pr1[i] = __fmul_rn(v, deg[i]);
-    }
-}
-
-__global__ void __launch_bounds__(kT) pr_update(const float *out, const float *pr1, float *pr, uint64_t n,
-                                                float damping, float add, float eps, unsigned long long *conv)
-{
-    unsigned long long c = 0;
-    for (uint64_t i = blockIdx.x * (uint64_t)kT + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kT) {
+        const float d = deg[i];
+        const float p1 = __fmul_rn(in[i], d);
         const float p2 = __fadd_rn(__fmul_rn(out[i], damping), add);
-        c += fabsf(pr1[i] - p2) < eps ? 1ull : 0ull;
+        c += fabsf(p1 - p2) < eps ? 1u : 0u;
         pr[i] = p2;
+        in[i] = __fdiv_rn(p2, d);
     }
     for (int d = 32; d; d >>= 1) c += __shfl_xor(c, d, 64);
-    if ((threadIdx.x & 63) == 0 && c) atomicAdd(conv, c);
+    if ((threadIdx.x & 63) == 0) wave[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (int w = 0; w < kT / 64; w++) t += wave[w];
+        counts[blockIdx.x] = t;
+    }
 }
 
 // X = max(X * N, eps) / (D + eps), element-wise in FP32 with each step
@@ -96,42 +105,59 @@ fmx_status fmx_pagerank(fmx_ctx *ctx, const fmx_spm *A, const fmx_spm *At, int m
     const uint64_t n = A->nrows;
     if (iters) *iters = 0;
     if (n == 0) return FMX_OK;
+    // per-block counts of converged vertices, in the context's pinned memory
+    const uint32_t gs = (uint32_t)std::min<uint64_t>({(n + kT - 1) / kT, (uint64_t)ctx->num_cus * 2, 1024});
+    uint32_t *counts = (uint32_t *)((char *)ctx->pinned + kPinnedCounts);
     float *buf = nullptr;
-    unsigned long long *conv = nullptr;
-    FMX_HIP(ctx, hipMalloc(&buf, 4 * n * sizeof(float)));
-    if (hipMalloc(&conv, sizeof(unsigned long long)) != hipSuccess) {
+    hipEvent_t ev = nullptr;
+    FMX_HIP(ctx, hipMalloc(&buf, 3 * n * sizeof(float)));
+    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
         (void)hipFree(buf);
-        return fail(ctx, FMX_ENOMEM, "PageRank counter");
+        return fail(ctx, FMX_EHIP, "PageRank event");
     }
-    float *deg = buf, *in = buf + n, *out = buf + 2 * n, *pr1 = buf + 3 * n;
+    float *deg = buf, *in = buf + n, *out = buf + 2 * n;
     const uint32_t g = grid_for_n(ctx, n);
     fmx_status st = FMX_OK;
     // out_deg = max(A * 1, 1); the ones vector lives in `in` for this step
     hipLaunchKernelGGL(pr_fill, dim3(g), dim3(kT), 0, s, in, n, 1.0f);
     st = fmx_spmm(ctx, A, FMX_F32, 1, in, 1, deg, 1, s);
     if (!st) {
-        hipLaunchKernelGGL(pr_init, dim3(g), dim3(kT), 0, s, deg, pr, n, (float)(1.0 / (double)n));
+        hipLaunchKernelGGL(pr_init, dim3(g), dim3(kT), 0, s, deg, pr, in, n, (float)(1.0 / (double)n));
         const float eps = (float)(0.001 / (double)n);
         const float add = (float)((1.0 - (double)damping) / (double)n);
+        // The next SpMV is launched before the host waits for this step's
+        // counts, which would leave the GPU idle for 22 us an iteration; it
+        // touches only `out`, which nothing reads if this was the last step.
+        // That one SpMV is then for nothing, so it is only done where it
+        // takes less than ten such gaps (0.2 ms: about 2^25 non-zeros).
+        const bool ahead = !At->streamed() && At->nnz <= (1ull << 25);
         int it = 0;
-        unsigned long long c = 0;
-        while (c < n && it < max_iters) {
-            hipLaunchKernelGGL(pr_prepare, dim3(g), dim3(kT), 0, s, pr, deg, in, pr1, n, conv);
-            st = fmx_spmm(ctx, At, FMX_F32, 1, in, 1, out, 1, s);
+        if (max_iters) st = fmx_spmm(ctx, At, FMX_F32, 1, in, 1, out, 1, s);
+        while (!st && it < max_iters) {
+            hipLaunchKernelGGL(pr_step, dim3(gs), dim3(kT), 0, s, out, deg, pr, in, n, damping, add, eps,
+                               counts);
+            if (hipGetLastError() != hipSuccess) {
+                st = fail(ctx, FMX_EHIP, "PageRank step");
+                break;
+            }
+            if (++it == max_iters) break;  // the counts no longer matter
+            bool ok = hipEventRecord(ev, s) == hipSuccess;
+            if (ok && ahead) st = fmx_spmm(ctx, At, FMX_F32, 1, in, 1, out, 1, s);
             if (st) break;
-            hipLaunchKernelGGL(pr_update, dim3(g), dim3(kT), 0, s, out, pr1, pr, n, damping, add, eps, conv);
-            if (hipMemcpyAsync(&c, conv, sizeof(c), hipMemcpyDeviceToHost, s) != hipSuccess ||
-                hipStreamSynchronize(s) != hipSuccess) {
+            if (!ok || hipEventSynchronize(ev) != hipSuccess) {
                 st = fail(ctx, FMX_EHIP, "PageRank convergence count");
                 break;
             }
-            it++;
+            uint64_t c = 0;
+            for (uint32_t b = 0; b < gs; b++) c += ((volatile uint32_t *)counts)[b];
+            if (c >= n) break;
+            if (!ahead) st = fmx_spmm(ctx, At, FMX_F32, 1, in, 1, out, 1, s);
         }
         if (iters) *iters = it;
     }
-    (void)hipStreamSynchronize(s);
+    if (hipStreamSynchronize(s) != hipSuccess && !st) st = fail(ctx, FMX_EHIP, "PageRank");
+    (void)hipEventDestroy(ev);
     (void)hipFree(buf);
-    (void)hipFree(conv);
     return st;
 }
 

@@ -118,3 +118,24 @@ def test_nmf_directed_streamed_and_errors(fmx, orc, directed):
     with pytest.raises(fmx.FmxError) as e:
         fmx.nmf(Wm, 2, 1, At=Wm)
     assert e.value.status == fmx.EUNSUPPORTED
+
+
+@pytest.mark.parametrize("n,iters", [(2, 3), (255, 1), (257, 4), (70001, 3)])
+def test_pagerank_counts_every_block(fmx, orc, n, iters):
+    """Vertex counts around the edges of the step's blocks, few iterations:
+    the same ranks as the oracle's, and the count of converged vertices ends
+    a ring (converged in its first iteration) whatever its last block holds."""
+    import torch
+    rng = np.random.default_rng(n)
+    s, d = rng.integers(0, n, 6 * n).astype(np.int32), rng.integers(0, n, 6 * n).astype(np.int32)
+    A = fmx.SparseMatrix.build(torch.from_numpy(s).cuda(), torch.from_numpy(d).cuda(), n=n, log2_h=9, log2_w=12)
+    At = fmx.SparseMatrix.build(torch.from_numpy(d).cuda(), torch.from_numpy(s).cuda(), n=n, log2_h=9, log2_w=12)
+    oA = orc.build_2d(s.view(np.uint32), d.view(np.uint32), n=n, log2h=9, log2w=12)
+    oAt = orc.build_2d(d.view(np.uint32), s.view(np.uint32), n=n, log2h=9, log2w=12)
+    pr, it = fmx.pagerank(A, At, max_iters=iters)
+    ref, rit = orc.pagerank(oA, oAt, iters, 0.85)
+    assert it == rit
+    assert np.abs(pr.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+    ring = torch.arange(n, dtype=torch.int32, device="cuda")
+    R = fmx.SparseMatrix.build(ring, (ring + 1) % n, n=n, log2_h=9, log2_w=12)
+    assert fmx.pagerank(R, fmx.SparseMatrix.build((ring + 1) % n, ring, n=n, log2_h=9, log2_w=12), max_iters=5)[1] == 1
