@@ -73,8 +73,8 @@ __device__ __forceinline__ const T *xrow(const SpmmArgs &a, uint32_t gcol)
                          : (const T *)a.X + (uint64_t)(gcol - a.nhot) * a.ldx;
 }
 
-template <typename T, int E>
-struct alignas(sizeof(T) * E) Vec {
+template <typename T, int E, bool ALIGNED = true>
+struct alignas(ALIGNED ? sizeof(T) * E : sizeof(T)) Vec {
     T v[E];
 };
 
@@ -121,14 +121,64 @@ struct Lanes {
     static constexpr int NZP = 64 / L;                     // non-zeros per pass
 };
 
-// Band column of output column c for compile-time widths: lane q of a
-// non-zero's L lanes holds columns q*E .. q*E+E-1 and adds its i-th one at
-// band column i*L+q, so the L lanes of one add touch consecutive words.
+// Compiled row forms: K > 0 is a width of K columns, one of the powers of two
+// above; K < 0 is any width of at least -K columns, -K elements per lane
+// (Row below); K = 0 walks flat (entry, element) pairs, one element per lane
+// and step: rows wider than 64 lanes hold, and the sequential mode's runtime
+// widths.
 template <typename T, int K>
-__device__ __forceinline__ uint32_t band_col(uint32_t c)
+constexpr int row_elems()
 {
-    using C = Lanes<T, K>;
-    return (c % C::E) * C::L + c / C::E;
+    if constexpr (K > 0) return Lanes<T, K>::E;
+    else return K < 0 ? -K : 1;
+}
+
+// This lane's share of the rows in a batch: L lanes take one row, lane q of
+// them the E columns from col0 with one load, and nzp rows go side by side.
+// Element i is added at band column off[i]: the lanes of one add touch
+// consecutive words.  With a width that is no multiple of E the last lane's
+// load starts early, so that it ends with the row; the columns it shares
+// with its neighbour go to the band row's spare word, and lanes left over
+// (64 mod L) take no entries.  The loads then need only T's alignment (the
+// hardware takes 16 bytes at any dword).
+template <typename T, int K>
+struct Row {
+    static constexpr int E = row_elems<T, K>();
+    uint32_t q, g, nzp, col0, off[E];
+    bool on;
+    __device__ __forceinline__ Row(int k, int lane)
+    {
+        if constexpr (K > 0) {
+            using C = Lanes<T, K>;
+            q = lane % C::L;
+            g = lane / C::L;
+            nzp = C::NZP;
+            col0 = q * E;
+            on = true;
+#pragma unroll
+            for (int i = 0; i < E; i++) off[i] = i * C::L + q;
+        } else {
+            const uint32_t L = ((uint32_t)k + E - 1) / E;
+            nzp = 64 / L;
+            g = lane / L;
+            q = lane - g * L;
+            on = g < nzp;
+            col0 = min(q * E, (uint32_t)k - E);
+            const uint32_t skip = q * E - col0;
+#pragma unroll
+            for (uint32_t i = 0; i < (uint32_t)E; i++) off[i] = i < skip ? E * L : (i - skip) * L + q;
+        }
+    }
+};
+
+// Band column of output column c in the order of Row::off.
+template <typename T, int K>
+__device__ __forceinline__ uint32_t band_col(uint32_t c, uint32_t k)
+{
+    if constexpr (K == 0) return c;
+    constexpr uint32_t E = row_elems<T, K>();
+    const uint32_t L = K > 0 ? (uint32_t)(K > 0 ? K : 1) / E : (k + E - 1) / E;
+    return (c % E) * L + c / E;
 }
 
 // Queue entry e lives at slot e + e/P: the P-entry segments of the lane
@@ -319,22 +369,31 @@ __device__ __forceinline__ uint32_t window_advance(const uint2 *dreg, const bool
 }
 
 // ---------------------------------------------------------------------------
-// Drains (compile-time width K): gathers of P consecutive entries per lane
-// group, summed in registers per row run, added to the band at row changes.
-template <typename T, int K, int P, typename A, bool HOT>
-__device__ __forceinline__ void gather_batch(const SpmmArgs &a, const uint32_t *qcol, const uint16_t *qrow,
-                                             uint32_t base, uint32_t qn, int lane, Vec<T, Lanes<T, K>::E> *v,
-                                             uint32_t *rr)
+// Drains (K != 0): gathers of P consecutive entries per lane group, summed in
+// registers per row run, added to the band at row changes.
+template <typename T, int K>
+__device__ __forceinline__ void load_row(Vec<T, row_elems<T, K>()> &v, const T *p)
 {
-    using C = Lanes<T, K>;
-    const int q = lane % C::L;
-    const int g = lane / C::L;
+    if constexpr (K > 0) {
+        v = *(const Vec<T, row_elems<T, K>()> *)p;
+    } else {
+        const Vec<T, row_elems<T, K>(), false> u = *(const Vec<T, row_elems<T, K>(), false> *)p;
+#pragma unroll
+        for (int i = 0; i < row_elems<T, K>(); i++) v.v[i] = u.v[i];
+    }
+}
+
+template <typename T, int K, int P, bool HOT>
+__device__ __forceinline__ void gather_batch(const SpmmArgs &a, const Row<T, K> &row, const uint32_t *qcol,
+                                             const uint16_t *qrow, uint32_t base, uint32_t qn,
+                                             Vec<T, row_elems<T, K>()> *v, uint32_t *rr)
+{
     uint32_t gcs[P];
 #pragma unroll
     for (int pp = 0; pp < P; pp++) {
-        const uint32_t e = base + g * P + pp;
-        const uint32_t sl = qslot<P>(e);
-        const bool ok = e < qn;
+        const uint32_t e = base + row.g * P + pp;
+        const bool ok = row.on && e < qn;
+        const uint32_t sl = qslot<P>(K > 0 || ok ? e : 0u);
         const uint32_t qr = qrow[sl];
         gcs[pp] = ok ? qcol[sl] : 0u;
         rr[pp] = (ok && qr != 0xFFFFu) ? qr : 0xFFFFFFFFu;
@@ -342,16 +401,15 @@ __device__ __forceinline__ void gather_batch(const SpmmArgs &a, const uint32_t *
     // every queue read before the first gather, every gather before the first use
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int pp = 0; pp < P; pp++) v[pp] = *(const Vec<T, C::E> *)(xrow<T, HOT>(a, gcs[pp]) + q * C::E);
+    for (int pp = 0; pp < P; pp++) load_row<T, K>(v[pp], xrow<T, HOT>(a, gcs[pp]) + row.col0);
     __builtin_amdgcn_sched_barrier(0);
 }
 
 template <typename T, int K, int P, typename A>
-__device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, int lane, const Vec<T, Lanes<T, K>::E> *v,
-                                                 const uint32_t *rr)
+__device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, const Row<T, K> &row,
+                                                 const Vec<T, row_elems<T, K>()> *v, const uint32_t *rr)
 {
-    using C = Lanes<T, K>;
-    const int q = lane % C::L;
+    constexpr int E = row_elems<T, K>();
     if constexpr (sizeof(T) == 8) {
         // 8-byte data: each entry adds straight into the band.  Run sums
         // save few LDS adds (rows average 2.4 entries per tile on R-MAT)
@@ -360,37 +418,37 @@ __device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, int lane, 
 #pragma unroll
         for (int pp = 0; pp < P; pp++) {
             if (rr[pp] != 0xFFFFFFFFu) {
-                A *dst = band + rr[pp] * S + q;
+                A *dst = band + rr[pp] * S;
 #pragma unroll
-                for (int i = 0; i < C::E; i++) lds_add(dst + i * C::L, (A)v[pp].v[i]);
+                for (int i = 0; i < E; i++) lds_add(dst + row.off[i], (A)v[pp].v[i]);
             }
         }
         return;
     }
-    A acc[C::E];
+    A acc[E];
     uint32_t cur = rr[0];
 #pragma unroll
-    for (int i = 0; i < C::E; i++) acc[i] = (A)v[0].v[i];
+    for (int i = 0; i < E; i++) acc[i] = (A)v[0].v[i];
 #pragma unroll
     for (int pp = 1; pp < P; pp++) {
         if (rr[pp] != cur) {
             if (cur != 0xFFFFFFFFu) {
-                A *dst = band + cur * S + q;
+                A *dst = band + cur * S;
 #pragma unroll
-                for (int i = 0; i < C::E; i++) lds_add(dst + i * C::L, acc[i]);
+                for (int i = 0; i < E; i++) lds_add(dst + row.off[i], acc[i]);
             }
             cur = rr[pp];
 #pragma unroll
-            for (int i = 0; i < C::E; i++) acc[i] = (A)v[pp].v[i];
+            for (int i = 0; i < E; i++) acc[i] = (A)v[pp].v[i];
         } else {
 #pragma unroll
-            for (int i = 0; i < C::E; i++) acc[i] += (A)v[pp].v[i];
+            for (int i = 0; i < E; i++) acc[i] += (A)v[pp].v[i];
         }
     }
     if (cur != 0xFFFFFFFFu) {
-        A *dst = band + cur * S + q;
+        A *dst = band + cur * S;
 #pragma unroll
-        for (int i = 0; i < C::E; i++) lds_add(dst + i * C::L, acc[i]);
+        for (int i = 0; i < E; i++) lds_add(dst + row.off[i], acc[i]);
     }
 }
 
@@ -556,11 +614,8 @@ __device__ __forceinline__ void write_band(const SpmmArgs &a, const A *band, uin
                                            uint32_t rows, uint32_t slot, int lane, const RowScale &rs,
                                            double *scratch)
 {
-    const uint32_t k = K ? K : (uint32_t)a.k;
-    auto bcol = [&](uint32_t cc) -> uint32_t {
-        if constexpr (K > 0) return band_col<T, (K ? K : 1)>(cc);
-        else return cc;
-    };
+    const uint32_t k = K > 0 ? K : (uint32_t)a.k;
+    auto bcol = [&](uint32_t cc) -> uint32_t { return band_col<T, K>(cc, k); };
     if (slot == kNone) {
         T *dst = (T *)a.Y + row0 * (uint64_t)a.ldy;
         bool staged = false;
@@ -689,6 +744,7 @@ spmm_lane(SpmmArgs a)
 
     ItemState st = item_state(a, a.items[item_id]);
     const RowScale rs = prefetch_rscale<T>(a, st.row0, st.ic.rows, lane);
+    const Row<T, K> row(a.k, lane);
     const uint32_t S = a.band_stride;
     for (uint32_t i = lane; i < st.ic.rows * S; i += 64) band[i] = A(0);
     if (lane == 0) win[DWIN] = make_uint2(0xFFFFFFFFu, 0u);
@@ -719,22 +775,21 @@ spmm_lane(SpmmArgs a)
         };
         if constexpr (K == 0) fetch_next();
         wave_sync();
-        if constexpr (K > 0) {
+        if constexpr (K != 0) {
             // requested behind the first batch's gathers: a wait for the
             // gathers need not wait for these, and their latency overlaps
             // the gathers' instead of preceding them
-            using C = Lanes<T, K>;
             bool fetched = false;
-            for (uint32_t base = 0; base < qn; base += C::NZP * P) {
-                Vec<T, C::E> v[P];
+            for (uint32_t base = 0; base < qn; base += row.nzp * P) {
+                Vec<T, row_elems<T, K>()> v[P];
                 uint32_t rr[P];
-                gather_batch<T, K, P, A, HOT>(a, qcol, qrow, base, qn, lane, v, rr);
+                gather_batch<T, K, P, HOT>(a, row, qcol, qrow, base, qn, v, rr);
                 if (!fetched) {
                     fetch_next();
                     fetched = true;
                 }
                 if constexpr (SEQ) accumulate_batch_seq<T, K, P>(band, S, lane, v, rr);
-                else accumulate_batch<T, K, P, A>(band, S, lane, v, rr);
+                else accumulate_batch<T, K, P, A>(band, S, row, v, rr);
             }
             if (!fetched) fetch_next();
         } else if (qn) {
@@ -924,6 +979,7 @@ spmm_lane_w(SpmmArgs a)
 
     ItemState st = item_state(a, a.items[item_id]);
     const RowScale rs = prefetch_rscale<T>(a, st.row0, st.ic.rows, lane);
+    const Row<T, K> row(a.k, lane);
     const uint32_t S = a.band_stride;
     for (uint32_t i = lane; i < st.ic.rows * S; i += 64) band[i] = A(0);
     if (lane == 0) {
@@ -981,22 +1037,20 @@ spmm_lane_w(SpmmArgs a)
             }
         };
         if constexpr (K == 0) fetch_next();
-        if constexpr (K > 0) {
+        if constexpr (K != 0) {
             // requested behind the first batch's gathers and value loads (as
             // in spmm_lane)
-            using C = Lanes<T, K>;
-            const int q = lane % C::L;
-            const int g = lane / C::L;
+            constexpr int E = row_elems<T, K>();
             bool fetched = false;
-            for (uint32_t base = 0; base < qn; base += C::NZP * P) {
-                Vec<T, C::E> v[P];
+            for (uint32_t base = 0; base < qn; base += row.nzp * P) {
+                Vec<T, E> v[P];
                 uint32_t rr[P], gcs[P];
                 V vals[P];
 #pragma unroll
                 for (int pp = 0; pp < P; pp++) {
-                    const uint32_t e = base + g * P + pp;
-                    const uint32_t sl = qslot<P>(e);
-                    const bool ok = e < qn;
+                    const uint32_t e = base + row.g * P + pp;
+                    const bool ok = row.on && e < qn;
+                    const uint32_t sl = qslot<P>(K > 0 || ok ? e : 0u);
                     const uint32_t qr = qrow[sl];
                     gcs[pp] = ok ? qcol[sl] : 0u;
                     rr[pp] = (ok && qr != 0xFFFFu) ? qr : 0xFFFFFFFFu;
@@ -1005,7 +1059,7 @@ spmm_lane_w(SpmmArgs a)
                 }
 #pragma unroll
                 for (int pp = 0; pp < P; pp++)
-                    v[pp] = *(const Vec<T, C::E> *)(xrow<T, HOT>(a, gcs[pp]) + q * C::E);
+                    load_row<T, K>(v[pp], xrow<T, HOT>(a, gcs[pp]) + row.col0);
                 if (!fetched) {
                     fetch_next();
                     fetched = true;
@@ -1016,34 +1070,34 @@ spmm_lane_w(SpmmArgs a)
 #pragma unroll
                     for (int pp = 0; pp < P; pp++)
 #pragma unroll
-                        for (int i = 0; i < C::E; i++) v[pp].v[i] = v[pp].v[i] * (T)vals[pp];
+                        for (int i = 0; i < E; i++) v[pp].v[i] = v[pp].v[i] * (T)vals[pp];
                     accumulate_batch_seq<T, K, P>(band, S, lane, v, rr);
                     continue;
                 }
-                A acc[C::E];
+                A acc[E];
                 uint32_t cur = 0xFFFFFFFFu;
 #pragma unroll
-                for (int i = 0; i < C::E; i++) acc[i] = A(0);
+                for (int i = 0; i < E; i++) acc[i] = A(0);
 #pragma unroll
                 for (int pp = 0; pp < P; pp++) {
                     if (rr[pp] != cur) {
                         if (cur != 0xFFFFFFFFu) {
-                            A *dst = band + cur * S + q;
+                            A *dst = band + cur * S;
 #pragma unroll
-                            for (int i = 0; i < C::E; i++) lds_add(dst + i * C::L, acc[i]);
+                            for (int i = 0; i < E; i++) lds_add(dst + row.off[i], acc[i]);
                         }
                         cur = rr[pp];
 #pragma unroll
-                        for (int i = 0; i < C::E; i++) acc[i] = (A)v[pp].v[i] * (A)vals[pp];
+                        for (int i = 0; i < E; i++) acc[i] = (A)v[pp].v[i] * (A)vals[pp];
                     } else {
 #pragma unroll
-                        for (int i = 0; i < C::E; i++) acc[i] += (A)v[pp].v[i] * (A)vals[pp];
+                        for (int i = 0; i < E; i++) acc[i] += (A)v[pp].v[i] * (A)vals[pp];
                     }
                 }
                 if (cur != 0xFFFFFFFFu) {
-                    A *dst = band + cur * S + q;
+                    A *dst = band + cur * S;
 #pragma unroll
-                    for (int i = 0; i < C::E; i++) lds_add(dst + i * C::L, acc[i]);
+                    for (int i = 0; i < E; i++) lds_add(dst + row.off[i], acc[i]);
                 }
             }
             if (!fetched) fetch_next();
@@ -1108,7 +1162,7 @@ __global__ void __launch_bounds__(256) spmm_reduce(const Split *splits, const A 
 template <typename T, int K>
 constexpr int passes_for()
 {
-    if constexpr (K == 0) return 8;
+    if constexpr (K <= 0) return 8;
     else return 512 / Lanes<T, K>::NZP < 8 ? 512 / Lanes<T, K>::NZP : 8;
 }
 
@@ -1172,21 +1226,54 @@ fmx_status launch_k(fmx_ctx *ctx, SpmmArgs a, int vprim, hipStream_t stream)
     return launch_items<spmm_lane<T, K, kLaneR, P, SEQ, HOT>>(ctx, a, stream);
 }
 
+// Elements per lane of the runtime-width form for rows of k elements (0: the
+// flat form).  Four 4-byte or two 8-byte elements make 16-byte loads; three
+// 4-byte columns take two lanes of two.
+template <typename T>
+int runtime_elems(int k)
+{
+    const int e = sizeof(T) == 8 || k < 4 ? 2 : 4;
+    return k >= e && k <= 64 * e ? e : 0;
+}
+
+// Rows of a width without a form of its own, or not aligned for it.  The flat
+// form spends a division, a 4- or 8-byte load and an LDS add on each element,
+// this one a third of a load and an add per row run: 700,001 vertices x 10
+// FP32 columns 140 -> 115 us with the restaging of X, four NMF sweeps of rank
+// 20 over 260,000 vertices 2.63 -> 2.08 ms.
+template <typename T, bool SEQ, bool HOT>
+fmx_status launch_runtime(fmx_ctx *ctx, SpmmArgs a, int vprim, hipStream_t stream)
+{
+    if constexpr (!SEQ) {
+        const int e = runtime_elems<T>(a.k);
+        if (e) {
+            // a band row holds whole lanes and a spare word
+            a.band_stride = (uint32_t)((a.k + e - 1) / e * e + 1);
+            a.band_bytes = (uint32_t)(((uint64_t)a.hs * a.band_stride * sizeof(typename AccOf<T>::type) + 15) & ~15ull);
+        }
+        if constexpr (sizeof(T) == 4)
+            if (e == 4) return launch_k<T, -4, SEQ, HOT>(ctx, a, vprim, stream);
+        if (e == 2) return launch_k<T, -2, SEQ, HOT>(ctx, a, vprim, stream);
+    }
+    return launch_k<T, 0, SEQ, HOT>(ctx, a, vprim, stream);
+}
+
 // HOT (a gather-order image, rows narrower than a 128-byte line) has kernels
-// for the widths it is used with; other widths take the runtime-width form.
+// for the widths it is used with; k = 0 asks for the runtime-width form.
 template <typename T, bool SEQ, bool HOT>
 fmx_status launch_w(fmx_ctx *ctx, SpmmArgs a, int k, int vprim, hipStream_t stream)
 {
     constexpr int KMAX = HOT ? (int)(64 / sizeof(T)) : 64;
+    if (k > KMAX) k = 0;
     switch (k) {
     case 1: return launch_k<T, 1, SEQ, HOT>(ctx, a, vprim, stream);
     case 2: return launch_k<T, 2, SEQ, HOT>(ctx, a, vprim, stream);
     case 4: return launch_k<T, 4, SEQ, HOT>(ctx, a, vprim, stream);
     case 8: return launch_k<T, 8, SEQ, HOT>(ctx, a, vprim, stream);
-    case 16: return launch_k<T, (16 <= KMAX ? 16 : 0), SEQ, HOT>(ctx, a, vprim, stream);
-    case 32: return launch_k<T, (32 <= KMAX ? 32 : 0), SEQ, HOT>(ctx, a, vprim, stream);
-    case 64: return launch_k<T, (64 <= KMAX ? 64 : 0), SEQ, HOT>(ctx, a, vprim, stream);
-    default: return launch_k<T, 0, SEQ, HOT>(ctx, a, vprim, stream);
+    case 16: return launch_k<T, (16 <= KMAX ? 16 : 8), SEQ, HOT>(ctx, a, vprim, stream);
+    case 32: return launch_k<T, (32 <= KMAX ? 32 : 8), SEQ, HOT>(ctx, a, vprim, stream);
+    case 64: return launch_k<T, (64 <= KMAX ? 64 : 8), SEQ, HOT>(ctx, a, vprim, stream);
+    default: return launch_runtime<T, SEQ, HOT>(ctx, a, vprim, stream);
     }
 }
 

@@ -273,3 +273,33 @@ def test_config2_rmat22_spmm_parity(fmx, orc, lh):
     Yd = torch.empty_like(Xdt)
     spm.multiply_async(Xdt, Yd, seq=True)
     assert np.array_equal(Yd.cpu().numpy(), refd)
+
+
+@pytest.mark.parametrize("k,pad", [(2, 1), (3, 0), (5, 2), (6, 0), (7, 0), (9, 1), (10, 0), (16, 3), (20, 0), (33, 0),
+                                   (63, 0), (65, 0), (129, 0), (257, 0)])
+def test_runtime_widths(fmx, orc, k, pad):
+    """Widths without a compiled form, and aligned widths with odd strides: the
+    runtime-width form (one 16-byte load per lane, the last lane's starting
+    early) and, past 64 lanes, the flat one; binary and weighted.  Small whole
+    numbers, so every type must be exact; X ends with its last row."""
+    import torch
+    s, d = orc.rmat_edges(11, 16 << 11, seed=k)
+    n = (1 << 11) - 7
+    ok = (s < n) & (d < n)
+    s, d = s[ok], d[ok]
+    rng = np.random.default_rng(k)
+    img = orc.build_2d(s, d, n=n, log2h=6, log2w=10)
+    a = fmx.SparseMatrix.upload(img.data, img.offs)
+    for dt in (np.int32, np.int64, np.float32, np.float64):
+        vals = rng.integers(1, 5, s.size).astype(dt)
+        wimg = orc.build_2d_w(s, d, vals, n=n, log2h=6, log2w=10)
+        w = fmx.SparseMatrix.upload(wimg.data, wimg.offs)
+        X = rng.integers(-9, 10, (n, k)).astype(dt)
+        buf = torch.zeros(n * (k + pad) - pad, dtype=torch.from_numpy(X).dtype, device="cuda")
+        Xt = buf.as_strided((n, k), (k + pad, 1))
+        Xt.copy_(torch.from_numpy(X))
+        for spm, im in ((a, img), (w, wimg)):
+            Y = torch.full((n, k + pad), 77, dtype=Xt.dtype, device="cuda")
+            spm.multiply_async(Xt, Y[:, :k])
+            assert np.array_equal(Y[:, :k].cpu().numpy(), orc.spmm(im, X)), dt
+            assert bool((Y[:, k:] == 77).all())
