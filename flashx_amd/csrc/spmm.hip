@@ -7,20 +7,19 @@
 // Execution model (one wave = one work item, no cross-wave sharing):
 //   * an item is a contiguous word range of one block row (tile headers and
 //     all) plus a band of <= Hs output rows kept in LDS;
-//   * the range is decoded 64*R words at a time (a "chunk", 16-byte aligned):
-//     lane l owns R consecutive words, finds the tile holding its first word
-//     by a binary search of an LDS window of the tile directory, and
-//     classifies its words (tile header / row head / column) with per-lane
-//     state.  The row in effect at a lane's first word is the last row head
-//     of the nearest lane below it (ballot + shuffle), and a wave prefix sum
-//     of per-lane column counts writes the (global column, band row) entries
-//     in stream order to an LDS queue;
+//   * the range is decoded 512 words at a time (a "chunk", 16-byte aligned),
+//     lane l owning 8 consecutive words.  A header is 8 words and a tile at
+//     least 11, so a lane's entries belong to one tile, the last one that
+//     starts at or before its first word, and two 8-bit masks (row heads and
+//     entries) describe its words.  The row in effect at a lane's first word
+//     and its first queue position are wave scans (DPP), and the (global
+//     column, band row) entries go to an LDS queue in stream order;
 //   * the queue is drained with vector gathers of X rows (16 bytes per lane,
-//     L lanes per non-zero).  Lane group g takes P consecutive entries, so a
+//     L lanes per non-zero).  Lane group g takes 8 consecutive entries, so a
 //     run of one row (a row part of a tile) is summed in registers and reaches
 //     the band with one LDS add per element at each row change;
-//   * the next chunk's words are requested before the drain; a wave's own
-//     decode and gathers alternate, and the other resident waves (up to four
+//   * the next chunk's words are requested behind the first gathers; a wave's
+//     own decode and gathers alternate, and the other resident waves (five
 //     per SIMD, as LDS allows) keep gathers in flight meanwhile;
 //   * the band is written to Y once (rows without non-zeros are 0), or to a
 //     partial slot when a power-law band was split over several items; split
@@ -61,16 +60,34 @@ struct SpmmArgs {
     int ycol;              // Y column-major: element (r, j) at Y[j * ldy + r]
     const void *Xhot;      // gather-order images: rows of columns < nhot (leading dimension k)
     uint64_t nhot;         // columns c >= nhot are row c - nhot of X
+    const void *Xcold;     // narrow forms: X - nhot rows, so that row c of it is column c >= nhot
+    uint32_t xstride;      // narrow forms: bytes from row to row of X (and Xhot)
 };
 
-// Row gcol of the gathered operand: with HOT (a gather-order image) the
-// dense hot block for the first nhot columns and X for the others, else X.
-template <typename T, bool HOT>
-__device__ __forceinline__ const T *xrow(const SpmmArgs &a, uint32_t gcol)
+// Narrow: the columns fit 24 bits, the operand 32-bit byte offsets and the
+// band 8-bit row numbers (narrow_ok).  A queue entry is then one word, and a
+// row's address one 24-bit multiply-add onto a scalar base, instead of a
+// 64-bit product per gather.
+constexpr int kRowShift = 24;
+
+// Where element colb / sizeof(T) of row gcol of the gathered operand lies:
+// with HOT (a gather-order image) in the dense hot block for the first nhot
+// columns and in X for the others, else in X.
+template <typename T, bool HOT, bool NARROW>
+__device__ __forceinline__ const T *xrow(const SpmmArgs &a, uint32_t gcol, uint32_t colb)
 {
-    if constexpr (!HOT) return (const T *)a.X + (uint64_t)gcol * a.ldx;
-    return gcol < a.nhot ? (const T *)a.Xhot + (uint64_t)gcol * (uint32_t)a.k
-                         : (const T *)a.X + (uint64_t)(gcol - a.nhot) * a.ldx;
+    if constexpr (NARROW) {
+        const uint32_t off = __umul24(gcol, a.xstride) + colb;
+        if constexpr (!HOT) return (const T *)((const char *)a.X + off);
+        const char *base = gcol < (uint32_t)a.nhot ? (const char *)a.Xhot : (const char *)a.Xcold;
+        return (const T *)(base + off);
+    } else {
+        const T *p;
+        if constexpr (!HOT) p = (const T *)a.X + (uint64_t)gcol * a.ldx;
+        else p = gcol < a.nhot ? (const T *)a.Xhot + (uint64_t)gcol * (uint32_t)a.k
+                               : (const T *)a.X + (uint64_t)(gcol - a.nhot) * a.ldx;
+        return (const T *)((const char *)p + colb);
+    }
 }
 
 template <typename T, int E, bool ALIGNED = true>
@@ -79,8 +96,6 @@ struct alignas(ALIGNED ? sizeof(T) * E : sizeof(T)) Vec {
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint64_t mask_lt(int lane) { return (1ull << lane) - 1ull; }
 
 __device__ __forceinline__ uint32_t rdlane(uint32_t v, int l)
 {
@@ -105,6 +120,26 @@ __device__ __forceinline__ void wave_sync()
 {
     __builtin_amdgcn_wave_barrier();
     asm volatile("" ::: "memory");
+}
+
+// Inclusive scans over the wave's lanes on DPP moves (no LDS trip): within
+// rows of 16 lanes, then row 15's total into the next row and lane 31's into
+// the upper half.  Lanes without a source keep the identity.
+template <typename OP>
+__device__ __forceinline__ int wave_scan(int v, int identity, OP op)
+{
+    v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+    v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+    v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x114, 0xf, 0xf, false));  // row_shr:4
+    v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x118, 0xf, 0xf, false));  // row_shr:8
+    v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return v;
+}
+__device__ __forceinline__ int wave_sum(int v) { return wave_scan(v, 0, [](int a, int b) { return a + b; }); }
+__device__ __forceinline__ int wave_max(int v, int least)
+{
+    return wave_scan(v, least, [](int a, int b) { return a > b ? a : b; });
 }
 
 // LDS accumulator type: FP32 data accumulate in FP64 (ds_add_f64 is fast on
@@ -134,39 +169,39 @@ constexpr int row_elems()
 }
 
 // This lane's share of the rows in a batch: L lanes take one row, lane q of
-// them the E columns from col0 with one load, and nzp rows go side by side.
-// Element i is added at band column off[i]: the lanes of one add touch
+// them the E columns from byte colb with one load, and nzp rows go side by
+// side.  Element i is added at band column off[i]: the lanes of one add touch
 // consecutive words.  With a width that is no multiple of E the last lane's
-// load starts early, so that it ends with the row; the columns it shares
-// with its neighbour go to the band row's spare word, and lanes left over
-// (64 mod L) take no entries.  The loads then need only T's alignment (the
-// hardware takes 16 bytes at any dword).
+// load starts early, so that it ends with the row; the columns it shares with
+// its neighbour go to the band row's spare word, and so does everything of
+// the lanes left over (64 mod L, and beyond 32 rows), which repeat lane 0's
+// load.  The loads then need only T's alignment (the hardware takes 16 bytes
+// at any dword).
 template <typename T, int K>
 struct Row {
     static constexpr int E = row_elems<T, K>();
-    uint32_t q, g, nzp, col0, off[E];
-    bool on;
+    uint32_t g, nzp, colb, off[E];
     __device__ __forceinline__ Row(int k, int lane)
     {
         if constexpr (K > 0) {
             using C = Lanes<T, K>;
-            q = lane % C::L;
+            const uint32_t q = lane % C::L;
             g = lane / C::L;
             nzp = C::NZP;
-            col0 = q * E;
-            on = true;
+            colb = q * E * sizeof(T);
 #pragma unroll
             for (int i = 0; i < E; i++) off[i] = i * C::L + q;
-        } else {
+        } else if constexpr (K < 0) {
             const uint32_t L = ((uint32_t)k + E - 1) / E;
-            nzp = 64 / L;
+            nzp = min(64 / L, 32u);
             g = lane / L;
-            q = lane - g * L;
-            on = g < nzp;
-            col0 = min(q * E, (uint32_t)k - E);
-            const uint32_t skip = q * E - col0;
+            const uint32_t q = lane - g * L;
+            const uint32_t col0 = min(q * E, (uint32_t)k - E), skip = q * E - col0;
+            const bool on = g < nzp;
 #pragma unroll
-            for (uint32_t i = 0; i < (uint32_t)E; i++) off[i] = i < skip ? E * L : (i - skip) * L + q;
+            for (uint32_t i = 0; i < (uint32_t)E; i++) off[i] = !on || i < skip ? E * L : (i - skip) * L + q;
+            if (!on) g = 0;
+            colb = on ? col0 * sizeof(T) : 0;
         }
     }
 };
@@ -181,134 +216,182 @@ __device__ __forceinline__ uint32_t band_col(uint32_t c, uint32_t k)
     return (c % E) * L + c / E;
 }
 
-// Queue entry e lives at slot e + e/P: the P-entry segments of the lane
-// groups then start in different LDS banks.
-template <int P>
-__device__ __forceinline__ uint32_t qslot(uint32_t e) { return e + e / P; }
+constexpr int kP = 8;        // consecutive queue entries of a lane group per batch
+constexpr int kChunk = 512;  // words per chunk: 8 per lane
+constexpr int kWin = 64;     // directory window: a chunk meets at most (512 - 1) / 11 + 1 tile starts
+constexpr uint32_t kNoWord = 0x7FFFFFFFu;  // past every word of a block row
+
+// Queue entry e lives at slot e + e/8: the 8-entry segments of the lane
+// groups then start in different LDS banks.  The flat form (K = 0) reads in
+// order.  Whole batches are drained, so the slots past the last entry are
+// filled up: batches of at most 32 rows side by side (K < 0) end at entry 672
+// at the latest.
+template <int K>
+__device__ __forceinline__ uint32_t qslot(uint32_t e) { return K ? e + e / kP : e; }
+template <int K>
+constexpr int queue_slots() { return K > 0 ? kChunk + kChunk / kP + 1 : K < 0 ? 672 + 672 / kP + 1 : kChunk + 1; }
+
+// A wave's LDS: the band, the queue's columns, values and rows, the window,
+// the lanes' tile flags and the window's value words.
+struct Layout {
+    uint32_t val, row, win, flag, wval, bytes;
+};
+template <int K, bool WEIGHTED, bool NARROW>
+__host__ __device__ __forceinline__ Layout lds_layout(uint32_t band_bytes)
+{
+    constexpr uint32_t QS = queue_slots<K>();
+    Layout l;
+    l.val = band_bytes + QS * 4;
+    l.row = l.val + (WEIGHTED ? QS * 4 : 0);
+    l.win = (l.row + (NARROW ? 0 : QS * 2) + 7) & ~7u;
+    l.flag = l.win + (kWin + 1) * 8;
+    l.wval = l.flag + 64 * 4;
+    l.bytes = (l.wval + (WEIGHTED ? kWin * 4 : 0) + 15) & ~15u;
+    return l;
+}
+
+// Entry slots: the column, and the band row (`dump`, the row past the band,
+// for an entry outside it, whose column is 0 then).
+template <bool NARROW>
+struct Queue {
+    uint32_t *col;
+    uint16_t *row;
+    __device__ __forceinline__ void put(uint32_t sl, uint32_t c, uint32_t r) const
+    {
+        if constexpr (NARROW) {
+            col[sl] = r << kRowShift | c;
+        } else {
+            col[sl] = c;
+            row[sl] = (uint16_t)r;
+        }
+    }
+    __device__ __forceinline__ void get(uint32_t sl, uint32_t &c, uint32_t &r) const
+    {
+        c = col[sl];
+        if constexpr (NARROW) {
+            r = c >> kRowShift;
+            c &= (1u << kRowShift) - 1;
+        } else {
+            r = row[sl];
+        }
+    }
+};
 
 // ---------------------------------------------------------------------------
-// Lane-sequential decode
-template <int R>
-struct LaneCfg {
-    static constexpr int CW = 64 * R;                                // words per chunk
-    static constexpr int NB = 1 + (R + 10) / 11;                     // tiles a lane can touch
-    static constexpr int DWIN = ((CW - 1) / 11 + 2 + 63) / 64 * 64;  // window entries
-    static constexpr int DPL = DWIN / 64;
-};
-// A stored tile is >= 11 words (16-byte header, one entry, end marker; a
-// 16-byte stub only for an empty block row, which is an item by itself), so
-// a chunk meets at most (CW-1)/11+1 tile starts after the tile holding its
-// first word, and R words at most NB-1.
+// Decode.  A stored tile is >= 11 words (16-byte header, one entry, end
+// marker; a 16-byte stub only for an empty block row, which is an item by
+// itself).
 
 struct ItemCtx {
     uint64_t bw;          // absolute word index of the block row
     int32_t begin, pend;  // item words [begin, pend), relative to the block row
-    uint32_t sb_base, rows;
+    uint32_t sb_base, rows, dump;
     int log2w;
-    uint64_t ncols;
+    uint32_t last_col;
 };
 
+// One directory entry of the window per lane, and (weighted) its values word.
+struct Window {
+    uint2 e;
+    uint32_t v;
+    bool live;  // inside the block row
+};
+
+__device__ __forceinline__ int32_t clamp8(int32_t x) { return x < 0 ? 0 : x > 8 ? 8 : x; }
+
 // Decodes the chunk starting at absolute word c (8-word aligned) from this
-// lane's R words in wreg and the directory window win (DWIN entries and a
-// sentinel).  Writes the chunk's entries in stream order at queue slots
-// qslot<SEGP>(e) -- band row 0xFFFF for an entry outside the band -- and
+// lane's 8 words in wreg and the directory window, whose entry 0 holds the
+// chunk's first item word.  Writes the chunk's entries in stream order and
 // returns their number; carry becomes the row in effect after the chunk.
-template <int R, int SEGP>
+// Weighted images (W): a tile's values follow its COO region, one per
+// non-zero in stream order (SCSR values, then COO values,
+// sparse_matrix_format.h:233-241).  Words at or past the values region are
+// not entries, and the value of an entry is as many values behind the
+// region's start as entries of its tile come before it: those decoded in the
+// chunk before the tile's first lane do not count, and c0 of window tile 0's
+// came in earlier chunks.  Work items start at tile starts (rotation and
+// splits), so no value position is carried into an item.  tiles: how many
+// tiles of the window have lanes in this chunk; qt: the entry that the value
+// positions of lane 63's tile count from.
+template <int K, bool W, bool NARROW>
 __device__ __forceinline__ uint32_t decode_chunk(const ItemCtx &ic, uint64_t c, const uint32_t *wreg,
-                                                 const uint2 *win, int &carry, uint32_t *qcol, uint16_t *qrow,
-                                                 int lane)
+                                                 const Window &w, uint2 *win, uint32_t *flag, uint32_t *wval, int c0,
+                                                 int vwords, int &carry, const Queue<NARROW> &q, uint32_t *qval,
+                                                 int lane, int &tiles, int &qt)
 {
-    using LC = LaneCfg<R>;
-    constexpr int NB = LC::NB, DWIN = LC::DWIN;
-    const int32_t p0 = (int32_t)((int64_t)c - (int64_t)ic.bw) + lane * R;
-    const int32_t q = p0 > ic.begin ? p0 : ic.begin;
-    // last window tile starting at or before q (window entry 0 holds the
-    // chunk's first item word, sentinels compare greater)
-    uint32_t j = 0;
-#pragma unroll
-    for (int st = DWIN / 2; st >= 1; st >>= 1)
-        if (win[j + st].x <= (uint32_t)q) j += st;
-    uint32_t ts0[NB], tb0[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        const uint32_t jj = j + b < DWIN ? j + b : DWIN;
-        const uint2 e = win[jj];
-        ts0[b] = e.x;
-        tb0[b] = e.y;
+    const int32_t cb = (int32_t)((int64_t)c - (int64_t)ic.bw);
+    const int32_t p0 = cb + lane * 8;
+    // Window tile t rules the lanes from the first one whose words start at
+    // or behind it (tile 0: from lane 0); no two tiles begin with one lane.
+    // Lanes leave their tile's mark there, valid in this chunk only.
+    win[lane] = w.live ? w.e : make_uint2(kNoWord, 0u);
+    if constexpr (W) wval[lane] = w.v;
+    const int32_t f = lane == 0 ? 0 : ((int32_t)w.e.x - cb + 7) >> 3;
+    if (w.live && f < 64) flag[f] = (uint32_t)cb;
+    wave_sync();
+    const bool begins = flag[lane] == (uint32_t)cb;
+    const uint64_t bm = __ballot(begins);
+    const uint32_t j = __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u)) +
+                       (begins ? 0u : ~0u);
+    const uint2 t = win[j];
+    int32_t stop = (int32_t)win[j + 1].x;
+    stop = stop < ic.pend ? stop : ic.pend;
+    uint32_t tv = 0;
+    if constexpr (W) {
+        tv = wval[j];
+        stop = stop < (int32_t)tv ? stop : (int32_t)tv;
     }
-    // pass 1: column count and last row head of this lane
-    int cnt = 0, lrow = 0;
-    bool hh = false;
-    {
-        uint32_t ts[NB];
-#pragma unroll
-        for (int b = 0; b < NB; b++) ts[b] = ts0[b];
-#pragma unroll
-        for (int i = 0; i < R; i++) {
-            const int32_t pos = p0 + i;
-            const uint32_t w = (wreg[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu;
-            const bool valid = pos >= ic.begin && pos < ic.pend;
-            if (NB > 1 && valid && (uint32_t)pos >= ts[NB > 1 ? 1 : 0]) {
-#pragma unroll
-                for (int b = 0; b + 1 < NB; b++) ts[b] = ts[b + 1];
-                ts[NB - 1] = 0xFFFFFFFFu;
-            }
-            const bool body = valid && ((uint32_t)pos - ts[0]) >= 8u;
-            if (body && (w & 0x8000u)) {
-                lrow = (int)(w & 0x7FFFu);
-                hh = true;
-            }
-            cnt += (body && !(w & 0x8000u)) ? 1 : 0;
-        }
-    }
-    // row in effect at this lane's first word; row after the chunk
-    const uint64_t hm = __ballot(hh);
-    const uint64_t below = hm & mask_lt(lane);
-    const int src = below ? 63 - __clzll(below) : 0;
-    const int prow = __shfl(lrow, src);
-    const int row_in = below ? prow : carry;
-    if (hm) carry = (int)rdlane((uint32_t)lrow, 63 - __clzll(hm));
-    int incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int t = __shfl_up(incl, d);
-        if (lane >= d) incl += t;
-    }
+    // this lane's item words behind the tile's header and before its end
+    const int32_t from = (int32_t)t.x + 8 > ic.begin ? (int32_t)t.x + 8 : ic.begin;
+    const int32_t lo = clamp8(from - p0), hi = clamp8(stop - p0);
+    const uint32_t body = hi > lo ? ((1u << (hi - lo)) - 1u) << lo : 0u;
+    // bit i: word i has the head bit (the top bytes of four words side by
+    // side, their top bits weighted 1, 2, 4, 8 by a dot product)
+    const uint32_t y0 = __builtin_amdgcn_perm(wreg[1], wreg[0], 0x07050301u);
+    const uint32_t y1 = __builtin_amdgcn_perm(wreg[3], wreg[2], 0x07050301u);
+    const uint32_t hb = __builtin_amdgcn_udot4((y1 >> 7) & 0x01010101u, 0x80402010u,
+                                               __builtin_amdgcn_udot4((y0 >> 7) & 0x01010101u, 0x08040201u, 0u, false),
+                                               false);
+    const uint32_t heads = body & hb, ents = body & ~hb;
+    // the last head's row, scanned together with its lane: the nearest lane
+    // below with a head gives the row in effect at this lane's first word
+    const int last = 31 - __clz((int)heads);
+    const uint32_t w01 = last & 2 ? wreg[1] : wreg[0], w23 = last & 2 ? wreg[3] : wreg[2];
+    const uint32_t lw = (last & 4 ? w23 : w01) >> ((last & 1) * 16);
+    const int key = wave_max(heads ? (lane << 16) | (int)(lw & 0x7FFFu) : -1, -1);
+    const int below = __builtin_amdgcn_update_dpp(-1, key, 0x138, 0xf, 0xf, false);  // wave_shr:1
+    int r = below >= 0 ? below & 0x7FFF : carry;
+    const int top = (int)rdlane((uint32_t)key, 63);
+    if (top >= 0) carry = top & 0x7FFF;
+    const int cnt = __popc(ents);
+    const int incl = wave_sum(cnt);
     const uint32_t qn = rdlane((uint32_t)incl, 63);
-    // pass 2: entries in stream order
-    {
-        uint32_t ts[NB], tb[NB];
+    uint32_t o = (uint32_t)(incl - cnt);
+    uint32_t vw = 0;
+    if constexpr (W) {
+        // (the counts never fall, so the latest tile start has the largest)
+        int q0 = wave_max(begins ? incl - cnt : 0, 0);
+        q0 = j == 0 ? -c0 : q0;
+        vw = tv + (uint32_t)((int)o - q0) * (uint32_t)vwords;
+        tiles = __popcll(bm);
+        qt = (int)rdlane((uint32_t)q0, 63);
+    }
+    const uint32_t colbase = t.y << ic.log2w;
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            ts[b] = ts0[b];
-            tb[b] = tb0[b];
-        }
-        int r = row_in;
-        uint32_t o = (uint32_t)(incl - cnt);
-#pragma unroll
-        for (int i = 0; i < R; i++) {
-            const int32_t pos = p0 + i;
-            const uint32_t w = (wreg[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu;
-            const bool valid = pos >= ic.begin && pos < ic.pend;
-            if (NB > 1 && valid && (uint32_t)pos >= ts[NB > 1 ? 1 : 0]) {
-#pragma unroll
-                for (int b = 0; b + 1 < NB; b++) {
-                    ts[b] = ts[b + 1];
-                    tb[b] = tb[b + 1];
-                }
-                ts[NB - 1] = 0xFFFFFFFFu;
+    for (int i = 0; i < 8; i++) {
+        const uint32_t word = (wreg[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu;
+        if (heads & (1u << i)) r = (int)(word & 0x7FFFu);
+        if (ents & (1u << i)) {
+            const uint32_t br = (uint32_t)r - ic.sb_base;  // no row in effect: r = -1, past any band
+            const bool keep = br < ic.rows;
+            const uint32_t gcol = min(colbase | word, ic.last_col);
+            const uint32_t sl = qslot<K>(o);
+            q.put(sl, keep ? gcol : 0u, keep ? br : ic.dump);
+            if constexpr (W) {
+                qval[sl] = vw;
+                vw += (uint32_t)vwords;
             }
-            const bool body = valid && ((uint32_t)pos - ts[0]) >= 8u;
-            if (body && (w & 0x8000u)) r = (int)(w & 0x7FFFu);
-            if (body && !(w & 0x8000u)) {
-                const uint32_t br = (uint32_t)(r - (int)ic.sb_base);
-                const uint32_t gcol = (tb[0] << ic.log2w) | w;
-                const bool keep = r >= 0 && br < ic.rows && gcol < ic.ncols;
-                const uint32_t sl = qslot<SEGP>(o);
-                qcol[sl] = keep ? gcol : 0u;
-                qrow[sl] = keep ? (uint16_t)br : (uint16_t)0xFFFFu;
-                o++;
-            }
+            o++;
         }
     }
     return qn;
@@ -318,57 +401,28 @@ __device__ __forceinline__ uint32_t decode_chunk(const ItemCtx &ic, uint64_t c, 
 // the item's last word lastw (always inside the image allocation, whose size
 // is a multiple of 4096 bytes).  The image is streamed once: non-temporal
 // loads, so it does not displace X in L2.
-template <int R>
-__device__ __forceinline__ void load_words(const uint16_t *img, uint64_t c, uint64_t lastw, int lane,
-                                           uint32_t *wreg)
+__device__ __forceinline__ void load_words(const uint16_t *img, uint64_t c, uint64_t lastw, int lane, uint32_t *wreg)
 {
-    static_assert(R % 8 == 0, "lane word count");
     const uint64_t last8 = lastw & ~7ull;
-#pragma unroll
-    for (int h = 0; h < R / 8; h++) {
-        uint64_t g = c + (uint64_t)lane * R + h * 8;
-        g = g < last8 ? g : last8;
-        const u32x4 v = __builtin_nontemporal_load((const u32x4 *)(img + g));
-        wreg[h * 4 + 0] = v.x;
-        wreg[h * 4 + 1] = v.y;
-        wreg[h * 4 + 2] = v.z;
-        wreg[h * 4 + 3] = v.w;
-    }
+    uint64_t g = c + (uint64_t)lane * 8;
+    g = g < last8 ? g : last8;
+    const u32x4 v = __builtin_nontemporal_load((const u32x4 *)(img + g));
+    wreg[0] = v.x;
+    wreg[1] = v.y;
+    wreg[2] = v.z;
+    wreg[3] = v.w;
 }
 
-// Directory entries ct + h*64 + lane (clamped); `live` marks those inside the
-// block row, the others become sentinels when the window is stored.
-template <int DPL>
-__device__ __forceinline__ void load_window(const uint2 *dir, uint32_t ct, uint32_t dlast, int lane, uint2 *dreg,
-                                            bool *live)
+// Directory entry ct + lane (clamped); `live` marks one inside the block row.
+template <bool W>
+__device__ __forceinline__ void load_window(const SpmmArgs &a, uint32_t ct, uint32_t dlast, int lane, Window &w)
 {
-#pragma unroll
-    for (int h = 0; h < DPL; h++) {
-        const uint32_t t = ct + h * 64 + lane;
-        live[h] = t <= dlast;
-        dreg[h] = dir[t < dlast ? t : dlast];
-    }
+    const uint32_t t = ct + lane;
+    w.live = t <= dlast;
+    w.e = a.dir[t < dlast ? t : dlast];
+    if constexpr (W) w.v = a.vdir[t < dlast ? t : dlast];
 }
 
-template <int DPL>
-__device__ __forceinline__ void store_window(uint2 *win, const uint2 *dreg, const bool *live, int lane)
-{
-#pragma unroll
-    for (int h = 0; h < DPL; h++) win[h * 64 + lane] = live[h] ? dreg[h] : make_uint2(0xFFFFFFFFu, 0u);
-}
-
-// Start of the next chunk's window: entries of this window starting at or
-// before its first word (the window is sorted, sentinels compare greater).
-template <int DPL>
-__device__ __forceinline__ uint32_t window_advance(const uint2 *dreg, const bool *live, uint32_t pn)
-{
-    int n = 0;
-#pragma unroll
-    for (int h = 0; h < DPL; h++) n += __popcll(__ballot(live[h] && dreg[h].x <= pn));
-    return (uint32_t)n;
-}
-
-// ---------------------------------------------------------------------------
 // Drains (K != 0): gathers of P consecutive entries per lane group, summed in
 // registers per row run, added to the band at row changes.
 template <typename T, int K>
@@ -383,70 +437,68 @@ __device__ __forceinline__ void load_row(Vec<T, row_elems<T, K>()> &v, const T *
     }
 }
 
-template <typename T, int K, int P, bool HOT>
-__device__ __forceinline__ void gather_batch(const SpmmArgs &a, const Row<T, K> &row, const uint32_t *qcol,
-                                             const uint16_t *qrow, uint32_t base, uint32_t qn,
-                                             Vec<T, row_elems<T, K>()> *v, uint32_t *rr)
+// The batch of entries from `base` (a multiple of 8): lane group g's are
+// g * 8 .. g * 8 + 7 of it.
+template <typename T, int K, bool HOT, bool NARROW>
+__device__ __forceinline__ void gather_batch(const SpmmArgs &a, const Row<T, K> &row, const Queue<NARROW> &q,
+                                             uint32_t base, Vec<T, row_elems<T, K>()> *v, uint32_t *rr)
 {
-    uint32_t gcs[P];
+    uint32_t gcs[kP];
+    const uint32_t s0 = qslot<K>(base) + row.g * (kP + 1);
 #pragma unroll
-    for (int pp = 0; pp < P; pp++) {
-        const uint32_t e = base + row.g * P + pp;
-        const bool ok = row.on && e < qn;
-        const uint32_t sl = qslot<P>(K > 0 || ok ? e : 0u);
-        const uint32_t qr = qrow[sl];
-        gcs[pp] = ok ? qcol[sl] : 0u;
-        rr[pp] = (ok && qr != 0xFFFFu) ? qr : 0xFFFFFFFFu;
-    }
+    for (int pp = 0; pp < kP; pp++) q.get(s0 + pp, gcs[pp], rr[pp]);
     // every queue read before the first gather, every gather before the first use
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int pp = 0; pp < P; pp++) load_row<T, K>(v[pp], xrow<T, HOT>(a, gcs[pp]) + row.col0);
+    for (int pp = 0; pp < kP; pp++) load_row<T, K>(v[pp], xrow<T, HOT, NARROW>(a, gcs[pp], row.colb));
     __builtin_amdgcn_sched_barrier(0);
 }
 
-template <typename T, int K, int P, typename A>
-__device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, const Row<T, K> &row,
-                                                 const Vec<T, row_elems<T, K>()> *v, const uint32_t *rr)
+// Fills the slots from entry qn up to entry `end` with row-less entries.
+template <int K, bool NARROW>
+__device__ __forceinline__ void fill_queue(const Queue<NARROW> &q, uint32_t *qval, uint32_t qn, uint32_t end,
+                                           uint32_t dump, int lane)
+{
+    for (uint32_t e = qn + lane; e < end; e += 64) {
+        q.put(qslot<K>(e), 0u, dump);
+        if (qval) qval[qslot<K>(e)] = 0u;  // a safe address
+    }
+    wave_sync();
+}
+
+// Adds a batch to the band, run by run; scale(pp, i, x) is entry pp's element
+// i in the accumulator's type (times its value).
+template <typename T, int K, typename A, bool RUNS, typename F>
+__device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, const Row<T, K> &row, const uint32_t *rr, F elem)
 {
     constexpr int E = row_elems<T, K>();
-    if constexpr (sizeof(T) == 8) {
-        // 8-byte data: each entry adds straight into the band.  Run sums
-        // save few LDS adds (rows average 2.4 entries per tile on R-MAT)
-        // and their divergent branches cost more than that for E <= 2
-        // (FP64 k = 16: 1.17 ms against 1.34 ms with run sums)
+    if constexpr (!RUNS) {
 #pragma unroll
-        for (int pp = 0; pp < P; pp++) {
-            if (rr[pp] != 0xFFFFFFFFu) {
-                A *dst = band + rr[pp] * S;
+        for (int pp = 0; pp < kP; pp++) {
+            A *dst = band + __umul24(rr[pp], S);
 #pragma unroll
-                for (int i = 0; i < E; i++) lds_add(dst + row.off[i], (A)v[pp].v[i]);
-            }
+            for (int i = 0; i < E; i++) lds_add(dst + row.off[i], elem(pp, i));
         }
-        return;
-    }
-    A acc[E];
-    uint32_t cur = rr[0];
+    } else {
+        A acc[E];
+        uint32_t cur = rr[0];
 #pragma unroll
-    for (int i = 0; i < E; i++) acc[i] = (A)v[0].v[i];
+        for (int i = 0; i < E; i++) acc[i] = elem(0, i);
 #pragma unroll
-    for (int pp = 1; pp < P; pp++) {
-        if (rr[pp] != cur) {
-            if (cur != 0xFFFFFFFFu) {
-                A *dst = band + cur * S;
+        for (int pp = 1; pp < kP; pp++) {
+            if (rr[pp] != cur) {
+                A *dst = band + __umul24(cur, S);
 #pragma unroll
                 for (int i = 0; i < E; i++) lds_add(dst + row.off[i], acc[i]);
+                cur = rr[pp];
+#pragma unroll
+                for (int i = 0; i < E; i++) acc[i] = elem(pp, i);
+            } else {
+#pragma unroll
+                for (int i = 0; i < E; i++) acc[i] += elem(pp, i);
             }
-            cur = rr[pp];
-#pragma unroll
-            for (int i = 0; i < E; i++) acc[i] = (A)v[pp].v[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < E; i++) acc[i] += (A)v[pp].v[i];
         }
-    }
-    if (cur != 0xFFFFFFFFu) {
-        A *dst = band + cur * S;
+        A *dst = band + __umul24(cur, S);
 #pragma unroll
         for (int i = 0; i < E; i++) lds_add(dst + row.off[i], acc[i]);
     }
@@ -464,7 +516,7 @@ __device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, const Row<
 // (one wave's LDS accesses execute in program order).  A run of one row
 // inside a group is chained in registers, which is the same sequence of
 // roundings.
-template <typename T, int K, int P>
+template <typename T, int K>
 __device__ __forceinline__ void accumulate_batch_seq(T *band, uint32_t S, int lane, const Vec<T, Lanes<T, K>::E> *v,
                                                      const uint32_t *rr)
 {
@@ -475,70 +527,27 @@ __device__ __forceinline__ void accumulate_batch_seq(T *band, uint32_t S, int la
     for (int gg = 0; gg < C::NZP; gg++) {
         if (g == gg) {
             T acc[C::E];
-            uint32_t cur = 0xFFFFFFFFu;
+            uint32_t cur = rr[0];
+            T *at = band + cur * S + q;
 #pragma unroll
-            for (int i = 0; i < C::E; i++) acc[i] = T(0);
+            for (int i = 0; i < C::E; i++) acc[i] = at[i * C::L];
 #pragma unroll
-            for (int pp = 0; pp < P; pp++) {
+            for (int pp = 0; pp < kP; pp++) {
                 if (rr[pp] != cur) {
-                    if (cur != 0xFFFFFFFFu) {
-                        T *dst = band + cur * S + q;
 #pragma unroll
-                        for (int i = 0; i < C::E; i++) dst[i * C::L] = acc[i];
-                    }
+                    for (int i = 0; i < C::E; i++) at[i * C::L] = acc[i];
                     cur = rr[pp];
-                    if (cur != 0xFFFFFFFFu) {
-                        const T *src = band + cur * S + q;
+                    at = band + cur * S + q;
 #pragma unroll
-                        for (int i = 0; i < C::E; i++) acc[i] = src[i * C::L];
-                    }
+                    for (int i = 0; i < C::E; i++) acc[i] = at[i * C::L];
                 }
-                if (cur != 0xFFFFFFFFu) {
 #pragma unroll
-                    for (int i = 0; i < C::E; i++) acc[i] = acc[i] + v[pp].v[i];
-                }
+                for (int i = 0; i < C::E; i++) acc[i] = acc[i] + v[pp].v[i];
             }
-            if (cur != 0xFFFFFFFFu) {
-                T *dst = band + cur * S + q;
 #pragma unroll
-                for (int i = 0; i < C::E; i++) dst[i * C::L] = acc[i];
-            }
+            for (int i = 0; i < C::E; i++) at[i * C::L] = acc[i];
         }
         wave_sync();
-    }
-}
-
-// Sequential mode at runtime widths: lane j owns output column j (of each
-// 64-column slice) and adds the queue's entries in order.  Weighted images
-// (W) multiply each gathered element by the entry's value of type V first,
-// rounded in T, as `src_row[j] * data` is.
-template <typename T, typename V, int P, bool W>
-__device__ __forceinline__ void drain_generic_seq(const SpmmArgs &a, T *band, uint32_t S, const uint32_t *qcol,
-                                                  const uint16_t *qrow, const uint32_t *qval, const uint16_t *vimg,
-                                                  uint32_t qn, int lane);
-
-// Runtime width: flat (entry, element) pairs, one element per lane.
-template <typename T, int P, typename A, bool HOT>
-__device__ __forceinline__ void drain_generic(const SpmmArgs &a, A *band, uint32_t S, const uint32_t *qcol,
-                                              const uint16_t *qrow, uint32_t qn, int lane)
-{
-    const uint32_t k = (uint32_t)a.k;
-    const uint32_t tot = qn * k;
-    for (uint32_t base = 0; base < tot; base += 64 * P) {
-        T v[P];
-        uint32_t dst[P];
-#pragma unroll
-        for (int pp = 0; pp < P; pp++) {
-            const uint32_t f = base + pp * 64 + lane;
-            const uint32_t fc = f < tot ? f : tot - 1;
-            const uint32_t e = fc / k, j = fc - e * k;
-            const uint32_t qr = qrow[e];
-            v[pp] = xrow<T, HOT>(a, qcol[e])[j];
-            dst[pp] = (f < tot && qr != 0xFFFFu) ? qr * S + j : 0xFFFFFFFFu;
-        }
-#pragma unroll
-        for (int pp = 0; pp < P; pp++)
-            if (dst[pp] != 0xFFFFFFFFu) lds_add(band + dst[pp], (A)v[pp]);
     }
 }
 
@@ -557,30 +566,62 @@ __device__ __forceinline__ T load_value(const uint16_t *p)
     }
 }
 
-template <typename T, typename V, int P, bool W>
-__device__ __forceinline__ void drain_generic_seq(const SpmmArgs &a, T *band, uint32_t S, const uint32_t *qcol,
-                                                  const uint16_t *qrow, const uint32_t *qval, const uint16_t *vimg,
-                                                  uint32_t qn, int lane)
+// Runtime width: flat (entry, element) pairs, one element per lane; weighted
+// images (V) multiply it by the entry's value.
+template <typename T, typename V, typename A, bool HOT, bool NARROW>
+__device__ __forceinline__ void drain_generic(const SpmmArgs &a, A *band, uint32_t S, const Queue<NARROW> &q,
+                                              const uint32_t *qval, const uint16_t *vimg, uint32_t qn, int lane)
+{
+    const uint32_t k = (uint32_t)a.k;
+    const uint32_t tot = qn * k;
+    for (uint32_t base = 0; base < tot; base += 64 * kP) {
+        A v[kP];
+        uint32_t dst[kP];
+#pragma unroll
+        for (int pp = 0; pp < kP; pp++) {
+            const uint32_t f = base + pp * 64 + lane;
+            const uint32_t fc = f < tot ? f : tot - 1;
+            const uint32_t e = fc / k, j = fc - e * k;
+            uint32_t gc, qr;
+            q.get(e, gc, qr);
+            v[pp] = (A)*xrow<T, HOT, NARROW>(a, gc, j * sizeof(T));
+            if constexpr (!std::is_void<V>::value) v[pp] *= (A)load_value<V>(vimg + qval[e]);
+            dst[pp] = f < tot ? qr * S + j : 0xFFFFFFFFu;
+        }
+#pragma unroll
+        for (int pp = 0; pp < kP; pp++)
+            if (dst[pp] != 0xFFFFFFFFu) lds_add(band + dst[pp], v[pp]);
+    }
+}
+
+// Sequential mode at runtime widths: lane j owns output column j (of each
+// 64-column slice) and adds the queue's entries in order.  Weighted images
+// multiply each gathered element by the entry's value of type V first,
+// rounded in T, as `src_row[j] * data` is.
+template <typename T, typename V, bool NARROW>
+__device__ __forceinline__ void drain_generic_seq(const SpmmArgs &a, T *band, uint32_t S, const Queue<NARROW> &q,
+                                                  const uint32_t *qval, const uint16_t *vimg, uint32_t qn, int lane)
 {
 #pragma clang fp contract(off)
     const uint32_t k = (uint32_t)a.k;
     for (uint32_t j0 = 0; j0 < k; j0 += 64) {
         const uint32_t j = j0 + (uint32_t)lane;
         const bool act = j < k;
-        for (uint32_t e0 = 0; e0 < qn; e0 += P) {
-            T v[P];
-            uint32_t dst[P];
+        for (uint32_t e0 = 0; e0 < qn; e0 += kP) {
+            T v[kP];
+            uint32_t dst[kP];
 #pragma unroll
-            for (int pp = 0; pp < P; pp++) {
+            for (int pp = 0; pp < kP; pp++) {
                 const uint32_t e = e0 + pp;
                 const uint32_t ec = e < qn ? e : qn - 1;
-                const uint32_t qr = qrow[ec];
-                v[pp] = xrow<T, false>(a, qcol[ec])[act ? j : 0u];
-                if constexpr (W) v[pp] = v[pp] * (T)load_value<V>(vimg + qval[ec]);
-                dst[pp] = (e < qn && act && qr != 0xFFFFu) ? qr * S + j : 0xFFFFFFFFu;
+                uint32_t gc, qr;
+                q.get(ec, gc, qr);
+                v[pp] = *xrow<T, false, NARROW>(a, gc, (act ? j : 0u) * sizeof(T));
+                if constexpr (!std::is_void<V>::value) v[pp] = v[pp] * (T)load_value<V>(vimg + qval[ec]);
+                dst[pp] = (e < qn && act) ? qr * S + j : 0xFFFFFFFFu;
             }
 #pragma unroll
-            for (int pp = 0; pp < P; pp++)
+            for (int pp = 0; pp < kP; pp++)
                 if (dst[pp] != 0xFFFFFFFFu) band[dst[pp]] = band[dst[pp]] + v[pp];
         }
     }
@@ -696,8 +737,9 @@ __device__ __forceinline__ ItemState item_state(const SpmmArgs &a, const Item &i
     s.ic.pend = (int32_t)(it.begin + it.nwords);  // nwords >= 1
     s.ic.sb_base = it.sb_base;
     s.ic.rows = it.rows;
+    s.ic.dump = a.hs;
     s.ic.log2w = a.log2w;
-    s.ic.ncols = a.ncols;
+    s.ic.last_col = (uint32_t)(a.ncols - 1);
     s.dlast = it.dir_end - 1;
     s.row0 = ((uint64_t)it.row0_hi << 32) | it.row0_lo;
     s.slot = it.slot;
@@ -713,22 +755,19 @@ __device__ __forceinline__ ItemState item_state(const SpmmArgs &a, const Item &i
 }
 
 // ---------------------------------------------------------------------------
-// The SpMM kernel: chunks of 64*R words, each decoded and then drained
-// batch by batch.  The next chunk's words and window are requested behind
-// the first batch's gathers, so their latency overlaps the gathers'; the
-// gathers of one wave are not overlapped with its own decode, other resident
-// waves fill that gap (four per SIMD where LDS allows).
+// The SpMM kernel: chunks of 512 words, each decoded and then drained batch
+// by batch.  The next chunk's words and window are requested behind the
+// first batch's gathers, so their latency overlaps the gathers'; the gathers
+// of one wave are not overlapped with its own decode, other resident waves
+// fill that gap.
+// V: the type of a weighted image's values, void for a binary one.
 // SEQ: the sequential mode (accumulate_batch_seq): the band holds T and
 // every element is summed in the reference's order; the plan of such a call
 // neither splits nor rotates items.
-template <typename T, int K, int R, int P, bool SEQ, bool HOT>
-__global__ void __launch_bounds__(64 * kWPB) __attribute__((amdgpu_waves_per_eu(5, 5)))
-spmm_lane(SpmmArgs a)
+template <typename T, typename V, int K, bool SEQ, bool HOT, bool NARROW>
+__device__ __forceinline__ void spmm_body(const SpmmArgs &a)
 {
-    using LC = LaneCfg<R>;
-    constexpr int CW = LC::CW, DWIN = LC::DWIN, DPL = LC::DPL;
-    constexpr int SEGP = K ? P : (1 << 30);
-    constexpr int QS = CW + CW / (K ? P : CW) + 1;
+    constexpr bool W = !std::is_void<V>::value;
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63;
     const uint32_t wv = uni(threadIdx.x >> 6);
@@ -737,399 +776,123 @@ spmm_lane(SpmmArgs a)
 
     unsigned char *wbase = smem + wv * a.wave_bytes;
     using A = typename std::conditional<SEQ, T, typename AccOf<T>::type>::type;
+    const Layout l = lds_layout<K, W, NARROW>(a.band_bytes);
     A *band = (A *)wbase;
-    uint32_t *qcol = (uint32_t *)(wbase + a.band_bytes);
-    uint16_t *qrow = (uint16_t *)(qcol + QS);
-    uint2 *win = (uint2 *)(wbase + ((a.band_bytes + QS * 6 + 7) & ~7u));
+    const Queue<NARROW> q{(uint32_t *)(wbase + a.band_bytes), (uint16_t *)(wbase + l.row)};
+    uint32_t *qval = W ? (uint32_t *)(wbase + l.val) : nullptr;
+    uint2 *win = (uint2 *)(wbase + l.win);
+    uint32_t *flag = (uint32_t *)(wbase + l.flag);
+    uint32_t *wval = W ? (uint32_t *)(wbase + l.wval) : nullptr;
 
     ItemState st = item_state(a, a.items[item_id]);
     const RowScale rs = prefetch_rscale<T>(a, st.row0, st.ic.rows, lane);
     const Row<T, K> row(a.k, lane);
     const uint32_t S = a.band_stride;
     for (uint32_t i = lane; i < st.ic.rows * S; i += 64) band[i] = A(0);
-    if (lane == 0) win[DWIN] = make_uint2(0xFFFFFFFFu, 0u);
-
-    for (int seg = 0; seg < 2; seg++) {
-    if (!select_segment(st, seg)) break;
-    const uint64_t abs_end = st.ic.bw + (uint64_t)st.ic.pend;
-    const uint64_t lastw = abs_end - 1;
-    uint64_t c = (st.ic.bw + (uint64_t)st.ic.begin) & ~7ull;
-    uint32_t wreg[R / 2];
-    uint2 dreg[DPL];
-    bool live[DPL];
-    load_words<R>(a.img, c, lastw, lane, wreg);
-    load_window<DPL>(a.dir, st.ct, st.dlast, lane, dreg, live);
-
-    while (c < abs_end) {
-        store_window<DPL>(win, dreg, live, lane);
-        wave_sync();
-        const uint32_t qn = decode_chunk<R, SEGP>(st.ic, c, wreg, win, st.carry, qcol, qrow, lane);
-        const uint64_t cn = c + CW;
-        // the next chunk's words and window (this chunk's are in LDS now)
-        auto fetch_next = [&]() {
-            if (cn < abs_end) {
-                st.ct += window_advance<DPL>(dreg, live, (uint32_t)((int64_t)cn - (int64_t)st.ic.bw)) - 1;
-                load_words<R>(a.img, cn, lastw, lane, wreg);
-                load_window<DPL>(a.dir, st.ct, st.dlast, lane, dreg, live);
-            }
-        };
-        if constexpr (K == 0) fetch_next();
-        wave_sync();
-        if constexpr (K != 0) {
-            // requested behind the first batch's gathers: a wait for the
-            // gathers need not wait for these, and their latency overlaps
-            // the gathers' instead of preceding them
-            bool fetched = false;
-            for (uint32_t base = 0; base < qn; base += row.nzp * P) {
-                Vec<T, row_elems<T, K>()> v[P];
-                uint32_t rr[P];
-                gather_batch<T, K, P, HOT>(a, row, qcol, qrow, base, qn, v, rr);
-                if (!fetched) {
-                    fetch_next();
-                    fetched = true;
-                }
-                if constexpr (SEQ) accumulate_batch_seq<T, K, P>(band, S, lane, v, rr);
-                else accumulate_batch<T, K, P, A>(band, S, row, v, rr);
-            }
-            if (!fetched) fetch_next();
-        } else if (qn) {
-            if constexpr (SEQ) drain_generic_seq<T, T, P, false>(a, band, S, qcol, qrow, nullptr, nullptr, qn, lane);
-            else drain_generic<T, P, A, HOT>(a, band, S, qcol, qrow, qn, lane);
-        }
-        wave_sync();
-        c = cn;
-    }
-    }
-    write_band<T, K, A>(a, band, S, st.row0, st.ic.rows, st.slot, lane, rs, (double *)qcol);
-}
-
-
-// ---------------------------------------------------------------------------
-// Weighted images (entry_size 4 or 8): each tile's values follow its COO
-// region, one per non-zero in stream order (SCSR values, then COO values,
-// sparse_matrix_format.h:233-241).  The decode is decode_chunk's plus two
-// facts per entry: words at or past the tile's values region are not
-// entries, and the entry's value is the tile's (o - wq[j])-th, where o is
-// the entry's index in the chunk and wq[j] the chunk index at which window
-// tile j starts (minus the columns of tile 0 seen in earlier chunks, for
-// j = 0).  Work items start at tile starts (rotation and splits), so no
-// value position is carried into an item.
-template <int R, int SEGP>
-__device__ __forceinline__ uint32_t decode_chunk_w(const ItemCtx &ic, uint64_t c, const uint32_t *wreg,
-                                                   const uint2 *win, const uint32_t *wvb, int32_t *wq, int c0,
-                                                   int vwords, int &carry, uint32_t *qcol, uint16_t *qrow,
-                                                   uint32_t *qval, int lane)
-{
-    using LC = LaneCfg<R>;
-    constexpr int NB = LC::NB, DWIN = LC::DWIN;
-    const int32_t p0 = (int32_t)((int64_t)c - (int64_t)ic.bw) + lane * R;
-    const int32_t q = p0 > ic.begin ? p0 : ic.begin;
-    uint32_t j = 0;
-#pragma unroll
-    for (int st = DWIN / 2; st >= 1; st >>= 1)
-        if (win[j + st].x <= (uint32_t)q) j += st;
-    uint32_t ts0[NB], tb0[NB], tv0[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        const uint32_t jj = j + b < DWIN ? j + b : DWIN;
-        const uint2 e = win[jj];
-        ts0[b] = e.x;
-        tb0[b] = e.y;
-        tv0[b] = wvb[jj];
-    }
-    // pass 1: counts, last row head, and the column count at each tile
-    // start inside this lane's words (a tile starting exactly at the lane's
-    // first item word counts too, unless it is window tile 0)
-    int cnt = 0, lrow = 0;
-    bool hh = false;
-    int nx = 0;
-    int xcnt[NB];
-    uint32_t xj[NB];
-    {
-        uint32_t ts[NB], tv[NB];
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            ts[b] = ts0[b];
-            tv[b] = tv0[b];
-            xcnt[b] = 0;
-            xj[b] = 0;
-        }
-        if (j > 0 && ts0[0] == (uint32_t)q && q < ic.pend) {
-            xcnt[0] = 0;
-            xj[0] = j;
-            nx = 1;
-        }
-        uint32_t jc = j;
-#pragma unroll
-        for (int i = 0; i < R; i++) {
-            const int32_t pos = p0 + i;
-            const uint32_t w = (wreg[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu;
-            const bool valid = pos >= ic.begin && pos < ic.pend;
-            if (NB > 1 && valid && (uint32_t)pos >= ts[NB > 1 ? 1 : 0]) {
-#pragma unroll
-                for (int b = 0; b + 1 < NB; b++) {
-                    ts[b] = ts[b + 1];
-                    tv[b] = tv[b + 1];
-                }
-                ts[NB - 1] = 0xFFFFFFFFu;
-                tv[NB - 1] = 0xFFFFFFFFu;
-                jc++;
-                if (nx < NB) {
-                    xcnt[nx] = cnt;
-                    xj[nx] = jc;
-                    nx++;
-                }
-            }
-            const bool body = valid && ((uint32_t)pos - ts[0]) >= 8u && (uint32_t)pos < tv[0];
-            if (body && (w & 0x8000u)) {
-                lrow = (int)(w & 0x7FFFu);
-                hh = true;
-            }
-            cnt += (body && !(w & 0x8000u)) ? 1 : 0;
-        }
-    }
-    const uint64_t hm = __ballot(hh);
-    const uint64_t below = hm & mask_lt(lane);
-    const int src = below ? 63 - __clzll(below) : 0;
-    const int prow = __shfl(lrow, src);
-    const int row_in = below ? prow : carry;
-    if (hm) carry = (int)rdlane((uint32_t)lrow, 63 - __clzll(hm));
-    int incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int t = __shfl_up(incl, d);
-        if (lane >= d) incl += t;
-    }
-    const uint32_t qn = rdlane((uint32_t)incl, 63);
-    const int base = incl - cnt;
-    if (lane == 0) wq[0] = -c0;
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-        if (b < nx) wq[xj[b]] = base + xcnt[b];
-    wave_sync();
-    // pass 2: entries with their value words
-    {
-        uint32_t ts[NB], tb[NB], tv[NB];
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            ts[b] = ts0[b];
-            tb[b] = tb0[b];
-            tv[b] = tv0[b];
-        }
-        int qt = wq[j];
-        int r = row_in;
-        uint32_t o = (uint32_t)base;
-#pragma unroll
-        for (int i = 0; i < R; i++) {
-            const int32_t pos = p0 + i;
-            const uint32_t w = (wreg[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu;
-            const bool valid = pos >= ic.begin && pos < ic.pend;
-            if (NB > 1 && valid && (uint32_t)pos >= ts[NB > 1 ? 1 : 0]) {
-#pragma unroll
-                for (int b = 0; b + 1 < NB; b++) {
-                    ts[b] = ts[b + 1];
-                    tb[b] = tb[b + 1];
-                    tv[b] = tv[b + 1];
-                }
-                ts[NB - 1] = 0xFFFFFFFFu;
-                tv[NB - 1] = 0xFFFFFFFFu;
-                qt = (int)o;
-            }
-            const bool body = valid && ((uint32_t)pos - ts[0]) >= 8u && (uint32_t)pos < tv[0];
-            if (body && (w & 0x8000u)) r = (int)(w & 0x7FFFu);
-            if (body && !(w & 0x8000u)) {
-                const uint32_t br = (uint32_t)(r - (int)ic.sb_base);
-                const uint32_t gcol = (tb[0] << ic.log2w) | w;
-                const bool keep = r >= 0 && br < ic.rows && gcol < ic.ncols;
-                const uint32_t sl = qslot<SEGP>(o);
-                qcol[sl] = keep ? gcol : 0u;
-                qrow[sl] = keep ? (uint16_t)br : (uint16_t)0xFFFFu;
-                qval[sl] = tv[0] + (uint32_t)((int)o - qt) * (uint32_t)vwords;
-                o++;
-            }
-        }
-    }
-    return qn;
-}
-
-template <typename T, typename V, int K, int R, int P, bool SEQ, bool HOT>
-__global__ void __launch_bounds__(64 * kWPB) __attribute__((amdgpu_waves_per_eu(4, 4)))
-spmm_lane_w(SpmmArgs a)
-{
-    using LC = LaneCfg<R>;
-    constexpr int CW = LC::CW, DWIN = LC::DWIN, DPL = LC::DPL;
-    constexpr int SEGP = K ? P : (1 << 30);
-    constexpr int QS = CW + CW / (K ? P : CW) + 1;
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63;
-    const uint32_t wv = uni(threadIdx.x >> 6);
-    const uint32_t item_id = blockIdx.x * kWPB + wv;
-    if (item_id >= a.nitems) return;
-
-    unsigned char *wbase = smem + wv * a.wave_bytes;
-    using A = typename std::conditional<SEQ, T, typename AccOf<T>::type>::type;
-    A *band = (A *)wbase;
-    uint32_t *qcol = (uint32_t *)(wbase + a.band_bytes);
-    uint32_t *qval = qcol + QS;
-    uint16_t *qrow = (uint16_t *)(qval + QS);
-    const uint32_t win_off = (a.band_bytes + QS * 10 + 7) & ~7u;
-    uint2 *win = (uint2 *)(wbase + win_off);
-    uint32_t *wvb = (uint32_t *)(wbase + win_off + (DWIN + 1) * 8);
-    int32_t *wq = (int32_t *)(wbase + win_off + (DWIN + 1) * 12);
-
-    ItemState st = item_state(a, a.items[item_id]);
-    const RowScale rs = prefetch_rscale<T>(a, st.row0, st.ic.rows, lane);
-    const Row<T, K> row(a.k, lane);
-    const uint32_t S = a.band_stride;
-    for (uint32_t i = lane; i < st.ic.rows * S; i += 64) band[i] = A(0);
-    if (lane == 0) {
-        win[DWIN] = make_uint2(0xFFFFFFFFu, 0u);
-        wvb[DWIN] = 0xFFFFFFFFu;
-    }
+    if (lane == 0) win[kWin] = make_uint2(kNoWord, 0u);
     const uint16_t *vimg = a.img + st.ic.bw;
 
     for (int seg = 0; seg < 2; seg++) {
     if (!select_segment(st, seg)) break;
+    flag[lane] = kNoWord;
     const uint64_t abs_end = st.ic.bw + (uint64_t)st.ic.pend;
     const uint64_t lastw = abs_end - 1;
     uint64_t c = (st.ic.bw + (uint64_t)st.ic.begin) & ~7ull;
-    int c0 = 0;  // columns of window tile 0 decoded in earlier chunks
-    uint32_t wreg[R / 2];
-    uint2 dreg[DPL];
-    uint32_t vreg[DPL];
-    bool live[DPL];
-    load_words<R>(a.img, c, lastw, lane, wreg);
-    load_window<DPL>(a.dir, st.ct, st.dlast, lane, dreg, live);
-#pragma unroll
-    for (int h = 0; h < DPL; h++) {
-        const uint32_t t = st.ct + h * 64 + lane;
-        vreg[h] = a.vdir[t < st.dlast ? t : st.dlast];
-    }
+    int c0 = 0;  // weighted: entries of window tile 0 decoded in earlier chunks
+    uint32_t wreg[4];
+    Window w;
+    load_words(a.img, c, lastw, lane, wreg);
+    load_window<W>(a, st.ct, st.dlast, lane, w);
 
     while (c < abs_end) {
-        store_window<DPL>(win, dreg, live, lane);
-#pragma unroll
-        for (int h = 0; h < DPL; h++) wvb[h * 64 + lane] = live[h] ? vreg[h] : 0xFFFFFFFFu;
+        int tiles = 0, qt = 0;
+        const uint32_t qn = decode_chunk<K, W, NARROW>(st.ic, c, wreg, w, win, flag, wval, c0, a.vwords, st.carry, q,
+                                                       qval, lane, tiles, qt);
+        const uint64_t cn = c + kChunk;
         wave_sync();
-        const uint32_t qn = decode_chunk_w<R, SEGP>(st.ic, c, wreg, win, wvb, wq, c0, a.vwords, st.carry,
-                                                    qcol, qrow, qval, lane);
-        const uint64_t cn = c + CW;
-        wave_sync();
-        // the next chunk's words, window and value-directory entries (this
-        // chunk's are in LDS now)
+        // the next chunk's words and window (this chunk's are in LDS now),
+        // whose entry 0 is this window's last tile starting at or before it
         auto fetch_next = [&]() {
             if (cn < abs_end) {
                 const uint32_t pn = (uint32_t)((int64_t)cn - (int64_t)st.ic.bw);
-                const uint32_t adv = window_advance<DPL>(dreg, live, pn);
-                // the next chunk's window tile 0 is window tile adv-1; one
-                // that starts exactly at the next chunk's first word has no
-                // columns in this chunk, and its wq slot was not written by
-                // this decode
-                c0 = win[adv - 1].x == pn ? 0 : (int)qn - wq[adv - 1];
-                st.ct += adv - 1;
-                load_words<R>(a.img, cn, lastw, lane, wreg);
-                load_window<DPL>(a.dir, st.ct, st.dlast, lane, dreg, live);
-#pragma unroll
-                for (int h = 0; h < DPL; h++) {
-                    const uint32_t t = st.ct + h * 64 + lane;
-                    vreg[h] = a.vdir[t < st.dlast ? t : st.dlast];
-                }
+                const int adv = __popcll(__ballot(w.live && w.e.x <= pn));
+                // that tile has entries in this chunk if lanes of it began here
+                if constexpr (W) c0 = adv > tiles ? 0 : (int)qn - qt;
+                st.ct += (uint32_t)adv - 1;
+                load_words(a.img, cn, lastw, lane, wreg);
+                load_window<W>(a, st.ct, st.dlast, lane, w);
             }
         };
-        if constexpr (K == 0) fetch_next();
         if constexpr (K != 0) {
-            // requested behind the first batch's gathers and value loads (as
-            // in spmm_lane)
+            // requested behind the first batch's gathers: a wait for the
+            // gathers need not wait for these, and their latency overlaps
+            // the gathers' instead of preceding them
             constexpr int E = row_elems<T, K>();
+            const uint32_t batch = row.nzp * kP;
             bool fetched = false;
-            for (uint32_t base = 0; base < qn; base += row.nzp * P) {
-                Vec<T, E> v[P];
-                uint32_t rr[P], gcs[P];
-                V vals[P];
+            for (uint32_t base = 0; base < qn; base += batch) {
+                if (base + batch > qn) fill_queue<K>(q, qval, qn, base + batch, st.ic.dump, lane);
+                Vec<T, E> v[kP];
+                uint32_t rr[kP];
+                typename std::conditional<W, V, int>::type vals[kP];
+                if constexpr (W) {
+                    const uint32_t s0 = qslot<K>(base) + row.g * (kP + 1);
 #pragma unroll
-                for (int pp = 0; pp < P; pp++) {
-                    const uint32_t e = base + row.g * P + pp;
-                    const bool ok = row.on && e < qn;
-                    const uint32_t sl = qslot<P>(K > 0 || ok ? e : 0u);
-                    const uint32_t qr = qrow[sl];
-                    gcs[pp] = ok ? qcol[sl] : 0u;
-                    rr[pp] = (ok && qr != 0xFFFFu) ? qr : 0xFFFFFFFFu;
-                    const uint32_t vo = ok ? qval[sl] : 0u;  // a safe address when unused
-                    vals[pp] = load_value<V>(vimg + vo);
+                    for (int pp = 0; pp < kP; pp++) vals[pp] = load_value<V>(vimg + qval[s0 + pp]);
                 }
-#pragma unroll
-                for (int pp = 0; pp < P; pp++)
-                    load_row<T, K>(v[pp], xrow<T, HOT>(a, gcs[pp]) + row.col0);
+                gather_batch<T, K, HOT, NARROW>(a, row, q, base, v, rr);
                 if (!fetched) {
                     fetch_next();
                     fetched = true;
                 }
                 if constexpr (SEQ) {
-                    // products rounded in T, then added in order
+                    if constexpr (W) {
+                        // products rounded in T, then added in order
 #pragma clang fp contract(off)
 #pragma unroll
-                    for (int pp = 0; pp < P; pp++)
+                        for (int pp = 0; pp < kP; pp++)
 #pragma unroll
-                        for (int i = 0; i < E; i++) v[pp].v[i] = v[pp].v[i] * (T)vals[pp];
-                    accumulate_batch_seq<T, K, P>(band, S, lane, v, rr);
-                    continue;
-                }
-                A acc[E];
-                uint32_t cur = 0xFFFFFFFFu;
-#pragma unroll
-                for (int i = 0; i < E; i++) acc[i] = A(0);
-#pragma unroll
-                for (int pp = 0; pp < P; pp++) {
-                    if (rr[pp] != cur) {
-                        if (cur != 0xFFFFFFFFu) {
-                            A *dst = band + cur * S;
-#pragma unroll
-                            for (int i = 0; i < E; i++) lds_add(dst + row.off[i], acc[i]);
-                        }
-                        cur = rr[pp];
-#pragma unroll
-                        for (int i = 0; i < E; i++) acc[i] = (A)v[pp].v[i] * (A)vals[pp];
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < E; i++) acc[i] += (A)v[pp].v[i] * (A)vals[pp];
+                            for (int i = 0; i < E; i++) v[pp].v[i] = v[pp].v[i] * (T)vals[pp];
                     }
-                }
-                if (cur != 0xFFFFFFFFu) {
-                    A *dst = band + cur * S;
-#pragma unroll
-                    for (int i = 0; i < E; i++) lds_add(dst + row.off[i], acc[i]);
+                    accumulate_batch_seq<T, K>(band, S, lane, v, rr);
+                } else if constexpr (W) {
+                    accumulate_batch<T, K, A, true>(band, S, row, rr,
+                                                    [&](int pp, int i) { return (A)v[pp].v[i] * (A)vals[pp]; });
+                } else {
+                    // 8-byte data: each entry adds straight into the band.
+                    // Run sums save few LDS adds (rows average 2.4 entries
+                    // per tile on R-MAT) and their divergent branches cost
+                    // more than that for E <= 2 (FP64 k = 16: 1.17 ms
+                    // against 1.34 ms with run sums)
+                    accumulate_batch<T, K, A, sizeof(T) != 8>(band, S, row, rr,
+                                                              [&](int pp, int i) { return (A)v[pp].v[i]; });
                 }
             }
             if (!fetched) fetch_next();
-        } else if (SEQ) {
-            if (qn) drain_generic_seq<T, V, P, true>(a, (T *)band, S, qcol, qrow, qval, vimg, qn, lane);
         } else {
-            const uint32_t k = (uint32_t)a.k;
-            const uint32_t tot = qn * k;
-            for (uint32_t base = 0; base < tot; base += 64 * P) {
-                T xv[P];
-                V vv[P];
-                uint32_t dst[P];
-#pragma unroll
-                for (int pp = 0; pp < P; pp++) {
-                    const uint32_t f = base + pp * 64 + lane;
-                    const uint32_t fc = f < tot ? f : tot - 1;
-                    const uint32_t e = fc / k, jj = fc - e * k;
-                    const uint32_t qr = qrow[e];
-                    xv[pp] = xrow<T, HOT>(a, qcol[e])[jj];
-                    vv[pp] = load_value<V>(vimg + qval[e]);
-                    dst[pp] = (f < tot && qr != 0xFFFFu) ? qr * S + jj : 0xFFFFFFFFu;
-                }
-#pragma unroll
-                for (int pp = 0; pp < P; pp++)
-                    if (dst[pp] != 0xFFFFFFFFu) lds_add(band + dst[pp], (A)xv[pp] * (A)vv[pp]);
+            fetch_next();
+            if (qn) {
+                if constexpr (SEQ) drain_generic_seq<T, V>(a, band, S, q, qval, vimg, qn, lane);
+                else drain_generic<T, V, A, HOT>(a, band, S, q, qval, vimg, qn, lane);
             }
         }
         wave_sync();
         c = cn;
     }
     }
-    write_band<T, K, A>(a, band, S, st.row0, st.ic.rows, st.slot, lane, rs, (double *)qcol);
+    write_band<T, K, A>(a, band, S, st.row0, st.ic.rows, st.slot, lane, rs, (double *)(wbase + a.band_bytes));
+}
+
+template <typename T, int K, bool SEQ, bool HOT, bool NARROW>
+__global__ void __launch_bounds__(64 * kWPB) __attribute__((amdgpu_waves_per_eu(5, 5))) spmm_lane(SpmmArgs a)
+{
+    spmm_body<T, void, K, SEQ, HOT, NARROW>(a);
+}
+
+template <typename T, typename V, int K, bool SEQ, bool HOT, bool NARROW>
+__global__ void __launch_bounds__(64 * kWPB) __attribute__((amdgpu_waves_per_eu(4, 4))) spmm_lane_w(SpmmArgs a)
+{
+    spmm_body<T, V, K, SEQ, HOT, NARROW>(a);
 }
 
 // Y rows of a split band = partial slots summed in stream order.
@@ -1152,21 +915,12 @@ __global__ void __launch_bounds__(256) spmm_reduce(const Split *splits, const A 
     }
 }
 
-// Gathers in flight per lane group.  Eight 16-byte gathers per lane keep
-// spmm_lane under 80 VGPRs, so the LDS of its band and queue, not registers,
-// bounds the waves per CU.  More resident waves with short batches put more
+// Gathers in flight per lane group (kP): eight 16-byte gathers per lane keep
+// spmm_lane under 96 VGPRs.  More resident waves with short batches put more
 // gathers in flight than fewer waves with long ones: on R-MAT scale 22, FP32
 // k = 16, 64x32768 tiles, 0.93 ms against 1.30 ms for 512-entry batches
 // overlapped with the next decode at two waves per SIMD (the best earlier
 // schedule), and 57 ms against 92 ms on scale 27, FP32 k = 32.
-template <typename T, int K>
-constexpr int passes_for()
-{
-    if constexpr (K <= 0) return 8;
-    else return 512 / Lanes<T, K>::NZP < 8 ? 512 / Lanes<T, K>::NZP : 8;
-}
-
-constexpr int kLaneR = 8;  // words per lane: 512-word chunks
 
 // Raises a kernel's dynamic LDS limit once per process.
 template <void (*KERN)(SpmmArgs)>
@@ -1196,34 +950,43 @@ fmx_status launch_items(fmx_ctx *ctx, const SpmmArgs &a, hipStream_t stream)
     return FMX_OK;
 }
 
-// Weighted images; V is the type of the stored values (T, or float values
-// with FP64 dense data: spmm_creator<double, float>).
-template <typename T, typename V, int K, bool SEQ, bool HOT>
-fmx_status launch_kw(fmx_ctx *ctx, SpmmArgs a, hipStream_t stream)
+template <typename T, int K, bool SEQ, bool HOT, bool NARROW>
+fmx_status launch_n(fmx_ctx *ctx, SpmmArgs a, int vprim, hipStream_t stream)
 {
-    constexpr int P = passes_for<T, K>();
-    constexpr int R = kLaneR;
-    constexpr int CW = 64 * R;
-    constexpr int QS = CW + CW / (K ? P : CW) + 1;
-    const uint32_t win_off = (a.band_bytes + QS * 10 + 7) & ~7u;
-    a.wave_bytes = (win_off + (LaneCfg<R>::DWIN + 1) * 16 + 15) & ~15u;
-    return launch_items<spmm_lane_w<T, V, K, R, P, SEQ, HOT>>(ctx, a, stream);
+    // the band and its dump row
+    a.band_bytes = (uint32_t)(((uint64_t)(a.hs + 1) * a.band_stride *
+                                   sizeof(typename std::conditional<SEQ, T, typename AccOf<T>::type>::type) + 15) & ~15ull);
+    a.wave_bytes = a.vdir ? lds_layout<K, true, NARROW>(a.band_bytes).bytes
+                          : lds_layout<K, false, NARROW>(a.band_bytes).bytes;
+    if (a.vdir) {
+        // the stored values are of type T, or float with FP64 dense data
+        // (spmm_creator<double, float>)
+        if constexpr (std::is_same<T, double>::value)
+            if (vprim == 8) return launch_items<spmm_lane_w<double, float, K, SEQ, HOT, NARROW>>(ctx, a, stream);
+        return launch_items<spmm_lane_w<T, T, K, SEQ, HOT, NARROW>>(ctx, a, stream);
+    }
+    return launch_items<spmm_lane<T, K, SEQ, HOT, NARROW>>(ctx, a, stream);
+}
+
+// The narrow forms' limits; with a hot block its rows and X's are one stride
+// apart.
+template <typename T>
+bool narrow_ok(const SpmmArgs &a)
+{
+    const uint64_t stride = (uint64_t)a.ldx * sizeof(T);
+    return a.ncols <= (1u << kRowShift) && a.hs < 256 && stride < (1u << 24) &&
+           a.ncols * stride + (uint64_t)a.k * sizeof(T) < (1ull << 32) && (!a.nhot || a.ldx == a.k);
 }
 
 template <typename T, int K, bool SEQ, bool HOT>
 fmx_status launch_k(fmx_ctx *ctx, SpmmArgs a, int vprim, hipStream_t stream)
 {
-    if (a.vdir) {
-        if constexpr (std::is_same<T, double>::value)
-            if (vprim == 8) return launch_kw<double, float, K, SEQ, HOT>(ctx, a, stream);
-        return launch_kw<T, T, K, SEQ, HOT>(ctx, a, stream);
+    if (narrow_ok<T>(a)) {
+        a.xstride = (uint32_t)(a.ldx * sizeof(T));
+        a.Xcold = (const char *)a.X - (size_t)a.nhot * a.xstride;
+        return launch_n<T, K, SEQ, HOT, true>(ctx, a, vprim, stream);
     }
-    constexpr int P = passes_for<T, K>();
-    constexpr int CW = 64 * kLaneR;
-    constexpr int QS = CW + CW / (K ? P : CW) + 1;
-    const uint32_t win_off = (a.band_bytes + QS * 6 + 7) & ~7u;
-    a.wave_bytes = (win_off + (LaneCfg<kLaneR>::DWIN + 1) * 8 + 15) & ~15u;
-    return launch_items<spmm_lane<T, K, kLaneR, P, SEQ, HOT>>(ctx, a, stream);
+    return launch_n<T, K, SEQ, HOT, false>(ctx, a, vprim, stream);
 }
 
 // Elements per lane of the runtime-width form for rows of k elements (0: the
@@ -1246,11 +1009,7 @@ fmx_status launch_runtime(fmx_ctx *ctx, SpmmArgs a, int vprim, hipStream_t strea
 {
     if constexpr (!SEQ) {
         const int e = runtime_elems<T>(a.k);
-        if (e) {
-            // a band row holds whole lanes and a spare word
-            a.band_stride = (uint32_t)((a.k + e - 1) / e * e + 1);
-            a.band_bytes = (uint32_t)(((uint64_t)a.hs * a.band_stride * sizeof(typename AccOf<T>::type) + 15) & ~15ull);
-        }
+        if (e) a.band_stride = (uint32_t)((a.k + e - 1) / e * e + 1);  // whole lanes and a spare word
         if constexpr (sizeof(T) == 4)
             if (e == 4) return launch_k<T, -4, SEQ, HOT>(ctx, a, vprim, stream);
         if (e == 2) return launch_k<T, -2, SEQ, HOT>(ctx, a, vprim, stream);
@@ -1299,9 +1058,7 @@ fmx_status launch_t(fmx_ctx *ctx, const fmx_spm *spm, const Plan *plan, int k,
     // pad band rows by one element to spread the LDS adds over the banks
     static const bool no_pad = getenv("FMX_NO_PAD") != nullptr;  // read once per process
     a.band_stride = (uint32_t)k + ((k >= 4 && !no_pad) ? 1u : 0u);
-    const uint64_t acc = seq ? sizeof(T) : sizeof(typename AccOf<T>::type);
-    a.band_bytes = (uint32_t)(((uint64_t)plan->hs * a.band_stride * acc + 15) & ~15ull);
-    a.wave_bytes = 0;
+    a.band_bytes = a.wave_bytes = 0;  // launch_n
     a.log2w = spm->log2w;
     a.k = k;
     a.ncols = spm->ncols;
