@@ -938,8 +938,18 @@ fmx_status gram(fmx_ctx *ctx, fmx_dtype dt, int mode, uint64_t n, int ka, int kb
         // most 8 per CU (the 48- to 96-row products ran 5-8% slower with three
         // waves, and more waves only add partials to reduce)
         const bool occ3 = dt == FMX_F32 && sym;
-        // waves of at least 1024 rows (a multiple of 16)
-        uint64_t waves = (n + 1023) / 1024;
+        // Waves of at least 128 rows (a multiple of 16), of 64 up to 512
+        // waves, so that a short operand fills the chip too: with 1024-row
+        // waves 260,000 x 20 FP32 took 57 us (now 26, sym), 8,192 x 96 by 16
+        // FP64 162 us (22), 524,288 x 96 by 16 FP32 122 us (64).  Each block
+        // writes its partial sums, so wide outputs stop at 2^22 of them in
+        // all: 524,288 x 128 by 32 takes 138 us at 1024 waves, 160 at 2048.
+        uint64_t waves = std::max((n + 127) / 128, std::min<uint64_t>((n + 63) / 64, 512));
+        waves = std::min(waves, std::max<uint64_t>((1u << 22) / nout, (n + 1023) / 1024));
+        // whole rounds of a block per CU (2^20 x 48 FP64: 317 us at 1820
+        // waves, 264 at 1024)
+        const uint64_t round = (uint64_t)ctx->num_cus * (kT / 64);
+        if (waves > round) waves -= waves % round;
         uint64_t cap = (uint64_t)ctx->num_cus * (occ3 ? 12 : 8);
         if (fixed_ws) {
             const uint64_t fit = fixed_bytes / ((size_t)nout * sizeof(double));  // blocks whose partials fit
@@ -1022,7 +1032,7 @@ fmx_status gram(fmx_ctx *ctx, fmx_dtype dt, int mode, uint64_t n, int ka, int kb
 #undef FMX_GRAMS_I
 #undef FMX_GRAMS
         FMX_HIP(ctx, hipGetLastError());
-        if (nblk > 256)  // many partials: 16 segments per output instead of 4
+        if (nblk > 16)  // many partials: 16 segments per output instead of 4
             hipLaunchKernelGGL(reduce_partials_seg<double>, dim3((nout + 15) / 16), dim3(kT), 0, s,
                                (const double *)ws, (int)nblk, nout, G);
         else

@@ -156,3 +156,21 @@ def test_colnorm_and_row_scale(fmx, orc):
         d = rng.standard_normal(123457)
         Y = fmx.row_scale(dev(d), dev(A)).cpu().numpy()
         assert np.array_equal(Y, (A.astype(np.float64) * d[:, None]).astype(dt))
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 65, 129, 4097, 33001])
+def test_gram_short_operands(fmx, n):
+    """Row counts around a stage (16 rows), a wave's least share (64) and the
+    wave count from which waves take 128 rows, for narrow and wide outputs:
+    A^T B and A^T A against the FP64 product, to its own rounding."""
+    import torch
+    g = torch.Generator().manual_seed(n)
+    for ka, kb in ((16, 16), (20, 20), (96, 16), (64, 64), (128, 32)):
+        for dt in (torch.float32, torch.float64):
+            A, B = torch.randn((n, ka), generator=g).to(dt), torch.randn((n, kb), generator=g).to(dt)
+            for X, Y in ((A, B), (A, A)):
+                G = fmx.gram(X.cuda(), Y.cuda() if Y is B else X.cuda()).cpu()
+                x, y = X.double(), Y.double()
+                assert ((G - x.t() @ y).abs() <= 1e-13 * (x.abs().t() @ y.abs()) + 1e-300).all(), (ka, kb, dt)
+            Ad = A.cuda()
+            assert torch.equal(fmx.gram(Ad, Ad), fmx.gram(Ad, Ad))
