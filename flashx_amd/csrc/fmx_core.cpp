@@ -671,7 +671,7 @@ static int value_prim(fmx_dtype dt)
 // The SpMM entries (fmx_spmm, fmx_spmm_ex, fmx_spmm_scaled).
 fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, const double *pre,
                      const double *post, const void *X, int64_t ldx, void *Y, int64_t ldy, uint32_t flags,
-                     bool mixed, hipStream_t s)
+                     bool mixed, hipStream_t s, bool round_first)
 {
     if (!ctx || !cspm) return fail(ctx, FMX_EINVAL, "null context or matrix");
     fmx_spm *spm = const_cast<fmx_spm *>(cspm);
@@ -741,7 +741,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
         X = ctx->xstage.ptr;
         ldx = k;
     }
-    const uint32_t kflags = flags & (FMX_SPMM_SEQ | FMX_SPMM_Y_COLMAJOR);
+    const uint32_t kflags = (flags & (FMX_SPMM_SEQ | FMX_SPMM_Y_COLMAJOR)) | (round_first ? kSpmmRoundFirst : 0u);
     if (hot) {
         // X's hot rows, densely, in the gather-order image's column order
         const size_t hb = orig->nhot * (size_t)k * es;
@@ -765,12 +765,6 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
         return launch_spmm(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, spm->partial.ptr, s,
                            (const uint16_t *)spm->d_image, 0, plan->nitems, true, post, kflags);
     return spmm_streamed(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, s, post, kflags);
-}
-
-fmx_status spmm_scaled(fmx_ctx *ctx, const fmx_spm *spm, fmx_dtype dtype, int k, const void *X, int64_t ldx,
-                       void *Y, int64_t ldy, const double *rscale, hipStream_t s)
-{
-    return spmm_exec(ctx, spm, dtype, k, nullptr, rscale, X, ldx, Y, ldy, 0, false, s);
 }
 
 }  // namespace fmx

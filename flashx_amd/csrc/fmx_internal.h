@@ -198,6 +198,9 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *spm, uint32_t hs, bool ordered, Plan 
 // Band height for element size s and width k.
 uint32_t band_rows(const fmx_spm *spm, int k, int s);
 
+// launch_spmm's flag beside FMX_SPMM_*: spmm_exec's round_first.
+constexpr uint32_t kSpmmRoundFirst = 1u << 31;
+
 // Launches the SpMM kernel over plan items [item_begin, item_end) with the
 // image at img (absolute u16 word w of the image is img[w]) and, if reduce,
 // the in-order reduction of the plan's split bands.
@@ -223,14 +226,11 @@ fmx_status stage_dense_rows(fmx_ctx *ctx, fmx_dtype dt, uint64_t n, int k, const
 // Y = diag(post) A diag(pre) X with FMX_SPMM_* flags; pre / post may be null.
 // The weighted-value type may differ from dtype only when mixed is set
 // (FP64 dense data with FP32 values, spmm_creator<double, float>).
+// round_first: a scaled row's sum is rounded to dtype before post multiplies
+// it (and rounded again), as a product followed by a row scaling rounds.
 fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *spm, fmx_dtype dtype, int k, const double *pre,
                      const double *post, const void *X, int64_t ldx, void *Y, int64_t ldy, uint32_t flags,
-                     bool mixed, hipStream_t stream);
-
-// fmx_spmm with each output row r scaled by rscale[r] (FP32/FP64 data; null:
-// none), applied to the FP64 sum before its single rounding.
-fmx_status spmm_scaled(fmx_ctx *ctx, const fmx_spm *spm, fmx_dtype dtype, int k, const void *X, int64_t ldx,
-                       void *Y, int64_t ldy, const double *rscale, hipStream_t stream);
+                     bool mixed, hipStream_t s, bool round_first = false);
 
 }  // namespace fmx
 

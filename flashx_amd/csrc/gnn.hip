@@ -5,15 +5,17 @@
 // matrix/eigensolver/FM_MultiVector.h:164-168).  Network, for the normalised
 // adjacency N = D^-1/2 A D^-1/2:
 //   H0 = X0 (n x 16: log(1+deg), 8 uniform features, 7 zeros)
-//   Agg_l = N H_l                      (fmx_spmm + two row scalings)
+//   Agg_l = N H_l                      (an SpMM with its output rows scaled;
+//                                       the product before it also writes D^-1/2 H_l)
 //   H_{l+1} = relu(H_l Ws_l + Agg_l Wn_l + b_l),  l = 0, 1, 2  (hidden 64)
 //   Y = H_3 Wo                         (n x 16)
 // Dense products run as v_mfma_f32_16x16x32_bf16 with BF16 operands (weights
 // and activations rounded to BF16) and FP32 accumulation; a plain-FP32 mode
-// exists for gradient checking.  Weight gradients are Gram products
-// (fmx_gram, BF16 MFMA or FP64), the bias gradient a column sum.
+// exists for gradient checking.  Weight gradients are Gram products (BF16
+// MFMA, or FP64), the bias gradient a column sum in the same kernel.
 // Parameters, flat FP32: per layer Ws (din x 64), Wn (din x 64), b (64);
 // then Wo (64 x 16); din = 16, 64, 64 (19,648 values).
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -25,7 +27,6 @@ namespace {
 
 constexpr int kIn = 16, kHid = 64, kOut = 16, kLayers = 3;
 constexpr int kT = 256;
-constexpr int kRows = 64;       // rows per block tile
 constexpr int kKMax = 128;      // max inner dimension
 constexpr int kPad = 8;
 
@@ -49,107 +50,320 @@ size_t layer_off(int l)
     return o;
 }
 
-// out[r][c] = act( sum_k A[r][k] B[k][c] + bias[c] + add[r][c] ), A = [A1 | A2]
-// (n x K), B = W (K x dout row-major) or W^T (W dout x K row-major, wtrans).
-template <bool BF16>
-__global__ void __launch_bounds__(kT) gnn_gemm_kernel(const float *A1, int64_t lda1, int d1, const float *A2,
-                                                      int64_t lda2, int d2, const float *W, int wtrans,
-                                                      int dout, const float *bias, const float *add,
-                                                      int64_t ldadd, int relu, float *out, int64_t ldo,
-                                                      uint64_t n)
+// What a dense product's epilogue does with out[r][c] = sum_k A[r][k] B[k][c],
+// A = [A1 | A2] (n x K), in this order: adds bias[c], adds add[r][c], clears a
+// negative value (relu), clears it where gate[r][c] is not positive (the ReLU's
+// backward step); then stores the value to out and, times scale[r], to outs.
+// Every matrix of it is n x dout without gaps; a null pointer leaves its step
+// out.
+struct Epilogue {
+    const float *bias = nullptr, *add = nullptr, *gate = nullptr;
+    const double *scale = nullptr;
+    int relu = 0;
+    float *out = nullptr, *outs = nullptr;
+};
+
+// N floats moved by one load or store, at any float's address.
+template <int N>
+struct FV {
+    float v[N];
+};
+using F4 = FV<4>;
+
+__device__ __forceinline__ bf16x8 to_bf16(const F4 &a, const F4 &b)
 {
+    bf16x8 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        r[i] = (__bf16)a.v[i];
+        r[i + 4] = (__bf16)b.v[i];
+    }
+    return r;
+}
+
+// BF16 MFMA form, K = d1 + d2 <= 32 * KS, dout = 16 * NT; B = W (K x dout) or
+// W^T (W dout x K, wtrans).  Bound by the operands' bytes: each wave takes 16
+// rows at a time straight from memory into the MFMA operand (a lane's 8
+// consecutive k of one row are two 16-byte loads; rounded to BF16 by the
+// hardware's pair conversion), B stays in registers for the whole kernel, and
+// output tile t of lane p is column NT * p + t, so that a lane stores NT
+// consecutive columns.  131,072 rows, 128 -> 64: 46 us with both operands
+// staged in LDS by 4-byte loads and 11 us for the scaled copy in a kernel of
+// its own, 37 us together like this (100 MB moved, 2.7 TB/s); 64 -> 64 20 us.
+template <int KS, int NT>
+__global__ void __launch_bounds__(kT) gnn_mfma_kernel(const float *A1, int d1, const float *A2, int d2,
+                                                      const float *W, int wtrans, Epilogue ep, uint64_t n)
+{
+    constexpr int KP = KS * 32, DO = NT * 16, LD = KP + kPad;
+    __shared__ unsigned short Bt[DO * LD];
     const int K = d1 + d2;
-    const int KP = (K + 31) & ~31;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if constexpr (BF16) {
-        __shared__ unsigned short As[kRows * (kKMax + kPad)];
-        __shared__ unsigned short Bt[kHid * (kKMax + kPad)];
-        const int ld = KP + kPad;
-        for (int e = threadIdx.x; e < dout * KP; e += kT) {
-            const int c = e / KP, k = e - c * KP;
-            float v = 0.f;
-            if (k < K) v = wtrans ? W[(size_t)c * K + k] : W[(size_t)k * dout + c];
-            Bt[c * ld + k] = f2bf(v);
+    // (DO * KP is a multiple of 2 * kT; consecutive threads read consecutive
+    // words of W, several in flight)
+    constexpr int PER = DO * KP / kT, STEP = PER < 8 ? PER : 8;
+    for (int i0 = 0; i0 < PER; i0 += STEP) {
+        float v[STEP];
+#pragma unroll
+        for (int i = 0; i < STEP; i++) {
+            const int e = (i0 + i) * kT + threadIdx.x;
+            const int c = wtrans ? e / KP : e % DO, k = wtrans ? e % KP : e / DO, kc = k < K ? k : 0;
+            v[i] = W[wtrans ? c * K + kc : kc * DO + c];
+            if (k >= K) v[i] = 0.f;
         }
-        const int nct = dout / 16;
-        for (uint64_t r0 = blockIdx.x * (uint64_t)kRows; r0 < n; r0 += (uint64_t)gridDim.x * kRows) {
-            __syncthreads();
-            for (int e = threadIdx.x; e < kRows * KP; e += kT) {
-                const int r = e / KP, k = e - r * KP;
-                const uint64_t row = r0 + r;
-                float v = 0.f;
-                if (row < n && k < K) v = k < d1 ? A1[row * lda1 + k] : A2[row * lda2 + (k - d1)];
-                As[r * ld + k] = f2bf(v);
-            }
-            __syncthreads();
-            floatx4 acc[4];
 #pragma unroll
-            for (int t = 0; t < 4; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-            for (int ks = 0; ks < KP; ks += 32) {
-                const int k0 = ks + (lane >> 4) * 8;
-                const bf16x8 a = *(const bf16x8 *)(As + (w * 16 + (lane & 15)) * ld + k0);
+        for (int i = 0; i < STEP; i++) {
+            const int e = (i0 + i) * kT + threadIdx.x;
+            const int c = wtrans ? e / KP : e % DO, k = wtrans ? e % KP : e / DO;
+            Bt[c * LD + k] = f2bf(v[i]);
+        }
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, p = lane & 15, kg = (lane >> 4) * 8;
+    bf16x8 b[KS][NT];
 #pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    if (t < nct) {
-                        const bf16x8 b = *(const bf16x8 *)(Bt + (t * 16 + (lane & 15)) * ld + k0);
-                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
-                    }
-                }
-            }
+    for (int s = 0; s < KS; s++)
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                if (t >= nct) continue;
-                const int c = t * 16 + (lane & 15);
+        for (int t = 0; t < NT; t++) b[s][t] = *(const bf16x8 *)(Bt + (NT * p + t) * LD + s * 32 + kg);
+    FV<NT> bias{};
+    if (ep.bias) bias = *(const FV<NT> *)(ep.bias + NT * p);
+    const uint64_t waves = (uint64_t)gridDim.x * (kT / 64);
+    for (uint64_t r0 = (blockIdx.x * (uint64_t)(kT / 64) + (threadIdx.x >> 6)) * 16; r0 < n; r0 += waves * 16) {
+        const uint64_t ar = r0 + p < n ? r0 + p : n - 1;  // rows past the end are not stored
+        F4 x[KS][2];
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const uint64_t row = r0 + w * 16 + (lane >> 4) * 4 + q;
-                    if (row >= n) continue;
-                    float v = acc[t][q];
-                    if (bias) v += bias[c];
-                    if (add) v += add[row * ldadd + c];
-                    if (relu) v = v > 0.f ? v : 0.f;
-                    out[row * ldo + c] = v;
-                }
+        for (int s = 0; s < KS; s++) {
+            const int k = s * 32 + kg;
+            // (d1 is a multiple of 8, so a lane's k all lie in one operand)
+            const float *src = k < d1 ? A1 + ar * d1 + k : A2 + ar * d2 + (k - d1);
+            if (k < K) {
+                x[s][0] = *(const F4 *)src;
+                x[s][1] = *(const F4 *)(src + 4);
+            } else {
+                x[s][0] = x[s][1] = F4{{0.f, 0.f, 0.f, 0.f}};
             }
         }
-    } else {
-        constexpr int kR = kRows / 2;  // 32-row tiles keep the FP32 operands in 48 KiB
-        __shared__ float As[kR * (kKMax + 1)];
-        __shared__ float Bs[kKMax * kHid];
-        for (int e = threadIdx.x; e < K * dout; e += kT) {
-            const int k = e / dout, c = e - k * dout;
-            Bs[e] = wtrans ? W[(size_t)c * K + k] : W[(size_t)k * dout + c];
+        floatx4 acc[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            const bf16x8 a = to_bf16(x[s][0], x[s][1]);
+#pragma unroll
+            for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[s][t], acc[t], 0, 0, 0);
         }
-        for (uint64_t r0 = blockIdx.x * (uint64_t)kR; r0 < n; r0 += (uint64_t)gridDim.x * kR) {
-            __syncthreads();
-            for (int e = threadIdx.x; e < kR * K; e += kT) {
-                const int r = e / K, k = e - r * K;
-                const uint64_t row = r0 + r;
-                float v = 0.f;
-                if (row < n) v = k < d1 ? A1[row * lda1 + k] : A2[row * lda2 + (k - d1)];
-                As[r * (kKMax + 1) + k] = v;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint64_t row = r0 + (lane >> 4) * 4 + q;
+            if (row >= n) continue;
+            const uint64_t at = row * DO + NT * p;
+            FV<NT> y, ys;
+#pragma unroll
+            for (int t = 0; t < NT; t++) y.v[t] = acc[t][q];
+            if (ep.bias) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) y.v[t] += bias.v[t];
             }
-            __syncthreads();
-            for (int o = threadIdx.x; o < kR * dout; o += kT) {
-                const int r = o / dout, c = o - r * dout;
-                const uint64_t row = r0 + r;
-                if (row >= n) continue;
-                float v = 0.f;
-                for (int k = 0; k < K; k++) v = fmaf(As[r * (kKMax + 1) + k], Bs[k * dout + c], v);
-                if (bias) v += bias[c];
-                if (add) v += add[row * ldadd + c];
-                if (relu) v = v > 0.f ? v : 0.f;
-                out[row * ldo + c] = v;
+            if (ep.add) {
+                const FV<NT> x = *(const FV<NT> *)(ep.add + at);
+#pragma unroll
+                for (int t = 0; t < NT; t++) y.v[t] += x.v[t];
+            }
+            if (ep.relu) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) y.v[t] = y.v[t] > 0.f ? y.v[t] : 0.f;
+            }
+            if (ep.gate) {
+                const FV<NT> x = *(const FV<NT> *)(ep.gate + at);
+#pragma unroll
+                for (int t = 0; t < NT; t++) y.v[t] = x.v[t] > 0.f ? y.v[t] : 0.f;
+            }
+            if (ep.out) *(FV<NT> *)(ep.out + at) = y;
+            if (ep.outs) {
+                const double d = ep.scale[row];
+#pragma unroll
+                for (int t = 0; t < NT; t++) ys.v[t] = (float)((double)y.v[t] * d);
+                *(FV<NT> *)(ep.outs + at) = ys;
             }
         }
     }
 }
 
-// dZ = dH * (H > 0), in place on dH
-__global__ void __launch_bounds__(kT) relu_back_kernel(const float *H, float *dH, uint64_t tot)
+// FP32 form: 32-row tiles keep the operands in 48 KiB.
+__global__ void __launch_bounds__(kT) gnn_f32_kernel(const float *A1, int d1, const float *A2, int d2, const float *W,
+                                                     int wtrans, int dout, Epilogue ep, uint64_t n)
 {
-    for (uint64_t e = blockIdx.x * (uint64_t)kT + threadIdx.x; e < tot; e += (uint64_t)gridDim.x * kT)
-        if (!(H[e] > 0.f)) dH[e] = 0.f;
+    constexpr int kR = 32;
+    __shared__ float As[kR * (kKMax + 1)];
+    __shared__ float Bs[kKMax * kHid];
+    const int K = d1 + d2;
+    for (int e = threadIdx.x; e < K * dout; e += kT) {
+        const int k = e / dout, c = e - k * dout;
+        Bs[e] = wtrans ? W[(size_t)c * K + k] : W[(size_t)k * dout + c];
+    }
+    for (uint64_t r0 = blockIdx.x * (uint64_t)kR; r0 < n; r0 += (uint64_t)gridDim.x * kR) {
+        __syncthreads();
+        for (int e = threadIdx.x; e < kR * K; e += kT) {
+            const int r = e / K, k = e - r * K;
+            const uint64_t row = r0 + r;
+            float v = 0.f;
+            if (row < n) v = k < d1 ? A1[row * d1 + k] : A2[row * d2 + (k - d1)];
+            As[r * (kKMax + 1) + k] = v;
+        }
+        __syncthreads();
+        for (int o = threadIdx.x; o < kR * dout; o += kT) {
+            const int r = o / dout, c = o - r * dout;
+            const uint64_t row = r0 + r;
+            if (row >= n) continue;
+            float v = 0.f;
+            for (int k = 0; k < K; k++) v = fmaf(As[r * (kKMax + 1) + k], Bs[k * dout + c], v);
+            const uint64_t at = row * dout + c;
+            if (ep.bias) v += ep.bias[c];
+            if (ep.add) v += ep.add[at];
+            if (ep.relu) v = v > 0.f ? v : 0.f;
+            if (ep.gate) v = ep.gate[at] > 0.f ? v : 0.f;
+            if (ep.out) ep.out[at] = v;
+            if (ep.outs) ep.outs[at] = (float)((double)v * ep.scale[row]);
+        }
+    }
+}
+
+// ---- weight gradients ----------------------------------------------------------
+// partial[y][block] = A_y^T Z over the block's rows (ka = 16 TI by kb = 16 TJ,
+// BF16 MFMA, FP32 accumulation; y = blockIdx.y picks A0 or A1) and, with
+// bpartial and y = 0, the column sums of Z in FP64.  Bound by the operands'
+// bytes: the rows are the MFMA's K dimension, and a lane's 8 rows of a 32-row
+// step come straight from memory, TI (TJ) consecutive columns per load, so
+// that 16 lanes read whole rows; tile t of lane p is then column TI * p + t.
+// Blocks of 128-row steps, few enough that their partials stay a small part
+// of the traffic.  131,072 rows, 64 x 64: 200 us for one A from operands
+// staged and transposed in LDS by 4-byte loads in 128 blocks, 22 us for both
+// like this, and 6 us to add the partials up; the column sums took 17 + 121 us
+// in kernels of their own.
+template <int TI, int TJ>
+__global__ void __launch_bounds__(kT) gnn_grad_kernel(const float *A0, const float *A1, const float *Z, uint64_t n,
+                                                      uint64_t rows_per_blk, float *partial, double *bpartial)
+{
+    constexpr int KA = 16 * TI, KB = 16 * TJ, NOUT = KA * KB;
+    __shared__ float red[2][NOUT];
+    __shared__ double bred[kT / 64][KB];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, p = lane & 15, rg = (lane >> 4) * 8;
+    const float *A = blockIdx.y ? A1 : A0;
+    const bool bias = bpartial && blockIdx.y == 0;
+    floatx4 acc[TI][TJ];
+    double bs[TJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < TJ; j++) bs[j] = 0.0;
+    const uint64_t b0 = blockIdx.x * rows_per_blk, b1 = min(n, b0 + rows_per_blk);
+    for (uint64_t r0 = b0 + w * 32; r0 < b1; r0 += 32 * (kT / 64)) {
+        FV<TI> a[8];
+        FV<TJ> z[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint64_t r = r0 + rg + i, rc = r < b1 ? r : b1 - 1;
+            a[i] = *(const FV<TI> *)(A + rc * KA + TI * p);
+            z[i] = *(const FV<TJ> *)(Z + rc * KB + TJ * p);
+            if (r >= b1) {
+#pragma unroll
+                for (int t = 0; t < TI; t++) a[i].v[t] = 0.f;
+#pragma unroll
+                for (int t = 0; t < TJ; t++) z[i].v[t] = 0.f;
+            }
+        }
+        if (bias)
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int t = 0; t < TJ; t++) bs[t] += (double)z[i].v[t];
+        bf16x8 zb[TJ];
+#pragma unroll
+        for (int t = 0; t < TJ; t++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) zb[t][i] = (__bf16)z[i].v[t];
+#pragma unroll
+        for (int ti = 0; ti < TI; ti++) {
+            bf16x8 ab;
+#pragma unroll
+            for (int i = 0; i < 8; i++) ab[i] = (__bf16)a[i].v[ti];
+#pragma unroll
+            for (int tj = 0; tj < TJ; tj++)
+                acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab, zb[tj], acc[ti][tj], 0, 0, 0);
+        }
+    }
+    // the block's four waves combine as (w0 + w2) + (w1 + w3)
+    auto each = [&](auto fn) {
+#pragma unroll
+        for (int ti = 0; ti < TI; ti++)
+#pragma unroll
+            for (int tj = 0; tj < TJ; tj++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    fn(acc[ti][tj][q], (TI * ((lane >> 4) * 4 + q) + ti) * KB + TJ * p + tj);
+    };
+    if (w >= 2) each([&](float v, int o) { red[w - 2][o] = v; });
+    if (bias) {
+#pragma unroll
+        for (int t = 0; t < TJ; t++) {
+            bs[t] += __shfl_xor(bs[t], 16, 64);
+            bs[t] += __shfl_xor(bs[t], 32, 64);
+            if (lane < 16) bred[w][TJ * p + t] = bs[t];
+        }
+    }
+    __syncthreads();
+    if (w < 2) {
+#pragma unroll
+        for (int ti = 0; ti < TI; ti++)
+#pragma unroll
+            for (int tj = 0; tj < TJ; tj++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int o = (TI * ((lane >> 4) * 4 + q) + ti) * KB + TJ * p + tj;
+                    acc[ti][tj][q] += red[w][o];
+                    if (w == 1) red[1][o] = acc[ti][tj][q];
+                }
+    }
+    __syncthreads();
+    if (w == 0) {
+        float *out = partial + ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * NOUT;
+        each([&](float v, int o) { out[o] = v + red[1][o]; });
+    }
+    if (bias && threadIdx.x < KB) {
+        double t = 0.0;
+        for (int q = 0; q < kT / 64; q++) t += bred[q][threadIdx.x];
+        bpartial[(uint64_t)blockIdx.x * KB + threadIdx.x] = t;
+    }
+}
+
+// out[o] = the sum of nblk partials of output o, in FP64: 16 interleaved
+// segments (q, q + 16, ...), each in block order, then the segments in order.
+// Outputs 0 .. na - 1 are pa's (FP32), the nb behind them pb's (FP64).
+template <int SEG>
+__device__ __forceinline__ double seg_sum(double mine, double *red)
+{
+    red[threadIdx.x] = mine;
+    __syncthreads();
+    double t = 0.0;
+    if (threadIdx.x < kT / SEG)
+        for (int q = 0; q < SEG; q++) t += red[q * (kT / SEG) + threadIdx.x];
+    return t;
+}
+
+__global__ void __launch_bounds__(kT) gnn_grad_reduce(const float *pa, int ny, int nout, const double *pb, int nb,
+                                                      int nblk, float *out)
+{
+    __shared__ double red[kT];
+    const int o = blockIdx.x * 16 + (threadIdx.x & 15), sg = threadIdx.x >> 4;
+    double s = 0.0;
+    if (o < ny * nout) {
+        const float *p = pa + (uint64_t)(o / nout) * nblk * nout + o % nout;
+        for (int b = sg; b < nblk; b += 16) s += (double)p[(uint64_t)b * nout];
+    } else if (o < ny * nout + nb) {
+        for (int b = sg; b < nblk; b += 16) s += pb[(uint64_t)b * nb + (o - ny * nout)];
+    }
+    const double t = seg_sum<16>(s, red);
+    if (threadIdx.x < 16 && o < ny * nout + nb) out[o] = (float)t;
 }
 
 __global__ void __launch_bounds__(kT) colsum_kernel(const float *A, uint64_t n, int k, uint64_t rpb,
@@ -169,15 +383,6 @@ __global__ void __launch_bounds__(kT) colsum_kernel(const float *A, uint64_t n, 
         double t = 0.0;
         for (int q = 0; q < per; q++) t += red[q * k + threadIdx.x];
         partial[(uint64_t)blockIdx.x * k + threadIdx.x] = t;
-    }
-}
-
-__global__ void __launch_bounds__(kT) colsum_finish(const double *partial, int nblk, int k, float *out)
-{
-    for (int j = threadIdx.x; j < k; j += kT) {
-        double s = 0.0;
-        for (int b = 0; b < nblk; b++) s += partial[(uint64_t)b * k + j];
-        out[j] = (float)s;
     }
 }
 
@@ -226,41 +431,93 @@ uint32_t grid_n(fmx_ctx *ctx, uint64_t work)
     return (uint32_t)(b < 1 ? 1 : (b > cap ? cap : b));
 }
 
-fmx_status gemm(fmx_ctx *ctx, int mode, const float *A1, int64_t lda1, int d1, const float *A2, int64_t lda2,
-                int d2, const float *W, int wtrans, int dout, const float *bias, const float *add,
-                int64_t ldadd, int relu, float *out, int64_t ldo, uint64_t n, hipStream_t s)
+// [A1 | A2] B with the epilogue; dout is 16 or 64, d1 and d2 multiples of 16.
+fmx_status gemm(fmx_ctx *ctx, int mode, const float *A1, int d1, const float *A2, int d2, const float *W, int wtrans,
+                int dout, const Epilogue &ep, uint64_t n, hipStream_t s)
 {
-    const uint64_t tiles = (n + kRows - 1) / kRows;
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(tiles ? tiles : 1, (uint64_t)ctx->num_cus * 8);
-    if (mode == 0)
-        hipLaunchKernelGGL(gnn_gemm_kernel<true>, dim3(grid), dim3(kT), 0, s, A1, lda1, d1, A2, lda2, d2, W,
-                           wtrans, dout, bias, add, ldadd, relu, out, ldo, n);
-    else
-        hipLaunchKernelGGL(gnn_gemm_kernel<false>, dim3(grid), dim3(kT), 0, s, A1, lda1, d1, A2, lda2, d2, W,
-                           wtrans, dout, bias, add, ldadd, relu, out, ldo, n);
+    if (!n) return FMX_OK;
+    const int K = d1 + d2;
+    if (mode != 0) {
+        const uint32_t grid = (uint32_t)std::min<uint64_t>((n + 31) / 32, (uint64_t)ctx->num_cus * 8);
+        hipLaunchKernelGGL(gnn_f32_kernel, dim3(grid), dim3(kT), 0, s, A1, d1, A2, d2, W, wtrans, dout, ep, n);
+        FMX_HIP(ctx, hipGetLastError());
+        return FMX_OK;
+    }
+    // at most four blocks per CU: a wave's B then serves several row tiles
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((n + 63) / 64, (uint64_t)ctx->num_cus * 4);
+#define FMX_GNN(KS, NT)                                                                                        \
+    hipLaunchKernelGGL((gnn_mfma_kernel<KS, NT>), dim3(grid), dim3(kT), 0, s, A1, d1, A2, d2, W, wtrans, ep, n)
+    if (dout == 64) {
+        if (K <= 32) FMX_GNN(1, 4);
+        else if (K <= 64) FMX_GNN(2, 4);
+        else FMX_GNN(4, 4);
+    } else {
+        if (K <= 32) FMX_GNN(1, 1);
+        else if (K <= 64) FMX_GNN(2, 1);
+        else FMX_GNN(4, 1);
+    }
+#undef FMX_GNN
     FMX_HIP(ctx, hipGetLastError());
     return FMX_OK;
 }
 
-// out = N X for d columns: row scale, SpMM, row scale (T is n x d scratch)
-fmx_status norm_agg(fmx_ctx *ctx, const fmx_spm *spm, const double *dinv, const float *X, int d, float *T,
-                    float *out, hipStream_t s)
+// out = N X for d columns, XS being X with its rows scaled already; the sums
+// are rounded before and after the outer scaling
+fmx_status norm_agg(fmx_ctx *ctx, const fmx_spm *spm, const double *dinv, const float *XS, int d, float *out,
+                    hipStream_t s)
 {
-    const uint64_t n = spm->nrows;
-    fmx_status st = row_scale(ctx, FMX_F32, n, d, dinv, X, d, T, d, s);
-    if (st) return st;
-    st = fmx_spmm(ctx, spm, FMX_F32, d, T, d, out, d, s);
-    if (st) return st;
-    return row_scale(ctx, FMX_F32, n, d, dinv, out, d, out, d, s);
+    return spmm_exec(ctx, spm, FMX_F32, d, nullptr, dinv, XS, d, out, d, 0, false, s, true);
 }
 
-// grads (FP32) <- Gram(A, B) through an FP64 scratch
-fmx_status gram_grad(fmx_ctx *ctx, int mode, uint64_t n, int ka, int kb, const float *A, const float *B,
-                     double *g64, float *out, hipStream_t s)
+// out (FP32) = A0^T Z, then A1^T Z, then (bias) the column sums of Z; A0 and
+// A1 (or NULL) are n x ka, Z n x kb.
+fmx_status grads(fmx_ctx *ctx, int mode, uint64_t n, int ka, int kb, const float *A0, const float *A1, const float *Z,
+                 bool bias, float *out, hipStream_t s)
 {
-    fmx_status st = gram(ctx, FMX_F32, mode == 0 ? FMX_GRAM_BF16 : FMX_GRAM_F64, n, ka, kb, A, ka, B, kb, g64, s);
+    const int nout = ka * kb, ny = A1 ? 2 : 1, nb = bias ? kb : 0;
+    if (mode != 0) {
+        double *g64 = nullptr, *part = nullptr;
+        const uint32_t nblk = 512;
+        FMX_HIP(ctx, hipMalloc(&g64, ((size_t)nout + (size_t)nblk * kHid) * sizeof(double)));
+        part = g64 + nout;
+        fmx_status st = FMX_OK;
+        for (int y = 0; y < ny && !st; y++) {
+            st = gram(ctx, FMX_F32, FMX_GRAM_F64, n, ka, kb, y ? A1 : A0, ka, Z, kb, g64, s);
+            if (st) break;
+            hipLaunchKernelGGL(f64_to_f32, dim3(16), dim3(kT), 0, s, g64, out + y * nout, nout);
+        }
+        if (!st && bias) {
+            hipLaunchKernelGGL(colsum_kernel, dim3(nblk), dim3(kT), 0, s, Z, n, kb, (n + nblk - 1) / nblk, part);
+            hipLaunchKernelGGL(gnn_grad_reduce, dim3((nb + 15) / 16), dim3(kT), 0, s, nullptr, 0, nout, part, nb,
+                               (int)nblk, out + ny * nout);
+        }
+        if (!st && hipGetLastError() != hipSuccess) st = fail(ctx, FMX_EHIP, "gradient launch");
+        (void)hipStreamSynchronize(s);
+        (void)hipFree(g64);
+        return st;
+    }
+    // 256 blocks, more where the rows' bytes dwarf the partials'
+    const uint64_t blocks = std::min<uint64_t>((n + 127) / 128, std::max<uint64_t>(256, std::min<uint64_t>(n / 2048, 1024)));
+    const uint64_t rpb = blocks ? ((n + blocks - 1) / blocks + 127) / 128 * 128 : 128;
+    const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, (n + rpb - 1) / rpb);
+    const size_t fb = (size_t)ny * nblk * nout * sizeof(float);
+    void *ws = nullptr;
+    fmx_status st = ctx_scratch(ctx, fb + (size_t)nblk * kb * sizeof(double), &ws);
     if (st) return st;
-    hipLaunchKernelGGL(f64_to_f32, dim3(16), dim3(kT), 0, s, g64, out, ka * kb);
+    float *pa = (float *)ws;
+    double *pb = bias ? (double *)((char *)ws + fb) : nullptr;
+#define FMX_GRAD(TI, TJ)                                                                                       \
+    hipLaunchKernelGGL((gnn_grad_kernel<TI, TJ>), dim3(nblk, ny), dim3(kT), 0, s, A0, A1, Z, n, rpb, pa, pb)
+    if (kb == 64) {
+        if (ka == 64) FMX_GRAD(4, 4);
+        else FMX_GRAD(1, 4);
+    } else {
+        FMX_GRAD(4, 1);
+    }
+#undef FMX_GRAD
+    FMX_HIP(ctx, hipGetLastError());
+    hipLaunchKernelGGL(gnn_grad_reduce, dim3((ny * nout + nb + 15) / 16), dim3(kT), 0, s, pa, ny, nout, pb, nb,
+                       (int)nblk, out);
     FMX_HIP(ctx, hipGetLastError());
     return FMX_OK;
 }
@@ -310,22 +567,32 @@ fmx_status fmx_gnn_forward(fmx_ctx *ctx, const fmx_spm *spm, const double *dinv,
     hipStream_t s = (hipStream_t)stream;
     const uint64_t n = spm->nrows;
     const float *H = X0;
-    float *a = acts;
-    for (int l = 0; l < kLayers; l++) {
+    float *a = acts, *T = work;  // T: the next aggregation's operand, D^-1/2 H
+    fmx_status st = row_scale(ctx, FMX_F32, n, kIn, dinv, X0, kIn, T, kIn, s);
+    for (int l = 0; l < kLayers && !st; l++) {
         const int d = din_of(l);
         float *Agg = a;
         a += n * d;
         float *Hn = a;
         a += n * kHid;
-        fmx_status st = norm_agg(ctx, spm, dinv, H, d, work, Agg, s);
+        st = norm_agg(ctx, spm, dinv, T, d, Agg, s);
         if (st) return st;
         const float *Wl = P + layer_off(l);
-        st = gemm(ctx, mode, H, d, d, Agg, d, d, Wl, 0, kHid, Wl + 2 * (size_t)d * kHid, nullptr, 0, 1, Hn, kHid, n, s);
-        if (st) return st;
+        Epilogue ep;
+        ep.bias = Wl + 2 * (size_t)d * kHid;
+        ep.relu = 1;
+        ep.out = Hn;
+        if (l + 1 < kLayers) {
+            ep.scale = dinv;
+            ep.outs = T;
+        }
+        st = gemm(ctx, mode, H, d, Agg, d, Wl, 0, kHid, ep, n, s);
         H = Hn;
     }
-    return gemm(ctx, mode, H, kHid, kHid, nullptr, 0, 0, P + layer_off(kLayers), 0, kOut, nullptr, nullptr, 0, 0, Y,
-                kOut, n, s);
+    if (st) return st;
+    Epilogue ep;
+    ep.out = Y;
+    return gemm(ctx, mode, H, kHid, nullptr, 0, P + layer_off(kLayers), 0, kOut, ep, n, s);
 }
 
 fmx_status fmx_gnn_backward(fmx_ctx *ctx, const fmx_spm *spm, const double *dinv, const float *P,
@@ -347,44 +614,35 @@ fmx_status fmx_gnn_backward(fmx_ctx *ctx, const fmx_spm *spm, const double *dinv
         Hs[l + 1] = a;
         a += n * kHid;
     }
-    float *dH = work, *T = work + n * kHid, *T2 = work + 2 * n * kHid, *T3 = work + 3 * n * kHid;
-    double *g64 = nullptr, *part = nullptr;
-    FMX_HIP(ctx, hipMalloc(&g64, (size_t)kHid * kHid * sizeof(double)));
-    const uint32_t nblk = 512;
-    FMX_HIP(ctx, hipMalloc(&part, (size_t)nblk * kHid * sizeof(double)));
-    fmx_status st = FMX_OK;
+    float *dZ = work, *next = work + n * kHid, *T2 = work + 2 * n * kHid, *T3 = work + 3 * n * kHid;
     const float *Wo = P + layer_off(kLayers);
-    float *dWo = G + layer_off(kLayers);
-    st = gram_grad(ctx, mode, n, kHid, kOut, Hs[kLayers], dY, g64, dWo, s);
-    // dH3 = dY Wo^T  (Wo is 64 x 16 = dout x K)
-    if (!st) st = gemm(ctx, mode, dY, kOut, kOut, nullptr, 0, 0, Wo, 1, kHid, nullptr, nullptr, 0, 0, dH, kHid, n, s);
+    fmx_status st = grads(ctx, mode, n, kHid, kOut, Hs[kLayers], nullptr, dY, false, G + layer_off(kLayers), s);
+    {
+        // dZ_3 = (dY Wo^T) where H_3 > 0  (Wo is 64 x 16 = dout x K)
+        Epilogue ep;
+        ep.gate = Hs[kLayers];
+        ep.out = dZ;
+        if (!st) st = gemm(ctx, mode, dY, kOut, nullptr, 0, Wo, 1, kHid, ep, n, s);
+    }
     for (int l = kLayers - 1; l >= 0 && !st; l--) {
         const int d = din_of(l);
         const float *Wl = P + layer_off(l);
-        float *Gl = G + layer_off(l);
-        hipLaunchKernelGGL(relu_back_kernel, dim3(grid_n(ctx, n * kHid)), dim3(kT), 0, s, Hs[l + 1], dH, n * kHid);
-        if (hipGetLastError() != hipSuccess) { st = FMX_EHIP; break; }
-        st = gram_grad(ctx, mode, n, d, kHid, Hs[l], dH, g64, Gl, s);
-        if (!st) st = gram_grad(ctx, mode, n, d, kHid, Agg[l], dH, g64, Gl + (size_t)d * kHid, s);
-        if (!st) {
-            const uint64_t rpb = (n + nblk - 1) / nblk;
-            hipLaunchKernelGGL(colsum_kernel, dim3(nblk), dim3(kT), 0, s, dH, n, kHid, rpb, part);
-            hipLaunchKernelGGL(colsum_finish, dim3(1), dim3(kT), 0, s, part, (int)nblk, kHid,
-                               Gl + 2 * (size_t)d * kHid);
-            if (hipGetLastError() != hipSuccess) st = FMX_EHIP;
-        }
+        st = grads(ctx, mode, n, d, kHid, Hs[l], Agg[l], dZ, true, G + layer_off(l), s);
         if (st || l == 0) break;
-        // dH_l = dZ Ws^T + N (dZ Wn^T); Ws, Wn are d x 64 = dout x K
-        st = gemm(ctx, mode, dH, kHid, kHid, nullptr, 0, 0, Wl + (size_t)d * kHid, 1, d, nullptr, nullptr, 0, 0, T,
-                  d, n, s);
-        if (!st) st = norm_agg(ctx, spm, dinv, T, d, T2, T3, s);
-        if (!st) st = gemm(ctx, mode, dH, kHid, kHid, nullptr, 0, 0, Wl, 1, d, nullptr, T3, d, 0, T, d, n, s);
-        if (!st && hipMemcpyAsync(dH, T, n * d * sizeof(float), hipMemcpyDeviceToDevice, s) != hipSuccess)
-            st = FMX_EHIP;
+        // dZ_l = (dZ Ws^T + N (dZ Wn^T)) where H_l > 0; Ws, Wn are d x 64 = dout x K
+        Epilogue ea;
+        ea.scale = dinv;
+        ea.outs = T2;
+        st = gemm(ctx, mode, dZ, kHid, nullptr, 0, Wl + (size_t)d * kHid, 1, d, ea, n, s);
+        if (!st) st = norm_agg(ctx, spm, dinv, T2, d, T3, s);
+        Epilogue eb;
+        eb.add = T3;
+        eb.gate = Hs[l];
+        eb.out = next;
+        if (!st) st = gemm(ctx, mode, dZ, kHid, nullptr, 0, Wl, 1, d, eb, n, s);
+        std::swap(dZ, next);
     }
-    (void)hipStreamSynchronize(s);
-    (void)hipFree(g64);
-    (void)hipFree(part);
+    if (hipStreamSynchronize(s) != hipSuccess && !st) st = FMX_EHIP;
     return st ? fail(ctx, st, "gnn backward failed") : FMX_OK;
 }
 

@@ -58,6 +58,7 @@ struct SpmmArgs {
     int vwords;            // weighted images: u16 words per value (2 or 4)
     const double *rscale;  // floating-point data: Y row r is scaled by rscale[r] (or null)
     int ycol;              // Y column-major: element (r, j) at Y[j * ldy + r]
+    int round_first;       // a scaled row's sum is rounded to T before it is scaled
     const void *Xhot;      // gather-order images: rows of columns < nhot (leading dimension k)
     uint64_t nhot;         // columns c >= nhot are row c - nhot of X
     const void *Xcold;     // narrow forms: X - nhot rows, so that row c of it is column c >= nhot
@@ -627,6 +628,14 @@ __device__ __forceinline__ void drain_generic_seq(const SpmmArgs &a, T *band, ui
     }
 }
 
+// A row's sum times its output scale: rounded to T once, by the caller's
+// store, or (round_first) also before the scaling.
+template <typename T, typename A>
+__device__ __forceinline__ A scaled(int round_first, A sum, double scale)
+{
+    return (A)((round_first ? (double)(T)sum : (double)sum) * scale);
+}
+
 // The output scales of a band's first 128 rows, requested when the item
 // starts so that their latency is hidden by the item's work.
 struct RowScale {
@@ -678,7 +687,7 @@ __device__ __forceinline__ void write_band(const SpmmArgs &a, const A *band, uin
                 const uint32_t cc = i / rows, r = i - cc * rows;
                 A v = band[r * S + bcol(cc)];
                 if constexpr (std::is_floating_point<T>::value)
-                    if (a.rscale) v = (A)((double)v * (staged ? scratch[r] : a.rscale[row0 + r]));
+                    if (a.rscale) v = scaled<T>(a.round_first, v, staged ? scratch[r] : a.rscale[row0 + r]);
                 __builtin_nontemporal_store((T)v, &dc[cc * (uint64_t)a.ldy + r]);
             }
             return;
@@ -687,7 +696,7 @@ __device__ __forceinline__ void write_band(const SpmmArgs &a, const A *band, uin
             const uint32_t r = i / k, cc = i - r * k;
             A v = band[r * S + bcol(cc)];
             if constexpr (std::is_floating_point<T>::value)
-                if (a.rscale) v = (A)((double)v * (staged ? scratch[r] : a.rscale[row0 + r]));  // one rounding
+                if (a.rscale) v = scaled<T>(a.round_first, v, staged ? scratch[r] : a.rscale[row0 + r]);
             // written once and not read here: non-temporal
             __builtin_nontemporal_store((T)v, &dst[r * (uint64_t)a.ldy + cc]);
         }
@@ -899,7 +908,7 @@ __global__ void __launch_bounds__(64 * kWPB) __attribute__((amdgpu_waves_per_eu(
 template <typename T, typename A>
 __global__ void __launch_bounds__(256) spmm_reduce(const Split *splits, const A *partial,
                                                     uint32_t hs, uint32_t k, T *Y, int64_t ldy,
-                                                    const double *rscale, int ycol)
+                                                    const double *rscale, int ycol, int round_first)
 {
     const Split sp = splits[blockIdx.x];
     const uint32_t tot = sp.rows * k;
@@ -909,7 +918,7 @@ __global__ void __launch_bounds__(256) spmm_reduce(const Split *splits, const A 
             acc += partial[(uint64_t)(sp.slot_begin + s) * hs * k + i];
         uint32_t r = i / k, c = i - r * k;
         if constexpr (std::is_floating_point<T>::value)
-            if (rscale) acc = (A)((double)acc * rscale[sp.row0 + r]);
+            if (rscale) acc = scaled<T>(round_first, acc, rscale[sp.row0 + r]);
         if (ycol) Y[c * (uint64_t)ldy + sp.row0 + r] = (T)acc;
         else Y[(sp.row0 + r) * (uint64_t)ldy + c] = (T)acc;
     }
@@ -1066,6 +1075,7 @@ fmx_status launch_t(fmx_ctx *ctx, const fmx_spm *spm, const Plan *plan, int k,
     a.vwords = (int)(spm->esz / 2);
     a.rscale = rscale;
     a.ycol = (flags & FMX_SPMM_Y_COLMAJOR) ? 1 : 0;
+    a.round_first = (flags & kSpmmRoundFirst) ? 1 : 0;
     a.Xhot = Xhot;
     a.nhot = Xhot ? nhot : 0;
     // 16-byte vector gathers need aligned rows; otherwise the runtime-width path.
@@ -1085,7 +1095,8 @@ fmx_status launch_t(fmx_ctx *ctx, const fmx_spm *spm, const Plan *plan, int k,
     if (reduce && plan->nsplits) {
         using A = typename AccOf<T>::type;
         hipLaunchKernelGGL((spmm_reduce<T, A>), dim3(plan->nsplits), dim3(256), 0, stream,
-                           plan->d_splits, (const A *)partial, plan->hs, (uint32_t)k, (T *)Y, ldy, rscale, a.ycol);
+                           plan->d_splits, (const A *)partial, plan->hs, (uint32_t)k, (T *)Y, ldy, rscale, a.ycol,
+                           a.round_first);
         FMX_HIP(ctx, hipGetLastError());
     }
     return FMX_OK;

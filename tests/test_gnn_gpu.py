@@ -120,3 +120,65 @@ def test_dcsbm_generator_matches_oracle(fmx, orc):
         so, do = orc.dcsbm_edges(n, bstart, wtab, 20, n * 8, seed)
         assert np.array_equal(s.cpu().numpy().view(np.uint32), so)
         assert np.array_equal(d.cpu().numpy().view(np.uint32), do)
+
+
+@pytest.mark.parametrize("n", [1, 17, 200, 1031, 33000])
+def test_mfma_products_ragged_rows(fmx, n):
+    """The BF16 products and gradients at row counts around their tiles (16
+    rows a wave, 32 a gradient step, 128 a block step), against the same
+    network in FP64 with the operands of every product rounded to BF16.
+    dY is given, so nothing depends on the loss.  What remains is FP32
+    accumulation and the odd operand that rounds the other way: 1e-2 of each
+    block's largest value, as above."""
+    import torch
+    g = torch.Generator().manual_seed(n)
+    e = torch.randint(0, n, (2, 5 * n), generator=g).int()
+    spm = fmx.SparseMatrix.build(e[0].contiguous().cuda(), e[1].contiguous().cuda(), n=n, log2_h=7, log2_w=12,
+                                 flags=fmx.BUILD_DEDUP | fmx.BUILD_SYMMETRIZE)
+    r, c = torch.cat([e[0], e[1]]).long(), torch.cat([e[1], e[0]]).long()
+    key = torch.unique((r * n + c)[r != c])
+    r, c = key // n, key % n
+    deg = torch.bincount(r, minlength=n).double()
+    dinv = torch.where(deg > 0, deg.clamp(min=1).rsqrt(), torch.zeros_like(deg))
+    f32 = lambda x: x.float().double()
+    bf = lambda x: x.float().bfloat16().double()
+    spread = lambda x: torch.zeros_like(x).index_add_(0, r, x[c])
+    agg = lambda x: f32(f32(spread(f32(x * dinv[:, None]))) * dinv[:, None])
+    L, ctx = fmx.lib(), fmx.default_context()
+    P = (torch.randn(L.fmx_gnn_param_count(), generator=g) * 0.15)
+    X0, dY = torch.randn((n, 16), generator=g), torch.randn((n, 16), generator=g)
+    at, W = 0, []
+    for d in (16, 64, 64):
+        W.append((P[at:at + 64 * d].view(d, 64).double(), P[at + 64 * d:at + 128 * d].view(d, 64).double(),
+                  P[at + 128 * d:at + 128 * d + 64].double()))
+        at += 128 * d + 64
+    Wo = P[at:].view(64, 16).double()
+    Hs, Ag = [X0.double()], []
+    for Ws, Wn, b in W:
+        Ag.append(agg(Hs[-1]))
+        Hs.append(f32(torch.relu(bf(Hs[-1]) @ bf(Ws) + bf(Ag[-1]) @ bf(Wn) + b)))
+    want_Y = bf(Hs[3]) @ bf(Wo)
+    grads = [bf(Hs[3]).t() @ bf(dY)]
+    dZ = f32(bf(dY) @ bf(Wo).t()) * (Hs[3] > 0)
+    for l in (2, 1, 0):
+        Ws, Wn, _ = W[l]
+        grads[:0] = [bf(Hs[l]).t() @ bf(dZ), bf(Ag[l]).t() @ bf(dZ), dZ.sum(0)]
+        if l:
+            dZ = f32(bf(dZ) @ bf(Ws).t() + agg(f32(bf(dZ) @ bf(Wn).t()))) * (Hs[l] > 0)
+    acts = torch.empty(L.fmx_gnn_acts_floats(n), device="cuda")
+    work = torch.empty(L.fmx_gnn_work_floats(n), device="cuda")
+    Y, G = torch.empty((n, 16), device="cuda"), torch.full((P.numel(),), 7.0, device="cuda")
+    X0d, dYd, Pd, dv = X0.cuda(), dY.cuda(), P.cuda(), dinv.cuda()
+    ctx.check(L.fmx_gnn_forward(ctx.handle, spm.handle, dv.data_ptr(), Pd.data_ptr(), X0d.data_ptr(),
+                                acts.data_ptr(), Y.data_ptr(), work.data_ptr(), 0, None), "forward")
+    ctx.check(L.fmx_gnn_backward(ctx.handle, spm.handle, dv.data_ptr(), Pd.data_ptr(), X0d.data_ptr(),
+                                 acts.data_ptr(), dYd.data_ptr(), G.data_ptr(), work.data_ptr(), 0, None), "backward")
+    torch.cuda.synchronize()
+    assert (Y.cpu().double() - want_Y).abs().max() <= 1e-2 * want_Y.abs().max()
+    got = G.cpu().double()
+    at = 0
+    for w in grads:
+        part = got[at:at + w.numel()].view(w.shape)
+        assert (part - w).abs().max() <= 1e-2 * w.abs().max() + 1e-12, (at, w.shape)
+        at += w.numel()
+    assert at == got.numel()
