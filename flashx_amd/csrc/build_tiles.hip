@@ -46,6 +46,8 @@ struct KeyFmt {
     }
     __host__ __device__ uint32_t rrel(uint64_t k) const { return (uint32_t)((k >> lw) & (H - 1)); }
     __host__ __device__ uint32_t crel(uint64_t k) const { return (uint32_t)(k & (W - 1)); }
+    __host__ __device__ uint32_t row(uint64_t k) const { return br(k) << lh | rrel(k); }
+    __host__ __device__ uint32_t col(uint64_t k) const { return bc(k) << lw | crel(k); }
 };
 
 __device__ __forceinline__ uint64_t gtid() { return blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; }
@@ -149,6 +151,37 @@ __global__ void __launch_bounds__(kB) emit_keys_w(const uint32_t *src, const uin
             keys[p + 1] = f.key(b, a);
             eidx[p + 1] = (uint32_t)i;
         }
+    }
+}
+
+// The same non-zeros' keys in another image's format: column c becomes
+// newid[c], or stays c without one.
+__global__ void __launch_bounds__(kB) rekey(const uint64_t *k, uint64_t n, KeyFmt f, KeyFmt g, const uint32_t *newid,
+                                            uint64_t *out)
+{
+    for (uint64_t i = gtid(); i < n; i += gstride()) {
+        const uint64_t key = k[i];
+        const uint32_t r = f.row(key), c = f.col(key);
+        out[i] = g.key(r, newid ? newid[c] : c);
+    }
+}
+
+// Non-zeros per column, counted in `copies` copies of the counters (of ncols
+// words each): adds to one word pass one by one, some 5 ns each, and a
+// power-law graph's most used column takes one in a few hundred of all.
+__global__ void __launch_bounds__(kB) count_columns(const uint64_t *k, uint64_t n, KeyFmt f, uint32_t *uses,
+                                                    uint64_t ncols, uint32_t copies)
+{
+    uint32_t *u = uses + (uint64_t)(blockIdx.x % copies) * ncols;
+    for (uint64_t i = gtid(); i < n; i += gstride()) atomicAdd(&u[f.col(k[i])], 1u);
+}
+
+__global__ void __launch_bounds__(kB) add_copies(uint32_t *uses, uint64_t ncols, uint32_t copies)
+{
+    for (uint64_t c = gtid(); c < ncols; c += gstride()) {
+        uint32_t t = 0;
+        for (uint32_t q = 0; q < copies; q++) t += uses[(uint64_t)q * ncols + c];
+        uses[c] = t;
     }
 }
 
@@ -414,155 +447,32 @@ uint32_t grid_for(fmx_ctx *ctx, uint64_t n)
     return (uint32_t)(b ? b : 1);
 }
 
-}  // namespace
-
-
-}  // namespace fmx
-
-using namespace fmx;
-
-namespace fmx {
-
-// vals (device, esz bytes per edge) != nullptr builds a weighted image.
-// ncols != 0 builds an nrows = n by ncols matrix (ids below max(n, ncols);
-// the library's own work images); internal skips the work images of the
-// result.
-fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, size_t m, uint64_t n,
-                      uint32_t log2_h, uint32_t log2_w, uint32_t flags, const void *vals, uint32_t esz,
-                      int32_t prim_type, fmx_spm **out, uint64_t ncols, bool internal)
+KeyFmt key_fmt(uint32_t log2_h, uint32_t log2_w, uint64_t ncols)
 {
-    if (!ctx || !out) return fail(ctx, FMX_EINVAL, "null argument");
-    *out = nullptr;
-    if (m && (!src || !dst)) return fail(ctx, FMX_EINVAL, "null edge list");
-    if (log2_h > 15 || log2_w > 15) return fail(ctx, FMX_EINVAL, "tile dimensions must be <= 32768");
-    if (flags & ~7u) return fail(ctx, FMX_EINVAL, "unknown build flags");
-    FMX_HIP(ctx, hipSetDevice(ctx->device));
-    // the edge list may come from any stream: construction is synchronous
-    FMX_HIP(ctx, hipDeviceSynchronize());
-    hipStream_t s = ctx->stream;
-    // device time of the construction, from the first kernel to the last
-    // write (host waits for totals in between are included)
-    struct EvPair {
-        hipEvent_t a = nullptr, b = nullptr;
-        ~EvPair()
-        {
-            if (a) (void)hipEventDestroy(a);
-            if (b) (void)hipEventDestroy(b);
-        }
-    } ev;
-    FMX_HIP(ctx, hipEventCreate(&ev.a));
-    FMX_HIP(ctx, hipEventCreate(&ev.b));
-    FMX_HIP(ctx, hipEventRecord(ev.a, s));
-
-    // n = max id + 1 (fm_utils.cpp:730-739), or a caller-given n above every id
-    if (m) {
-        uint32_t mx = 0;
-        fmx_status st = max_u32_pair(ctx, src, dst, m, &mx, s);
-        if (st) return st;
-        if (n == 0) n = (uint64_t)mx + 1;
-        else if ((uint64_t)mx >= std::max(n, ncols)) return fail(ctx, FMX_EDIM, "vertex id >= n");
-    } else if (n == 0) {
-        return fail(ctx, FMX_EINVAL, "empty edge list needs an explicit n");
-    }
-    if (ncols == 0) ncols = n;
-    if (n > (1ull << 32) || ncols > (1ull << 32)) return fail(ctx, FMX_EINVAL, "n exceeds 2^32");
-    const uint64_t H = 1ull << log2_h, W = 1ull << log2_w;
-    const uint64_t nbr = (n + H - 1) / H, nbc = (ncols + W - 1) / W;
     KeyFmt f;
     f.lh = (int)log2_h;
     f.lw = (int)log2_w;
-    f.bbc = bits_for(nbc);
-    f.H = (uint32_t)H;
-    f.W = (uint32_t)W;
-    const int keybits = bits_for(nbr) + f.bbc + f.lh + f.lw;
-    const int sym = (flags & FMX_BUILD_SYMMETRIZE) != 0;
-    const uint64_t cap = sym ? 2 * (uint64_t)m : (uint64_t)m;
+    f.H = 1u << log2_h;
+    f.W = 1u << log2_w;
+    f.bbc = bits_for((ncols + f.W - 1) / f.W);
+    return f;
+}
 
-    // 1. keys (weighted: in edge order, with the edge index as payload)
-    const int keep_self = (flags & FMX_BUILD_KEEP_SELF) ? 1 : 0;
-    DevBuf<uint64_t> keys, tmp;
-    DevBuf<uint32_t> eidx, etmp;
-    DevBuf<unsigned long long> counter;
-    FMX_HIP(ctx, keys.alloc(cap));
-    FMX_HIP(ctx, tmp.alloc(cap));
-    FMX_HIP(ctx, counter.alloc(1));
-    FMX_HIP(ctx, hipMemsetAsync(counter.p, 0, sizeof(unsigned long long), s));
-    unsigned long long nk64 = 0;
+// Steps 3 to 6: the image of the nk sorted keys K, an n x ncols matrix;
+// weighted (vals): V[i] is the edge whose value non-zero i takes.  done is
+// recorded behind the last kernel.
+fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint64_t nk, const KeyFmt &f, uint64_t n,
+                       uint64_t ncols, const void *vals, uint32_t esz, int32_t prim_type, hipEvent_t done,
+                       std::unique_ptr<fmx_spm> &out)
+{
+    hipStream_t s = ctx->stream;
+    const uint64_t H = f.H, W = f.W;
+    const uint64_t nbr = (n + H - 1) / H, nbc = (ncols + W - 1) / W;
+    // 3. runs
     fmx_status st = FMX_OK;
-    if (vals) {
-        if (m >= (1ull << 31)) return fail(ctx, FMX_EUNSUPPORTED, "weighted builds take fewer than 2^31 edges");
-        FMX_HIP(ctx, eidx.alloc(cap));
-        FMX_HIP(ctx, etmp.alloc(cap));
-        DevBuf<uint32_t> pos;
-        FMX_HIP(ctx, pos.alloc((uint64_t)m + 1));
-        uint32_t total = 0;
-        if (m) {
-            hipLaunchKernelGGL(count_keys_w, dim3(grid_for(ctx, m)), dim3(kB), 0, s, src, dst, (uint64_t)m,
-                               keep_self, sym, pos.p);
-            FMX_HIP(ctx, hipGetLastError());
-            st = scan_exclusive<uint32_t>(ctx, pos.p, pos.p, m, &total, s);
-            if (st) return st;
-            hipLaunchKernelGGL(emit_keys_w, dim3(grid_for(ctx, m)), dim3(kB), 0, s, src, dst, (uint64_t)m, f,
-                               keep_self, sym, pos.p, keys.p, eidx.p);
-            FMX_HIP(ctx, hipGetLastError());
-        }
-        nk64 = total;
-    } else {
-        if (m) {
-            hipLaunchKernelGGL(make_keys, dim3(grid_for(ctx, m)), dim3(kB), 0, s, src, dst, (uint64_t)m, f,
-                               keep_self, sym, keys.p, counter.p);
-            FMX_HIP(ctx, hipGetLastError());
-        }
-        FMX_HIP(ctx, hipMemcpyAsync(&nk64, counter.p, sizeof(nk64), hipMemcpyDeviceToHost, s));
-        FMX_HIP(ctx, hipStreamSynchronize(s));
-    }
-    if (nk64 >= (1ull << 32)) return fail(ctx, FMX_EUNSUPPORTED, "more than 2^32 - 1 non-zeros");
-
-    // 2. sort + unique (a stable sort: equal keys keep edge order)
-    uint64_t *K = keys.p;
-    uint32_t *V = eidx.p;
-    st = radix_sort_u64_kv(ctx, keys.p, tmp.p, vals ? eidx.p : nullptr, vals ? etmp.p : nullptr, nk64, keybits,
-                           &K, &V, s);
-    if (st) return st;
-    uint64_t *other = (K == keys.p) ? tmp.p : keys.p;
-    uint32_t *vother = (V == eidx.p) ? etmp.p : eidx.p;
-    uint64_t nk = nk64;
+    uint32_t R = 0;
     DevBuf<uint32_t> flag;
     FMX_HIP(ctx, flag.alloc(nk + 1));
-    if ((flags & FMX_BUILD_DEDUP) && nk) {
-        hipLaunchKernelGGL(group_flags, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, 0, flag.p);
-        FMX_HIP(ctx, hipGetLastError());
-        uint32_t nu = 0;
-        st = scan_exclusive<uint32_t>(ctx, flag.p, flag.p, nk, &nu, s);
-        if (st) return st;
-        if (vals) {
-            hipLaunchKernelGGL(compact_unique_kv, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, V, nk, flag.p,
-                               other, vother);
-            V = vother;
-        } else {
-            hipLaunchKernelGGL(compact_unique, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, flag.p, other);
-        }
-        FMX_HIP(ctx, hipGetLastError());
-        K = other;
-        nk = nu;
-    }
-    // the key (and payload) buffer that does not hold the result is not read
-    // again: its memory goes back before the run and tile arrays are made
-    // (17 GB at 2^31 edges)
-    FMX_HIP(ctx, hipStreamSynchronize(s));
-    for (DevBuf<uint64_t> *b : {&keys, &tmp})
-        if (b->p && b->p != K) {
-            FMX_HIP(ctx, hipFree(b->p));
-            b->p = nullptr;
-        }
-    for (DevBuf<uint32_t> *b : {&eidx, &etmp})
-        if (b->p && b->p != V) {
-            FMX_HIP(ctx, hipFree(b->p));
-            b->p = nullptr;
-        }
-
-    // 3. runs
-    uint32_t R = 0;
     if (nk) {
         hipLaunchKernelGGL(group_flags, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, f.lw, flag.p);
         FMX_HIP(ctx, hipGetLastError());
@@ -687,7 +597,7 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
     hipLaunchKernelGGL(check_dir, dim3(grid_for(ctx, nbr)), dim3(kB), 0, s, spm->d_dir, spm->d_vdir, bdir.p,
                        offs_ex.p, nbr, nbc, (uint64_t)ndir, vals ? 1 : 0, bad.p);
     FMX_HIP(ctx, hipGetLastError());
-    FMX_HIP(ctx, hipEventRecord(ev.b, s));
+    if (done) FMX_HIP(ctx, hipEventRecord(done, s));
     // the host keeps the block-row offsets and first directory indices; the
     // directory itself stays in HBM (plans copy the few block rows they split)
     std::vector<uint64_t> oex(nbr + 1);
@@ -698,10 +608,6 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
     FMX_HIP(ctx, hipMemcpyAsync(&hbad, bad.p, sizeof(unsigned int), hipMemcpyDeviceToHost, s));
     FMX_HIP(ctx, hipStreamSynchronize(s));
     if (hbad) return fail(ctx, FMX_EINVAL, "internal error: inconsistent device-built directory");
-    float build_ms = 0.f;
-    FMX_HIP(ctx, hipEventElapsedTime(&build_ms, ev.a, ev.b));
-    spm->build_ns = (uint64_t)((double)build_ms * 1e6);
-    spm->edges_in = m;
     spm->offs.resize(nbr + 1);
     for (uint64_t b = 0; b <= nbr; b++) spm->offs[b] = (int64_t)(4096 + oex[b]);
     spm->bytes = bytes;
@@ -710,16 +616,231 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
     spm->nnz = nk;
     spm->H = H;
     spm->W = W;
-    spm->log2h = (int)log2_h;
-    spm->log2w = (int)log2_w;
+    spm->log2h = f.lh;
+    spm->log2w = f.lw;
     spm->nbr = nbr;
     spm->nbc = nbc;
     spm->esz = vals ? esz : 0;
     spm->prim = vals ? prim_type : 0;
     spm->ntiles = ndir;
+    out = std::move(spm);
+    return FMX_OK;
+}
+
+// The work images of a matrix from its own keys (K, V: nk sorted keys in
+// format f and, if weighted, their edges; vals: the edges' values).  Re-cut
+// (tiles taller than an SpMM band): the keys are in order inside each of the
+// new block rows already, so a stable sort by block row is all they need.
+// Gather order: the columns' uses are counted and ranked, and the relabelled
+// keys sorted anew.
+fmx_status work_images(fmx_ctx *ctx, fmx_spm *spm, const uint64_t *K, const uint32_t *V, const KeyFmt &f,
+                       const void *vals)
+{
+    hipStream_t s = ctx->stream;
+    const uint64_t nk = spm->nnz;
+    const uint32_t h2 = work_rows_for(spm);
+    const bool fast = wants_fast(spm);
+    if (!h2 && !fast) return FMX_OK;
+    DevBuf<uint64_t> keys, tmp;
+    DevBuf<uint32_t> va, vb;
+    FMX_HIP(ctx, keys.alloc(nk));
+    FMX_HIP(ctx, tmp.alloc(nk));
+    if (vals) {
+        FMX_HIP(ctx, va.alloc(nk));
+        FMX_HIP(ctx, vb.alloc(nk));
+    }
+    auto image = [&](uint32_t log2_h, uint32_t log2_w, uint64_t ncols, const uint32_t *newid, bool in_order,
+                     std::unique_ptr<fmx_spm> &out) -> fmx_status {
+        const KeyFmt g = key_fmt(log2_h, log2_w, ncols);
+        const int low = g.lh + g.lw + g.bbc;
+        uint64_t *k2 = keys.p;
+        uint32_t *v2 = va.p;
+        if (nk) {
+            hipLaunchKernelGGL(rekey, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, f, g, newid, keys.p);
+            FMX_HIP(ctx, hipGetLastError());
+            if (vals) FMX_HIP(ctx, hipMemcpyAsync(va.p, V, nk * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
+        }
+        fmx_status st = radix_sort_u64_kv(ctx, keys.p, tmp.p, vals ? va.p : nullptr, vals ? vb.p : nullptr, nk,
+                                          in_order ? low : 0, low + bits_for((spm->nrows + g.H - 1) / g.H), &k2, &v2,
+                                          s);
+        if (!st) st = write_image(ctx, k2, v2, nk, g, spm->nrows, ncols, vals, (uint32_t)spm->esz, spm->prim, nullptr,
+                                  out);
+        return st;
+    };
+    if (h2) {
+        fmx_status st = image((uint32_t)bits_for(h2), (uint32_t)spm->log2w, spm->ncols, nullptr, true, spm->work);
+        if (st) return st;
+    }
+    if (!fast) return FMX_OK;
+    DevBuf<uint32_t> newid, hot;
+    uint64_t nhot = 0;
+    {
+        const uint32_t copies = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, (16ull << 20) / spm->ncols));
+        DevBuf<uint32_t> uses;
+        FMX_HIP(ctx, uses.alloc(spm->ncols * copies));
+        FMX_HIP(ctx, hipMemsetAsync(uses.p, 0, spm->ncols * copies * sizeof(uint32_t), s));
+        hipLaunchKernelGGL(count_columns, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, f, uses.p, spm->ncols, copies);
+        hipLaunchKernelGGL(add_copies, dim3(grid_for(ctx, spm->ncols)), dim3(kB), 0, s, uses.p, spm->ncols, copies);
+        FMX_HIP(ctx, hipGetLastError());
+        fmx_status st = rank_columns(ctx, uses.p, spm->ncols, nk, hot_permille(), &newid.p, &hot.p, &nhot);
+        if (st || !nhot) return st;
+    }
+    fmx_status st = image(fast_log2_rows(spm), 15, nhot + spm->ncols, newid.p, false, spm->fast);
+    if (st) return st;
+    spm->d_hot = hot.release();
+    spm->nhot = nhot;
+    return FMX_OK;
+}
+
+}  // namespace
+
+
+}  // namespace fmx
+
+using namespace fmx;
+
+namespace fmx {
+
+// vals (device, esz bytes per edge) != nullptr builds a weighted image.
+// ncols != 0 builds an nrows = n by ncols matrix (ids below max(n, ncols);
+// the library's own work images); internal skips the work images of the
+// result.
+fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, size_t m, uint64_t n,
+                      uint32_t log2_h, uint32_t log2_w, uint32_t flags, const void *vals, uint32_t esz,
+                      int32_t prim_type, fmx_spm **out, uint64_t ncols, bool internal)
+{
+    if (!ctx || !out) return fail(ctx, FMX_EINVAL, "null argument");
+    *out = nullptr;
+    if (m && (!src || !dst)) return fail(ctx, FMX_EINVAL, "null edge list");
+    if (log2_h > 15 || log2_w > 15) return fail(ctx, FMX_EINVAL, "tile dimensions must be <= 32768");
+    if (flags & ~7u) return fail(ctx, FMX_EINVAL, "unknown build flags");
+    FMX_HIP(ctx, hipSetDevice(ctx->device));
+    // the edge list may come from any stream: construction is synchronous
+    FMX_HIP(ctx, hipDeviceSynchronize());
+    hipStream_t s = ctx->stream;
+    // device time of the construction, from the first kernel to the last
+    // write (host waits for totals in between are included)
+    struct EvPair {
+        hipEvent_t a = nullptr, b = nullptr;
+        ~EvPair()
+        {
+            if (a) (void)hipEventDestroy(a);
+            if (b) (void)hipEventDestroy(b);
+        }
+    } ev;
+    FMX_HIP(ctx, hipEventCreate(&ev.a));
+    FMX_HIP(ctx, hipEventCreate(&ev.b));
+    FMX_HIP(ctx, hipEventRecord(ev.a, s));
+
+    // n = max id + 1 (fm_utils.cpp:730-739), or a caller-given n above every id
+    if (m && !internal) {
+        uint32_t mx = 0;
+        fmx_status st = max_u32_pair(ctx, src, dst, m, &mx, s);
+        if (st) return st;
+        if (n == 0) n = (uint64_t)mx + 1;
+        else if ((uint64_t)mx >= std::max(n, ncols)) return fail(ctx, FMX_EDIM, "vertex id >= n");
+    } else if (n == 0) {
+        return fail(ctx, FMX_EINVAL, "empty edge list needs an explicit n");
+    }
+    if (ncols == 0) ncols = n;
+    if (n > (1ull << 32) || ncols > (1ull << 32)) return fail(ctx, FMX_EINVAL, "n exceeds 2^32");
+    const KeyFmt f = key_fmt(log2_h, log2_w, ncols);
+    const int keybits = bits_for((n + f.H - 1) / f.H) + f.bbc + f.lh + f.lw;
+    const int sym = (flags & FMX_BUILD_SYMMETRIZE) != 0;
+    const uint64_t cap = sym ? 2 * (uint64_t)m : (uint64_t)m;
+
+    // 1. keys (weighted: in edge order, with the edge index as payload)
+    const int keep_self = (flags & FMX_BUILD_KEEP_SELF) ? 1 : 0;
+    DevBuf<uint64_t> keys, tmp;
+    DevBuf<uint32_t> eidx, etmp;
+    DevBuf<unsigned long long> counter;
+    FMX_HIP(ctx, keys.alloc(cap));
+    FMX_HIP(ctx, tmp.alloc(cap));
+    FMX_HIP(ctx, counter.alloc(1));
+    FMX_HIP(ctx, hipMemsetAsync(counter.p, 0, sizeof(unsigned long long), s));
+    unsigned long long nk64 = 0;
+    fmx_status st = FMX_OK;
+    if (vals) {
+        if (m >= (1ull << 31)) return fail(ctx, FMX_EUNSUPPORTED, "weighted builds take fewer than 2^31 edges");
+        FMX_HIP(ctx, eidx.alloc(cap));
+        FMX_HIP(ctx, etmp.alloc(cap));
+        DevBuf<uint32_t> pos;
+        FMX_HIP(ctx, pos.alloc((uint64_t)m + 1));
+        uint32_t total = 0;
+        if (m) {
+            hipLaunchKernelGGL(count_keys_w, dim3(grid_for(ctx, m)), dim3(kB), 0, s, src, dst, (uint64_t)m,
+                               keep_self, sym, pos.p);
+            FMX_HIP(ctx, hipGetLastError());
+            st = scan_exclusive<uint32_t>(ctx, pos.p, pos.p, m, &total, s);
+            if (st) return st;
+            hipLaunchKernelGGL(emit_keys_w, dim3(grid_for(ctx, m)), dim3(kB), 0, s, src, dst, (uint64_t)m, f,
+                               keep_self, sym, pos.p, keys.p, eidx.p);
+            FMX_HIP(ctx, hipGetLastError());
+        }
+        nk64 = total;
+    } else {
+        if (m) {
+            hipLaunchKernelGGL(make_keys, dim3(grid_for(ctx, m)), dim3(kB), 0, s, src, dst, (uint64_t)m, f,
+                               keep_self, sym, keys.p, counter.p);
+            FMX_HIP(ctx, hipGetLastError());
+        }
+        FMX_HIP(ctx, hipMemcpyAsync(&nk64, counter.p, sizeof(nk64), hipMemcpyDeviceToHost, s));
+        FMX_HIP(ctx, hipStreamSynchronize(s));
+    }
+    if (nk64 >= (1ull << 32)) return fail(ctx, FMX_EUNSUPPORTED, "more than 2^32 - 1 non-zeros");
+
+    // 2. sort + unique (a stable sort: equal keys keep edge order)
+    uint64_t *K = keys.p;
+    uint32_t *V = eidx.p;
+    st = radix_sort_u64_kv(ctx, keys.p, tmp.p, vals ? eidx.p : nullptr, vals ? etmp.p : nullptr, nk64, 0,
+                           keybits, &K, &V, s);
+    if (st) return st;
+    uint64_t *other = (K == keys.p) ? tmp.p : keys.p;
+    uint32_t *vother = (V == eidx.p) ? etmp.p : eidx.p;
+    uint64_t nk = nk64;
+    if ((flags & FMX_BUILD_DEDUP) && nk) {
+        DevBuf<uint32_t> flag;
+        FMX_HIP(ctx, flag.alloc(nk + 1));
+        hipLaunchKernelGGL(group_flags, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, 0, flag.p);
+        FMX_HIP(ctx, hipGetLastError());
+        uint32_t nu = 0;
+        st = scan_exclusive<uint32_t>(ctx, flag.p, flag.p, nk, &nu, s);
+        if (st) return st;
+        if (vals) {
+            hipLaunchKernelGGL(compact_unique_kv, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, V, nk, flag.p,
+                               other, vother);
+            V = vother;
+        } else {
+            hipLaunchKernelGGL(compact_unique, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, flag.p, other);
+        }
+        FMX_HIP(ctx, hipGetLastError());
+        K = other;
+        nk = nu;
+    }
+    // the key (and payload) buffer that does not hold the result is not read
+    // again: its memory goes back before the run and tile arrays are made
+    // (17 GB at 2^31 edges)
+    FMX_HIP(ctx, hipStreamSynchronize(s));
+    for (DevBuf<uint64_t> *b : {&keys, &tmp})
+        if (b->p && b->p != K) {
+            FMX_HIP(ctx, hipFree(b->p));
+            b->p = nullptr;
+        }
+    for (DevBuf<uint32_t> *b : {&eidx, &etmp})
+        if (b->p && b->p != V) {
+            FMX_HIP(ctx, hipFree(b->p));
+            b->p = nullptr;
+        }
+
+    std::unique_ptr<fmx_spm> spm;
+    st = write_image(ctx, K, V, nk, f, n, ncols, vals, esz, prim_type, ev.b, spm);
+    if (st) return st;
+    float build_ms = 0.f;
+    FMX_HIP(ctx, hipEventElapsedTime(&build_ms, ev.a, ev.b));
+    spm->build_ns = (uint64_t)((double)build_ms * 1e6);
+    spm->edges_in = m;
     if (!internal) {
-        st = prepare_work(ctx, spm.get());
-        if (!st) st = prepare_fast(ctx, spm.get());
+        st = work_images(ctx, spm.get(), K, V, f, vals);
         if (st) return st;
     }
     *out = spm.release();

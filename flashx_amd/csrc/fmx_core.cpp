@@ -487,37 +487,6 @@ fmx_status prepare_work(fmx_ctx *ctx, fmx_spm *s)
 {
     const uint32_t h2 = work_rows_for(s);
     if (!h2) return FMX_OK;
-    if (!s->host_bytes() && s->d_image) {
-        // built on the device, without a host copy: the non-zeros listed in
-        // stream order and built again in h2-row tiles (every entry as it
-        // is, so the result is the re-cut of the same image)
-        struct Lists {
-            uint32_t *rows = nullptr, *cols = nullptr;
-            void *vals = nullptr;
-            ~Lists()
-            {
-                if (rows) (void)hipFree(rows);
-                if (cols) (void)hipFree(cols);
-                if (vals) (void)hipFree(vals);
-            }
-        } l;
-        const uint64_t nz = s->nnz ? s->nnz : 1;
-        if (hipMalloc(&l.rows, nz * 4) != hipSuccess || hipMalloc(&l.cols, nz * 4) != hipSuccess ||
-            (s->esz && hipMalloc(&l.vals, nz * s->esz) != hipSuccess))
-            return fail(ctx, FMX_ENOMEM, "re-cut work image");
-        fmx_status st = decode_lists(ctx, s, l.rows, l.cols, l.vals, nullptr);
-        if (st) return st;
-        int lh2 = 0;
-        while ((1u << lh2) < h2) lh2++;
-        fmx_spm *w = nullptr;
-        st = build_impl(ctx, l.rows, l.cols, s->nnz, s->nrows, (uint32_t)lh2, (uint32_t)s->log2w, FMX_BUILD_KEEP_SELF,
-                        s->esz ? l.vals : nullptr, (uint32_t)s->esz, s->prim, &w, s->ncols, true);
-        if (st) return st;
-        std::unique_ptr<fmx_spm> wp(w);
-        if (wp->nnz != s->nnz) return fail(ctx, FMX_EINVAL, "internal error: the re-cut work image lost non-zeros");
-        s->work = std::move(wp);
-        return FMX_OK;
-    }
     std::unique_ptr<fmx_spm> w(new fmx_spm());
     w->ctx = ctx;
     retile_image(s, h2, w->h_image, w->offs);

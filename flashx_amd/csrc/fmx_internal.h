@@ -153,7 +153,8 @@ int elem_size(fmx_dtype dt);
 // Validates a host image and fills the matrix fields + directory.
 fmx_status analyse_image(fmx_ctx *ctx, fmx_spm *spm);
 // Device construction (build_tiles.hip); ncols != 0: an n x ncols matrix;
-// internal: the result gets no work images of its own.
+// internal: a work image of another matrix, whose ids are known to be in
+// range and which gets no work images of its own.
 fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, size_t m, uint64_t n,
                       uint32_t log2_h, uint32_t log2_w, uint32_t flags, const void *vals, uint32_t esz,
                       int32_t prim_type, fmx_spm **out, uint64_t ncols, bool internal);
@@ -162,6 +163,17 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
 // stream_chunk != 0: the image is streamed from pinned host memory in
 // chunks of that many bytes, as the matrix it belongs to.
 fmx_status prepare_fast(fmx_ctx *ctx, fmx_spm *spm, uint64_t stream_chunk = 0);
+// The gather order of ncols columns with the given uses (device; image_dev.hip):
+// *newid (device, allocated here) maps a column to its new id, *hot lists the
+// nhot columns that cover `permille` of the nnz non-zeros in their new order.
+// *nhot = 0 (and nothing allocated) when there are none.  On ctx->stream.
+fmx_status rank_columns(fmx_ctx *ctx, const uint32_t *uses, uint64_t ncols, uint64_t nnz, uint64_t permille,
+                        uint32_t **newid, uint32_t **hot, uint64_t *nhot);
+// The share of the non-zeros that the hot columns of a gather-order image
+// cover, and its tile height; whether a matrix gets one.
+uint64_t hot_permille();
+uint32_t fast_log2_rows(const fmx_spm *spm);
+bool wants_fast(const fmx_spm *spm);
 // The non-zeros of the image in HBM of src (image_dev.hip) in stream order
 // into device lists rows, cols (relabelled into gather order) and vals (esz
 // bytes each, if weighted); *hot (device, allocated here) lists the nhot

@@ -18,11 +18,13 @@
 // sums in the reference's column order and keeps using the image in that
 // order.
 //
-// The image is built once, when the matrix is created: the column degrees
-// and the relabelled (row, column[, value]) list come from the image in HBM
-// (image_dev.hip) or, for a matrix streamed from host memory, from its
-// host copy (below); the device builder (build_tiles.hip) then writes the
-// new image in tiles of at most 64 rows by 32768 columns.
+// The image is built once, when the matrix is created, in tiles of at most
+// 64 rows by 32768 columns.  A matrix built on the device counts and relabels
+// the columns of the sorted keys it was written from (build_tiles.hip).  For
+// an uploaded matrix the column degrees and the relabelled (row, column[,
+// value]) list come from the image in HBM (image_dev.hip), for one streamed
+// from host memory from its host copy (below), and the device builder writes
+// the new image from that list.
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -175,14 +177,26 @@ fmx_status host_lists(fmx_ctx *ctx, const fmx_spm *src, uint64_t ncols, uint64_t
 
 }  // namespace
 
-fmx_status prepare_fast(fmx_ctx *ctx, fmx_spm *s, uint64_t stream_chunk)
+bool wants_fast(const fmx_spm *s)
 {
     const char *e = getenv("FMX_HOT_COLS");  // "0" turns the gather-order image off
-    if ((e && !strcmp(e, "0")) || s->nnz == 0 || s->nnz >= (1ull << 31)) return FMX_OK;
-    const fmx_spm *src = s->work ? s->work.get() : s;  // either walks the same non-zeros
-    // the share of the non-zeros the hot columns cover (FMX_HOT_PERMILLE)
+    return !(e && !strcmp(e, "0")) && s->nnz != 0 && s->nnz < (1ull << 31);
+}
+
+// the share of the non-zeros the hot columns cover (FMX_HOT_PERMILLE)
+uint64_t hot_permille()
+{
     const char *pm = getenv("FMX_HOT_PERMILLE");
-    const uint64_t permille = std::min<uint64_t>(1000, pm ? strtoull(pm, nullptr, 10) : 950);
+    return std::min<uint64_t>(1000, pm ? strtoull(pm, nullptr, 10) : 950);
+}
+
+uint32_t fast_log2_rows(const fmx_spm *s) { return (uint32_t)std::min(s->log2h, 6); }
+
+fmx_status prepare_fast(fmx_ctx *ctx, fmx_spm *s, uint64_t stream_chunk)
+{
+    if (!wants_fast(s)) return FMX_OK;
+    const fmx_spm *src = s->work ? s->work.get() : s;  // either walks the same non-zeros
+    const uint64_t permille = hot_permille();
     struct Lists {
         uint32_t *rows = nullptr, *cols = nullptr, *hot = nullptr;
         void *vals = nullptr;
@@ -204,7 +218,7 @@ fmx_status prepare_fast(fmx_ctx *ctx, fmx_spm *s, uint64_t stream_chunk)
     if (st || nhot == 0) return st;
     fmx_spm *f = nullptr;
     {
-        const uint32_t lh = (uint32_t)std::min(s->log2h, 6), lw = 15;
+        const uint32_t lh = fast_log2_rows(s), lw = 15;
         // every non-zero as it is: self edges kept, duplicates kept (in
         // stream order, so a weighted row keeps its value order)
         st = build_impl(ctx, l.rows, l.cols, s->nnz, s->nrows, lh, lw, FMX_BUILD_KEEP_SELF,

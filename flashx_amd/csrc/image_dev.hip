@@ -1,7 +1,6 @@
-// image_dev.hip -- walks of an image resident in HBM, on the device.  A
-// matrix built on the device has no host copy of its image; what the host
-// walks of an uploaded or streamed image compute (hotcols.cpp, retile.cpp,
-// the carries of get_plan) is computed here for it.
+// image_dev.hip -- walks of an image resident in HBM, on the device: the
+// gather-order relabelling of an uploaded image, the column ranking that a
+// device build shares, and the cuts of a device-built image's work plans.
 //
 // decode_lists: every non-zero as (row, column[, value]) in stream order
 // (block rows ascending; in each block row its tiles in directory order; in
@@ -13,15 +12,14 @@
 //                 non-zeros (and counts each column's uses, atomically, when
 //                 asked).
 //
-// gather_order_lists: the same lists with the columns relabelled so that the
-// nhot most used columns become 0..nhot-1 in descending order of use (ties by
-// column) and every other column c becomes nhot + c, and the list of the hot
-// columns in their new order:
+// rank_columns: the nhot most used columns become 0..nhot-1 in descending
+// order of use (ties by column) and every other column c becomes nhot + c:
 //   rank          sort keys ((2^31 - uses) << 32 | column): descending use,
 //                 ascending column among equals;
 //   cut           the first rank at which the running sum of uses reaches
 //                 the wanted share (or the uses reach 0) is nhot;
-//   relabel       new ids, then every column of the list.
+//   new ids       of all columns, and the list of the hot ones in new order.
+// gather_order_lists: decode_lists' lists with the columns relabelled so.
 //
 // plan_cuts: the split items of a work plan, whose ranges come as fractions
 // of their block row, moved to where an item may start (one wave per item:
@@ -235,49 +233,62 @@ fmx_status decode_lists(fmx_ctx *ctx, const fmx_spm *src, uint32_t *rows, uint32
     return FMX_OK;
 }
 
-fmx_status gather_order_lists(fmx_ctx *ctx, const fmx_spm *src, uint64_t ncols, uint64_t permille,
-                              uint32_t *rows, uint32_t *cols, void *vals, uint32_t **hot_out, uint64_t *nhot_out)
+fmx_status rank_columns(fmx_ctx *ctx, const uint32_t *uses, uint64_t ncols, uint64_t nnz, uint64_t permille,
+                        uint32_t **newid_out, uint32_t **hot_out, uint64_t *nhot_out)
 {
-    *hot_out = nullptr;
+    *newid_out = *hot_out = nullptr;
     *nhot_out = 0;
     hipStream_t s = ctx->stream;
-    DevBuf<uint32_t> uses, newid;
-    FMX_HIP(ctx, uses.alloc(ncols));
-    FMX_HIP(ctx, hipMemsetAsync(uses.p, 0, ncols * sizeof(uint32_t), s));
-    fmx_status st = decode_lists(ctx, src, rows, cols, vals, uses.p);
-    if (st) return st;
     DevBuf<uint64_t> keys, ktmp, before, nhot;
     FMX_HIP(ctx, keys.alloc(ncols));
     FMX_HIP(ctx, ktmp.alloc(ncols));
     FMX_HIP(ctx, before.alloc(ncols));
     FMX_HIP(ctx, nhot.alloc(1));
-    hipLaunchKernelGGL(rank_keys, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, uses.p, ncols, keys.p);
+    hipLaunchKernelGGL(rank_keys, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, uses, ncols, keys.p);
     FMX_HIP(ctx, hipGetLastError());
     uint64_t *sorted = nullptr;
-    st = radix_sort_u64(ctx, keys.p, ktmp.p, ncols, 64, &sorted, s);
+    // by the uses only: the keys start in column order and the sort is stable
+    fmx_status st = radix_sort_u64(ctx, keys.p, ktmp.p, ncols, 32, 64, &sorted, s);
     if (st) return st;
     hipLaunchKernelGGL(ranked_uses, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, sorted, ncols, before.p);
     FMX_HIP(ctx, hipGetLastError());
     st = scan_exclusive<uint64_t>(ctx, before.p, before.p, ncols, nullptr, s);
     if (st) return st;
     FMX_HIP(ctx, hipMemcpyAsync(nhot.p, &ncols, sizeof(uint64_t), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(cut, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, sorted, before.p, ncols,
-                       src->nnz * permille, nhot.p);
+    hipLaunchKernelGGL(cut, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, sorted, before.p, ncols, nnz * permille,
+                       nhot.p);
     FMX_HIP(ctx, hipGetLastError());
     uint64_t nh = 0;
     FMX_HIP(ctx, hipMemcpyAsync(&nh, nhot.p, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     FMX_HIP(ctx, hipStreamSynchronize(s));
     if (nh == 0 || nh + ncols > (1ull << 32)) return FMX_OK;  // no hot columns, or ids past 32 bits
-    DevBuf<uint32_t> hot;
+    DevBuf<uint32_t> newid, hot;
     FMX_HIP(ctx, newid.alloc(ncols));
     FMX_HIP(ctx, hot.alloc(nh));
     hipLaunchKernelGGL(new_ids, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, ncols, nh, newid.p);
     hipLaunchKernelGGL(hot_ids, dim3(grid_for(ctx, nh)), dim3(kT), 0, s, sorted, nh, newid.p, hot.p);
+    FMX_HIP(ctx, hipGetLastError());
+    *newid_out = newid.release();
+    *hot_out = hot.release();
+    *nhot_out = nh;
+    return FMX_OK;
+}
+
+fmx_status gather_order_lists(fmx_ctx *ctx, const fmx_spm *src, uint64_t ncols, uint64_t permille,
+                              uint32_t *rows, uint32_t *cols, void *vals, uint32_t **hot_out, uint64_t *nhot_out)
+{
+    hipStream_t s = ctx->stream;
+    *hot_out = nullptr;
+    *nhot_out = 0;
+    DevBuf<uint32_t> uses, newid;
+    FMX_HIP(ctx, uses.alloc(ncols));
+    FMX_HIP(ctx, hipMemsetAsync(uses.p, 0, ncols * sizeof(uint32_t), s));
+    fmx_status st = decode_lists(ctx, src, rows, cols, vals, uses.p);
+    if (!st) st = rank_columns(ctx, uses.p, ncols, src->nnz, permille, &newid.p, hot_out, nhot_out);
+    if (st || !*nhot_out) return st;
     hipLaunchKernelGGL(relabel, dim3(grid_for(ctx, src->nnz)), dim3(kT), 0, s, cols, src->nnz, newid.p);
     FMX_HIP(ctx, hipGetLastError());
     FMX_HIP(ctx, hipStreamSynchronize(s));
-    *hot_out = hot.release();
-    *nhot_out = nh;
     return FMX_OK;
 }
 
