@@ -110,7 +110,7 @@ fmx_status fmx_pagerank(fmx_ctx *ctx, const fmx_spm *A, const fmx_spm *At, int m
     uint32_t *counts = (uint32_t *)((char *)ctx->pinned + kPinnedCounts);
     float *buf = nullptr;
     hipEvent_t ev = nullptr;
-    FMX_HIP(ctx, hipMalloc(&buf, 3 * n * sizeof(float)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&buf, 3 * n * sizeof(float)));
     if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
         (void)hipFree(buf);
         return fail(ctx, FMX_EHIP, "PageRank event");
@@ -193,8 +193,8 @@ fmx_status fmx_nmf(fmx_ctx *ctx, const fmx_spm *A, const fmx_spm *At, int k, int
     float *buf = nullptr;
     double *g = nullptr;
     const uint64_t big = std::max(n, m) * (uint64_t)k;
-    FMX_HIP(ctx, hipMalloc(&buf, 2 * big * sizeof(float)));
-    if (hipMalloc(&g, 2 * (size_t)k * k * sizeof(double)) != hipSuccess) {
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&buf, 2 * big * sizeof(float)));
+    if (dev_malloc(ctx, (void **)&g, 2 * (size_t)k * k * sizeof(double)) != hipSuccess) {
         (void)hipFree(buf);
         return fail(ctx, FMX_ENOMEM, "NMF Gram buffers");
     }

@@ -472,7 +472,7 @@ fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint6
     fmx_status st = FMX_OK;
     uint32_t R = 0;
     DevBuf<uint32_t> flag;
-    FMX_HIP(ctx, flag.alloc(nk + 1));
+    FMX_HIP(ctx, flag.alloc(ctx, nk + 1));
     if (nk) {
         hipLaunchKernelGGL(group_flags, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, f.lw, flag.p);
         FMX_HIP(ctx, hipGetLastError());
@@ -481,11 +481,11 @@ fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint6
     }
     DevBuf<uint32_t> run_start, tflag, coo_ex, tile_of_run;
     DevBuf<uint64_t> scsr_ex;
-    FMX_HIP(ctx, run_start.alloc((uint64_t)R + 1));
-    FMX_HIP(ctx, tflag.alloc((uint64_t)R + 1));
-    FMX_HIP(ctx, coo_ex.alloc((uint64_t)R + 1));
-    FMX_HIP(ctx, scsr_ex.alloc((uint64_t)R + 1));
-    FMX_HIP(ctx, tile_of_run.alloc((uint64_t)R + 1));
+    FMX_HIP(ctx, run_start.alloc(ctx, (uint64_t)R + 1));
+    FMX_HIP(ctx, tflag.alloc(ctx, (uint64_t)R + 1));
+    FMX_HIP(ctx, coo_ex.alloc(ctx, (uint64_t)R + 1));
+    FMX_HIP(ctx, scsr_ex.alloc(ctx, (uint64_t)R + 1));
+    FMX_HIP(ctx, tile_of_run.alloc(ctx, (uint64_t)R + 1));
     const int tshift = f.lh + f.lw;
     uint32_t T = 0;
     if (nk) {
@@ -508,15 +508,15 @@ fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint6
     DevBuf<uint64_t> tsize, tile_off, offs_ex;
     DevBuf<unsigned long long> brsize;
     DevBuf<uint8_t> had;
-    FMX_HIP(ctx, tile_first_run.alloc((uint64_t)T + 1));
-    FMX_HIP(ctx, tsize.alloc((uint64_t)T + 1));
-    FMX_HIP(ctx, tile_off.alloc((uint64_t)T + 1));
-    FMX_HIP(ctx, brsize.alloc(nbr + 1));
-    FMX_HIP(ctx, offs_ex.alloc(nbr + 1));
-    FMX_HIP(ctx, br_first.alloc(nbr + 1));
-    FMX_HIP(ctx, had.alloc(nbr + 1));
+    FMX_HIP(ctx, tile_first_run.alloc(ctx, (uint64_t)T + 1));
+    FMX_HIP(ctx, tsize.alloc(ctx, (uint64_t)T + 1));
+    FMX_HIP(ctx, tile_off.alloc(ctx, (uint64_t)T + 1));
+    FMX_HIP(ctx, brsize.alloc(ctx, nbr + 1));
+    FMX_HIP(ctx, offs_ex.alloc(ctx, nbr + 1));
+    FMX_HIP(ctx, br_first.alloc(ctx, nbr + 1));
+    FMX_HIP(ctx, had.alloc(ctx, nbr + 1));
     DevBuf<uint32_t> bdir;  // directory entries per block row, then their exclusive scan
-    FMX_HIP(ctx, bdir.alloc(nbr + 1));
+    FMX_HIP(ctx, bdir.alloc(ctx, nbr + 1));
     FMX_HIP(ctx, hipMemsetAsync(brsize.p, 0, (nbr + 1) * sizeof(unsigned long long), s));
     if (T) {
         hipLaunchKernelGGL(fill_tiles, dim3(grid_for(ctx, R)), dim3(kB), 0, s, K, run_start.p, R, tshift,
@@ -545,11 +545,11 @@ fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint6
     spm->ctx = ctx;
     const uint64_t bytes = 4096 + tiles_total;
     const uint64_t padded = (bytes + 4095) & ~4095ull;
-    FMX_HIP(ctx, hipMalloc(&spm->d_image, padded));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&spm->d_image, padded));
     FMX_HIP(ctx, hipMemsetAsync(spm->d_image + bytes, 0, padded - bytes, s));
     {
-        uint8_t hdr[4096];
-        memset(hdr, 0, sizeof(hdr));
+        uint8_t *hdr = (uint8_t *)ctx->pinned + kPinnedHeader;
+        memset(hdr, 0, kHeaderBytes);
         const int64_t magic = 0x0123456789FFFFFFLL;
         const int32_t ver = 2, type = 2, layout = 2, prim = vals ? prim_type : 0;
         const uint64_t hesz = vals ? esz : 0;
@@ -563,8 +563,7 @@ fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint6
         memcpy(hdr + 44, &prim, 4);
         memcpy(hdr + 48, &H, 8);
         memcpy(hdr + 56, &W, 8);
-        FMX_HIP(ctx, hipMemcpyAsync(spm->d_image, hdr, 4096, hipMemcpyHostToDevice, s));
-        FMX_HIP(ctx, hipStreamSynchronize(s));
+        FMX_HIP(ctx, hipMemcpyAsync(spm->d_image, hdr, kHeaderBytes, hipMemcpyHostToDevice, s));
     }
     if (T) {
         hipLaunchKernelGGL(write_tiles, dim3(grid_for(ctx, T)), dim3(kB), 0, s, K, f, run_start.p,
@@ -585,14 +584,14 @@ fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint6
     uint32_t ndir = 0;
     st = scan_exclusive<uint32_t>(ctx, bdir.p, bdir.p, nbr + 1, &ndir, s);
     if (st) return st;
-    FMX_HIP(ctx, hipMalloc(&spm->d_dir, std::max<uint64_t>(1, ndir) * sizeof(uint2)));
-    if (vals) FMX_HIP(ctx, hipMalloc(&spm->d_vdir, std::max<uint64_t>(1, ndir) * sizeof(uint32_t)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&spm->d_dir, std::max<uint64_t>(1, ndir) * sizeof(uint2)));
+    if (vals) FMX_HIP(ctx, dev_malloc(ctx, (void **)&spm->d_vdir, std::max<uint64_t>(1, ndir) * sizeof(uint32_t)));
     hipLaunchKernelGGL(fill_dir, dim3(grid_for(ctx, std::max<uint64_t>(T, nbr))), dim3(kB), 0, s, K, f,
                        run_start.p, tile_first_run.p, T, offs_ex.p, br_first.p, tile_off.p, bdir.p, had.p, nbr,
                        vals ? 1 : 0, spm->d_dir, spm->d_vdir);
     FMX_HIP(ctx, hipGetLastError());
     DevBuf<unsigned int> bad;
-    FMX_HIP(ctx, bad.alloc(1));
+    FMX_HIP(ctx, bad.alloc(ctx, 1));
     FMX_HIP(ctx, hipMemsetAsync(bad.p, 0, sizeof(unsigned int), s));
     hipLaunchKernelGGL(check_dir, dim3(grid_for(ctx, nbr)), dim3(kB), 0, s, spm->d_dir, spm->d_vdir, bdir.p,
                        offs_ex.p, nbr, nbc, (uint64_t)ndir, vals ? 1 : 0, bad.p);
@@ -603,10 +602,15 @@ fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint6
     std::vector<uint64_t> oex(nbr + 1);
     unsigned int hbad = 0;
     spm->brow_dir.resize(nbr + 1);
-    FMX_HIP(ctx, hipMemcpyAsync(oex.data(), offs_ex.p, (nbr + 1) * 8, hipMemcpyDeviceToHost, s));
-    FMX_HIP(ctx, hipMemcpyAsync(spm->brow_dir.data(), bdir.p, (nbr + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    FMX_HIP(ctx, hipMemcpyAsync(&hbad, bad.p, sizeof(unsigned int), hipMemcpyDeviceToHost, s));
+    const size_t ob = (nbr + 1) * 8, bb = (nbr + 1) * sizeof(uint32_t);
+    st = pinned_fetch(ctx, &hbad, bad.p, sizeof(unsigned int), 0, s);
+    if (!st) st = pinned_fetch(ctx, oex.data(), offs_ex.p, ob, 64, s);
+    if (!st) st = pinned_fetch(ctx, spm->brow_dir.data(), bdir.p, bb, 64 + ob, s);
+    if (st) return st;
     FMX_HIP(ctx, hipStreamSynchronize(s));
+    pinned_get(ctx, &hbad, sizeof(unsigned int), 0);
+    pinned_get(ctx, oex.data(), ob, 64);
+    pinned_get(ctx, spm->brow_dir.data(), bb, 64 + ob);
     if (hbad) return fail(ctx, FMX_EINVAL, "internal error: inconsistent device-built directory");
     spm->offs.resize(nbr + 1);
     for (uint64_t b = 0; b <= nbr; b++) spm->offs[b] = (int64_t)(4096 + oex[b]);
@@ -643,11 +647,11 @@ fmx_status work_images(fmx_ctx *ctx, fmx_spm *spm, const uint64_t *K, const uint
     if (!h2 && !fast) return FMX_OK;
     DevBuf<uint64_t> keys, tmp;
     DevBuf<uint32_t> va, vb;
-    FMX_HIP(ctx, keys.alloc(nk));
-    FMX_HIP(ctx, tmp.alloc(nk));
+    FMX_HIP(ctx, keys.alloc(ctx, nk));
+    FMX_HIP(ctx, tmp.alloc(ctx, nk));
     if (vals) {
-        FMX_HIP(ctx, va.alloc(nk));
-        FMX_HIP(ctx, vb.alloc(nk));
+        FMX_HIP(ctx, va.alloc(ctx, nk));
+        FMX_HIP(ctx, vb.alloc(ctx, nk));
     }
     auto image = [&](uint32_t log2_h, uint32_t log2_w, uint64_t ncols, const uint32_t *newid, bool in_order,
                      std::unique_ptr<fmx_spm> &out) -> fmx_status {
@@ -677,7 +681,7 @@ fmx_status work_images(fmx_ctx *ctx, fmx_spm *spm, const uint64_t *K, const uint
     {
         const uint32_t copies = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, (16ull << 20) / spm->ncols));
         DevBuf<uint32_t> uses;
-        FMX_HIP(ctx, uses.alloc(spm->ncols * copies));
+        FMX_HIP(ctx, uses.alloc(ctx, spm->ncols * copies));
         FMX_HIP(ctx, hipMemsetAsync(uses.p, 0, spm->ncols * copies * sizeof(uint32_t), s));
         hipLaunchKernelGGL(count_columns, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, f, uses.p, spm->ncols, copies);
         hipLaunchKernelGGL(add_copies, dim3(grid_for(ctx, spm->ncols)), dim3(kB), 0, s, uses.p, spm->ncols, copies);
@@ -717,6 +721,7 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
     FMX_HIP(ctx, hipSetDevice(ctx->device));
     // the edge list may come from any stream: construction is synchronous
     FMX_HIP(ctx, hipDeviceSynchronize());
+    BlockScope scope(ctx->blocks);
     hipStream_t s = ctx->stream;
     // device time of the construction, from the first kernel to the last
     // write (host waits for totals in between are included)
@@ -754,18 +759,18 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
     DevBuf<uint64_t> keys, tmp;
     DevBuf<uint32_t> eidx, etmp;
     DevBuf<unsigned long long> counter;
-    FMX_HIP(ctx, keys.alloc(cap));
-    FMX_HIP(ctx, tmp.alloc(cap));
-    FMX_HIP(ctx, counter.alloc(1));
+    FMX_HIP(ctx, keys.alloc(ctx, cap));
+    FMX_HIP(ctx, tmp.alloc(ctx, cap));
+    FMX_HIP(ctx, counter.alloc(ctx, 1));
     FMX_HIP(ctx, hipMemsetAsync(counter.p, 0, sizeof(unsigned long long), s));
     unsigned long long nk64 = 0;
     fmx_status st = FMX_OK;
     if (vals) {
         if (m >= (1ull << 31)) return fail(ctx, FMX_EUNSUPPORTED, "weighted builds take fewer than 2^31 edges");
-        FMX_HIP(ctx, eidx.alloc(cap));
-        FMX_HIP(ctx, etmp.alloc(cap));
+        FMX_HIP(ctx, eidx.alloc(ctx, cap));
+        FMX_HIP(ctx, etmp.alloc(ctx, cap));
         DevBuf<uint32_t> pos;
-        FMX_HIP(ctx, pos.alloc((uint64_t)m + 1));
+        FMX_HIP(ctx, pos.alloc(ctx, (uint64_t)m + 1));
         uint32_t total = 0;
         if (m) {
             hipLaunchKernelGGL(count_keys_w, dim3(grid_for(ctx, m)), dim3(kB), 0, s, src, dst, (uint64_t)m,
@@ -784,8 +789,10 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
                                keep_self, sym, keys.p, counter.p);
             FMX_HIP(ctx, hipGetLastError());
         }
-        FMX_HIP(ctx, hipMemcpyAsync(&nk64, counter.p, sizeof(nk64), hipMemcpyDeviceToHost, s));
+        st = pinned_fetch(ctx, &nk64, counter.p, sizeof(nk64), 0, s);
+        if (st) return st;
         FMX_HIP(ctx, hipStreamSynchronize(s));
+        pinned_get(ctx, &nk64, sizeof(nk64), 0);
     }
     if (nk64 >= (1ull << 32)) return fail(ctx, FMX_EUNSUPPORTED, "more than 2^32 - 1 non-zeros");
 
@@ -800,7 +807,7 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
     uint64_t nk = nk64;
     if ((flags & FMX_BUILD_DEDUP) && nk) {
         DevBuf<uint32_t> flag;
-        FMX_HIP(ctx, flag.alloc(nk + 1));
+        FMX_HIP(ctx, flag.alloc(ctx, nk + 1));
         hipLaunchKernelGGL(group_flags, dim3(grid_for(ctx, nk)), dim3(kB), 0, s, K, nk, 0, flag.p);
         FMX_HIP(ctx, hipGetLastError());
         uint32_t nu = 0;
@@ -820,17 +827,10 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
     // the key (and payload) buffer that does not hold the result is not read
     // again: its memory goes back before the run and tile arrays are made
     // (17 GB at 2^31 edges)
-    FMX_HIP(ctx, hipStreamSynchronize(s));
     for (DevBuf<uint64_t> *b : {&keys, &tmp})
-        if (b->p && b->p != K) {
-            FMX_HIP(ctx, hipFree(b->p));
-            b->p = nullptr;
-        }
+        if (b->p != K) b->reset();
     for (DevBuf<uint32_t> *b : {&eidx, &etmp})
-        if (b->p && b->p != V) {
-            FMX_HIP(ctx, hipFree(b->p));
-            b->p = nullptr;
-        }
+        if (b->p != V) b->reset();
 
     std::unique_ptr<fmx_spm> spm;
     st = write_image(ctx, K, V, nk, f, n, ncols, vals, esz, prim_type, ev.b, spm);

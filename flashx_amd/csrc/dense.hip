@@ -854,7 +854,7 @@ fmx_status ctx_scratch(fmx_ctx *ctx, size_t bytes, void **out)
         if (ctx->ws) FMX_HIP(ctx, hipFree(ctx->ws));
         ctx->ws = nullptr;
         ctx->ws_bytes = 0;
-        FMX_HIP(ctx, hipMalloc(&ctx->ws, bytes));
+        FMX_HIP(ctx, dev_malloc(ctx, (void **)&ctx->ws, bytes));
         ctx->ws_bytes = bytes;
     }
     *out = ctx->ws;

@@ -29,12 +29,27 @@ fmx_status radix_sort_u64_kv(fmx_ctx *ctx, uint64_t *keys, uint64_t *tmp, uint32
 fmx_status max_u32_pair(fmx_ctx *ctx, const uint32_t *a, const uint32_t *b, uint64_t n,
                         uint32_t *out, hipStream_t s);
 
-// RAII device buffer.
+// RAII device buffer, from the context's block cache (fmx_internal.h).
 template <typename T>
 struct DevBuf {
     T *p = nullptr;
-    ~DevBuf() { if (p) (void)hipFree(p); }
-    hipError_t alloc(uint64_t n) { return hipMalloc(&p, (n ? n : 1) * sizeof(T)); }
+    size_t bytes = 0;
+    fmx_ctx *ctx = nullptr;
+    DevBuf() = default;
+    DevBuf(const DevBuf &) = delete;
+    DevBuf &operator=(const DevBuf &) = delete;
+    ~DevBuf() { reset(); }
+    void reset()
+    {
+        if (p && ctx) ctx->blocks.put(p, bytes);
+        else if (p) (void)hipFree(p);
+        p = nullptr;
+    }
+    hipError_t alloc(fmx_ctx *c, uint64_t n)
+    {
+        ctx = c;
+        return c->blocks.get((n ? n : 1) * sizeof(T), (void **)&p, &bytes);
+    }
     T *release() { T *q = p; p = nullptr; return q; }
 };
 

@@ -107,7 +107,7 @@ fmx_status scan_rec(fmx_ctx *ctx, const T *in, T *out, uint64_t n, T *d_total, h
         return FMX_OK;
     }
     DevBuf<T> partials;
-    FMX_HIP(ctx, partials.alloc(nb));
+    FMX_HIP(ctx, partials.alloc(ctx, nb));
     hipLaunchKernelGGL(scan_reduce<T>, dim3((uint32_t)nb), dim3(kT), 0, s, in, n, partials.p);
     FMX_HIP(ctx, hipGetLastError());
     fmx_status st = scan_rec<T>(ctx, partials.p, partials.p, nb, d_total, s);
@@ -115,8 +115,8 @@ fmx_status scan_rec(fmx_ctx *ctx, const T *in, T *out, uint64_t n, T *d_total, h
     hipLaunchKernelGGL(scan_tile<T>, dim3((uint32_t)nb), dim3(kT), 0, s, in, out, n,
                        (const T *)partials.p, (T *)nullptr);
     FMX_HIP(ctx, hipGetLastError());
-    // partials must outlive the kernels that read them
-    FMX_HIP(ctx, hipStreamSynchronize(s));
+    // outside a construction the partials are freed at once: after the kernels
+    if (!ctx->blocks.scopes) FMX_HIP(ctx, hipStreamSynchronize(s));
     return FMX_OK;
 }
 
@@ -261,7 +261,7 @@ template <typename T>
 fmx_status scan_exclusive(fmx_ctx *ctx, const T *in, T *out, uint64_t n, T *total, hipStream_t s)
 {
     DevBuf<T> d_total;
-    FMX_HIP(ctx, d_total.alloc(1));
+    FMX_HIP(ctx, d_total.alloc(ctx, 1));
     if (n == 0) {
         if (total) *total = 0;
         return FMX_OK;
@@ -269,9 +269,11 @@ fmx_status scan_exclusive(fmx_ctx *ctx, const T *in, T *out, uint64_t n, T *tota
     fmx_status st = scan_rec<T>(ctx, in, out, n, d_total.p, s);
     if (st) return st;
     if (total) {
-        FMX_HIP(ctx, hipMemcpyAsync(total, d_total.p, sizeof(T), hipMemcpyDeviceToHost, s));
+        st = pinned_fetch(ctx, total, d_total.p, sizeof(T), 0, s);
+        if (st) return st;
     }
-    FMX_HIP(ctx, hipStreamSynchronize(s));
+    if (total || !ctx->blocks.scopes) FMX_HIP(ctx, hipStreamSynchronize(s));
+    if (total) pinned_get(ctx, total, sizeof(T), 0);
     return FMX_OK;
 }
 
@@ -304,7 +306,7 @@ fmx_status radix_sort_u64_kv(fmx_ctx *ctx, uint64_t *keys, uint64_t *tmp, uint32
     if (nb64 >= (1ull << 32) / 256) return fail(ctx, FMX_EUNSUPPORTED, "too many keys to sort");
     const uint32_t nb = (uint32_t)nb64;
     DevBuf<uint64_t> hist;
-    FMX_HIP(ctx, hist.alloc((uint64_t)nb * 256));
+    FMX_HIP(ctx, hist.alloc(ctx, (uint64_t)nb * 256));
     uint64_t *a = keys, *b = tmp;
     uint32_t *va = vals, *vb = vtmp;
     for (int shift = from; shift < bits; shift += 8) {
@@ -325,7 +327,7 @@ fmx_status radix_sort_u64_kv(fmx_ctx *ctx, uint64_t *keys, uint64_t *tmp, uint32
         va = vb;
         vb = vt;
     }
-    FMX_HIP(ctx, hipStreamSynchronize(s));
+    if (!ctx->blocks.scopes) FMX_HIP(ctx, hipStreamSynchronize(s));
     *sorted = a;
     *sorted_vals = va;
     return FMX_OK;
@@ -335,15 +337,17 @@ fmx_status max_u32_pair(fmx_ctx *ctx, const uint32_t *a, const uint32_t *b, uint
                         uint32_t *out, hipStream_t s)
 {
     DevBuf<uint32_t> d;
-    FMX_HIP(ctx, d.alloc(1));
+    FMX_HIP(ctx, d.alloc(ctx, 1));
     FMX_HIP(ctx, hipMemsetAsync(d.p, 0, sizeof(uint32_t), s));
     uint64_t blocks = (n + kT - 1) / kT;
     if (blocks > (uint64_t)ctx->num_cus * 4) blocks = (uint64_t)ctx->num_cus * 4;
     if (blocks == 0) blocks = 1;
     hipLaunchKernelGGL(max_pair_kernel, dim3((uint32_t)blocks), dim3(kT), 0, s, a, b, n, d.p);
     FMX_HIP(ctx, hipGetLastError());
-    FMX_HIP(ctx, hipMemcpyAsync(out, d.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    fmx_status st = pinned_fetch(ctx, out, d.p, sizeof(uint32_t), 0, s);
+    if (st) return st;
     FMX_HIP(ctx, hipStreamSynchronize(s));
+    pinned_get(ctx, out, sizeof(uint32_t), 0);
     return FMX_OK;
 }
 

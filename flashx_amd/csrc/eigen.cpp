@@ -128,36 +128,36 @@ template <typename T>
 fmx_status Solver<T>::alloc()
 {
     const uint64_t n = n_ ? n_ : 1;
-    FMX_HIP(ctx_, hipMalloc(&V_.p, n * m_ * sizeof(T)));
-    FMX_HIP(ctx_, hipMalloc(&W_.p, n * b_ * sizeof(T)));
-    FMX_HIP(ctx_, hipMalloc(&T1_.p, n * b_ * sizeof(T)));
-    FMX_HIP(ctx_, hipMalloc(&dinv_.p, n * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&deg_.p, n * sizeof(float)));
-    FMX_HIP(ctx_, hipMalloc(&H_.p, (size_t)m_ * m_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&S_.p, (size_t)m_ * m_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&Ssel_.p, (size_t)m_ * m_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&Scols_.p, (size_t)m_ * m_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&ev_.p, (size_t)m_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&C1_.p, (size_t)m_ * b_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&C2_.p, (size_t)m_ * b_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&G_.p, (size_t)b_ * b_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&Rinv_.p, (size_t)b_ * b_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&info_.p, 4 * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&rot_.p, small_sym_eig_ws(m_)));
-    FMX_HIP(ctx_, hipMalloc(&X64_.p, n * o_.nev * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&Y64_.p, n * o_.nev * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&Z64_.p, n * o_.nev * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&theta_.p, (size_t)m_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&rn_.p, (size_t)m_ * sizeof(double)));
-    FMX_HIP(ctx_, hipMalloc(&part_.p, (size_t)1024 * 256 * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&V_.p, n * m_ * sizeof(T)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&W_.p, n * b_ * sizeof(T)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&T1_.p, n * b_ * sizeof(T)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&dinv_.p, n * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&deg_.p, n * sizeof(float)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&H_.p, (size_t)m_ * m_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&S_.p, (size_t)m_ * m_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&Ssel_.p, (size_t)m_ * m_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&Scols_.p, (size_t)m_ * m_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&ev_.p, (size_t)m_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&C1_.p, (size_t)m_ * b_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&C2_.p, (size_t)m_ * b_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&G_.p, (size_t)b_ * b_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&Rinv_.p, (size_t)b_ * b_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&info_.p, 4 * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&rot_.p, small_sym_eig_ws(m_)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&X64_.p, n * o_.nev * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&Y64_.p, n * o_.nev * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&Z64_.p, n * o_.nev * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&theta_.p, (size_t)m_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&rn_.p, (size_t)m_ * sizeof(double)));
+    FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&part_.p, (size_t)1024 * 256 * sizeof(double)));
     const int keep = std::min(m_ - b_, ((o_.nev + b_ - 1) / b_) * b_ + b_);
     shadow_ = std::is_same<T, float>::value && o_.precision == FMX_EIG_MIXED && b_ % 8 == 0 && m_ % 8 == 0 &&
               m_ <= 128 && keep <= 32;
-    if (shadow_) FMX_HIP(ctx_, hipMalloc(&Vb_.p, n * m_ * sizeof(unsigned short)));
+    if (shadow_) FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&Vb_.p, n * m_ * sizeof(unsigned short)));
     if (op_ == FMX_EIG_OP_SVD) {
         const uint64_t nm = nmid_ ? nmid_ : 1;
-        FMX_HIP(ctx_, hipMalloc(&T2_.p, nm * b_ * sizeof(T)));
-        FMX_HIP(ctx_, hipMalloc(&M64_.p, nm * o_.nev * sizeof(double)));
+        FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&T2_.p, nm * b_ * sizeof(T)));
+        FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&M64_.p, nm * o_.nev * sizeof(double)));
     }
     return FMX_OK;
 }
@@ -284,7 +284,7 @@ fmx_status Solver<T>::run(const void *X0, int64_t ldx0, fmx_dtype x0_dt, double 
     // degrees and D^-1/2 (NA_eigen_Operator ctor, test-eigen.cpp:93-110)
     if (op_ == FMX_EIG_OP_NORMALIZED) {
         Dev<float> ones;
-        FMX_HIP(ctx_, hipMalloc(&ones.p, (n_ ? n_ : 1) * sizeof(float)));
+        FMX_HIP(ctx_, dev_malloc(ctx_, (void **)&ones.p, (n_ ? n_ : 1) * sizeof(float)));
         std::vector<float> h1(n_, 1.0f);
         FMX_HIP(ctx_, hipMemcpyAsync(ones.p, h1.data(), n_ * sizeof(float), hipMemcpyHostToDevice, s_));
         TRY(fmx_spmm(ctx_, spm_, FMX_F32, 1, ones.p, 1, deg_.p, 1, s_));

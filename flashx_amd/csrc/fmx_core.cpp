@@ -24,6 +24,70 @@ Scratch::~Scratch()
     if (ptr) (void)hipFree(ptr);
 }
 
+hipError_t BlockCache::get(size_t bytes, void **p, size_t *got)
+{
+    // the smallest block that fits and wastes no more than half
+    size_t best = free_.size();
+    for (size_t i = 0; scopes && i < free_.size(); i++)
+        if (free_[i].first >= bytes && free_[i].first / 2 <= bytes + 32768 &&
+            (best == free_.size() || free_[i].first < free_[best].first))
+            best = i;
+    if (best < free_.size()) {
+        *got = free_[best].first;
+        *p = free_[best].second;
+        held_ -= *got;
+        free_.erase(free_.begin() + best);
+        return hipSuccess;
+    }
+    *got = bytes;
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess || free_.empty()) return e;
+    (void)hipGetLastError();
+    trim(0);
+    return hipMalloc(p, bytes);
+}
+
+void BlockCache::put(void *p, size_t bytes)
+{
+    if (scopes && held_ + bytes <= kKeep) {
+        free_.emplace_back(bytes, p);
+        held_ += bytes;
+    } else {
+        (void)hipFree(p);
+    }
+}
+
+void BlockCache::trim(size_t most)
+{
+    std::sort(free_.begin(), free_.end());
+    while (held_ > most) {
+        (void)hipFree(free_.back().second);
+        held_ -= free_.back().first;
+        free_.pop_back();
+    }
+}
+
+hipError_t dev_malloc(fmx_ctx *ctx, void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    ctx->blocks.trim(0);
+    return hipMalloc(p, bytes);
+}
+
+fmx_status pinned_fetch(fmx_ctx *ctx, void *dst, const void *src, size_t bytes, size_t at, hipStream_t s)
+{
+    if (kPinnedStage + at + bytes <= kPinnedBytes) dst = (char *)ctx->pinned + kPinnedStage + at;
+    FMX_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+    return FMX_OK;
+}
+
+void pinned_get(fmx_ctx *ctx, void *dst, size_t bytes, size_t at)
+{
+    if (kPinnedStage + at + bytes <= kPinnedBytes) memcpy(dst, (char *)ctx->pinned + kPinnedStage + at, bytes);
+}
+
 fmx_status fail(fmx_ctx *ctx, fmx_status st, const std::string &msg)
 {
     if (ctx) ctx->last_error = msg;
@@ -439,7 +503,7 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
         // context's pinned buffer where they fit (a pageable copy of 64 KB
         // takes 35 us, a pinned one 12)
         const size_t ib = plan->nitems * sizeof(Item), all = ib + plan->nsplits * sizeof(Split);
-        FMX_HIP(ctx, hipMalloc(&plan->d_items, all));
+        FMX_HIP(ctx, dev_malloc(ctx, (void **)&plan->d_items, all));
         plan->d_splits = (Split *)((char *)plan->d_items + ib);
         std::vector<char> host;
         char *src = (char *)ctx->pinned + kPinnedStage;
@@ -474,10 +538,10 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
 // Tile directory (and, for weighted images, the values directory) to HBM.
 fmx_status upload_dirs(fmx_ctx *ctx, fmx_spm *s)
 {
-    FMX_HIP(ctx, hipMalloc(&s->d_dir, std::max<size_t>(1, s->dir.size()) * sizeof(uint2)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&s->d_dir, std::max<size_t>(1, s->dir.size()) * sizeof(uint2)));
     FMX_HIP(ctx, hipMemcpy(s->d_dir, s->dir.data(), s->dir.size() * sizeof(uint2), hipMemcpyHostToDevice));
     if (s->esz) {
-        FMX_HIP(ctx, hipMalloc(&s->d_vdir, std::max<size_t>(1, s->vdir.size()) * sizeof(uint32_t)));
+        FMX_HIP(ctx, dev_malloc(ctx, (void **)&s->d_vdir, std::max<size_t>(1, s->vdir.size()) * sizeof(uint32_t)));
         FMX_HIP(ctx, hipMemcpy(s->d_vdir, s->vdir.data(), s->vdir.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     }
     return FMX_OK;
@@ -494,7 +558,7 @@ fmx_status prepare_work(fmx_ctx *ctx, fmx_spm *s)
     if (st) return fail(ctx, FMX_EINVAL, "internal error: the re-cut work image is invalid: " + ctx->last_error);
     if (w->nnz != s->nnz) return fail(ctx, FMX_EINVAL, "internal error: the re-cut work image lost non-zeros");
     const size_t padded = (w->bytes + 4095) & ~size_t(4095);
-    FMX_HIP(ctx, hipMalloc(&w->d_image, padded));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&w->d_image, padded));
     FMX_HIP(ctx, hipMemcpy(w->d_image, w->h_image.data(), w->bytes, hipMemcpyHostToDevice));
     if (padded > w->bytes) FMX_HIP(ctx, hipMemset(w->d_image + w->bytes, 0, padded - w->bytes));
     st = upload_dirs(ctx, w.get());
@@ -603,7 +667,7 @@ fmx_status finish_streamed_chunks(fmx_ctx *ctx, fmx_spm *s, uint64_t chunk_bytes
     s->chunk_br.push_back(s->nbr);
     FMX_HIP(ctx, hipSetDevice(ctx->device));
     for (int b = 0; b < 2; b++) {
-        FMX_HIP(ctx, hipMalloc(&s->d_stage[b], std::max<uint64_t>(s->stage_bytes, 16)));
+        FMX_HIP(ctx, dev_malloc(ctx, (void **)&s->d_stage[b], std::max<uint64_t>(s->stage_bytes, 16)));
         FMX_HIP(ctx, hipEventCreateWithFlags(&s->ev_copied[b], hipEventDisableTiming));
         FMX_HIP(ctx, hipEventCreateWithFlags(&s->ev_free[b], hipEventDisableTiming));
     }
@@ -689,7 +753,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
         if (spm->partial.ptr) FMX_HIP(ctx, hipFree(spm->partial.ptr));
         spm->partial.ptr = nullptr;
         spm->partial.bytes = 0;
-        FMX_HIP(ctx, hipMalloc(&spm->partial.ptr, need));
+        FMX_HIP(ctx, dev_malloc(ctx, (void **)&spm->partial.ptr, need));
         spm->partial.bytes = need;
     }
     // a column-major or pre-scaled X is restaged row-major first (the
@@ -702,7 +766,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
             if (ctx->xstage.ptr) FMX_HIP(ctx, hipFree(ctx->xstage.ptr));
             ctx->xstage.ptr = nullptr;
             ctx->xstage.bytes = 0;
-            FMX_HIP(ctx, hipMalloc(&ctx->xstage.ptr, xb));
+            FMX_HIP(ctx, dev_malloc(ctx, (void **)&ctx->xstage.ptr, xb));
             ctx->xstage.bytes = xb;
         }
         st = stage_dense_rows(ctx, dtype, orig->ncols, k, X, ldx, xcol, pre, ctx->xstage.ptr, s);
@@ -718,7 +782,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
             if (ctx->xhot.ptr) FMX_HIP(ctx, hipFree(ctx->xhot.ptr));
             ctx->xhot.ptr = nullptr;
             ctx->xhot.bytes = 0;
-            FMX_HIP(ctx, hipMalloc(&ctx->xhot.ptr, hb));
+            FMX_HIP(ctx, dev_malloc(ctx, (void **)&ctx->xhot.ptr, hb));
             ctx->xhot.bytes = hb;
         }
         st = stage_hot_rows(ctx, dtype, orig->nhot, k, X, ldx, orig->d_hot, ctx->xhot.ptr, s);
@@ -853,7 +917,7 @@ fmx_status fmx_spm_upload(fmx_ctx *ctx, const void *image, size_t bytes,
     fmx_status st = analyse_image(ctx, s.get());
     if (st) return st;
     size_t padded = (s->bytes + 4095) & ~size_t(4095);
-    FMX_HIP(ctx, hipMalloc(&s->d_image, padded));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&s->d_image, padded));
     FMX_HIP(ctx, hipMemcpy(s->d_image, s->h_image.data(), s->bytes, hipMemcpyHostToDevice));
     if (padded > s->bytes) FMX_HIP(ctx, hipMemset(s->d_image + s->bytes, 0, padded - s->bytes));
     st = upload_dirs(ctx, s.get());
@@ -1094,8 +1158,8 @@ fmx_status fmx_spmm_host(fmx_ctx *ctx, const fmx_spm *spm, fmx_dtype dtype, int 
     FMX_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t s = (hipStream_t)stream;
     void *dx = nullptr, *dy = nullptr;
-    FMX_HIP(ctx, hipMalloc(&dx, std::max<uint64_t>(spm->ncols * kb * es, 16)));
-    if (hipMalloc(&dy, spm->nrows * kb * es) != hipSuccess) {
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&dx, std::max<uint64_t>(spm->ncols * kb * es, 16)));
+    if (dev_malloc(ctx, (void **)&dy, spm->nrows * kb * es) != hipSuccess) {
         (void)hipFree(dx);
         return fail(ctx, FMX_ENOMEM, "dense panel");
     }

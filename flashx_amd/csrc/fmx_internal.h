@@ -15,6 +15,7 @@
 #include <map>
 #include <memory>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/fmx.h"
@@ -69,9 +70,40 @@ struct Plan {
     ~Plan();
 };
 
+// Device blocks of constructions (inside a BlockScope), kept for reuse: a
+// build makes and drops some hundred buffers, and hipMalloc + hipFree take
+// 25 us from 4 MB and 360 us from 256 MB (a build of 16.8 M edges spent 11 of
+// its 16.5 ms in them).  Everything that uses them runs on the context's
+// stream, so a block may be handed on while kernels that use it are still
+// queued.  At most kKeep bytes are kept while a scope is open and kRest when
+// it is closed, the largest blocks going back first; all of them go back when
+// an allocation fails and with the context, which one host thread uses at a
+// time.  Blocks outside a scope are allocated and freed as they come.
+class BlockCache {
+public:
+    ~BlockCache() { trim(0); }
+    hipError_t get(size_t bytes, void **p, size_t *got);
+    void put(void *p, size_t bytes);
+    void trim(size_t most);
+    int scopes = 0;
+    static constexpr size_t kKeep = size_t(2) << 30, kRest = size_t(1) << 30;
+
+private:
+    std::vector<std::pair<size_t, void *>> free_;
+    size_t held_ = 0;
+};
+
+struct BlockScope {
+    BlockCache &c;
+    explicit BlockScope(BlockCache &cache) : c(cache) { c.scopes++; }
+    ~BlockScope() { if (--c.scopes == 0) c.trim(BlockCache::kRest); }
+};
+
 // The context's pinned host memory: counts that a kernel writes and the host
-// reads, a kernel's error flag, and a staging area for small uploads.
-constexpr size_t kPinnedCounts = 0, kPinnedFlag = 4096, kPinnedStage = 8192, kPinnedBytes = 8192 + (256 << 10);
+// reads, a kernel's error flag, an image's header page, and a staging area
+// for small copies.
+constexpr size_t kPinnedCounts = 0, kPinnedFlag = 4096, kPinnedHeader = 8192, kPinnedStage = 12288,
+                 kPinnedBytes = kPinnedStage + (2 << 20);
 
 struct Scratch {
     void *ptr = nullptr;
@@ -94,6 +126,7 @@ struct fmx_ctx {
     void *noalloc_ws = nullptr;  // this device's copy of the fixed scratch (fmx_gram_noalloc)
     size_t noalloc_bytes = 0;
     void *pinned = nullptr;      // pinned host memory (kPinned*)
+    fmx::BlockCache blocks;
 };
 
 struct fmx_spm {
@@ -149,6 +182,14 @@ namespace fmx {
 fmx_status fail(fmx_ctx *ctx, fmx_status st, const std::string &msg);
 fmx_status hip_fail(fmx_ctx *ctx, hipError_t e, const char *what);
 int elem_size(fmx_dtype dt);
+// hipMalloc that gives the context's kept blocks back if memory is short.
+hipError_t dev_malloc(fmx_ctx *ctx, void **p, size_t bytes);
+// Queues a copy of `bytes` bytes of device memory to the context's pinned
+// staging area, for pinned_get after the stream has been synchronised; larger
+// ones go to dst at once (hipMemcpy's pageable copies of some 100 KB take
+// three times as long).
+fmx_status pinned_fetch(fmx_ctx *ctx, void *dst, const void *src, size_t bytes, size_t at, hipStream_t s);
+void pinned_get(fmx_ctx *ctx, void *dst, size_t bytes, size_t at);
 
 // Validates a host image and fills the matrix fields + directory.
 fmx_status analyse_image(fmx_ctx *ctx, fmx_spm *spm);

@@ -184,9 +184,9 @@ extern "C" fmx_status fmx_dcsbm_edges(fmx_ctx *ctx, uint64_t n, int nblocks, con
     hipStream_t s = (hipStream_t)stream;
     uint64_t *C = nullptr;
     uint32_t *dwt = nullptr, *dbs = nullptr;
-    FMX_HIP(ctx, hipMalloc(&C, (n + 1) * sizeof(uint64_t)));
-    FMX_HIP(ctx, hipMalloc(&dwt, 1024 * sizeof(uint32_t)));
-    FMX_HIP(ctx, hipMalloc(&dbs, (nblocks + 1) * sizeof(uint32_t)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&C, (n + 1) * sizeof(uint64_t)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&dwt, 1024 * sizeof(uint32_t)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&dbs, (nblocks + 1) * sizeof(uint32_t)));
     FMX_HIP(ctx, hipMemcpyAsync(dwt, wtab, 1024 * 4, hipMemcpyHostToDevice, s));
     FMX_HIP(ctx, hipMemcpyAsync(dbs, bstart, (nblocks + 1) * 4, hipMemcpyHostToDevice, s));
     PermKeys pk;

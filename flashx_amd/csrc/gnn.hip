@@ -478,7 +478,7 @@ fmx_status grads(fmx_ctx *ctx, int mode, uint64_t n, int ka, int kb, const float
     if (mode != 0) {
         double *g64 = nullptr, *part = nullptr;
         const uint32_t nblk = 512;
-        FMX_HIP(ctx, hipMalloc(&g64, ((size_t)nout + (size_t)nblk * kHid) * sizeof(double)));
+        FMX_HIP(ctx, dev_malloc(ctx, (void **)&g64, ((size_t)nout + (size_t)nblk * kHid) * sizeof(double)));
         part = g64 + nout;
         fmx_status st = FMX_OK;
         for (int y = 0; y < ny && !st; y++) {
@@ -541,8 +541,8 @@ fmx_status fmx_gnn_features(fmx_ctx *ctx, const fmx_spm *spm, uint64_t seed, flo
     hipStream_t s = (hipStream_t)stream;
     const uint64_t n = spm->nrows;
     float *ones = nullptr, *deg = nullptr;
-    FMX_HIP(ctx, hipMalloc(&ones, n * sizeof(float)));
-    FMX_HIP(ctx, hipMalloc(&deg, n * sizeof(float)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&ones, n * sizeof(float)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&deg, n * sizeof(float)));
     std::vector<float> h1(n, 1.0f);
     fmx_status st = FMX_OK;
     if (hipMemcpyAsync(ones, h1.data(), n * 4, hipMemcpyHostToDevice, s) != hipSuccess) st = FMX_EHIP;
@@ -653,9 +653,9 @@ fmx_status fmx_subspace_loss(fmx_ctx *ctx, uint64_t n, int k, const float *Y, co
     FMX_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t s = (hipStream_t)stream;
     double *dG = nullptr, *dC = nullptr, *dM = nullptr;
-    FMX_HIP(ctx, hipMalloc(&dG, (size_t)k * k * sizeof(double)));
-    FMX_HIP(ctx, hipMalloc(&dC, (size_t)k * k * sizeof(double)));
-    FMX_HIP(ctx, hipMalloc(&dM, 2 * (size_t)k * k * sizeof(double)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&dG, (size_t)k * k * sizeof(double)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&dC, (size_t)k * k * sizeof(double)));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&dM, 2 * (size_t)k * k * sizeof(double)));
     std::vector<double> G(k * k), C(k * k), Gi(k * k), B(k * k), M1(k * k), M2(k * k), T(k * k);
     fmx_status st = gram(ctx, FMX_F32, FMX_GRAM_F64, n, k, k, Y, k, Y, k, dG, s);
     if (!st) st = gram(ctx, FMX_F32, FMX_GRAM_F64, n, k, k, U, k, Y, k, dC, s);

@@ -165,7 +165,7 @@ fmx_status host_lists(fmx_ctx *ctx, const fmx_spm *src, uint64_t ncols, uint64_t
         (esz && hipMemcpy(d_vals, vals, nnz * esz, hipMemcpyHostToDevice) != hipSuccess))
         return fail(ctx, FMX_EHIP, "gather-order image upload");
     uint32_t *hot = nullptr;
-    FMX_HIP(ctx, hipMalloc(&hot, nhot * 4));
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&hot, nhot * 4));
     if (hipMemcpy(hot, order.data(), nhot * 4, hipMemcpyHostToDevice) != hipSuccess) {
         (void)hipFree(hot);
         return fail(ctx, FMX_EHIP, "gather-order image upload");
@@ -197,6 +197,7 @@ fmx_status prepare_fast(fmx_ctx *ctx, fmx_spm *s, uint64_t stream_chunk)
     if (!wants_fast(s)) return FMX_OK;
     const fmx_spm *src = s->work ? s->work.get() : s;  // either walks the same non-zeros
     const uint64_t permille = hot_permille();
+    BlockScope scope(ctx->blocks);
     struct Lists {
         uint32_t *rows = nullptr, *cols = nullptr, *hot = nullptr;
         void *vals = nullptr;
@@ -208,8 +209,9 @@ fmx_status prepare_fast(fmx_ctx *ctx, fmx_spm *s, uint64_t stream_chunk)
             if (hot) (void)hipFree(hot);
         }
     } l;
-    if (hipMalloc(&l.rows, s->nnz * 4) != hipSuccess || hipMalloc(&l.cols, s->nnz * 4) != hipSuccess ||
-        (s->esz && hipMalloc(&l.vals, s->nnz * s->esz) != hipSuccess))
+    if (dev_malloc(ctx, (void **)&l.rows, s->nnz * 4) != hipSuccess ||
+        dev_malloc(ctx, (void **)&l.cols, s->nnz * 4) != hipSuccess ||
+        (s->esz && dev_malloc(ctx, &l.vals, s->nnz * s->esz) != hipSuccess))
         return fail(ctx, FMX_ENOMEM, "gather-order image");
     uint64_t nhot = 0;
     fmx_status st = src->d_image

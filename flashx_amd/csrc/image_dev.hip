@@ -89,8 +89,9 @@ __global__ void __launch_bounds__(kT) rank_keys(const uint32_t *uses, uint64_t n
         keys[c] = ((kMaxUses - uses[c]) << 32) | c;
 }
 
-__global__ void __launch_bounds__(kT) ranked_uses(const uint64_t *keys, uint64_t ncols, uint64_t *u)
+__global__ void __launch_bounds__(kT) ranked_uses(const uint64_t *keys, uint64_t ncols, uint64_t *u, uint64_t *nhot)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *nhot = ncols;  // what cut leaves if every rank is hot
     for (uint64_t i = blockIdx.x * (uint64_t)kT + threadIdx.x; i < ncols; i += (uint64_t)gridDim.x * kT)
         u[i] = kMaxUses - (keys[i] >> 32);
 }
@@ -212,10 +213,10 @@ fmx_status decode_lists(fmx_ctx *ctx, const fmx_spm *src, uint32_t *rows, uint32
     const uint64_t nbr = src->nbr, ntiles = src->brow_dir[nbr];
     DevBuf<int64_t> offs;
     DevBuf<uint32_t> bdir, tbr, tnnz;
-    FMX_HIP(ctx, offs.alloc(nbr + 1));
-    FMX_HIP(ctx, bdir.alloc(nbr + 1));
-    FMX_HIP(ctx, tbr.alloc(ntiles));
-    FMX_HIP(ctx, tnnz.alloc(ntiles));
+    FMX_HIP(ctx, offs.alloc(ctx, nbr + 1));
+    FMX_HIP(ctx, bdir.alloc(ctx, nbr + 1));
+    FMX_HIP(ctx, tbr.alloc(ctx, ntiles));
+    FMX_HIP(ctx, tnnz.alloc(ctx, ntiles));
     FMX_HIP(ctx, hipMemcpyAsync(offs.p, src->offs.data(), (nbr + 1) * sizeof(int64_t), hipMemcpyHostToDevice, s));
     FMX_HIP(ctx, hipMemcpyAsync(bdir.p, src->brow_dir.data(), (nbr + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(tile_origin, dim3(grid_for(ctx, nbr)), dim3(kT), 0, s, bdir.p, nbr, tbr.p);
@@ -240,31 +241,33 @@ fmx_status rank_columns(fmx_ctx *ctx, const uint32_t *uses, uint64_t ncols, uint
     *nhot_out = 0;
     hipStream_t s = ctx->stream;
     DevBuf<uint64_t> keys, ktmp, before, nhot;
-    FMX_HIP(ctx, keys.alloc(ncols));
-    FMX_HIP(ctx, ktmp.alloc(ncols));
-    FMX_HIP(ctx, before.alloc(ncols));
-    FMX_HIP(ctx, nhot.alloc(1));
+    FMX_HIP(ctx, keys.alloc(ctx, ncols));
+    FMX_HIP(ctx, ktmp.alloc(ctx, ncols));
+    FMX_HIP(ctx, before.alloc(ctx, ncols));
+    FMX_HIP(ctx, nhot.alloc(ctx, 1));
     hipLaunchKernelGGL(rank_keys, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, uses, ncols, keys.p);
     FMX_HIP(ctx, hipGetLastError());
     uint64_t *sorted = nullptr;
     // by the uses only: the keys start in column order and the sort is stable
     fmx_status st = radix_sort_u64(ctx, keys.p, ktmp.p, ncols, 32, 64, &sorted, s);
     if (st) return st;
-    hipLaunchKernelGGL(ranked_uses, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, sorted, ncols, before.p);
+    hipLaunchKernelGGL(ranked_uses, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, sorted, ncols, before.p,
+                       nhot.p);
     FMX_HIP(ctx, hipGetLastError());
     st = scan_exclusive<uint64_t>(ctx, before.p, before.p, ncols, nullptr, s);
     if (st) return st;
-    FMX_HIP(ctx, hipMemcpyAsync(nhot.p, &ncols, sizeof(uint64_t), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(cut, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, sorted, before.p, ncols, nnz * permille,
                        nhot.p);
     FMX_HIP(ctx, hipGetLastError());
     uint64_t nh = 0;
-    FMX_HIP(ctx, hipMemcpyAsync(&nh, nhot.p, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+    st = pinned_fetch(ctx, &nh, nhot.p, sizeof(uint64_t), 0, s);
+    if (st) return st;
     FMX_HIP(ctx, hipStreamSynchronize(s));
+    pinned_get(ctx, &nh, sizeof(uint64_t), 0);
     if (nh == 0 || nh + ncols > (1ull << 32)) return FMX_OK;  // no hot columns, or ids past 32 bits
     DevBuf<uint32_t> newid, hot;
-    FMX_HIP(ctx, newid.alloc(ncols));
-    FMX_HIP(ctx, hot.alloc(nh));
+    FMX_HIP(ctx, newid.alloc(ctx, ncols));
+    FMX_HIP(ctx, hot.alloc(ctx, nh));
     hipLaunchKernelGGL(new_ids, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, ncols, nh, newid.p);
     hipLaunchKernelGGL(hot_ids, dim3(grid_for(ctx, nh)), dim3(kT), 0, s, sorted, nh, newid.p, hot.p);
     FMX_HIP(ctx, hipGetLastError());
@@ -281,7 +284,7 @@ fmx_status gather_order_lists(fmx_ctx *ctx, const fmx_spm *src, uint64_t ncols, 
     *hot_out = nullptr;
     *nhot_out = 0;
     DevBuf<uint32_t> uses, newid;
-    FMX_HIP(ctx, uses.alloc(ncols));
+    FMX_HIP(ctx, uses.alloc(ctx, ncols));
     FMX_HIP(ctx, hipMemsetAsync(uses.p, 0, ncols * sizeof(uint32_t), s));
     fmx_status st = decode_lists(ctx, src, rows, cols, vals, uses.p);
     if (!st) st = rank_columns(ctx, uses.p, ncols, src->nnz, permille, &newid.p, hot_out, nhot_out);
