@@ -4,12 +4,11 @@
 // The SpMM kernel gives each work item one band of rows of one block row and
 // walks that block row's words; when a tile is taller than the band (the
 // reference's default 32768 x 32768 tiles, flash-graph/utils/fg2fm.cpp:
-// 155-156, against bands of 64-2048 rows), every band walks the whole block
+// 155-156, against bands of 32-2048 rows), every band walks the whole block
 // row to pick out its own rows.  Such an image is therefore re-cut once, when
-// the matrix is created, into a work image of 64-row tiles (work_rows_for)
+// the matrix is created, into a work image of 32-row tiles (work_rows_for)
 // with the same tile width: every row part and single-entry row of a tile
-// stays what
-// it is (its columns, its values, SCSR or COO), and moves to the tile of its
+// stays what it is (its columns, its values, SCSR or COO), and moves to the tile of its
 // new block row, in the same block column.  Row r of the matrix then
 // accumulates the same non-zeros in the same ascending-column order, so the
 // sequential mode is bit-identical on both images.  Resident and streamed
@@ -187,11 +186,20 @@ void retile_image(const fmx_spm *s, uint32_t h2, std::vector<uint8_t> &img, std:
 }
 
 // Tile height of the work image (0: none); FMX_WORK_ROWS overrides it (0
-// turns re-cutting off), read at every matrix creation.
+// turns the work image off).  Taller tiles than 64 rows are re-cut to 32: a
+// 32-row band of 16 FP32 columns and its queue leave room in LDS for as many
+// waves as the registers do, a 64-row one for 13 of those 20.  64 against 32
+// rows: four NMF sweeps of rank 20 over 260,000 vertices 1.53 / 1.32 ms, a
+// training step at 131,072 vertices (k = 64) 0.88 / 0.80 ms, scale 16 FP64
+// k = 8 22 / 20 us, 700,001 x 10 FP32 106 / 106; one column, which pays for
+// every tile header, is slower (a PageRank sweep of 2^20 vertices 109 / 117
+// us).  16 rows lose 10% at k = 10 and 23% at k = 1.  A 64-row image stays as
+// it is.
 uint32_t work_rows_for(const fmx_spm *s)
 {
-    uint64_t h2 = 64;
+    uint64_t h2 = 32;
     if (const char *e = getenv("FMX_WORK_ROWS")) h2 = strtoull(e, nullptr, 10);
+    else if (s->H <= 64) return 0;
     if (h2 == 0 || (h2 & (h2 - 1)) || s->H <= h2) return 0;
     return (uint32_t)h2;
 }
