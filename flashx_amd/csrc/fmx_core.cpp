@@ -701,6 +701,28 @@ static int value_prim(fmx_dtype dt)
     }
 }
 
+// Whether an SpMM with X rows of rb bytes runs on the matrix's gather-order
+// image.  Never for rows of a full 128-byte line, which gain nothing from
+// lying next to another hot row.  Otherwise by the number of columns: the
+// narrower the rows, the more of them a line of the hot block serves, and
+// copying the hot rows has to be worth while.  R-MAT, 16 edges a vertex, plain /
+// gather-order image, us:
+//   4-byte rows   2^19 columns 44 / 39, 2^20 95 / 76, 2^21 225 / 154
+//   16-byte rows  2^18 35 / 37, 2^19 65 / 57, 2^20 148 / 102, 2^21 382 / 210
+//   40-byte rows  2^19 75 / 81, 700,001 85 / 85, 2^20 171 / 144
+//   64-byte rows  2^19 68 / 82, 2^20 144 / 143, 2^21 354 / 296
+// A weighted matrix is cut at tile starts only, and the hot columns' tiles are
+// large, so it gains later (2^20: 64-byte rows 205 / 285, 16-byte 261 / 224;
+// 2^21 with 8 edges a vertex: 273 / 279 and 395 / 246).
+// (FMX_HOT_MIN_BYTES, read at every call, puts an X-size threshold instead.)
+static bool gather_order_pays(const fmx_spm *s, uint64_t rb)
+{
+    if (rb >= 128) return false;
+    if (const char *hm = getenv("FMX_HOT_MIN_BYTES")) return s->ncols * rb > strtoull(hm, nullptr, 10);
+    if (s->esz) return s->ncols > std::max<uint64_t>(32768 * rb, 1500000);
+    return s->ncols > std::max<uint64_t>(16384 * rb, 300000);
+}
+
 // The SpMM entries (fmx_spmm, fmx_spmm_ex, fmx_spmm_scaled).
 fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, const double *pre,
                      const double *post, const void *X, int64_t ldx, void *Y, int64_t ldy, uint32_t flags,
@@ -735,14 +757,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     // in the sequential mode the reference's column order, re-cut if its
     // tiles are taller than a band
     const fmx_spm *orig = spm;
-    // the gather-order image pays where X's rows share 128-byte lines and X
-    // is larger than the XCDs' L2s together (32 MB): a row of a full line
-    // gains nothing from being next to another hot row, and a small X stays
-    // in L2 anyway, so only the restaging would remain
-    // (FMX_HOT_MIN_BYTES, read at every call, moves the X-size threshold)
-    const char *hm = getenv("FMX_HOT_MIN_BYTES");
-    const uint64_t min_x = hm ? strtoull(hm, nullptr, 10) : (32ull << 20);
-    const bool hot = !seq && spm->fast && (uint64_t)k * es < 128 && spm->ncols * (uint64_t)k * es > min_x;
+    const bool hot = !seq && spm->fast && gather_order_pays(spm, (uint64_t)k * es);
     if (hot) spm = spm->fast.get();
     else if (spm->work) spm = spm->work.get();
     Plan *plan = nullptr;
