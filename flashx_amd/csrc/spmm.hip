@@ -904,24 +904,35 @@ __global__ void __launch_bounds__(64 * kWPB) __attribute__((amdgpu_waves_per_eu(
     spmm_body<T, V, K, SEQ, HOT, NARROW>(a);
 }
 
-// Y rows of a split band = partial slots summed in stream order.
+// Y rows of a split band = partial slots summed in stream order: one element
+// per thread, four slots' loads in flight (a block per split that walked its
+// elements and slots one load at a time took 26 us after each rank-20 SpMM of
+// 260,000 vertices; 5 us like this).
 template <typename T, typename A>
 __global__ void __launch_bounds__(256) spmm_reduce(const Split *splits, const A *partial,
                                                     uint32_t hs, uint32_t k, T *Y, int64_t ldy,
                                                     const double *rscale, int ycol, int round_first)
 {
     const Split sp = splits[blockIdx.x];
-    const uint32_t tot = sp.rows * k;
-    for (uint32_t i = threadIdx.x; i < tot; i += blockDim.x) {
-        A acc = partial[(uint64_t)sp.slot_begin * hs * k + i];
-        for (uint32_t s = 1; s < sp.nslots; s++)
-            acc += partial[(uint64_t)(sp.slot_begin + s) * hs * k + i];
-        uint32_t r = i / k, c = i - r * k;
-        if constexpr (std::is_floating_point<T>::value)
-            if (rscale) acc = scaled<T>(round_first, acc, rscale[sp.row0 + r]);
-        if (ycol) Y[c * (uint64_t)ldy + sp.row0 + r] = (T)acc;
-        else Y[(sp.row0 + r) * (uint64_t)ldy + c] = (T)acc;
+    const uint32_t i = blockIdx.y * 256 + threadIdx.x;
+    if (i >= sp.rows * k) return;
+    const uint64_t step = (uint64_t)hs * k;
+    const A *p = partial + (uint64_t)sp.slot_begin * step + i;
+    A acc = p[0];
+    uint32_t s = 1;
+    for (; s + 4 <= sp.nslots; s += 4) {
+        A v[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) v[t] = p[(s + t) * step];
+#pragma unroll
+        for (int t = 0; t < 4; t++) acc += v[t];
     }
+    for (; s < sp.nslots; s++) acc += p[s * step];
+    const uint32_t r = i / k, c = i - r * k;
+    if constexpr (std::is_floating_point<T>::value)
+        if (rscale) acc = scaled<T>(round_first, acc, rscale[sp.row0 + r]);
+    if (ycol) Y[c * (uint64_t)ldy + sp.row0 + r] = (T)acc;
+    else Y[(sp.row0 + r) * (uint64_t)ldy + c] = (T)acc;
 }
 
 // Gathers in flight per lane group (kP): eight 16-byte gathers per lane keep
@@ -1094,7 +1105,7 @@ fmx_status launch_t(fmx_ctx *ctx, const fmx_spm *spm, const Plan *plan, int k,
     if (st) return st;
     if (reduce && plan->nsplits) {
         using A = typename AccOf<T>::type;
-        hipLaunchKernelGGL((spmm_reduce<T, A>), dim3(plan->nsplits), dim3(256), 0, stream,
+        hipLaunchKernelGGL((spmm_reduce<T, A>), dim3(plan->nsplits, (plan->hs * (uint32_t)k + 255) / 256), dim3(256), 0, stream,
                            plan->d_splits, (const A *)partial, plan->hs, (uint32_t)k, (T *)Y, ldy, rscale, a.ycol,
                            a.round_first);
         FMX_HIP(ctx, hipGetLastError());
