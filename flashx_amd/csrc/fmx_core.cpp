@@ -327,17 +327,14 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     std::unique_ptr<Plan> plan(new Plan());
     plan->hs = hs;
 
-    struct Band { uint64_t br; uint64_t row0; uint32_t sb_base, rows; uint32_t words; };
-    std::vector<Band> bands;
-    uint64_t total = 0;
+    auto rows_of = [&](uint64_t br) { return std::min<uint64_t>(s->H, s->nrows - br * s->H); };
+    auto words_of = [&](uint64_t br) { return (uint32_t)((s->offs[br + 1] - s->offs[br]) / 2); };
+    auto row_block = [&](const Item &t) { return (((uint64_t)t.row0_hi << 32) | t.row0_lo) >> s->log2h; };
+    uint64_t total = 0, nbands = 0;
     for (uint64_t br = 0; br < s->nbr; br++) {
-        uint64_t rows_here = std::min<uint64_t>(s->H, s->nrows - br * s->H);
-        uint32_t words = (uint32_t)((s->offs[br + 1] - s->offs[br]) / 2);
-        for (uint64_t sb = 0; sb * hs < rows_here; sb++) {
-            uint32_t rows = (uint32_t)std::min<uint64_t>(hs, rows_here - sb * hs);
-            bands.push_back({br, br * s->H + sb * hs, (uint32_t)(sb * hs), rows, words});
-            total += words;
-        }
+        const uint64_t nb = (rows_of(br) + hs - 1) / hs;
+        nbands += nb;
+        total += nb * words_of(br);
     }
     // Work cap: a band whose stream exceeds it is split into near-equal word
     // ranges reduced in order afterwards (power-law hub rows).  A matrix with
@@ -348,7 +345,7 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     // 25 at 1024 words, 26 at 512, 31 at 2048; 260,000 vertices, k = 20, four
     // NMF sweeps 4.6 ms, 2.5 at 2048, 2.7 at 1024, 3.0 at 4096; scale 20
     // weighted 485 us at 8192, 491 at 4096, 515 at 2048.
-    uint64_t avg = bands.empty() ? 0 : total / bands.size();
+    uint64_t avg = nbands ? total / nbands : 0;
     const uint64_t share = total / ((uint64_t)ctx->num_cus * 16);
     uint64_t cap = std::min(std::max<uint64_t>(8192, 4 * avg), std::max<uint64_t>(1024, share));
     const char *e = getenv("FMX_ITEM_CAP");
@@ -361,55 +358,58 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     // only: the ranges of split bands leave the host as plain fractions of
     // their block row, and a kernel moves them to where an item may start.
     const bool dev_cuts = s->dir.empty();
-    for (const Band &b : bands) {
-        uint32_t pieces = (uint32_t)(b.words / cap + (b.words % cap != 0));
+    std::vector<Item> items;  // in row order
+    items.reserve(nbands + std::min<uint64_t>(nbands, total / cap));
+    std::vector<uint32_t> cut, dirs, carries, keep;
+    for (uint64_t br = 0; br < s->nbr; br++)
+    for (uint64_t sb = 0, rows_here = rows_of(br); sb < rows_here; sb += hs) {
+        const uint32_t words = words_of(br);
+        const uint64_t row0 = br * s->H + sb;
+        uint32_t pieces = (uint32_t)(words / cap + (words % cap != 0));
         if (pieces < 1) pieces = 1;
         Item base{};
-        base.brow_word = (uint64_t)s->offs[b.br] / 2;
-        base.dir_end = s->brow_dir[b.br + 1];
-        base.row0_lo = (uint32_t)b.row0;
-        base.row0_hi = (uint32_t)(b.row0 >> 32);
-        base.sb_base = b.sb_base;
-        base.rows = b.rows;
+        base.brow_word = (uint64_t)s->offs[br] / 2;
+        base.dir_begin = s->brow_dir[br];
+        base.dir_end = s->brow_dir[br + 1];
+        base.row0_lo = (uint32_t)row0;
+        base.row0_hi = (uint32_t)(row0 >> 32);
+        base.sb_base = (uint32_t)sb;
+        base.rows = (uint32_t)std::min<uint64_t>(hs, rows_here - sb);
+        base.nwords = words;
+        base.carry = kNone;
+        base.slot = kNone;
         if (pieces == 1) {
-            Item t = base;
-            t.begin = 0;
-            t.nwords = b.words;
-            t.dir_begin = s->brow_dir[b.br];
-            t.carry = kNone;
-            t.slot = kNone;
-            plan->items.push_back(t);
+            items.push_back(base);
             continue;
         }
-        std::vector<uint32_t> cut(pieces + 1), dirs(pieces + 1, base.dir_end), carries(pieces + 1, kNone);
-        cut[0] = 0;
-        dirs[0] = s->brow_dir[b.br];
-        const uint2 *d = dev_cuts ? nullptr : s->dir.data() + s->brow_dir[b.br];
+        cut.assign(pieces + 1, 0);
+        dirs.assign(pieces + 1, s->brow_dir[br]);
+        carries.assign(pieces + 1, kNone);
+        const uint2 *d = dev_cuts ? nullptr : s->dir.data() + s->brow_dir[br];
         for (uint32_t i = 1; i < pieces; i++) {
-            uint32_t p = (uint32_t)((uint64_t)b.words * i / pieces);
-            dirs[i] = s->brow_dir[b.br];
+            uint32_t p = (uint32_t)((uint64_t)words * i / pieces);
             if (!dev_cuts) {
                 if (p <= cut[i - 1]) p = cut[i - 1] + 1;
-                const uint32_t t = tile_at(s, b.br, d, p);
-                const uint32_t tx = d[t - s->brow_dir[b.br]].x;
+                const uint32_t t = tile_at(s, br, d, p);
+                const uint32_t tx = d[t - s->brow_dir[br]].x;
                 if (s->esz) {
                     // weighted: cut at the tile start at or before p, so no row
                     // and no value position is carried into a piece
                     p = std::max(tx, cut[i - 1]);
                 } else {
                     if (p < tx + 8) p = tx + 8;  // out of the tile header
-                    carries[i] = carry_at(s, (uint64_t)s->offs[b.br] / 2, p);
+                    carries[i] = carry_at(s, (uint64_t)s->offs[br] / 2, p);
                 }
                 dirs[i] = t;
             }
             cut[i] = p;
         }
-        cut[pieces] = b.words;
+        cut[pieces] = words;
         // drop pieces emptied by header adjustment
-        std::vector<uint32_t> keep;
+        keep.clear();
         for (uint32_t i = 0; i < pieces; i++)
             if (cut[i] < cut[i + 1]) keep.push_back(i);
-        Split sp{b.row0, b.rows, nslots, (uint32_t)keep.size(), 0};
+        Split sp{row0, base.rows, nslots, (uint32_t)keep.size(), 0};
         for (uint32_t i : keep) {
             Item t = base;
             t.begin = cut[i];
@@ -417,13 +417,37 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
             t.dir_begin = dirs[i];
             t.carry = carries[i];
             t.slot = nslots++;
-            plan->items.push_back(t);
+            items.push_back(t);
         }
         splits.push_back(sp);
     }
-    // Longest items first, so the hardware dispatcher approximates LPT.
-    std::stable_sort(plan->items.begin(), plan->items.end(),
-                     [](const Item &a, const Item &b) { return a.nwords > b.nwords; });
+    // Longest items first, so the hardware dispatcher approximates LPT
+    // (streamed: the items of each chunk together, longest first within it):
+    // a stable counting sort of their places by size, in 4096 steps.
+    std::vector<uint32_t> order(items.size());
+    {
+        uint32_t longest = 0;
+        for (const Item &t : items) longest = std::max(longest, t.nwords);
+        int sh = 0;
+        while ((longest >> sh) >= 4096) sh++;
+        std::vector<uint32_t> at(4097, 0);
+        for (const Item &t : items) at[4096 - (t.nwords >> sh)]++;
+        for (int i = 1; i <= 4096; i++) at[i] += at[i - 1];
+        for (size_t i = 0; i < items.size(); i++) order[at[4095 - (items[i].nwords >> sh)]++] = (uint32_t)i;
+    }
+    if (s->streamed()) {
+        const std::vector<uint64_t> &cb = s->chunk_br;
+        const size_t nch = cb.size() - 1;
+        auto chunk_of = [&](const Item &t) {
+            return (size_t)(std::upper_bound(cb.begin(), cb.end(), row_block(t)) - cb.begin()) - 1;
+        };
+        plan->chunk_items.assign(nch + 1, 0);
+        for (const Item &t : items) plan->chunk_items[chunk_of(t) + 1]++;
+        for (size_t c = 0; c < nch; c++) plan->chunk_items[c + 1] += plan->chunk_items[c];
+        std::vector<uint32_t> at(plan->chunk_items.begin(), plan->chunk_items.end() - 1), by(order.size());
+        for (uint32_t i : order) by[at[chunk_of(items[i])]++] = i;
+        order.swap(by);
+    }
     // Column rotation (off unless FMX_ROT_SLOTS is set): item i (in dispatch
     // order) starts at the first of its tiles in block column
     // >= (i * nbc / slots) mod nbc and wraps around, so that items resident
@@ -434,8 +458,8 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     // every rotation rate tried was 5-10% slower than none.
     const char *re = getenv("FMX_ROT_SLOTS");
     const uint64_t slots = (re && !ordered && !s->dir.empty()) ? strtoull(re, nullptr, 10) : 0;
-    for (size_t i = 0; i < plan->items.size(); i++) {
-        Item &t = plan->items[i];
+    for (size_t i = 0; i < items.size(); i++) {
+        Item &t = items[order[i]];
         t.rot_begin = t.begin;
         t.rot_dir = t.dir_begin;
         if (slots == 0 || s->nbc < 2) continue;
@@ -453,11 +477,11 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
         }
     }
     // The kernel trusts these invariants; check them before anything runs.
-    for (const Item &t : plan->items) {
+    for (const Item &t : items) {
         // the first tile of the item starts at or before the item: the block
         // row's first tile at word 0, or the tile a cut fell in (plan_cuts
         // finds and checks that one for an image in HBM only)
-        const uint64_t br = (((uint64_t)t.row0_hi << 32) | t.row0_lo) / s->H;
+        const uint64_t br = row_block(t);
         bool first_ok = br < s->nbr;
         if (first_ok && (t.begin == 0 || dev_cuts)) {
             first_ok = t.dir_begin == s->brow_dir[br];
@@ -473,29 +497,17 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
         if (!ok) return fail(ctx, FMX_EINVAL, "internal error: inconsistent SpMM work item");
     }
     if (s->streamed()) {
-        // streamed: the items of each chunk together, longest first within it
-        const std::vector<uint64_t> &cb = s->chunk_br;
-        auto chunk_of = [&](const Item &t) {
-            const uint64_t br = (uint64_t)(((uint64_t)t.row0_hi << 32 | t.row0_lo) / s->H);
-            return (size_t)(std::upper_bound(cb.begin(), cb.end(), br) - cb.begin()) - 1;
-        };
-        std::stable_sort(plan->items.begin(), plan->items.end(),
-                         [&](const Item &a, const Item &b) { return chunk_of(a) < chunk_of(b); });
-        const size_t nch = cb.size() - 1;
-        plan->chunk_items.assign(nch + 1, 0);
-        for (const Item &t : plan->items) plan->chunk_items[chunk_of(t) + 1]++;
-        for (size_t c = 0; c < nch; c++) plan->chunk_items[c + 1] += plan->chunk_items[c];
         // a chunk's items stay inside the bytes staged for it
-        for (size_t c = 0; c < nch; c++)
+        for (size_t c = 0; c + 1 < s->chunk_br.size(); c++)
             for (uint32_t i = plan->chunk_items[c]; i < plan->chunk_items[c + 1]; i++) {
-                const Item &t = plan->items[i];
+                const Item &t = items[order[i]];
                 const uint64_t lo = 2 * ((t.brow_word + t.begin) & ~7ull);
                 const uint64_t hi = 2 * (((t.brow_word + t.begin + t.nwords - 1) | 7ull) + 1);
                 if (lo < s->chunk_lo[c] || hi > s->chunk_hi[c])
                     return fail(ctx, FMX_EINVAL, "internal error: work item outside its chunk");
             }
     }
-    plan->nitems = (uint32_t)plan->items.size();
+    plan->nitems = (uint32_t)items.size();
     plan->nslots = nslots;
     plan->nsplits = (uint32_t)splits.size();
     if (plan->nitems) {
@@ -511,13 +523,12 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
             host.resize(all);
             src = host.data();
         }
-        if (dev_cuts)  // plan_cuts takes a split item's block-row length from here
-            for (Item &t : plan->items)
-                if (t.slot != kNone) {
-                    const uint64_t br = (((uint64_t)t.row0_hi << 32) | t.row0_lo) / s->H;
-                    t.rot_begin = (uint32_t)((s->offs[br + 1] - s->offs[br]) / 2);
-                }
-        memcpy(src, plan->items.data(), ib);
+        Item *dst = (Item *)src;
+        for (size_t i = 0; i < items.size(); i++) {
+            dst[i] = items[order[i]];
+            // plan_cuts takes a split item's block-row length from here
+            if (dev_cuts && dst[i].slot != kNone) dst[i].rot_begin = words_of(row_block(dst[i]));
+        }
         if (plan->nsplits) memcpy(src + ib, splits.data(), all - ib);
         FMX_HIP(ctx, hipMemcpyAsync(plan->d_items, src, all, hipMemcpyHostToDevice, ctx->stream));
         const bool moved = dev_cuts && nslots;

@@ -64,7 +64,6 @@ struct Plan {
     uint32_t nsplits = 0;
     Item *d_items = nullptr;
     Split *d_splits = nullptr;  // in d_items' allocation
-    std::vector<Item> items;    // as built on the host (plan_cuts moves split ones on the device)
     // streamed matrices: the items of chunk c are [chunk_items[c], chunk_items[c+1])
     std::vector<uint32_t> chunk_items;
     ~Plan();
