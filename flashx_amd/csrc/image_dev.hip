@@ -148,9 +148,10 @@ __device__ __forceinline__ uint32_t tile_before(const uint2 *dir, uint32_t lo, u
 // a range inside one tile then becomes empty and its partial zero).  The row
 // in force at a binary item's first word, kNone if that word is a header
 // (row part or COO entry), is that of the nearest header before it: the
-// lanes read 64 words back at a time and a ballot finds it (a hub row's part
-// can be thousands of words long; the word behind the tile header always has
-// the header bit, so the search ends inside the tile).
+// lanes read 512 words back at a time and a ballot finds it (a hub row's part
+// can be 32768 words long, and 64 words a step made this the longest part of
+// a plan; the word behind the tile header always has the header bit, so the
+// search ends inside the tile).
 __global__ void __launch_bounds__(kT) fix_items(const uint16_t *img, const uint2 *dir, Item *items, uint32_t n,
                                                 int weighted, uint32_t *bad)
 {
@@ -173,17 +174,36 @@ __global__ void __launch_bounds__(kT) fix_items(const uint16_t *img, const uint2
     uint32_t carry = kNone;
     if (!weighted && end[0] != 0) {
         const uint16_t *w = img + t.brow_word;
-        const int64_t q = end[0];
+        const uint32_t q = end[0];
         if (!(w[q] & 0x8000u)) {
-            for (int64_t hi = q - 1;; hi -= 64) {
-                const int64_t at = hi - lane;
-                const uint32_t v = at >= 0 ? w[at] : 0x8000u;
-                const uint64_t m = __ballot((v & 0x8000u) != 0);
+            // 8-word groups of the image, aligned as the image is: lane l
+            // looks at group `top - l`, whose words before q and inside the
+            // block row count
+            const uint64_t at = t.brow_word + q;  // first word not looked at
+            for (uint64_t top = (at - 1) >> 3;; top -= 64) {
+                uint32_t head = 0;
+                bool any = false;
+                if (top >= (uint64_t)lane && (top - lane) * 8 + 7 >= t.brow_word) {
+                    const uint64_t g = (top - lane) * 8;
+                    const uint4 v = *(const uint4 *)(img + g);
+                    const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        const uint32_t word = (x[j >> 1] >> ((j & 1) * 16)) & 0xFFFFu;
+                        if (g + j >= t.brow_word && g + j < at && (word & 0x8000u)) {
+                            head = word;
+                            any = true;
+                        }
+                    }
+                }
+                const uint64_t m = __ballot(any);
                 if (m) {
-                    const int l0 = __ffsll((unsigned long long)m) - 1;  // nearest to q
-                    carry = __shfl(v, l0, 64) & 0x7FFFu;
+                    // the lowest such lane is the nearest group, its last
+                    // head the nearest word
+                    carry = __shfl(head, __ffsll((unsigned long long)m) - 1, 64) & 0x7FFFu;
                     break;
                 }
+                if (top < 64 || (top - 63) * 8 <= t.brow_word) break;  // (not reached: the tile has a header)
             }
         }
     }
