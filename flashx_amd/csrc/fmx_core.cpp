@@ -19,9 +19,66 @@ Plan::~Plan()
     if (d_items) (void)hipFree(d_items);  // d_splits lies behind them
 }
 
-Scratch::~Scratch()
+StreamScratch::~StreamScratch()
 {
-    if (ptr) (void)hipFree(ptr);
+    for (const Buf &b : bufs_) (void)hipFree(b.ptr);
+}
+
+fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, void **out)
+{
+    *out = nullptr;
+    if (!bytes) return FMX_OK;
+    calls_++;
+    unsigned long long graph = 0;
+    if (s) {  // the null stream cannot be captured
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamGetCaptureInfo(s, &cs, &graph) != hipSuccess) {
+            (void)hipGetLastError();
+            cs = hipStreamCaptureStatusNone;
+        }
+        if (cs != hipStreamCaptureStatusActive) graph = 0;
+        else if (!graph) graph = 1;
+    }
+    Buf *mine = nullptr, *eager = nullptr, *shared = nullptr;  // best of each kind
+    size_t neager = 0, ngraph = 0;
+    for (Buf &b : bufs_) {
+        if (b.stream == s && b.graph == graph && (!graph || b.bytes >= bytes)) mine = &b;
+        if (!b.graph) {
+            neager++;
+            // under capture the newest that is large enough, else the oldest
+            if (graph ? b.bytes >= bytes && (!eager || b.used > eager->used) : !eager || b.used < eager->used)
+                eager = &b;
+        } else {
+            ngraph++;
+            if (b.bytes >= bytes) shared = &b;
+        }
+    }
+    if (graph && !mine) {
+        mine = shared && (!eager || ngraph >= kGraphs) ? shared : eager;
+        if (mine && !mine->graph) {
+            mine->stream = s;
+            mine->graph = graph;
+        }
+    }
+    if (!graph && !mine && neager >= kStreams) {
+        FMX_HIP(ctx, hipDeviceSynchronize());
+        mine = eager;
+        mine->stream = s;
+    }
+    if (!mine || mine->bytes < bytes) {
+        if (mine) {
+            void *old = mine->ptr;
+            bufs_.erase(bufs_.begin() + (mine - bufs_.data()));
+            FMX_HIP(ctx, hipFree(old));
+        }
+        void *p = nullptr;
+        FMX_HIP(ctx, dev_malloc(ctx, &p, bytes));
+        bufs_.push_back({s, graph, calls_, p, bytes});
+        mine = &bufs_.back();
+    }
+    mine->used = calls_;
+    *out = mine->ptr;
+    return FMX_OK;
 }
 
 hipError_t BlockCache::get(size_t bytes, void **p, size_t *got)
@@ -586,8 +643,8 @@ fmx_status prepare_work(fmx_ctx *ctx, fmx_spm *s)
 // streams), and the copies wait for the caller's earlier work on its stream.
 // Split bands are reduced once, after the last chunk.
 fmx_status spmm_streamed(fmx_ctx *ctx, fmx_spm *spm, Plan *plan, fmx_dtype dtype, int k, const void *X,
-                         int64_t ldx, void *Y, int64_t ldy, hipStream_t s, const double *rscale, uint32_t flags,
-                         const void *Xhot = nullptr, uint64_t nhot = 0)
+                         int64_t ldx, void *Y, int64_t ldy, void *partial, hipStream_t s, const double *rscale,
+                         uint32_t flags, const void *Xhot = nullptr, uint64_t nhot = 0)
 {
     const size_t nch = spm->chunk_br.size() - 1;
     FMX_HIP(ctx, hipEventRecord(spm->ev_start, s));
@@ -604,7 +661,7 @@ fmx_status spmm_streamed(fmx_ctx *ctx, fmx_spm *spm, Plan *plan, fmx_dtype dtype
         FMX_HIP(ctx, hipStreamWaitEvent(s, spm->ev_copied[b], 0));
         // absolute word w of the image is at staging byte 2w - lo
         const uint16_t *img = (const uint16_t *)(spm->d_stage[b] - lo);
-        fmx_status st = launch_spmm(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, spm->partial.ptr, s, img,
+        fmx_status st = launch_spmm(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, partial, s, img,
                                     plan->chunk_items[c], plan->chunk_items[c + 1], c + 1 == nch, rscale, flags,
                                     Xhot, nhot);
         if (st) return st;
@@ -775,55 +832,43 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     fmx_status st = get_plan(ctx, spm, band_rows(spm, k, acc), seq, &plan);
     if (st) return st;
     size_t need = (size_t)plan->nslots * plan->hs * k * (dtype == FMX_F32 ? 8 : es);
-    if (need > spm->partial.bytes) {
-        if (spm->partial.ptr) FMX_HIP(ctx, hipFree(spm->partial.ptr));
-        spm->partial.ptr = nullptr;
-        spm->partial.bytes = 0;
-        FMX_HIP(ctx, dev_malloc(ctx, (void **)&spm->partial.ptr, need));
-        spm->partial.bytes = need;
-    }
+    void *partial = nullptr;
+    st = spm->partial.get(ctx, s, need, &partial);
+    if (st) return st;
     // a column-major or pre-scaled X is restaged row-major first (the
     // reference converts a non-row-major input, sparse_matrix.cpp:720-736)
     // X has orig's columns as rows: a gather-order image counts its hot
     // columns on top of them
     if ((xcol || pre) && orig->ncols) {
         const size_t xb = orig->ncols * (size_t)k * es;
-        if (xb > ctx->xstage.bytes) {
-            if (ctx->xstage.ptr) FMX_HIP(ctx, hipFree(ctx->xstage.ptr));
-            ctx->xstage.ptr = nullptr;
-            ctx->xstage.bytes = 0;
-            FMX_HIP(ctx, dev_malloc(ctx, (void **)&ctx->xstage.ptr, xb));
-            ctx->xstage.bytes = xb;
-        }
-        st = stage_dense_rows(ctx, dtype, orig->ncols, k, X, ldx, xcol, pre, ctx->xstage.ptr, s);
+        void *xs = nullptr;
+        st = ctx->xstage.get(ctx, s, xb, &xs);
         if (st) return st;
-        X = ctx->xstage.ptr;
+        st = stage_dense_rows(ctx, dtype, orig->ncols, k, X, ldx, xcol, pre, xs, s);
+        if (st) return st;
+        X = xs;
         ldx = k;
     }
     const uint32_t kflags = (flags & (FMX_SPMM_SEQ | FMX_SPMM_Y_COLMAJOR)) | (round_first ? kSpmmRoundFirst : 0u);
     if (hot) {
         // X's hot rows, densely, in the gather-order image's column order
         const size_t hb = orig->nhot * (size_t)k * es;
-        if (hb > ctx->xhot.bytes) {
-            if (ctx->xhot.ptr) FMX_HIP(ctx, hipFree(ctx->xhot.ptr));
-            ctx->xhot.ptr = nullptr;
-            ctx->xhot.bytes = 0;
-            FMX_HIP(ctx, dev_malloc(ctx, (void **)&ctx->xhot.ptr, hb));
-            ctx->xhot.bytes = hb;
-        }
-        st = stage_hot_rows(ctx, dtype, orig->nhot, k, X, ldx, orig->d_hot, ctx->xhot.ptr, s);
+        void *xh = nullptr;
+        st = ctx->xhot.get(ctx, s, hb, &xh);
+        if (st) return st;
+        st = stage_hot_rows(ctx, dtype, orig->nhot, k, X, ldx, orig->d_hot, xh, s);
         if (st) return st;
         if (spm->streamed())
-            return spmm_streamed(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, s, post, kflags, ctx->xhot.ptr,
+            return spmm_streamed(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, partial, s, post, kflags, xh,
                                  orig->nhot);
-        return launch_spmm(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, spm->partial.ptr, s,
-                           (const uint16_t *)spm->d_image, 0, plan->nitems, true, post, kflags, ctx->xhot.ptr,
+        return launch_spmm(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, partial, s,
+                           (const uint16_t *)spm->d_image, 0, plan->nitems, true, post, kflags, xh,
                            orig->nhot);
     }
     if (!spm->streamed())
-        return launch_spmm(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, spm->partial.ptr, s,
+        return launch_spmm(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, partial, s,
                            (const uint16_t *)spm->d_image, 0, plan->nitems, true, post, kflags);
-    return spmm_streamed(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, s, post, kflags);
+    return spmm_streamed(ctx, spm, plan, dtype, k, X, ldx, Y, ldy, partial, s, post, kflags);
 }
 
 }  // namespace fmx

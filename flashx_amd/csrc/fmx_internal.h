@@ -104,10 +104,31 @@ struct BlockScope {
 constexpr size_t kPinnedCounts = 0, kPinnedFlag = 4096, kPinnedHeader = 8192, kPinnedStage = 12288,
                  kPinnedBytes = kPinnedStage + (2 << 20);
 
-struct Scratch {
-    void *ptr = nullptr;
-    size_t bytes = 0;
-    ~Scratch();
+// Scratch of one purpose for calls on several streams: a buffer for each
+// stream that uses it, so that calls of one context on different streams do
+// not share one.  At most kStreams of them are kept; a further stream gets the
+// longest unused one, after the device has finished.  A buffer given to a call
+// under stream capture belongs to that capture's graph from then on (replays
+// may overlap any later call) and lives as long as its owner; nothing can be
+// allocated under capture, so that call takes a buffer that an earlier eager
+// call left, and, if there is none or captures hold kGraphs, shares an earlier
+// capture's.
+class StreamScratch {
+public:
+    ~StreamScratch();
+    fmx_status get(fmx_ctx *ctx, hipStream_t s, size_t bytes, void **out);
+
+private:
+    static constexpr size_t kStreams = 4, kGraphs = 8;
+    struct Buf {
+        hipStream_t stream;
+        unsigned long long graph;  // the capture it belongs to, 0 = none
+        uint64_t used;
+        void *ptr;
+        size_t bytes;
+    };
+    std::vector<Buf> bufs_;
+    uint64_t calls_ = 0;
 };
 
 }  // namespace fmx
@@ -120,8 +141,8 @@ struct fmx_ctx {
     size_t lds_per_block = 0;
     void *ws = nullptr;        // grow-only device workspace (dense-op partials)
     size_t ws_bytes = 0;
-    fmx::Scratch xstage;       // grow-only: a dense operand restaged row-major / pre-scaled
-    fmx::Scratch xhot;         // grow-only: the hot rows of X, densely (gather-order images)
+    fmx::StreamScratch xstage;  // a dense operand restaged row-major / pre-scaled
+    fmx::StreamScratch xhot;    // the hot rows of X, densely (gather-order images)
     void *noalloc_ws = nullptr;  // this device's copy of the fixed scratch (fmx_gram_noalloc)
     size_t noalloc_bytes = 0;
     void *pinned = nullptr;      // pinned host memory (kPinned*)
@@ -142,7 +163,7 @@ struct fmx_spm {
     std::vector<uint32_t> vdir;         // weighted images: values-region word (block-row relative)
     std::vector<uint32_t> brow_dir;     // first directory index per block row (+1)
     std::map<uint32_t, std::unique_ptr<fmx::Plan>> plans;
-    fmx::Scratch partial;               // partial bands of split items
+    fmx::StreamScratch partial;         // partial bands of split items
     // Out-of-core form (d_image == nullptr): the image stays in pinned host
     // memory and every SpMM streams it through two HBM staging buffers in
     // chunks of whole block rows; directory and plans stay in HBM.

@@ -303,3 +303,87 @@ def test_runtime_widths(fmx, orc, k, pad):
             spm.multiply_async(Xt, Y[:, :k])
             assert np.array_equal(Y[:, :k].cpu().numpy(), orc.spmm(im, X)), dt
             assert bool((Y[:, k:] == 77).all())
+
+
+@pytest.mark.parametrize("k,pad,tall", [(1, 0, True), (2, 1, True), (4, 0, True), (1, 2, False), (4, 4, False),
+                                        (5, 1, False), (8, 1, False), (16, 16, False)])
+def test_wide_queue_forms(fmx, orc, monkeypatch, k, pad, tall):
+    """Bands of 256 rows and more, and the gather order with X's rows further
+    apart than the hot block's: the forms whose queue entry holds a 32-bit
+    column and a 16-bit row.  Binary and weighted; small whole numbers, so
+    every type must be exact."""
+    import torch
+    if tall:
+        monkeypatch.setenv("FMX_WORK_ROWS", "0")
+        monkeypatch.setenv("FMX_HOT_MIN_BYTES", str(1 << 40))
+    else:
+        monkeypatch.setenv("FMX_HOT_MIN_BYTES", "0")
+    s, d = orc.rmat_edges(12, 16 << 12, seed=k)
+    n = (1 << 12) - 5
+    ok = (s < n) & (d < n)
+    s, d = s[ok], d[ok]
+    rng = np.random.default_rng(k)
+    lh = 12 if tall else 6
+    img = orc.build_2d(s, d, n=n, log2h=lh, log2w=10)
+    a = fmx.SparseMatrix.upload(img.data, img.offs)
+    for dt in (np.int32, np.int64, np.float32, np.float64):
+        vals = rng.integers(1, 5, s.size).astype(dt)
+        wimg = orc.build_2d_w(s, d, vals, n=n, log2h=lh, log2w=10)
+        w = fmx.SparseMatrix.upload(wimg.data, wimg.offs)
+        X = rng.integers(-9, 10, (n, k)).astype(dt)
+        buf = torch.zeros(n * (k + pad) - pad, dtype=torch.from_numpy(X).dtype, device="cuda")
+        Xt = buf.as_strided((n, k), (k + pad, 1))
+        Xt.copy_(torch.from_numpy(X))
+        for spm, im in ((a, img), (w, wimg)):
+            Y = torch.full((n, k), 77, dtype=Xt.dtype, device="cuda")
+            spm.multiply_async(Xt, Y)
+            assert np.array_equal(Y.cpu().numpy(), orc.spmm(im, X)), dt
+
+
+@pytest.mark.parametrize("hot", ["0", str(1 << 40)])
+def test_streams_and_graphs_keep_their_own_scratch(fmx, orc, rmat16, monkeypatch, hot):
+    """Calls on six streams at once, and a captured call replayed between
+    larger eager ones: the partial bands and the hot block of one never serve
+    another.  Integers, so every product must be exact."""
+    import torch
+    monkeypatch.setenv("FMX_HOT_MIN_BYTES", hot)
+    src, dst = rmat16
+    img = orc.build_2d(src, dst, n=1 << 16, log2h=15, log2w=15)
+    spm = fmx.SparseMatrix.upload(img.data, img.offs)
+    rng = np.random.default_rng(3)
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    X = [rng.integers(-9, 10, (img.n, 4)).astype(np.int32) for _ in streams]
+    ref = [orc.spmm(img, x) for x in X]
+    Xt = [to_dev(x) for x in X]
+    Y = [[torch.empty_like(x) for _ in range(4)] for x in Xt]
+    torch.cuda.synchronize()
+    for n in (2, 6):  # 2: one buffer each, 6: more streams than buffers
+        for r in range(4):
+            for i in range(n):
+                with torch.cuda.stream(streams[i]):
+                    spm.multiply_async(Xt[i], Y[i][r])
+        torch.cuda.synchronize()
+        for i in range(n):
+            for y in Y[i]:
+                assert np.array_equal(y.cpu().numpy(), ref[i]), (n, i)
+                y.zero_()
+        torch.cuda.synchronize()
+    Xg, Yg = Xt[0].clone(), torch.empty_like(Xt[0])
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        spm.multiply_async(Xg, Yg)
+    wide = rng.integers(-9, 10, (img.n, 16)).astype(np.int32)
+    Xw, refw = to_dev(wide), orc.spmm(img, wide)
+    Yw = torch.empty_like(Xw)
+    torch.cuda.synchronize()
+    for i in range(4):
+        Xg.copy_(Xt[i])
+        torch.cuda.synchronize()
+        Yg.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        with torch.cuda.stream(streams[i]):
+            spm.multiply_async(Xw, Yw)
+        torch.cuda.synchronize()
+        assert np.array_equal(Yg.cpu().numpy(), ref[i]), i
+        assert np.array_equal(Yw.cpu().numpy(), refw), i
