@@ -832,8 +832,12 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     fmx_status st = get_plan(ctx, spm, band_rows(spm, k, acc), seq, &plan);
     if (st) return st;
     size_t need = (size_t)plan->nslots * plan->hs * k * (dtype == FMX_F32 ? 8 : es);
+    // the partial bands of up to kSharedPartials lie in the context's buffer, so
+    // that a new matrix's first product does not allocate (57 to 390 us for
+    // 8 MB behind a freed matrix, against 34 for the product); larger ones
+    // are freed with their matrix
     void *partial = nullptr;
-    st = spm->partial.get(ctx, s, need, &partial);
+    st = (need <= kSharedPartials ? ctx->partial : spm->partial).get(ctx, s, need, &partial);
     if (st) return st;
     // a column-major or pre-scaled X is restaged row-major first (the
     // reference converts a non-row-major input, sparse_matrix.cpp:720-736)

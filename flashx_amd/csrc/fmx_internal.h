@@ -131,6 +131,8 @@ private:
     uint64_t calls_ = 0;
 };
 
+constexpr size_t kSharedPartials = size_t(64) << 20;
+
 }  // namespace fmx
 
 struct fmx_ctx {
@@ -143,6 +145,7 @@ struct fmx_ctx {
     size_t ws_bytes = 0;
     fmx::StreamScratch xstage;  // a dense operand restaged row-major / pre-scaled
     fmx::StreamScratch xhot;    // the hot rows of X, densely (gather-order images)
+    fmx::StreamScratch partial; // partial bands of split items, to kSharedPartials
     void *noalloc_ws = nullptr;  // this device's copy of the fixed scratch (fmx_gram_noalloc)
     size_t noalloc_bytes = 0;
     void *pinned = nullptr;      // pinned host memory (kPinned*)
@@ -163,7 +166,7 @@ struct fmx_spm {
     std::vector<uint32_t> vdir;         // weighted images: values-region word (block-row relative)
     std::vector<uint32_t> brow_dir;     // first directory index per block row (+1)
     std::map<uint32_t, std::unique_ptr<fmx::Plan>> plans;
-    fmx::StreamScratch partial;         // partial bands of split items
+    fmx::StreamScratch partial;         // partial bands of split items, above kSharedPartials
     // Out-of-core form (d_image == nullptr): the image stays in pinned host
     // memory and every SpMM streams it through two HBM staging buffers in
     // chunks of whole block rows; directory and plans stay in HBM.
