@@ -24,7 +24,7 @@
 // plan_cuts: the split items of a work plan, whose ranges come as fractions
 // of their block row, moved to where an item may start (one wave per item:
 // a binary search of the directory, then a search back for the row in
-// force, 64 words at a time).
+// force, 512 words at a time).
 #include "devprim.h"
 
 namespace fmx {

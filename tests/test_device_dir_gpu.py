@@ -111,3 +111,28 @@ def test_small_matrix_splits_by_its_share(fmx, n, lh, weighted):
         if not weighted:  # row 7 meets every column but its own
             want = X.double().sum(0) - X[7].double()
             assert np.array_equal(ya[7].double().cpu().numpy(), want.cpu().numpy())
+
+
+@pytest.mark.parametrize("n,lh,lw", [(32768, 6, 15), (32769, 15, 15), (100003, 6, 10), (100003, 4, 12),
+                                     ((1 << 23) + 5, 15, 15), ((1 << 24) + 1, 6, 13)])
+def test_column_counts_by_windows(fmx, monkeypatch, n, lh, lw):
+    """A device build counts its columns' uses by windows of 32768 columns (one
+    or two grouping passes; more than one window per block; block columns
+    narrower than a window); the host route counts them from the image.  The
+    gather-order images are the same, so FP32 sums agree to the bit."""
+    import torch
+    monkeypatch.setenv("FMX_HOT_MIN_BYTES", "0")
+    rng = np.random.default_rng(n + lh)
+    m = 200000
+    src = rng.integers(0, n, m).astype(np.int32)
+    dst = (n * rng.random(m) ** 3).astype(np.int32)  # some columns many times
+    dst[: m // 2 : 2] = n - 1 - (dst[: m // 2 : 2] % 40)
+    a = fmx.SparseMatrix.build(dev(src), dev(dst), n=n, log2_h=lh, log2_w=lw, flags=fmx.BUILD_DEDUP)
+    b, _ = host_route(fmx, a)
+    assert a.info.nnz == b.info.nnz
+    assert a.info.hot_columns == b.info.hot_columns > 0
+    X = torch.rand((n, 1), device="cuda")
+    ya, yb = torch.empty_like(X), torch.empty_like(X)
+    a.multiply_async(X, ya)
+    b.multiply_async(X, yb)
+    assert torch.equal(ya, yb)
