@@ -75,13 +75,115 @@ __global__ void __launch_bounds__(kT) pr_step(const float *out, const float *deg
     }
 }
 
-// X = max(X * N, eps) / (D + eps), element-wise in FP32 with each step
-// rounded (fm.pmax2(X * N, eps) / (den + eps), NMF.cpp:180-192,206-217).
-__global__ void __launch_bounds__(kT) nmf_mult_update(float *X, const float *N, const float *D, uint64_t len,
-                                                      float eps)
+// X = max(X * N, eps) / (X G + eps), X rows x k, G k x k: the denominators'
+// FP64 sums are rounded to FP32, and every FP32 step is rounded
+// (fm.pmax2(X * N, eps) / (den + eps), NMF.cpp:180-192,206-217).  The
+// denominators never reach memory: X and N are read and X written once, which
+// bounds it (260,000 x 20: 63 MB).  A block stages rows of X, and G, in LDS,
+// zero-padded to four columns; a thread keeps four rows by four columns, rows
+// `rg` apart so that neighbouring lanes read different banks.  FP64 FMAs and
+// the FP64 matrix cores run at one rate, and the former need no padding to 16.
+// 260,000 x 20: 19 us, where the product (22) and an element-wise update
+// reading its result (13) took 35; an iteration over 262,144 vertices, 8 edges
+// each: 122 / 97 us at 4 columns, 249 / 220 at 20, 949 / 683 at 64.
+constexpr int kUpdRows = 4, kUpdCols = 4;
+
+struct UpdShape {
+    int k, k4, cg, rg, ks;  // columns, padded to 4; column groups, row groups; LDS row stride of X (words)
+    __host__ __device__ explicit UpdShape(int k_) : k(k_)
+    {
+        k4 = (k + 3) & ~3;
+        cg = k4 / kUpdCols;
+        rg = kT / cg;
+        ks = k4 % 8 ? k4 : k4 + 4;
+    }
+    __host__ __device__ int rows() const { return kUpdRows * rg; }
+    size_t lds() const { return (size_t)k4 * k4 * 8 + (size_t)rows() * ks * 4; }
+};
+
+template <bool VEC>
+__global__ void __launch_bounds__(kT) nmf_update(float *X, const float *N, const double *G, uint64_t n, int k_,
+                                                 float eps)
 {
-    for (uint64_t i = blockIdx.x * (uint64_t)kT + threadIdx.x; i < len; i += (uint64_t)gridDim.x * kT)
-        X[i] = __fdiv_rn(fmaxf(__fmul_rn(X[i], N[i]), eps), __fadd_rn(D[i], eps));
+    extern __shared__ double lds_g[];
+    const UpdShape f(k_);
+    float *lds_x = (float *)(lds_g + f.k4 * f.k4);
+    for (int e = threadIdx.x; e < f.k4 * f.k4; e += kT) {
+        const int i = e / f.k4, j = e % f.k4;
+        lds_g[e] = i < f.k && j < f.k ? G[i * f.k + j] : 0.0;
+    }
+    const int r = threadIdx.x / f.cg, c0 = threadIdx.x % f.cg * kUpdCols;
+    for (uint64_t t0 = blockIdx.x * (uint64_t)f.rows(); t0 < n; t0 += gridDim.x * (uint64_t)f.rows()) {
+        const int rows = (int)min((uint64_t)f.rows(), n - t0);
+        __syncthreads();  // the last tile's rows are read
+        if constexpr (VEC) {
+            for (int e = threadIdx.x; e < rows * f.cg; e += kT)
+                *(float4 *)(lds_x + e / f.cg * f.ks + e % f.cg * 4) = *(const float4 *)(X + t0 * f.k + e * 4);
+        } else {
+            for (int e = threadIdx.x; e < rows * f.k4; e += kT) {
+                const int i = e / f.k4, j = e % f.k4;
+                lds_x[i * f.ks + j] = j < f.k ? X[(t0 + i) * f.k + j] : 0.0f;
+            }
+        }
+        __syncthreads();
+        if (r >= f.rg || r >= rows) continue;  // every thread reaches the next tile's barrier
+        float num[kUpdRows][kUpdCols];
+#pragma unroll
+        for (int q = 0; q < kUpdRows; q++) {
+            const int row = r + q * f.rg;
+            const float *p = N + (t0 + row) * f.k + c0;
+            if constexpr (VEC) {
+                const float4 v = row < rows ? *(const float4 *)p : float4{0, 0, 0, 0};
+                num[q][0] = v.x;
+                num[q][1] = v.y;
+                num[q][2] = v.z;
+                num[q][3] = v.w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < kUpdCols; j++) num[q][j] = row < rows && c0 + j < f.k ? p[j] : 0.0f;
+            }
+        }
+        double acc[kUpdRows][kUpdCols] = {};
+        const float *xr[kUpdRows];  // (rows past the end read the first row)
+#pragma unroll
+        for (int q = 0; q < kUpdRows; q++) xr[q] = lds_x + (r + q * f.rg < rows ? r + q * f.rg : r) * f.ks;
+        for (int i = 0; i < f.k4; i += 4) {
+            float x[kUpdRows][4];
+#pragma unroll
+            for (int q = 0; q < kUpdRows; q++) {
+                const float4 v = *(const float4 *)(xr[q] + i);
+                x[q][0] = v.x;
+                x[q][1] = v.y;
+                x[q][2] = v.z;
+                x[q][3] = v.w;
+            }
+#pragma unroll
+            for (int h = 0; h < 4; h++) {
+                const double *g = lds_g + (i + h) * f.k4 + c0;
+#pragma unroll
+                for (int j = 0; j < kUpdCols; j++)
+#pragma unroll
+                    for (int q = 0; q < kUpdRows; q++) acc[q][j] = fma((double)x[q][h], g[j], acc[q][j]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kUpdRows; q++) {
+            const int row = r + q * f.rg;
+            if (row >= rows) continue;
+            float y[kUpdCols];
+#pragma unroll
+            for (int j = 0; j < kUpdCols; j++)
+                y[j] = __fdiv_rn(fmaxf(__fmul_rn(xr[q][c0 + j], num[q][j]), eps), __fadd_rn((float)acc[q][j], eps));
+            float *p = X + (t0 + row) * f.k + c0;
+            if constexpr (VEC) {
+                *(float4 *)p = float4{y[0], y[1], y[2], y[3]};
+            } else {
+#pragma unroll
+                for (int j = 0; j < kUpdCols; j++)
+                    if (c0 + j < f.k) p[j] = y[j];
+            }
+        }
+    }
 }
 
 }  // namespace
@@ -198,23 +300,27 @@ fmx_status fmx_nmf(fmx_ctx *ctx, const fmx_spm *A, const fmx_spm *At, int k, int
         (void)hipFree(buf);
         return fail(ctx, FMX_ENOMEM, "NMF Gram buffers");
     }
-    float *P = buf, *Q = buf + big;  // (m|n) x k products and denominators
+    float *P = buf, *Q = buf + big;  // (m|n) x k products; the distance's tH W^T W
     double *G = g, *G2 = g + (size_t)k * k;
     std::vector<double> h1((size_t)k * k), h2((size_t)k * k);
-    auto upd = [&](float *X, const float *N, const float *D, uint64_t rows) {
-        const uint64_t len = rows * (uint64_t)k;
-        hipLaunchKernelGGL(nmf_mult_update, dim3(grid_for_n(ctx, len)), dim3(kT), 0, s, X, N, D, len, eps);
+    auto upd = [&](float *X, const double *den, uint64_t rows) {
+        const UpdShape f(k);
+        const uint64_t tiles = (rows + f.rows() - 1) / f.rows();
+        const dim3 grid((uint32_t)std::min<uint64_t>(tiles, (uint64_t)ctx->num_cus * 8));
+        if (!tiles) return FMX_OK;
+        if (k % 4 == 0 && (uintptr_t)X % 16 == 0)
+            hipLaunchKernelGGL(nmf_update<true>, grid, dim3(kT), f.lds(), s, X, P, den, rows, k, eps);
+        else
+            hipLaunchKernelGGL(nmf_update<false>, grid, dim3(kT), f.lds(), s, X, P, den, rows, k, eps);
         return hipGetLastError() == hipSuccess ? FMX_OK : fail(ctx, FMX_EHIP, "NMF update launch");
     };
     fmx_status st = gram(ctx, FMX_F32, FMX_GRAM_F64, n, k, k, W, k, W, k, G, s);  // W^T W
     for (int it = 0; !st && it < max_iters; it++) {
-        if (!st) st = gemm_tall(ctx, FMX_F32, m, k, k, 1.0, tH, k, G, 0.0, Q, k, s);
         if (!st) st = fmx_spmm(ctx, At, FMX_F32, k, W, k, P, k, s);
-        if (!st) st = upd(tH, P, Q, m);
+        if (!st) st = upd(tH, G, m);
         if (!st) st = gram(ctx, FMX_F32, FMX_GRAM_F64, m, k, k, tH, k, tH, k, G2, s);  // H H^T
-        if (!st) st = gemm_tall(ctx, FMX_F32, n, k, k, 1.0, W, k, G2, 0.0, Q, k, s);
         if (!st) st = fmx_spmm(ctx, A, FMX_F32, k, tH, k, P, k, s);
-        if (!st) st = upd(W, P, Q, n);
+        if (!st) st = upd(W, G2, n);
         if (!st) st = gram(ctx, FMX_F32, FMX_GRAM_F64, n, k, k, W, k, W, k, G, s);
         if (!st && dist && it % 5 == 0) {
             st = fmx_spmm(ctx, At, FMX_F32, k, W, k, P, k, s);                            // A^T W

@@ -139,3 +139,28 @@ def test_pagerank_counts_every_block(fmx, orc, n, iters):
     ring = torch.arange(n, dtype=torch.int32, device="cuda")
     R = fmx.SparseMatrix.build(ring, (ring + 1) % n, n=n, log2_h=9, log2_w=12)
     assert fmx.pagerank(R, fmx.SparseMatrix.build((ring + 1) % n, ring, n=n, log2_h=9, log2_w=12), max_iters=5)[1] == 1
+
+
+@pytest.mark.parametrize("k,off", [(1, 0), (4, 0), (4, 1), (5, 0), (20, 0), (32, 1), (33, 0), (64, 0)])
+def test_nmf_update_widths(fmx, orc, k, off):
+    """One iteration at widths around the update kernel's column groups, rows
+    that end inside a tile, and factors that are not 16-byte aligned."""
+    import torch
+    n = (1 << 12) + 3
+    s, d = orc.rmat_edges(12, 8 << 12, 9)
+    img = orc.build_2d(s, d, n=n, log2h=8, log2w=11, flags=orc.DEDUP | orc.SYMMETRIZE)
+    A = fmx.SparseMatrix.upload(img.data, img.offs)
+    rng = np.random.default_rng(k)
+    W0 = rng.random((n, k)).astype(np.float32)
+    tH0 = rng.random((n, k)).astype(np.float32)
+
+    def at(x):
+        buf = torch.zeros(n * k + off, dtype=torch.float32, device="cuda")
+        v = buf[off:].view(n, k)
+        v.copy_(torch.from_numpy(x))
+        return v
+
+    W, tH, dist = fmx.nmf(A, k, 1, W=at(W0), tH=at(tH0))
+    rW, rtH, rdist = orc.nmf(img, img, W0, tH0, 1, A.get_nnz())
+    assert _rel(W.cpu().numpy(), rW) <= 1e-5 and _rel(tH.cpu().numpy(), rtH) <= 1e-5
+    assert abs(dist[0] - rdist[0]) <= 1e-6 * abs(rdist[0])
