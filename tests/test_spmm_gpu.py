@@ -387,3 +387,34 @@ def test_streams_and_graphs_keep_their_own_scratch(fmx, orc, rmat16, monkeypatch
         torch.cuda.synchronize()
         assert np.array_equal(Yg.cpu().numpy(), ref[i]), i
         assert np.array_equal(Yw.cpu().numpy(), refw), i
+
+
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 1000])
+@pytest.mark.parametrize("k", [1, 2, 4, 7, 31, 32, 33, 64, 67])
+def test_restaged_operands(fmx, orc, n, k):
+    """Column-major and scaled operands at the edges of the restaging tiles
+    (128 rows, 32 columns, 16-byte pieces, unaligned bases and strides): a ring
+    moves each row of X to its neighbour, and powers of two scale exactly."""
+    import torch
+    i = np.arange(n, dtype=np.uint32)
+    img = orc.build_2d(i, (i + 1) % n, n=n, log2h=6, log2w=10, flags=orc.DEDUP | 2)
+    spm = fmx.SparseMatrix.upload(img.data, img.offs)
+    assert spm.get_nnz() == n
+    rng = np.random.default_rng(n + k)
+    pre = 2.0 ** rng.integers(-3, 4, n)
+    pd = torch.from_numpy(pre).cuda()
+    for dt in (np.int32, np.int64, np.float32, np.float64):
+        X = rng.integers(-99, 100, (n, k)).astype(dt)
+        td = torch.from_numpy(X).dtype
+        ref = np.roll(X, -1, axis=0)
+        col = torch.zeros((k, n + 3), dtype=td, device="cuda")[:, 1 : n + 1].t()
+        wide = torch.zeros((n, k + 5), dtype=td, device="cuda")[:, 1 : k + 1]
+        row = torch.zeros((n, k), dtype=td, device="cuda")
+        for x in (col, wide, row):
+            x.copy_(torch.from_numpy(X))
+            Y = torch.empty((n, k), dtype=td, device="cuda")
+            spm.multiply_async(x, Y)
+            assert np.array_equal(Y.cpu().numpy(), ref), (dt, x.stride())
+            if np.issubdtype(dt, np.floating):
+                spm.multiply_scaled_async(x, Y, pre=pd)
+                assert np.array_equal(Y.cpu().numpy(), np.roll(X * pre[:, None], -1, axis=0).astype(dt)), (dt, x.stride())
