@@ -400,11 +400,14 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     // bands' chunks one after the other, so its cap is its share of 16 waves
     // per CU, at least two chunks: R-MAT scale 16, FP64 k = 8, 73 us uncapped,
     // 25 at 1024 words, 26 at 512, 31 at 2048; 260,000 vertices, k = 20, four
-    // NMF sweeps 4.6 ms, 2.5 at 2048, 2.7 at 1024, 3.0 at 4096; scale 20
-    // weighted 485 us at 8192, 491 at 4096, 515 at 2048.
-    uint64_t avg = nbands ? total / nbands : 0;
-    const uint64_t share = total / ((uint64_t)ctx->num_cus * 16);
-    uint64_t cap = std::min(std::max<uint64_t>(8192, 4 * avg), std::max<uint64_t>(1024, share));
+    // NMF sweeps 4.6 ms, 2.5 at 2048, 2.7 at 1024, 3.0 at 4096.  A
+    // weighted image's words are counted without its values, which are only
+    // read by their entries: R-MAT scale 16 FP32 k = 16, 29 us at 1024 words
+    // in all, 24 at 2304 (1024 of entries), 28 at 6144, scale 20 (plain
+    // order) 245, 332 and 230 at 4096, 2048 and 6144, 215 at 18432.
+    const uint64_t avg = nbands ? total / nbands : 0, share = total / ((uint64_t)ctx->num_cus * 16);
+    const uint64_t img = s->bytes / 2, ent = std::max<uint64_t>(1, img - s->nnz * (s->esz / 2));
+    uint64_t cap = std::min(std::max<uint64_t>(8192 * img / ent, 4 * avg), std::max<uint64_t>(1024 * img / ent, share));
     const char *e = getenv("FMX_ITEM_CAP");
     if (e) cap = std::max<uint64_t>(64, strtoull(e, nullptr, 10));
     if (ordered) cap = UINT64_MAX;  // one item per band: its rows are summed in stream order
@@ -417,7 +420,7 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     const bool dev_cuts = s->dir.empty();
     std::vector<Item> items;  // in row order
     items.reserve(nbands + std::min<uint64_t>(nbands, total / cap));
-    std::vector<uint32_t> cut, dirs, carries, keep;
+    std::vector<uint32_t> cut, dirs, carries, befores, keep;
     for (uint64_t br = 0; br < s->nbr; br++)
     for (uint64_t sb = 0, rows_here = rows_of(br); sb < rows_here; sb += hs) {
         const uint32_t words = words_of(br);
@@ -442,21 +445,36 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
         cut.assign(pieces + 1, 0);
         dirs.assign(pieces + 1, s->brow_dir[br]);
         carries.assign(pieces + 1, kNone);
+        befores.assign(pieces + 1, 0);
+        uint32_t ctile = kNone, cpos = 0, centries = 0;  // weighted: entries of a tile counted so far
         const uint2 *d = dev_cuts ? nullptr : s->dir.data() + s->brow_dir[br];
         for (uint32_t i = 1; i < pieces; i++) {
             uint32_t p = (uint32_t)((uint64_t)words * i / pieces);
             if (!dev_cuts) {
-                if (p <= cut[i - 1]) p = cut[i - 1] + 1;
-                const uint32_t t = tile_at(s, br, d, p);
-                const uint32_t tx = d[t - s->brow_dir[br]].x;
+                if (p <= cut[i - 1] && !s->esz) p = cut[i - 1] + 1;
+                const uint32_t t = tile_at(s, br, d, p), l = t - s->brow_dir[br];
+                const uint32_t tx = d[l].x;
+                const uint64_t at = (uint64_t)s->offs[br] / 2;
                 if (s->esz) {
-                    // weighted: cut at the tile start at or before p, so no row
-                    // and no value position is carried into a piece
-                    p = std::max(tx, cut[i - 1]);
-                } else {
-                    if (p < tx + 8) p = tx + 8;  // out of the tile header
-                    carries[i] = carry_at(s, (uint64_t)s->offs[br] / 2, p);
+                    // weighted: the cut's place in the tile, values and all,
+                    // as a place among its entries' words (values are only
+                    // read by their entries, so a piece's work is its
+                    // entries); the piece needs the number of entries of the
+                    // tile before it to find its values
+                    const uint32_t te = l + 1 < s->brow_dir[br + 1] - s->brow_dir[br] ? d[l + 1].x : words;
+                    p = tx + 8 + (uint32_t)((uint64_t)(p - tx) * (s->vdir[t] - tx - 8) / (te - tx));
+                    const uint16_t *w = reinterpret_cast<const uint16_t *>(s->host_image()) + at;
+                    if (ctile != t) {
+                        ctile = t;
+                        cpos = tx + 8;
+                        centries = 0;
+                    }
+                    for (; cpos < p; cpos++) centries += !(w[cpos] & 0x8000);
+                    befores[i] = centries;
+                } else if (p < tx + 8) {
+                    p = tx + 8;  // out of the tile header
                 }
+                if (!s->esz || (p < s->vdir[t] && p > tx + 8)) carries[i] = carry_at(s, at, p);
                 dirs[i] = t;
             }
             cut[i] = p;
@@ -473,6 +491,7 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
             t.nwords = cut[i + 1] - cut[i];
             t.dir_begin = dirs[i];
             t.carry = carries[i];
+            t.before = befores[i];
             t.slot = nslots++;
             items.push_back(t);
         }
@@ -779,15 +798,16 @@ static int value_prim(fmx_dtype dt)
 //   16-byte rows  2^18 35 / 37, 2^19 65 / 57, 2^20 148 / 102, 2^21 382 / 210
 //   40-byte rows  2^19 75 / 81, 700,001 85 / 85, 2^20 171 / 144
 //   64-byte rows  2^19 68 / 82, 2^20 144 / 143, 2^21 354 / 296
-// A weighted matrix is cut at tile starts only, and the hot columns' tiles are
-// large, so it gains later (2^20: 64-byte rows 205 / 285, 16-byte 261 / 224;
-// 2^21 with 8 edges a vertex: 273 / 279 and 395 / 246).
+// A weighted matrix gains sooner, with fewer tiles to step through: at 2^17
+// 4- to 80-byte rows are even (64-byte 42 / 43), at 2^18 37 / 33, 16-byte
+// 54 / 47, 64-byte 64 / 59, 80-byte 77 / 71, at 2^20 134 / 108, 218 / 163,
+// 215 / 183, 280 / 257 (with 4 edges a vertex 54 / 49 to 106 / 106).
 // (FMX_HOT_MIN_BYTES, read at every call, puts an X-size threshold instead.)
 static bool gather_order_pays(const fmx_spm *s, uint64_t rb)
 {
     if (rb >= 128) return false;
     if (const char *hm = getenv("FMX_HOT_MIN_BYTES")) return s->ncols * rb > strtoull(hm, nullptr, 10);
-    if (s->esz) return s->ncols > std::max<uint64_t>(32768 * rb, 1500000);
+    if (s->esz) return s->ncols > 200000;
     return s->ncols > std::max<uint64_t>(16384 * rb, 300000);
 }
 

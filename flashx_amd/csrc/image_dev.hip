@@ -144,16 +144,18 @@ __device__ __forceinline__ uint32_t tile_before(const uint2 *dir, uint32_t lo, u
 // Split items (slot != kNone) of a plan: item words [begin, begin + nwords)
 // of a block row of rot_begin words, dir_begin its first directory entry.
 // Both ends move the same way, so neighbouring items still meet: out of the
-// header of the tile they fall in (binary), or back to its start (weighted;
-// a range inside one tile then becomes empty and its partial zero).  The row
-// in force at a binary item's first word, kNone if that word is a header
+// header of the tile they fall in (binary), or to the same fraction of its
+// entries' words as they have of the whole tile (weighted: the values behind
+// them are only read by their entries).  A weighted item also gets the number
+// of its tile's entries before it, the place of its first value.  The row
+// in force at an item's first word, kNone if that word is a header
 // (row part or COO entry), is that of the nearest header before it: the
 // lanes read 512 words back at a time and a ballot finds it (a hub row's part
 // can be 32768 words long, and 64 words a step made this the longest part of
 // a plan; the word behind the tile header always has the header bit, so the
 // search ends inside the tile).
-__global__ void __launch_bounds__(kT) fix_items(const uint16_t *img, const uint2 *dir, Item *items, uint32_t n,
-                                                int weighted, uint32_t *bad)
+__global__ void __launch_bounds__(kT) fix_items(const uint16_t *img, const uint2 *dir, const uint32_t *vdir,
+                                                Item *items, uint32_t n, uint32_t *bad)
 {
     const int lane = threadIdx.x & 63;
     const uint32_t i = blockIdx.x * (kT / 64) + (threadIdx.x >> 6);
@@ -161,18 +163,41 @@ __global__ void __launch_bounds__(kT) fix_items(const uint16_t *img, const uint2
     const Item t = items[i];
     if (t.slot == kNone) return;
     const uint32_t words = t.rot_begin, d0 = t.dir_begin, d1 = t.dir_end;
-    uint32_t end[2], tile = d0;
+    uint32_t end[2], tile = d0, inside = 0;  // words of the tile's entries before the item
     for (int e = 0; e < 2; e++) {
         uint32_t p = e ? t.begin + t.nwords : t.begin;
         if (p != 0 && p < words) {
             const uint32_t at = tile_before(dir, d0, d1, p), x = dir[at].x;
-            p = weighted ? x : max(p, x + 8);
-            if (e == 0) tile = at;
+            if (vdir) {
+                const uint32_t next = at + 1 < d1 ? dir[at + 1].x : words;
+                p = x + 8 + (uint32_t)((uint64_t)(p - x) * (vdir[at] - x - 8) / (next - x));
+            } else {
+                p = max(p, x + 8);
+            }
+            if (e == 0) {
+                tile = at;
+                inside = p - (x + 8);
+            }
         }
         end[e] = p;
     }
-    uint32_t carry = kNone;
-    if (!weighted && end[0] != 0) {
+    uint32_t carry = kNone, before = 0;
+    if (vdir && inside) {
+        // the entries among the `inside` words before the item
+        const uint64_t stop = t.brow_word + end[0], start = stop - inside;
+#pragma unroll 4
+        for (uint64_t g = (start & ~7ull) + lane * 8; g < stop; g += 512) {
+            const uint4 v = *(const uint4 *)(img + g);
+            const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint32_t word = x[j >> 1] >> ((j & 1) * 16);
+                before += g + j >= start && g + j < stop && !(word & 0x8000u);
+            }
+        }
+        for (int d = 32; d; d >>= 1) before += __shfl_xor(before, d, 64);
+    }
+    if (end[0] != 0 && (!vdir || (inside && end[0] < vdir[tile]))) {
         const uint16_t *w = img + t.brow_word;
         const uint32_t q = end[0];
         if (!(w[q] & 0x8000u)) {
@@ -214,6 +239,7 @@ __global__ void __launch_bounds__(kT) fix_items(const uint16_t *img, const uint2
     o->nwords = end[1] - end[0];
     o->dir_begin = o->rot_dir = tile;
     o->carry = carry;
+    o->before = before;
 }
 
 uint32_t grid_for(fmx_ctx *ctx, uint64_t n)
@@ -321,7 +347,7 @@ fmx_status plan_cuts(fmx_ctx *ctx, const fmx_spm *s, Item *items, uint32_t n)
     uint32_t *bad = (uint32_t *)((char *)ctx->pinned + kPinnedFlag);
     *(volatile uint32_t *)bad = 0;
     hipLaunchKernelGGL(fix_items, dim3((n + kT / 64 - 1) / (kT / 64)), dim3(kT), 0, ctx->stream,
-                       (const uint16_t *)s->d_image, s->d_dir, items, n, s->esz ? 1 : 0, bad);
+                       (const uint16_t *)s->d_image, s->d_dir, s->esz ? s->d_vdir : nullptr, items, n, bad);
     FMX_HIP(ctx, hipGetLastError());
     return FMX_OK;
 }

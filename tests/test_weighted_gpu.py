@@ -156,3 +156,29 @@ def test_weighted_tiles_starting_at_chunk_edges(fmx, orc, dt, lh, lw):
     for k in (1, 4, 16):
         X = (rng.integers(-7, 8, (n, k)) if np.issubdtype(dt, np.integer) else rng.random((n, k))).astype(dt)
         compare(spm.multiply(to_dev(X)).cpu().numpy(), orc.spmm(img, X))
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64, np.float32, np.float64])
+@pytest.mark.parametrize("lh,lw,cap,hot", [(6, 15, "64", False), (13, 15, "64", False), (6, 9, "100", False),
+                                           (6, 15, "96", True), (5, 8, "2000", True)])
+def test_weighted_cuts_inside_tiles(fmx, orc, monkeypatch, dt, lh, lw, cap, hot):
+    """Pieces of a split band start inside a tile's entries, with the row in
+    force and the place of the first value, on an uploaded image (cut on the
+    host) and a device-built one; small whole numbers, so every type must be
+    exact."""
+    import torch
+    monkeypatch.setenv("FMX_ITEM_CAP", cap)
+    monkeypatch.setenv("FMX_HOT_MIN_BYTES", "0" if hot else str(1 << 40))
+    n = (1 << 13) + 11
+    s, d = orc.rmat_edges(13, 12 << 13, seed=lw)
+    rng = np.random.default_rng(lh + lw)
+    v = rng.integers(1, 9, s.size).astype(dt)
+    img = orc.build_2d_w(s, d, v, n=n, log2h=lh, log2w=lw)
+    up = fmx.SparseMatrix.upload(img.data, img.offs)
+    dev = fmx.SparseMatrix.build_weighted(to_dev(s.astype(np.int32)), to_dev(d.astype(np.int32)), to_dev(v), n=n,
+                                          log2_h=lh, log2_w=lw, flags=fmx.BUILD_DEDUP)
+    for k in (1, 5, 16):
+        X = rng.integers(-7, 8, (n, k)).astype(dt)
+        ref = orc.spmm(img, X)
+        for a in (up, dev):
+            assert np.array_equal(a.multiply(to_dev(X)).cpu().numpy(), ref), k
