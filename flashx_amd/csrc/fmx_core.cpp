@@ -106,7 +106,7 @@ hipError_t BlockCache::get(size_t bytes, void **p, size_t *got)
 
 void BlockCache::put(void *p, size_t bytes)
 {
-    if (scopes && held_ + bytes <= kKeep) {
+    if (scopes) {
         free_.emplace_back(bytes, p);
         held_ += bytes;
     } else {

@@ -76,10 +76,14 @@ struct Plan {
 // 25 us from 4 MB and 360 us from 256 MB (a build of 16.8 M edges spent 11 of
 // its 16.5 ms in them).  Everything that uses them runs on the context's
 // stream, so a block may be handed on while kernels that use it are still
-// queued.  At most kKeep bytes are kept while a scope is open and kRest when
-// it is closed, the largest blocks going back first; all of them go back when
-// an allocation fails and with the context, which one host thread uses at a
-// time.  Blocks outside a scope are allocated and freed as they come.
+// queued.  While a scope is open every block is kept, and kRest bytes when it
+// is closed, the largest blocks going back first; all of them go back when an
+// allocation fails and with the context, which one host thread uses at a time.
+// kRest covers the buffers of some 2^27 edges: the driver clears what is freed
+// at about 200 GB/s behind the program's back, during which allocations wait
+// and copies from the host run at half their rate (a matrix streamed right
+// after builds that gave their buffers back: 8.0 ms a product instead of 4.0).
+// Blocks outside a scope are allocated and freed as they come.
 class BlockCache {
 public:
     ~BlockCache() { trim(0); }
@@ -87,7 +91,7 @@ public:
     void put(void *p, size_t bytes);
     void trim(size_t most);
     int scopes = 0;
-    static constexpr size_t kKeep = size_t(2) << 30, kRest = size_t(1) << 30;
+    static constexpr size_t kRest = size_t(8) << 30;
 
 private:
     std::vector<std::pair<size_t, void *>> free_;

@@ -310,8 +310,7 @@ __device__ __forceinline__ int32_t clamp8(int32_t x) { return x < 0 ? 0 : x > 8 
 // not entries, and the value of an entry is as many values behind the
 // region's start as entries of its tile come before it: those decoded in the
 // chunk before the tile's first lane do not count, and c0 of window tile 0's
-// came in earlier chunks.  Work items start at tile starts (rotation and
-// splits), so no value position is carried into an item.  tiles: how many
+// lie before this chunk (in earlier ones, or before the item).  tiles: how many
 // tiles of the window have lanes in this chunk; qt: the entry that the value
 // positions of lane 63's tile count from.
 template <int K, bool W, bool NARROW>
