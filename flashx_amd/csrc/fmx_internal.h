@@ -79,7 +79,7 @@ struct Plan {
 // queued.  While a scope is open every block is kept, and kRest bytes when it
 // is closed, the largest blocks going back first; all of them go back when an
 // allocation fails and with the context, which one host thread uses at a time.
-// kRest covers the buffers of some 2^27 edges: the driver clears what is freed
+// kRest covers the buffers of some 2^27 edges: the system clears what is freed
 // at about 200 GB/s behind the program's back, during which allocations wait
 // and copies from the host run at half their rate (a matrix streamed right
 // after builds that gave their buffers back: 8.0 ms a product instead of 4.0).
