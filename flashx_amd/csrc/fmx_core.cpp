@@ -24,45 +24,28 @@ StreamScratch::~StreamScratch()
     for (const Buf &b : bufs_) (void)hipFree(b.ptr);
 }
 
-fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, void **out)
+fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphScratch &graphs, void **out)
 {
     *out = nullptr;
     if (!bytes) return FMX_OK;
-    calls_++;
-    unsigned long long graph = 0;
     if (s) {  // the null stream cannot be captured
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        unsigned long long graph = 0;
         if (hipStreamGetCaptureInfo(s, &cs, &graph) != hipSuccess) {
             (void)hipGetLastError();
             cs = hipStreamCaptureStatusNone;
         }
-        if (cs != hipStreamCaptureStatusActive) graph = 0;
-        else if (!graph) graph = 1;
+        if (cs == hipStreamCaptureStatusActive) return graphs.get(ctx, this, s, graph, bytes, out);
     }
-    Buf *mine = nullptr, *eager = nullptr, *shared = nullptr;  // best of each kind
-    size_t neager = 0, ngraph = 0;
+    calls_++;
+    Buf *mine = nullptr, *oldest = nullptr;
     for (Buf &b : bufs_) {
-        if (b.stream == s && b.graph == graph && (!graph || b.bytes >= bytes)) mine = &b;
-        if (!b.graph) {
-            neager++;
-            // under capture the newest that is large enough, else the oldest
-            if (graph ? b.bytes >= bytes && (!eager || b.used > eager->used) : !eager || b.used < eager->used)
-                eager = &b;
-        } else {
-            ngraph++;
-            if (b.bytes >= bytes) shared = &b;
-        }
+        if (b.stream == s) mine = &b;
+        if (!oldest || b.used < oldest->used) oldest = &b;
     }
-    if (graph && !mine) {
-        mine = shared && (!eager || ngraph >= kGraphs) ? shared : eager;
-        if (mine && !mine->graph) {
-            mine->stream = s;
-            mine->graph = graph;
-        }
-    }
-    if (!graph && !mine && neager >= kStreams) {
+    if (!mine && bufs_.size() >= kStreams) {
         FMX_HIP(ctx, hipDeviceSynchronize());
-        mine = eager;
+        mine = oldest;
         mine->stream = s;
     }
     if (!mine || mine->bytes < bytes) {
@@ -73,11 +56,37 @@ fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, void **
         }
         void *p = nullptr;
         FMX_HIP(ctx, dev_malloc(ctx, &p, bytes));
-        bufs_.push_back({s, graph, calls_, p, bytes});
+        bufs_.push_back({s, calls_, p, bytes});
         mine = &bufs_.back();
     }
     mine->used = calls_;
     *out = mine->ptr;
+    return FMX_OK;
+}
+
+GraphScratch::~GraphScratch()
+{
+    for (const Buf &b : bufs_) (void)hipFree(b.ptr);
+}
+
+fmx_status GraphScratch::get(fmx_ctx *ctx, const void *purpose, hipStream_t s, unsigned long long graph, size_t bytes,
+                             void **out)
+{
+    for (const Buf &b : bufs_)
+        if (b.purpose == purpose && b.stream == s && b.graph == graph && b.bytes >= bytes) {
+            *out = b.ptr;
+            return FMX_OK;
+        }
+    // an allocation is no stream operation: this thread's capture mode must
+    // only not forbid it
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    FMX_HIP(ctx, hipThreadExchangeStreamCaptureMode(&mode));
+    void *p = nullptr;
+    const hipError_t e = dev_malloc(ctx, &p, bytes);
+    FMX_HIP(ctx, hipThreadExchangeStreamCaptureMode(&mode));
+    FMX_HIP(ctx, e);
+    bufs_.push_back({purpose, s, graph, p, bytes});
+    *out = p;
     return FMX_OK;
 }
 
@@ -845,6 +854,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     // in the sequential mode the reference's column order, re-cut if its
     // tiles are taller than a band
     const fmx_spm *orig = spm;
+    GraphScratch &graphs = spm->graphs;
     const bool hot = !seq && spm->fast && gather_order_pays(spm, (uint64_t)k * es);
     if (hot) spm = spm->fast.get();
     else if (spm->work) spm = spm->work.get();
@@ -857,7 +867,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     // 8 MB behind a freed matrix, against 34 for the product); larger ones
     // are freed with their matrix
     void *partial = nullptr;
-    st = (need <= kSharedPartials ? ctx->partial : spm->partial).get(ctx, s, need, &partial);
+    st = (need <= kSharedPartials ? ctx->partial : spm->partial).get(ctx, s, need, graphs, &partial);
     if (st) return st;
     // a column-major or pre-scaled X is restaged row-major first (the
     // reference converts a non-row-major input, sparse_matrix.cpp:720-736)
@@ -866,7 +876,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     if ((xcol || pre) && orig->ncols) {
         const size_t xb = orig->ncols * (size_t)k * es;
         void *xs = nullptr;
-        st = ctx->xstage.get(ctx, s, xb, &xs);
+        st = ctx->xstage.get(ctx, s, xb, graphs, &xs);
         if (st) return st;
         st = stage_dense_rows(ctx, dtype, orig->ncols, k, X, ldx, xcol, pre, xs, s);
         if (st) return st;
@@ -878,7 +888,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
         // X's hot rows, densely, in the gather-order image's column order
         const size_t hb = orig->nhot * (size_t)k * es;
         void *xh = nullptr;
-        st = ctx->xhot.get(ctx, s, hb, &xh);
+        st = ctx->xhot.get(ctx, s, hb, graphs, &xh);
         if (st) return st;
         st = stage_hot_rows(ctx, dtype, orig->nhot, k, X, ldx, orig->d_hot, xh, s);
         if (st) return st;

@@ -110,25 +110,47 @@ struct BlockScope {
 constexpr size_t kPinnedCounts = 0, kPinnedFlag = 4096, kPinnedHeader = 8192, kPinnedStage = 12288,
                  kPinnedBytes = kPinnedStage + (2 << 20);
 
+// Scratch of captured calls: a buffer for each capture, stream in it and
+// purpose, allocated for them and shared with nothing else.  Replays may
+// overlap any later call and each other, and two streams of one capture are
+// branches that run side by side; the captured calls of one stream run in
+// order and share.  How long a graph lives is not known (user objects are
+// released too early or never on ROCm 7.2), so a buffer lives as long as its
+// owner, without which the graph cannot be replayed: the matrix.
+class GraphScratch {
+public:
+    GraphScratch() = default;
+    GraphScratch(const GraphScratch &) = delete;
+    GraphScratch &operator=(const GraphScratch &) = delete;
+    ~GraphScratch();
+    fmx_status get(fmx_ctx *ctx, const void *purpose, hipStream_t s, unsigned long long graph, size_t bytes,
+                   void **out);
+
+private:
+    struct Buf {
+        const void *purpose;
+        hipStream_t stream;
+        unsigned long long graph;  // hipStreamGetCaptureInfo's id
+        void *ptr;
+        size_t bytes;
+    };
+    std::vector<Buf> bufs_;
+};
+
 // Scratch of one purpose for calls on several streams: a buffer for each
 // stream that uses it, so that calls of one context on different streams do
 // not share one.  At most kStreams of them are kept; a further stream gets the
-// longest unused one, after the device has finished.  A buffer given to a call
-// under stream capture belongs to that capture's graph from then on (replays
-// may overlap any later call) and lives as long as its owner; nothing can be
-// allocated under capture, so that call takes a buffer that an earlier eager
-// call left, and, if there is none or captures hold kGraphs, shares an earlier
-// capture's.
+// longest unused one, after the device has finished.  A call under stream
+// capture takes its buffer from `graphs`.
 class StreamScratch {
 public:
     ~StreamScratch();
-    fmx_status get(fmx_ctx *ctx, hipStream_t s, size_t bytes, void **out);
+    fmx_status get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphScratch &graphs, void **out);
 
 private:
-    static constexpr size_t kStreams = 4, kGraphs = 8;
+    static constexpr size_t kStreams = 4;
     struct Buf {
         hipStream_t stream;
-        unsigned long long graph;  // the capture it belongs to, 0 = none
         uint64_t used;
         void *ptr;
         size_t bytes;
@@ -173,6 +195,7 @@ struct fmx_spm {
     std::vector<uint32_t> brow_dir;     // first directory index per block row (+1)
     std::map<uint32_t, std::unique_ptr<fmx::Plan>> plans;
     fmx::StreamScratch partial;         // partial bands of split items, above kSharedPartials
+    fmx::GraphScratch graphs;           // all scratch of captured multiplies by this matrix
     // Out-of-core form (d_image == nullptr): the image stays in pinned host
     // memory and every SpMM streams it through two HBM staging buffers in
     // chunks of whole block rows; directory and plans stay in HBM.

@@ -4,6 +4,7 @@ Bars: integer operands bit-exact; FP64 within 1e-12 relative, FP32 within
 1e-5 relative of the oracle's reference-order product (the tolerances the
 path is specified with); rows without non-zeros exactly 0.
 """
+import gc
 import os
 
 import numpy as np
@@ -418,3 +419,95 @@ def test_restaged_operands(fmx, orc, n, k):
             if np.issubdtype(dt, np.floating):
                 spm.multiply_scaled_async(x, Y, pre=pd)
                 assert np.array_equal(Y.cpu().numpy(), np.roll(X * pre[:, None], -1, axis=0).astype(dt)), (dt, x.stride())
+
+
+def _two_matrices(fmx, n, k):
+    """Two matrices in gather order with split bands, integer operands, and
+    the exact products."""
+    import torch
+    out = []
+    for seed in (5, 6):
+        src, dst = fmx.rmat_edges((n - 1).bit_length(), 16 * n, seed)
+        spm = fmx.SparseMatrix.build(src, dst, n=n, log2_h=6, log2_w=15)
+        g = torch.Generator(device="cuda")
+        g.manual_seed(seed)
+        X = torch.randint(-9, 10, (n, k), device="cuda", generator=g, dtype=torch.int32)
+        out.append((spm, X, spm.multiply(X)))
+    return out
+
+
+def test_each_capture_gets_scratch_of_its_own(fmx, monkeypatch):
+    """Captured multiplies (nothing is replayed here): each capture allocates
+    the scratch it holds -- here the hot block, at least 3 MB -- whether an
+    earlier eager call left some or not, and an eager call keeps its own."""
+    import torch
+    monkeypatch.setenv("FMX_HOT_MIN_BYTES", "0")
+    pair = _two_matrices(fmx, 1 << 18, 16)
+    least = min(spm.info.hot_columns for spm, _, _ in pair) * 16 * 4
+    assert least > 3 << 20
+    Y = [torch.empty_like(X) for _, X, _ in pair]
+    warm = torch.cuda.Stream()
+    graphs = []
+    with torch.cuda.stream(warm):
+        for (spm, X, _), y in zip(pair, Y):
+            spm.multiply_async(X, y)
+    torch.cuda.synchronize()
+    for i in (0, 1, 0):
+        gc.collect()
+        torch.cuda.empty_cache()  # as a capture's start does
+        free = torch.cuda.mem_get_info()[0]
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=warm):
+            pair[i][0].multiply_async(pair[i][1], Y[i])
+        graphs.append(g)
+        torch.cuda.synchronize()
+        assert free - torch.cuda.mem_get_info()[0] >= least, len(graphs)
+
+
+@pytest.mark.parametrize("hot", ["0", str(1 << 40)])
+def test_captured_multiplies_replay_side_by_side(fmx, monkeypatch, hot):
+    """Graphs of two matrices and a second one of the first, captured after one
+    eager call each and replayed at once on three streams; and both matrices
+    in one graph, on two branches.  Integers, so every product must be exact."""
+    import torch
+    monkeypatch.setenv("FMX_HOT_MIN_BYTES", hot)
+    pair = _two_matrices(fmx, 1 << 16, 4)
+    pair.append((pair[0][0], pair[0][1].flip(0).contiguous(), None))
+    pair[2] = (pair[2][0], pair[2][1], pair[2][0].multiply(pair[2][1]))
+    Y = [torch.empty_like(X) for _, X, _ in pair]
+    torch.cuda.synchronize()
+    graphs = []
+    for (spm, X, _), y in zip(pair, Y):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            for _ in range(3):
+                spm.multiply_async(X, y)
+        graphs.append(g)
+    streams = [torch.cuda.Stream() for _ in graphs]
+    for _ in range(5):
+        for y in Y:
+            y.zero_()
+        torch.cuda.synchronize()
+        for _ in range(10):
+            for g, s in zip(graphs, streams):
+                with torch.cuda.stream(s):
+                    g.replay()
+        pair[1][0].multiply(pair[1][1])  # an eager call beside them
+        torch.cuda.synchronize()
+        for i, (y, (_, _, want)) in enumerate(zip(Y, pair)):
+            assert torch.equal(y, want), i
+    both, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(both):
+        main = torch.cuda.current_stream()
+        side.wait_stream(main)
+        for _ in range(4):
+            pair[0][0].multiply_async(pair[0][1], Y[0])
+            with torch.cuda.stream(side):
+                pair[1][0].multiply_async(pair[1][1], Y[1])
+        main.wait_stream(side)
+    for _ in range(5):
+        Y[0].zero_(), Y[1].zero_()
+        torch.cuda.synchronize()
+        both.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(Y[0], pair[0][2]) and torch.equal(Y[1], pair[1][2])
