@@ -21,12 +21,14 @@ Plan::~Plan()
 
 StreamScratch::~StreamScratch()
 {
-    for (const Buf &b : bufs_) (void)hipFree(b.ptr);
+    for (const Buf &b : bufs_) {
+        (void)hipFree(b.ptr);
+        if (b.last) (void)hipEventDestroy(b.last);
+    }
 }
 
-fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphScratch &graphs, void **out)
+fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphScratch &graphs, Lease &out)
 {
-    *out = nullptr;
     if (!bytes) return FMX_OK;
     if (s) {  // the null stream cannot be captured
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -35,33 +37,49 @@ fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphSc
             (void)hipGetLastError();
             cs = hipStreamCaptureStatusNone;
         }
-        if (cs == hipStreamCaptureStatusActive) return graphs.get(ctx, this, s, graph, bytes, out);
+        if (cs == hipStreamCaptureStatusActive) return graphs.get(ctx, this, s, graph, bytes, &out.ptr);
     }
     calls_++;
-    Buf *mine = nullptr, *oldest = nullptr;
-    for (Buf &b : bufs_) {
-        if (b.stream == s) mine = &b;
-        if (!oldest || b.used < oldest->used) oldest = &b;
+    size_t mine = bufs_.size(), oldest = 0;
+    for (size_t i = 0; i < bufs_.size(); i++) {
+        if (bufs_[i].stream == s) mine = i;
+        if (bufs_[i].used < bufs_[oldest].used) oldest = i;
     }
-    if (!mine && bufs_.size() >= kStreams) {
-        FMX_HIP(ctx, hipDeviceSynchronize());
+    if (mine == bufs_.size() && mine >= kStreams) {
+        // another stream's: behind its last call, which only a first round
+        // of turns has not marked
         mine = oldest;
-        mine->stream = s;
+        if (bufs_[mine].marked) FMX_HIP(ctx, hipStreamWaitEvent(s, bufs_[mine].last, 0));
+        else FMX_HIP(ctx, hipDeviceSynchronize());
+        turns_ = true;
+    } else if (mine == bufs_.size()) {
+        bufs_.emplace_back();
     }
-    if (!mine || mine->bytes < bytes) {
-        if (mine) {
-            void *old = mine->ptr;
-            bufs_.erase(bufs_.begin() + (mine - bufs_.data()));
-            FMX_HIP(ctx, hipFree(old));
-        }
-        void *p = nullptr;
-        FMX_HIP(ctx, dev_malloc(ctx, &p, bytes));
-        bufs_.push_back({s, calls_, p, bytes});
-        mine = &bufs_.back();
+    Buf &b = bufs_[mine];
+    b.stream = s;
+    b.used = calls_;
+    b.marked = false;
+    if (b.bytes < bytes) {
+        void *old = b.ptr;
+        b.ptr = nullptr;
+        b.bytes = 0;
+        if (old) FMX_HIP(ctx, hipFree(old));
+        FMX_HIP(ctx, dev_malloc(ctx, &b.ptr, bytes));
+        b.bytes = bytes;
     }
-    mine->used = calls_;
-    *out = mine->ptr;
+    out.ptr = b.ptr;
+    out.from = this;
+    out.stream = s;
     return FMX_OK;
+}
+
+StreamScratch::Lease::~Lease()
+{
+    if (!from || !from->turns_) return;
+    for (Buf &b : from->bufs_)
+        if (b.stream == stream)
+            b.marked = (b.last || hipEventCreateWithFlags(&b.last, hipEventDisableTiming) == hipSuccess) &&
+                       hipEventRecord(b.last, stream) == hipSuccess;
 }
 
 GraphScratch::~GraphScratch()
@@ -866,18 +884,19 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     // that a new matrix's first product does not allocate (57 to 390 us for
     // 8 MB behind a freed matrix, against 34 for the product); larger ones
     // are freed with their matrix
-    void *partial = nullptr;
-    st = (need <= kSharedPartials ? ctx->partial : spm->partial).get(ctx, s, need, graphs, &partial);
+    StreamScratch::Lease partials, staged, hots;
+    st = (need <= kSharedPartials ? ctx->partial : spm->partial).get(ctx, s, need, graphs, partials);
     if (st) return st;
+    void *const partial = partials.ptr;
     // a column-major or pre-scaled X is restaged row-major first (the
     // reference converts a non-row-major input, sparse_matrix.cpp:720-736)
     // X has orig's columns as rows: a gather-order image counts its hot
     // columns on top of them
     if ((xcol || pre) && orig->ncols) {
         const size_t xb = orig->ncols * (size_t)k * es;
-        void *xs = nullptr;
-        st = ctx->xstage.get(ctx, s, xb, graphs, &xs);
+        st = ctx->xstage.get(ctx, s, xb, graphs, staged);
         if (st) return st;
+        void *const xs = staged.ptr;
         st = stage_dense_rows(ctx, dtype, orig->ncols, k, X, ldx, xcol, pre, xs, s);
         if (st) return st;
         X = xs;
@@ -887,9 +906,9 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     if (hot) {
         // X's hot rows, densely, in the gather-order image's column order
         const size_t hb = orig->nhot * (size_t)k * es;
-        void *xh = nullptr;
-        st = ctx->xhot.get(ctx, s, hb, graphs, &xh);
+        st = ctx->xhot.get(ctx, s, hb, graphs, hots);
         if (st) return st;
+        void *const xh = hots.ptr;
         st = stage_hot_rows(ctx, dtype, orig->nhot, k, X, ldx, orig->d_hot, xh, s);
         if (st) return st;
         if (spm->streamed())

@@ -139,24 +139,42 @@ private:
 
 // Scratch of one purpose for calls on several streams: a buffer for each
 // stream that uses it, so that calls of one context on different streams do
-// not share one.  At most kStreams of them are kept; a further stream gets the
-// longest unused one, after the device has finished.  A call under stream
-// capture takes its buffer from `graphs`.
+// not share one.  At most kStreams of them are kept; a further stream takes
+// the longest unused one, its work queued behind the call that used it last
+// (the device waits, not the host).  A call under stream capture takes its
+// buffer from `graphs`.
 class StreamScratch {
 public:
+    // A call's hold on its buffer, to the end of the call that queued the
+    // work on it.
+    struct Lease {
+        void *ptr = nullptr;
+        StreamScratch *from = nullptr;
+        hipStream_t stream = nullptr;
+        Lease() = default;
+        Lease(const Lease &) = delete;
+        Lease &operator=(const Lease &) = delete;
+        ~Lease();
+    };
+    StreamScratch() = default;
+    StreamScratch(const StreamScratch &) = delete;
+    StreamScratch &operator=(const StreamScratch &) = delete;
     ~StreamScratch();
-    fmx_status get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphScratch &graphs, void **out);
+    fmx_status get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphScratch &graphs, Lease &out);
 
 private:
     static constexpr size_t kStreams = 4;
     struct Buf {
-        hipStream_t stream;
-        uint64_t used;
-        void *ptr;
-        size_t bytes;
+        hipStream_t stream = nullptr;
+        uint64_t used = 0;
+        void *ptr = nullptr;
+        size_t bytes = 0;
+        hipEvent_t last = nullptr;  // behind its last call, if marked
+        bool marked = false;
     };
     std::vector<Buf> bufs_;
     uint64_t calls_ = 0;
+    bool turns_ = false;  // there were more streams than buffers: calls leave marks
 };
 
 constexpr size_t kSharedPartials = size_t(64) << 20;

@@ -511,3 +511,41 @@ def test_captured_multiplies_replay_side_by_side(fmx, monkeypatch, hot):
         both.replay()
         torch.cuda.synchronize()
         assert torch.equal(Y[0], pair[0][2]) and torch.equal(Y[1], pair[1][2])
+
+
+@pytest.mark.parametrize("hot", ["0", str(1 << 40)])
+def test_many_streams_in_turn_do_not_wait_for_the_device(fmx, monkeypatch, hot):
+    """Eight streams in turn, more than there are scratch buffers: a call
+    queues its work and returns while another stream is busy (some 200 ms of
+    matrix products), and every product is exact."""
+    import torch
+    monkeypatch.setenv("FMX_HOT_MIN_BYTES", hot)
+    pair = _two_matrices(fmx, 1 << 15, 4)
+    streams = [torch.cuda.Stream() for _ in range(8)]
+    Y = [torch.empty_like(pair[0][1]) for _ in streams]
+    busy, done = torch.cuda.Stream(), torch.cuda.Event()
+    M = torch.rand((4096, 4096), device="cuda")
+    torch.mm(M, M)
+
+    def turns():
+        for i, s in enumerate(streams):
+            spm, X, _ = pair[i % 2]
+            with torch.cuda.stream(s):
+                spm.multiply_async(X, Y[i])
+
+    for _ in range(3):
+        turns()
+    torch.cuda.synchronize()
+    for y in Y:
+        y.zero_()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        for _ in range(200):
+            torch.mm(M, M)
+        done.record()
+    turns()
+    waited = done.query()
+    torch.cuda.synchronize()
+    for i, y in enumerate(Y):
+        assert torch.equal(y, pair[i % 2][2]), i
+    assert not waited
