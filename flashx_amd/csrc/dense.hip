@@ -848,30 +848,22 @@ fmx_status noalloc_scratch_lookup(fmx_ctx *ctx)
     return FMX_OK;
 }
 
-fmx_status ctx_scratch(fmx_ctx *ctx, size_t bytes, void **out)
+fmx_status ctx_scratch(fmx_ctx *ctx, hipStream_t s, size_t bytes, StreamScratch::Lease &out)
 {
-    if (bytes > ctx->ws_bytes) {
-        if (ctx->ws) FMX_HIP(ctx, hipFree(ctx->ws));
-        ctx->ws = nullptr;
-        ctx->ws_bytes = 0;
-        FMX_HIP(ctx, dev_malloc(ctx, (void **)&ctx->ws, bytes));
-        ctx->ws_bytes = bytes;
-    }
-    *out = ctx->ws;
-    return FMX_OK;
+    return ctx->ws.get(ctx, s, bytes, ctx->graphs, out);
 }
 
-// Per-block partial sums of the Gram kernels: the context's grow-only
-// workspace, or -- fixed != null -- a caller-given buffer of fixed_bytes,
+// Per-block partial sums of the Gram kernels: the context's workspace for
+// the stream, or -- fixed != null -- a caller-given buffer of fixed_bytes,
 // in which case the block count is capped so that the partials fit.
-static fmx_status gram_ws(fmx_ctx *ctx, void *fixed, size_t fixed_bytes, size_t per_block, uint32_t &nblk,
-                          void **ws)
+static fmx_status gram_ws(fmx_ctx *ctx, hipStream_t s, void *fixed, size_t fixed_bytes, size_t per_block,
+                          uint32_t &nblk, StreamScratch::Lease &ws)
 {
-    if (!fixed) return ctx_scratch(ctx, (size_t)nblk * per_block, ws);
+    if (!fixed) return ctx_scratch(ctx, s, (size_t)nblk * per_block, ws);
     const size_t fit = fixed_bytes / per_block;
     if (fit == 0) return fail(ctx, FMX_EDIM, "Gram output larger than the fixed scratch");
     if (nblk > fit) nblk = (uint32_t)fit;
-    *ws = fixed;
+    ws.ptr = fixed;
     return FMX_OK;
 }
 
@@ -887,9 +879,10 @@ fmx_status gram(fmx_ctx *ctx, fmx_dtype dt, int mode, uint64_t n, int ka, int kb
         const int kap = (ka + 15) & ~15, kbp = (kb + 15) & ~15;
         if ((kap / 16) * (kbp / 16) > 64) return fail(ctx, FMX_EDIM, "BF16 Gram output too large");
         uint32_t nblk = blocks_for(ctx, n, 1024);
-        void *ws;
-        fmx_status st = gram_ws(ctx, fixed_ws, fixed_bytes, (size_t)nout * sizeof(float), nblk, &ws);
+        StreamScratch::Lease lease;
+        fmx_status st = gram_ws(ctx, s, fixed_ws, fixed_bytes, (size_t)nout * sizeof(float), nblk, lease);
         if (st) return st;
+        void *const ws = lease.ptr;
         const uint64_t rpb = (n + nblk - 1) / nblk;
         const size_t lds = (size_t)(kap + kbp) * kBPad * sizeof(unsigned short);
         static bool attr = false;
@@ -962,9 +955,10 @@ fmx_status gram(fmx_ctx *ctx, fmx_dtype dt, int mode, uint64_t n, int ka, int kb
         waves = (n + rpw - 1) / rpw;
         if (waves < 1) waves = 1;
         uint32_t nblk = (uint32_t)((waves * 64 + kT - 1) / kT);  // waves past the rows add zeros
-        void *ws;
-        fmx_status st = gram_ws(ctx, fixed_ws, fixed_bytes, (size_t)nout * sizeof(double), nblk, &ws);
+        StreamScratch::Lease lease;
+        fmx_status st = gram_ws(ctx, s, fixed_ws, fixed_bytes, (size_t)nout * sizeof(double), nblk, lease);
         if (st) return st;
+        void *const ws = lease.ptr;
         const size_t glds = std::max(stage_lds, (size_t)2 * nout * sizeof(double));
         const int veca = ((uintptr_t)A % 16 == 0) && ((lda * es) % 16 == 0);
         const int vecb = ((uintptr_t)B % 16 == 0) && ((ldb * es) % 16 == 0);
@@ -1042,9 +1036,10 @@ fmx_status gram(fmx_ctx *ctx, fmx_dtype dt, int mode, uint64_t n, int ka, int kb
         return FMX_OK;
     }
     uint32_t nblk = blocks_for(ctx, n, 512);
-    void *ws;
-    fmx_status st = gram_ws(ctx, fixed_ws, fixed_bytes, (size_t)nout * sizeof(double), nblk, &ws);
+    StreamScratch::Lease lease;
+    fmx_status st = gram_ws(ctx, s, fixed_ws, fixed_bytes, (size_t)nout * sizeof(double), nblk, lease);
     if (st) return st;
+    void *const ws = lease.ptr;
     const uint64_t rpb = (n + nblk - 1) / nblk;
     const size_t lds = (size_t)kGRows * (ka + kb) * sizeof(double);
     dim3 grid(nblk, (nout + 4095) / 4096);
@@ -1206,9 +1201,10 @@ fmx_status gram_bf16_shadow(fmx_ctx *ctx, uint64_t n, int ka, int kb, const unsi
         return fail(ctx, FMX_EDIM, "BF16-operand Gram: widths, strides or alignment unsupported");
     const int nout = ka * kb;
     uint32_t nblk = blocks_for(ctx, n, 1024);
-    void *ws;
-    fmx_status st = ctx_scratch(ctx, (size_t)nblk * nout * sizeof(float), &ws);
+    StreamScratch::Lease lease;
+    fmx_status st = ctx_scratch(ctx, s, (size_t)nblk * nout * sizeof(float), lease);
     if (st) return st;
+    void *const ws = lease.ptr;
     const uint64_t rpb = (n + nblk - 1) / nblk;
     const size_t lds = (size_t)(kap + kbp) * kBPad * sizeof(unsigned short);
     static bool attr = false;
@@ -1345,9 +1341,10 @@ fmx_status colnorm(fmx_ctx *ctx, fmx_dtype dt, uint64_t n, int k, const void *A,
     if (lda < k) return fail(ctx, FMX_EDIM, "leading dimension too small");
     const uint32_t nblk = blocks_for(ctx, n, 2048);
     const uint64_t rpb = (n + nblk - 1) / nblk;
-    void *ws;
-    fmx_status st = ctx_scratch(ctx, (size_t)nblk * k * sizeof(double), &ws);
+    StreamScratch::Lease lease;
+    fmx_status st = ctx_scratch(ctx, s, (size_t)nblk * k * sizeof(double), lease);
     if (st) return st;
+    void *const ws = lease.ptr;
     if (dt == FMX_F32)
         hipLaunchKernelGGL(colsq_kernel<float>, dim3(nblk), dim3(kT), 0, s, (const float *)A, lda, n, k,
                            rpb, (double *)ws);

@@ -65,14 +65,14 @@ fmx_status fmx_gather_floor(fmx_ctx *ctx, uint64_t row_bytes, const void *X, int
     if (n && x_rows == 0) return fail(ctx, FMX_EDIM, "X has no rows");
     if (n == 0) return FMX_OK;
     FMX_HIP(ctx, hipSetDevice(ctx->device));
-    void *ws;
-    fmx_status st = ctx_scratch(ctx, 16, &ws);
+    hipStream_t s = (hipStream_t)stream;
+    StreamScratch::Lease ws;
+    fmx_status st = ctx_scratch(ctx, s, 16, ws);
     if (st) return st;
     const uint64_t waves = (n + kPerWave - 1) / kPerWave;
     const dim3 grid((uint32_t)((waves * 64 + kFloorT - 1) / kFloorT));
-    hipStream_t s = (hipStream_t)stream;
     const unsigned char *x = (const unsigned char *)X;
-    uint32_t *sink = (uint32_t *)ws;
+    uint32_t *sink = (uint32_t *)ws.ptr;
     switch (L) {
     case 1: hipLaunchKernelGGL(gather_floor<1>, grid, dim3(kFloorT), 0, s, x, ldx_bytes, x_rows, cols, n, sink); break;
     case 2: hipLaunchKernelGGL(gather_floor<2>, grid, dim3(kFloorT), 0, s, x, ldx_bytes, x_rows, cols, n, sink); break;

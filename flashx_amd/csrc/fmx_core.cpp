@@ -1003,7 +1003,6 @@ fmx_status fmx_ctx_destroy(fmx_ctx *ctx)
         (void)hipStreamSynchronize(ctx->stream);
         (void)hipStreamDestroy(ctx->stream);
     }
-    if (ctx->ws) (void)hipFree(ctx->ws);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     delete ctx;
     return FMX_OK;

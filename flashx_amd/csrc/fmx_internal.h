@@ -116,7 +116,8 @@ constexpr size_t kPinnedCounts = 0, kPinnedFlag = 4096, kPinnedHeader = 8192, kP
 // branches that run side by side; the captured calls of one stream run in
 // order and share.  How long a graph lives is not known (user objects are
 // released too early or never on ROCm 7.2), so a buffer lives as long as its
-// owner, without which the graph cannot be replayed: the matrix.
+// owner, without which the graph cannot be replayed: the matrix, or for
+// dense operations the context.
 class GraphScratch {
 public:
     GraphScratch() = default;
@@ -187,8 +188,8 @@ struct fmx_ctx {
     std::string last_error;
     int num_cus = 0;
     size_t lds_per_block = 0;
-    void *ws = nullptr;        // grow-only device workspace (dense-op partials)
-    size_t ws_bytes = 0;
+    fmx::GraphScratch graphs;   // workspaces of captured dense operations
+    fmx::StreamScratch ws;      // dense operations' partials
     fmx::StreamScratch xstage;  // a dense operand restaged row-major / pre-scaled
     fmx::StreamScratch xhot;    // the hot rows of X, densely (gather-order images)
     fmx::StreamScratch partial; // partial bands of split items, to kSharedPartials

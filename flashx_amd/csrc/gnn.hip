@@ -501,11 +501,11 @@ fmx_status grads(fmx_ctx *ctx, int mode, uint64_t n, int ka, int kb, const float
     const uint64_t rpb = blocks ? ((n + blocks - 1) / blocks + 127) / 128 * 128 : 128;
     const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, (n + rpb - 1) / rpb);
     const size_t fb = (size_t)ny * nblk * nout * sizeof(float);
-    void *ws = nullptr;
-    fmx_status st = ctx_scratch(ctx, fb + (size_t)nblk * kb * sizeof(double), &ws);
+    StreamScratch::Lease ws;
+    fmx_status st = ctx_scratch(ctx, s, fb + (size_t)nblk * kb * sizeof(double), ws);
     if (st) return st;
-    float *pa = (float *)ws;
-    double *pb = bias ? (double *)((char *)ws + fb) : nullptr;
+    float *pa = (float *)ws.ptr;
+    double *pb = bias ? (double *)((char *)ws.ptr + fb) : nullptr;
 #define FMX_GRAD(TI, TJ)                                                                                       \
     hipLaunchKernelGGL((gnn_grad_kernel<TI, TJ>), dim3(nblk, ny), dim3(kT), 0, s, A0, A1, Z, n, rpb, pa, pb)
     if (kb == 64) {

@@ -259,7 +259,7 @@ fmx_status fmx_gram(fmx_ctx *ctx, fmx_dtype dtype, int mode, uint64_t n, int ka,
  * allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  The per-block partial sums go to a fixed
  * 4 MiB device array that the library holds on every GPU it runs on until
- * the process ends, not to the context's grow-only workspace, and the block
+ * the process ends, not to a workspace of the context, and the block
  * count is capped so that they fit (a ka * kb * 8-byte output larger than
  * the array is FMX_EDIM; every ka, kb <= 256 fits).  Arguments, results and
  * errors are fmx_gram's; no device memory is allocated or freed.  All calls

@@ -174,3 +174,62 @@ def test_gram_short_operands(fmx, n):
                 assert ((G - x.t() @ y).abs() <= 1e-13 * (x.abs().t() @ y.abs()) + 1e-300).all(), (ka, kb, dt)
             Ad = A.cuda()
             assert torch.equal(fmx.gram(Ad, Ad), fmx.gram(Ad, Ad))
+
+
+def test_dense_operations_on_several_streams(fmx):
+    """Grams and column norms queued at once on several streams of one context,
+    and captured Grams replayed beside them: the partial sums of one never
+    serve another.  The operands are small whole numbers, so Grams are exact;
+    norms equal those computed alone."""
+    import torch
+    F = fmx
+    n, count = 1 << 18, 6
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(1)
+    A = [torch.randint(-4, 5, (n, 32), device="cuda", generator=gen).to(torch.float32) for _ in range(count)]
+    B = [torch.randint(-4, 5, (n, 16), device="cuda", generator=gen).to(torch.float32) for _ in range(count)]
+    want = [(a.double().t().contiguous() @ b.double()) for a, b in zip(A, B)]
+    ctx = F.default_context()
+    G = [torch.empty((32, 16), dtype=torch.float64, device="cuda") for _ in range(count)]
+    N = [torch.empty(32, dtype=torch.float64, device="cuda") for _ in range(count)]
+
+    def run_gram(i):
+        s = torch.cuda.current_stream().cuda_stream
+        ctx.check(F.lib().fmx_gram(ctx.handle, F.dtype_code(torch.float32), 0, n, 32, 16, A[i].data_ptr(), 32,
+                                   B[i].data_ptr(), 16, G[i].data_ptr(), s), "fmx_gram")
+
+    def run_norm(i):
+        s = torch.cuda.current_stream().cuda_stream
+        ctx.check(F.lib().fmx_colnorm(ctx.handle, F.dtype_code(torch.float32), n, 32, A[i].data_ptr(), 32,
+                                      N[i].data_ptr(), s), "fmx_colnorm")
+
+    norms = []
+    for i in range(count):
+        run_norm(i)
+        torch.cuda.synchronize()
+        norms.append(N[i].clone())
+    streams = [torch.cuda.Stream() for _ in range(count)]
+    graphs = []
+    for i in range(2):
+        run_gram(i)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            run_gram(i)
+        graphs.append(g)
+    for _ in range(5):
+        for x in G + N:
+            x.zero_()
+        torch.cuda.synchronize()
+        for _ in range(8):
+            for i, s in enumerate(streams):
+                with torch.cuda.stream(s):
+                    if i < 2:
+                        graphs[i].replay()
+                    else:
+                        run_gram(i)
+                    run_norm(i)
+        torch.cuda.synchronize()
+        for i in range(count):
+            assert torch.equal(G[i], want[i]), i
+            assert torch.equal(N[i], norms[i]), i
