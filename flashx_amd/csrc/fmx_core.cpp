@@ -40,9 +40,10 @@ fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphSc
         if (cs == hipStreamCaptureStatusActive) return graphs.get(ctx, this, s, graph, bytes, &out.ptr);
     }
     calls_++;
+    const StreamKey key(s);
     size_t mine = bufs_.size(), oldest = 0;
     for (size_t i = 0; i < bufs_.size(); i++) {
-        if (bufs_[i].stream == s) mine = i;
+        if (bufs_[i].stream == key) mine = i;
         if (bufs_[i].used < bufs_[oldest].used) oldest = i;
     }
     if (mine == bufs_.size() && mine >= kStreams) {
@@ -56,7 +57,7 @@ fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphSc
         bufs_.emplace_back();
     }
     Buf &b = bufs_[mine];
-    b.stream = s;
+    b.stream = key;
     b.used = calls_;
     b.marked = false;
     if (b.bytes < bytes) {
@@ -69,7 +70,7 @@ fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphSc
     }
     out.ptr = b.ptr;
     out.from = this;
-    out.stream = s;
+    out.stream = key;
     return FMX_OK;
 }
 
@@ -79,7 +80,7 @@ StreamScratch::Lease::~Lease()
     for (Buf &b : from->bufs_)
         if (b.stream == stream)
             b.marked = (b.last || hipEventCreateWithFlags(&b.last, hipEventDisableTiming) == hipSuccess) &&
-                       hipEventRecord(b.last, stream) == hipSuccess;
+                       hipEventRecord(b.last, stream.s) == hipSuccess;
 }
 
 GraphScratch::~GraphScratch()
@@ -90,8 +91,9 @@ GraphScratch::~GraphScratch()
 fmx_status GraphScratch::get(fmx_ctx *ctx, const void *purpose, hipStream_t s, unsigned long long graph, size_t bytes,
                              void **out)
 {
+    const StreamKey key(s);
     for (const Buf &b : bufs_)
-        if (b.purpose == purpose && b.stream == s && b.graph == graph && b.bytes >= bytes) {
+        if (b.purpose == purpose && b.stream == key && b.graph == graph && b.bytes >= bytes) {
             *out = b.ptr;
             return FMX_OK;
         }
@@ -103,7 +105,7 @@ fmx_status GraphScratch::get(fmx_ctx *ctx, const void *purpose, hipStream_t s, u
     const hipError_t e = dev_malloc(ctx, &p, bytes);
     FMX_HIP(ctx, hipThreadExchangeStreamCaptureMode(&mode));
     FMX_HIP(ctx, e);
-    bufs_.push_back({purpose, s, graph, p, bytes});
+    bufs_.push_back({purpose, key, graph, p, bytes});
     *out = p;
     return FMX_OK;
 }

@@ -15,6 +15,7 @@
 #include <map>
 #include <memory>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -110,6 +111,19 @@ struct BlockScope {
 constexpr size_t kPinnedCounts = 0, kPinnedFlag = 4096, kPinnedHeader = 8192, kPinnedStage = 12288,
                  kPinnedBytes = kPinnedStage + (2 << 20);
 
+// A stream in the order of whose work a buffer may be used again.  The
+// handle hipStreamPerThread is another stream in every host thread.
+struct StreamKey {
+    hipStream_t s = nullptr;
+    std::thread::id thread;
+    StreamKey() = default;
+    explicit StreamKey(hipStream_t stream) : s(stream)
+    {
+        if (s == hipStreamPerThread) thread = std::this_thread::get_id();
+    }
+    bool operator==(const StreamKey &o) const { return s == o.s && thread == o.thread; }
+};
+
 // Scratch of captured calls: a buffer for each capture, stream in it and
 // purpose, allocated for them and shared with nothing else.  Replays may
 // overlap any later call and each other, and two streams of one capture are
@@ -130,7 +144,7 @@ public:
 private:
     struct Buf {
         const void *purpose;
-        hipStream_t stream;
+        StreamKey stream;
         unsigned long long graph;  // hipStreamGetCaptureInfo's id
         void *ptr;
         size_t bytes;
@@ -151,7 +165,7 @@ public:
     struct Lease {
         void *ptr = nullptr;
         StreamScratch *from = nullptr;
-        hipStream_t stream = nullptr;
+        StreamKey stream;
         Lease() = default;
         Lease(const Lease &) = delete;
         Lease &operator=(const Lease &) = delete;
@@ -166,7 +180,7 @@ public:
 private:
     static constexpr size_t kStreams = 4;
     struct Buf {
-        hipStream_t stream = nullptr;
+        StreamKey stream;
         uint64_t used = 0;
         void *ptr = nullptr;
         size_t bytes = 0;

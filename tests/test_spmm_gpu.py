@@ -421,14 +421,14 @@ def test_restaged_operands(fmx, orc, n, k):
                 assert np.array_equal(Y.cpu().numpy(), np.roll(X * pre[:, None], -1, axis=0).astype(dt)), (dt, x.stride())
 
 
-def _two_matrices(fmx, n, k):
+def _two_matrices(fmx, n, k, ctx=None):
     """Two matrices in gather order with split bands, integer operands, and
     the exact products."""
     import torch
     out = []
     for seed in (5, 6):
         src, dst = fmx.rmat_edges((n - 1).bit_length(), 16 * n, seed)
-        spm = fmx.SparseMatrix.build(src, dst, n=n, log2_h=6, log2_w=15)
+        spm = fmx.SparseMatrix.build(src, dst, n=n, log2_h=6, log2_w=15, ctx=ctx)
         g = torch.Generator(device="cuda")
         g.manual_seed(seed)
         X = torch.randint(-9, 10, (n, k), device="cuda", generator=g, dtype=torch.int32)
@@ -549,3 +549,48 @@ def test_many_streams_in_turn_do_not_wait_for_the_device(fmx, monkeypatch, hot):
     for i, y in enumerate(Y):
         assert torch.equal(y, pair[i % 2][2]), i
     assert not waited
+
+
+def test_threads_own_streams_have_their_own_scratch(fmx, monkeypatch):
+    """hipStreamPerThread is one handle and another stream in each host thread:
+    a second thread's first call (nothing runs meanwhile) allocates scratch of
+    its own, and calls queued from both threads in turn keep theirs apart."""
+    import threading
+
+    import torch
+    monkeypatch.setenv("FMX_HOT_MIN_BYTES", "0")
+    ctx = fmx.Context()  # (without scratch of earlier calls' streams)
+    pair = _two_matrices(fmx, 1 << 18, 16, ctx)
+    least = min(spm.info.hot_columns for spm, _, _ in pair) * 16 * 4
+    Y = [torch.empty_like(X) for _, X, _ in pair]
+    torch.cuda.synchronize()
+    free, turn, errors = [], [threading.Semaphore(1), threading.Semaphore(0)], []
+
+    def worker(i):
+        spm, X, _ = pair[i]
+        for r in range(6):
+            turn[i].acquire()
+            try:
+                if r == 0:
+                    before = torch.cuda.mem_get_info()[0]
+                for _ in range(1 if r == 0 else 3):
+                    st = fmx.lib().fmx_spmm(ctx.handle, spm.handle, fmx.dtype_code(X.dtype), 16, X.data_ptr(), 16,
+                                            Y[i].data_ptr(), 16, 2)  # hipStreamPerThread
+                    if st:
+                        errors.append(st)
+                if r == 0:
+                    torch.cuda.synchronize()
+                    free.append(before - torch.cuda.mem_get_info()[0])
+            finally:
+                turn[1 - i].release()
+
+    threads = [threading.Thread(target=worker, args=(i,)) for i in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    assert all(f >= least for f in free), free
+    for y, (_, _, want) in zip(Y, pair):
+        assert torch.equal(y, want)
