@@ -819,25 +819,45 @@ static int value_prim(fmx_dtype dt)
 
 // Whether an SpMM with X rows of rb bytes runs on the matrix's gather-order
 // image.  Never for rows of a full 128-byte line, which gain nothing from
-// lying next to another hot row.  Otherwise by the number of columns: the
+// lying next to another hot row.  Otherwise by the number of columns (the
 // narrower the rows, the more of them a line of the hot block serves, and
-// copying the hot rows has to be worth while.  R-MAT, 16 edges a vertex, plain /
-// gather-order image, us:
-//   4-byte rows   2^19 columns 44 / 39, 2^20 95 / 76, 2^21 225 / 154
-//   16-byte rows  2^18 35 / 37, 2^19 65 / 57, 2^20 148 / 102, 2^21 382 / 210
-//   40-byte rows  2^19 75 / 81, 700,001 85 / 85, 2^20 171 / 144
-//   64-byte rows  2^19 68 / 82, 2^20 144 / 143, 2^21 354 / 296
-// A weighted matrix gains sooner, with fewer tiles to step through: at 2^17
-// 4- to 80-byte rows are even (64-byte 42 / 43), at 2^18 37 / 33, 16-byte
-// 54 / 47, 64-byte 64 / 59, 80-byte 77 / 71, at 2^20 134 / 108, 218 / 163,
-// 215 / 183, 280 / 257 (with 4 edges a vertex 54 / 49 to 106 / 106).
+// copying the hot rows has to be worth while) and by the share of them that is
+// hot.  Plain / gather-order image, us, FP32, re-cut default tiles:
+// R-MAT, 4 and 24 edges a vertex, a fifth of the columns hot, binary:
+//   4-byte rows   370,001 columns 19 / 16 and 42 / 35, 2^20 44 / 33 and 126 / 100
+//   16-byte rows  370,001 31 / 25 and 56 / 52, 2^20 81 / 54 and 186 / 133
+//   32-byte rows  370,001 25 / 26 and 58 / 58, 2^19 33 / 31 and 81 / 76
+//   40-byte rows  2^19 36 / 39 and 98 / 95, 741,001 49 / 49 and 152 / 131
+//   64-byte rows  741,001 44 / 49 and 124 / 129, 2^20 62 / 64 and 192 / 184
+//   96-byte rows  2^20 100 / 109 and 327 / 307, 1,500,001 152 / 151 and 512 / 457
+// and weighted, which has more tiles to step through:
+//   16-byte rows  230,001 27 / 25 and 65 / 54, 2^19 57 / 45 and 146 / 102
+//   32-byte rows  2^18 24 / 26 and 60 / 61, 370,001 33 / 32 and 82 / 75
+//   64-byte rows  2^18 25 / 32 and 65 / 71, 2^19 44 / 50 and 126 / 118,
+//                 741,001 60 / 64 and 179 / 165, 2^20 85 / 85 and 258 / 237
+//   96-byte rows  2^18 37 / 46 and 99 / 109, 741,001 94 / 101 and 270 / 271,
+//                 1,500,001 194 / 192 and 622 / 595
+// Columns picked evenly (4 and 16 edges, 85% and 91% of them hot), where
+// gathers get no denser and only rows of at most 16 bytes still gain, from
+// the taller tiles, when there are many:
+//   4-byte rows   2^19 18 / 25 and 44 / 54, 2^20 48 / 43 and 105 / 114
+//   16-byte rows  2^19 34 / 43 and 80 / 84, 2^20 105 / 80 and 234 / 237
+//   64-byte rows  2^20 95 / 117 and 312 / 334, 2^21 198 / 238 and 659 / 709
+// and with 62% and 75% hot:
+//   16-byte rows  2^19 33 / 40 and 65 / 68, 2^20 103 / 71 and 182 / 152
+//   32-byte rows  2^20 77 / 69 and 207 / 191
+//   64-byte rows  2^20 77 / 89 and 237 / 232, 2^21 170 / 183 and 536 / 522.
 // (FMX_HOT_MIN_BYTES, read at every call, puts an X-size threshold instead.)
 static bool gather_order_pays(const fmx_spm *s, uint64_t rb)
 {
     if (rb >= 128) return false;
     if (const char *hm = getenv("FMX_HOT_MIN_BYTES")) return s->ncols * rb > strtoull(hm, nullptr, 10);
-    if (s->esz) return s->ncols > 200000;
-    return s->ncols > std::max<uint64_t>(16384 * rb, 300000);
+    uint64_t least = s->esz ? std::max<uint64_t>(11500 * rb, 200000) : std::max<uint64_t>(16384 * rb, 300000);
+    if (8 * s->nhot > 5 * s->ncols) {
+        if (rb > 16 && 5 * s->nhot > 4 * s->ncols) return false;
+        least += least * 3 / 4;
+    }
+    return s->ncols > least;
 }
 
 // The SpMM entries (fmx_spmm, fmx_spmm_ex, fmx_spmm_scaled).

@@ -105,3 +105,45 @@ def test_gather_order_restages_x_rows_only(fmx, orc, rmat16, forced, n, k, col):
     staged = (X.astype(np.float64) * pre[:, None]).astype(np.float32).astype(np.float64)
     want = orc.spmm(img, staged) * post[:, None]
     assert rel(Y.cpu().numpy(), want) <= 2.0 ** -24 + 1e-15
+
+
+@pytest.mark.parametrize("graph,n,weighted,k,hot", [
+    ("even", 1 << 21, False, 16, False), ("even", 1 << 20, True, 16, False), ("even", 1 << 19, False, 4, False),
+    ("even", 1 << 20, False, 4, True), ("ring", 1 << 20, False, 10, False), ("rmat", 1 << 21, False, 16, True),
+    ("rmat", 1 << 20, True, 16, True), ("rmat", 1 << 18, True, 16, False), ("rmat", 1 << 21, True, 4, True)])
+def test_gather_order_where_columns_are_skewed(fmx, monkeypatch, graph, n, weighted, k, hot):
+    """Which image a multiply runs on, told by the hot block that the first
+    call of a context allocates: the gather order where a small share of the
+    columns is hot, the plain image where columns are picked evenly or there
+    are too few for the width; and the products are right on either."""
+    import torch
+    monkeypatch.delenv("FMX_HOT_MIN_BYTES", raising=False)
+    ctx = fmx.Context()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    if graph == "ring":
+        src = torch.arange(n, device="cuda", dtype=torch.int32).repeat(4)
+        dst = torch.cat([(src[:n] + j) % n for j in (1, 2, 3, 4)])
+    elif graph == "even":
+        src, dst = (torch.randint(0, n, (4 * n,), device="cuda", generator=g, dtype=torch.int32) for _ in range(2))
+    else:
+        src, dst = fmx.rmat_edges((n - 1).bit_length(), 4 * n, 7)
+    if weighted:
+        vals = torch.ones(src.numel(), device="cuda")
+        spm = fmx.SparseMatrix.build_weighted(src, dst, vals, n=n, log2_h=15, ctx=ctx)
+    else:
+        spm = fmx.SparseMatrix.build(src, dst, n=n, log2_h=15, ctx=ctx)
+    block = spm.info.hot_columns * k * 4
+    assert block > 3 << 20
+    X = torch.randint(-9, 10, (n, k), device="cuda", generator=g).float()
+    Y = torch.empty_like(X)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    spm.multiply_async(X, Y)
+    torch.cuda.synchronize()
+    taken = free - torch.cuda.mem_get_info()[0]
+    assert taken >= block if hot else taken < block, (taken, block)
+    monkeypatch.setenv("FMX_HOT_MIN_BYTES", "0" if not hot else str(1 << 60))
+    Z = torch.empty_like(X)
+    spm.multiply_async(X, Z)
+    assert torch.equal(Y, Z)
