@@ -856,8 +856,8 @@ fmx_status build_impl(fmx_ctx *ctx, const uint32_t *src, const uint32_t *dst, si
         nk = nu;
     }
     // the key (and payload) buffer that does not hold the result is not read
-    // again: its memory goes back before the run and tile arrays are made
-    // (17 GB at 2^31 edges)
+    // again: its block serves the work images' keys, or goes back if memory
+    // gets short (17 GB at 2^31 edges)
     for (DevBuf<uint64_t> *b : {&keys, &tmp})
         if (b->p != K) b->reset();
     for (DevBuf<uint32_t> *b : {&eidx, &etmp})

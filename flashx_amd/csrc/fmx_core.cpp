@@ -19,12 +19,16 @@ Plan::~Plan()
     if (d_items) (void)hipFree(d_items);  // d_splits lies behind them
 }
 
-StreamScratch::~StreamScratch()
+StreamScratch::~StreamScratch() { clear(); }
+
+void StreamScratch::clear()
 {
     for (const Buf &b : bufs_) {
-        (void)hipFree(b.ptr);
+        if (b.ptr) (void)hipFree(b.ptr);
         if (b.last) (void)hipEventDestroy(b.last);
     }
+    bufs_.clear();
+    turns_ = false;
 }
 
 fmx_status StreamScratch::get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphScratch &graphs, Lease &out)
@@ -1034,6 +1038,16 @@ fmx_status fmx_ctx_stream(fmx_ctx *ctx, void **stream)
 {
     if (!ctx || !stream) return FMX_EINVAL;
     *stream = ctx->stream;
+    return FMX_OK;
+}
+
+fmx_status fmx_ctx_trim(fmx_ctx *ctx)
+{
+    if (!ctx) return FMX_EINVAL;
+    FMX_HIP(ctx, hipSetDevice(ctx->device));
+    FMX_HIP(ctx, hipDeviceSynchronize());
+    ctx->blocks.trim(0);
+    for (StreamScratch *s : {&ctx->ws, &ctx->xstage, &ctx->xhot, &ctx->partial}) s->clear();
     return FMX_OK;
 }
 

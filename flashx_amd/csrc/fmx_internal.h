@@ -78,12 +78,13 @@ struct Plan {
 // its 16.5 ms in them).  Everything that uses them runs on the context's
 // stream, so a block may be handed on while kernels that use it are still
 // queued.  While a scope is open every block is kept, and kRest bytes when it
-// is closed, the largest blocks going back first; all of them go back when an
-// allocation fails and with the context, which one host thread uses at a time.
-// kRest covers the buffers of some 2^27 edges: the system clears what is freed
-// at about 200 GB/s behind the program's back, during which allocations wait
-// and copies from the host run at half their rate (a matrix streamed right
-// after builds that gave their buffers back: 8.0 ms a product instead of 4.0).
+// is closed, the largest blocks going back first; all of them go back when one of
+// the library's allocations fails, with fmx_ctx_trim and with the context, which
+// one host thread uses at a time.  kRest is what other allocators of the
+// process (torch's) have to do without: 1 GB covers the buffers of some 2^24
+// edges (2^20 vertices, 16 edges each: 0.8 GB kept, 3.5 ms a build, 4.3 with
+// 512 MB, 6.7 with none); larger builds are served in part (2^26 edges 14.5 ms,
+// 13.0 with 8 GB, 17.7 with none).
 // Blocks outside a scope are allocated and freed as they come.
 class BlockCache {
 public:
@@ -92,7 +93,7 @@ public:
     void put(void *p, size_t bytes);
     void trim(size_t most);
     int scopes = 0;
-    static constexpr size_t kRest = size_t(8) << 30;
+    static constexpr size_t kRest = size_t(1) << 30;
 
 private:
     std::vector<std::pair<size_t, void *>> free_;
@@ -176,6 +177,7 @@ public:
     StreamScratch &operator=(const StreamScratch &) = delete;
     ~StreamScratch();
     fmx_status get(fmx_ctx *ctx, hipStream_t s, size_t bytes, GraphScratch &graphs, Lease &out);
+    void clear();  // the device has finished
 
 private:
     static constexpr size_t kStreams = 4;

@@ -313,7 +313,8 @@ fmx_status rank_columns(fmx_ctx *ctx, const uint32_t *uses, uint64_t ncols, uint
     if (nh == 0 || nh + ncols > (1ull << 32)) return FMX_OK;  // no hot columns, or ids past 32 bits
     DevBuf<uint32_t> newid, hot;
     FMX_HIP(ctx, newid.alloc(ctx, ncols));
-    FMX_HIP(ctx, hot.alloc(ctx, nh));
+    // (stays with the matrix: of its own size, a kept block may be twice that)
+    FMX_HIP(ctx, dev_malloc(ctx, (void **)&hot.p, nh * sizeof(uint32_t)));
     hipLaunchKernelGGL(new_ids, dim3(grid_for(ctx, ncols)), dim3(kT), 0, s, ncols, nh, newid.p);
     hipLaunchKernelGGL(hot_ids, dim3(grid_for(ctx, nh)), dim3(kT), 0, s, sorted, nh, newid.p, hot.p);
     FMX_HIP(ctx, hipGetLastError());

@@ -63,6 +63,7 @@ SIGNATURES = {
     "fmx_ctx_destroy": (ctypes.c_int, [_vp]),
     "fmx_ctx_stream": (ctypes.c_int, [_vp, ctypes.POINTER(_vp)]),
     "fmx_ctx_sync": (ctypes.c_int, [_vp]),
+    "fmx_ctx_trim": (ctypes.c_int, [_vp]),
     "fmx_strerror": (ctypes.c_char_p, [ctypes.c_int]),
     "fmx_ctx_last_error": (ctypes.c_char_p, [_vp]),
     "fmx_spm_upload": (ctypes.c_int, [_vp, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t,
@@ -184,6 +185,10 @@ class Context:
 
     def sync(self):
         self.check(lib().fmx_ctx_sync(self.handle), "fmx_ctx_sync")
+
+    def trim(self):
+        """Gives back the device memory kept for later calls."""
+        self.check(lib().fmx_ctx_trim(self.handle), "fmx_ctx_trim")
 
     def close(self):
         if self.handle:

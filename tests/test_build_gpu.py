@@ -103,3 +103,33 @@ def test_build_errors(fmx):
     assert len(offs) == 4 and spm.get_nnz() == 0  # three empty block rows
     Y = spm.multiply(torch.ones((10, 3), device="cuda"))
     assert torch.all(Y == 0)
+
+
+def test_what_a_context_keeps_is_bounded_and_given_back(fmx):
+    """After builds whose buffers take some 4 GB the context holds at most the
+    gigabyte it may keep (and its fixed few megabytes); trim gives that and the
+    multiplies' scratch back, and building and multiplying go on as before."""
+    import torch
+    ctx = fmx.Context()
+    n = 1 << 22
+    src, dst = fmx.rmat_edges(22, 16 * n, 3)
+    X = torch.ones((n, 8), device="cuda", dtype=torch.int32)
+    Y = torch.empty_like(X)
+    torch.cuda.synchronize()
+
+    def used(before):
+        torch.cuda.synchronize()
+        return before - torch.cuda.mem_get_info()[0]
+
+    want = None
+    start = torch.cuda.mem_get_info()[0]
+    for _ in range(3):
+        a = fmx.SparseMatrix.build(src, dst, n=n, log2_h=6, ctx=ctx)
+        a.multiply_async(X, Y)
+        assert want is None or torch.equal(Y, want)
+        want = Y.clone() if want is None else want
+        del a
+        scratch = 2 * n * 8 * 4  # hot block and partial bands at most
+        assert used(start) - want.numel() * 4 <= (1 << 30) + scratch + (64 << 20)
+        ctx.trim()
+        assert used(start) - want.numel() * 4 <= 64 << 20
