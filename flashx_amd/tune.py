@@ -4,9 +4,8 @@ The tile height H trades image size (taller tiles: fewer tile headers, more
 rows per row part) against the LDS band each wave holds (H rows x k
 accumulators) and hence the number of resident waves.  The tuner builds the
 matrix on the device for each candidate (log2 H, log2 W), times a few SpMMs
-with the caller's width and type, and returns the fastest; of shapes within
-2% of each other, the spread of one shape's runs, the earlier candidate.
-Everything it runs is the product path (fmx_spm_build, fmx_spmm)."""
+with the caller's width and type, and returns the fastest.  Everything it
+runs is the product path (fmx_spm_build, fmx_spmm)."""
 import time
 
 from . import fmx as F
@@ -62,10 +61,7 @@ def autotune_tile(src, dst, n, k, dtype, flags=F.BUILD_DEDUP, candidates=DEFAULT
         if Y is None:
             Y = torch.empty((n, k), device=src.device, dtype=dtype)
         times[(lh, lw)] = _time_spmm(spm, X, Y, reps)
-        # (scale 22, FP32 k = 16: 64 rows take 0.670-0.673 ms and 128 rows 0.660-0.673, either way
-        # round, since both multiply in 64-row gather order; the taller shape
-        # also keeps a re-cut image)
-        if best is None or times[(lh, lw)] < 0.98 * times[best]:
+        if best is None or times[(lh, lw)] < times[best]:
             best, best_build, best_dev_ms = (lh, lw), build_s, spm.info.build_ns / 1e6
             best_spm = spm if keep and not lean else None
         del spm
