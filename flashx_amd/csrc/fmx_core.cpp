@@ -119,12 +119,12 @@ hipError_t BlockCache::get(size_t bytes, void **p, size_t *got)
     // the smallest block that fits and wastes no more than half
     size_t best = free_.size();
     for (size_t i = 0; scopes && i < free_.size(); i++)
-        if (free_[i].first >= bytes && free_[i].first / 2 <= bytes + 32768 &&
-            (best == free_.size() || free_[i].first < free_[best].first))
+        if (free_[i].bytes >= bytes && free_[i].bytes / 2 <= bytes + 32768 &&
+            (best == free_.size() || free_[i].bytes < free_[best].bytes))
             best = i;
     if (best < free_.size()) {
-        *got = free_[best].first;
-        *p = free_[best].second;
+        *got = free_[best].bytes;
+        *p = free_[best].p;
         held_ -= *got;
         free_.erase(free_.begin() + best);
         return hipSuccess;
@@ -140,7 +140,7 @@ hipError_t BlockCache::get(size_t bytes, void **p, size_t *got)
 void BlockCache::put(void *p, size_t bytes)
 {
     if (scopes) {
-        free_.emplace_back(bytes, p);
+        free_.push_back({bytes, p, build_});
         held_ += bytes;
     } else {
         (void)hipFree(p);
@@ -149,10 +149,12 @@ void BlockCache::put(void *p, size_t bytes)
 
 void BlockCache::trim(size_t most)
 {
-    std::sort(free_.begin(), free_.end());
+    std::stable_sort(free_.begin(), free_.end(), [](const Block &a, const Block &b) {
+        return a.build != b.build ? a.build > b.build : a.bytes < b.bytes;
+    });
     while (held_ > most) {
-        (void)hipFree(free_.back().second);
-        held_ -= free_.back().first;
+        (void)hipFree(free_.back().p);
+        held_ -= free_.back().bytes;
         free_.pop_back();
     }
 }

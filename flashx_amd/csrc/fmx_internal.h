@@ -78,13 +78,14 @@ struct Plan {
 // its 16.5 ms in them).  Everything that uses them runs on the context's
 // stream, so a block may be handed on while kernels that use it are still
 // queued.  While a scope is open every block is kept, and kRest bytes when it
-// is closed, the largest blocks going back first; all of them go back when one of
-// the library's allocations fails, with fmx_ctx_trim and with the context, which
-// one host thread uses at a time.  kRest is what other allocators of the
-// process (torch's) have to do without: 1 GB covers the buffers of some 2^24
-// edges (2^20 vertices, 16 edges each: 0.8 GB kept, 3.5 ms a build, 4.3 with
-// 512 MB, 6.7 with none); larger builds are served in part (2^26 edges 14.5 ms,
-// 13.0 with 8 GB, 17.7 with none).
+// is closed: first the blocks that the latest build did not use go back, then
+// its largest.  All of them go back when one of the library's allocations
+// fails, with fmx_ctx_trim and with the context, which one host thread uses at
+// a time.  kRest is what other allocators of the process (torch's) have to do
+// without; 2 GB (8 GB: 13.0 ms at 2^26 edges, none: 17.7) hold what builds of up
+// to 2^24 edges use, among blocks of other sizes too: with 1 GB, builds of
+// 2^20 vertices, 16 edges each, took 4.5 ms by themselves and 5.0 to 5.9 after
+// larger ones, whose blocks they take over.
 // Blocks outside a scope are allocated and freed as they come.
 class BlockCache {
 public:
@@ -93,16 +94,26 @@ public:
     void put(void *p, size_t bytes);
     void trim(size_t most);
     int scopes = 0;
-    static constexpr size_t kRest = size_t(1) << 30;
+    static constexpr size_t kRest = size_t(2) << 30;
 
 private:
-    std::vector<std::pair<size_t, void *>> free_;
+    struct Block {
+        size_t bytes;
+        void *p;
+        uint64_t build;  // that used it last
+    };
+    std::vector<Block> free_;
     size_t held_ = 0;
+    uint64_t build_ = 0;
+    friend struct BlockScope;
 };
 
 struct BlockScope {
     BlockCache &c;
-    explicit BlockScope(BlockCache &cache) : c(cache) { c.scopes++; }
+    explicit BlockScope(BlockCache &cache) : c(cache)
+    {
+        if (c.scopes++ == 0) c.build_++;
+    }
     ~BlockScope() { if (--c.scopes == 0) c.trim(BlockCache::kRest); }
 };
 

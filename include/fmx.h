@@ -82,7 +82,7 @@ fmx_status fmx_ctx_stream(fmx_ctx *ctx, void **stream);
 fmx_status fmx_ctx_sync(fmx_ctx *ctx);
 /* No counterpart in the reference.  Gives back the device memory that the
  * context keeps for later calls: the buffers of matrix constructions (at most
- * 1 GB stay between them) and the scratch of multiplies and dense operations,
+ * 2 GB stay between them) and the scratch of multiplies and dense operations,
  * for programs whose own allocations need it.  Waits for the device; what
  * matrices and captured graphs hold stays. */
 fmx_status fmx_ctx_trim(fmx_ctx *ctx);
