@@ -161,7 +161,7 @@ struct Lanes {
 // above; K < 0 is any width of at least -K columns, -K elements per lane
 // (Row below); K = 0 walks flat (entry, element) pairs, one element per lane
 // and step: rows wider than 64 lanes hold, and the sequential mode's runtime
-// widths.
+// widths (never in gather order).
 template <typename T, int K>
 constexpr int row_elems()
 {
@@ -568,7 +568,7 @@ __device__ __forceinline__ T load_value(const uint16_t *p)
 
 // Runtime width: flat (entry, element) pairs, one element per lane; weighted
 // images (V) multiply it by the entry's value.
-template <typename T, typename V, typename A, bool HOT, bool NARROW>
+template <typename T, typename V, typename A, bool NARROW>
 __device__ __forceinline__ void drain_generic(const SpmmArgs &a, A *band, uint32_t S, const Queue<NARROW> &q,
                                               const uint32_t *qval, const uint16_t *vimg, uint32_t qn, int lane)
 {
@@ -584,7 +584,7 @@ __device__ __forceinline__ void drain_generic(const SpmmArgs &a, A *band, uint32
             const uint32_t e = fc / k, j = fc - e * k;
             uint32_t gc, qr;
             q.get(e, gc, qr);
-            v[pp] = (A)*xrow<T, HOT, NARROW>(a, gc, j * sizeof(T));
+            v[pp] = (A)*xrow<T, false, NARROW>(a, gc, j * sizeof(T));
             if constexpr (!std::is_void<V>::value) v[pp] *= (A)load_value<V>(vimg + qval[e]);
             dst[pp] = f < tot ? qr * S + j : 0xFFFFFFFFu;
         }
@@ -900,7 +900,7 @@ __device__ __forceinline__ void spmm_body(const SpmmArgs &a)
             fetch_next();
             if (qn) {
                 if constexpr (SEQ) drain_generic_seq<T, V>(a, band, S, q, qval, vimg, qn, lane);
-                else drain_generic<T, V, A, HOT>(a, band, S, q, qval, vimg, qn, lane);
+                else drain_generic<T, V, A>(a, band, S, q, qval, vimg, qn, lane);
             }
         }
         wave_sync();
@@ -954,7 +954,7 @@ __global__ void __launch_bounds__(256) spmm_reduce(const Split *splits, const A 
 }
 
 // Gathers in flight per lane group (kP): eight 16-byte gathers per lane keep
-// spmm_lane under 96 VGPRs.  More resident waves with short batches put more
+// spmm_lane at 86 VGPRs at most (FP32 k = 16: 77).  More resident waves with short batches put more
 // gathers in flight than fewer waves with long ones: on R-MAT scale 22, FP32
 // k = 16, 64x32768 tiles, 0.93 ms against 1.30 ms for 512-entry batches
 // overlapped with the next decode at two waves per SIMD (the best earlier
@@ -1052,7 +1052,10 @@ fmx_status launch_runtime(fmx_ctx *ctx, SpmmArgs a, int vprim, hipStream_t strea
             if (e == 4) return launch_k<T, -4, SEQ, HOT>(ctx, a, vprim, stream);
         if (e == 2) return launch_k<T, -2, SEQ, HOT>(ctx, a, vprim, stream);
     }
-    return launch_k<T, 0, SEQ, HOT>(ctx, a, vprim, stream);
+    // gather-order rows are shorter than 128 bytes, so what is left of them is
+    // one column at an address of less than its own alignment
+    if constexpr (HOT) return launch_k<T, 1, SEQ, HOT>(ctx, a, vprim, stream);
+    else return launch_k<T, 0, SEQ, HOT>(ctx, a, vprim, stream);
 }
 
 // HOT (a gather-order image, rows narrower than a 128-byte line) has kernels
