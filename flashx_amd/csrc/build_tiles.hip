@@ -623,7 +623,7 @@ fmx_status write_image(fmx_ctx *ctx, const uint64_t *K, const uint32_t *V, uint6
     FMX_HIP(ctx, hipGetLastError());
     if (done) FMX_HIP(ctx, hipEventRecord(done, s));
     // the host keeps the block-row offsets and first directory indices; the
-    // directory itself stays in HBM (plans copy the few block rows they split)
+    // directory itself stays in HBM (plan_cuts reads it there)
     std::vector<uint64_t> oex(nbr + 1);
     unsigned int hbad = 0;
     spm->brow_dir.resize(nbr + 1);

@@ -655,8 +655,6 @@ fmx_status get_plan(fmx_ctx *ctx, fmx_spm *s, uint32_t hs, bool ordered, Plan **
     return FMX_OK;
 }
 
-// A device-built image: bring the host copy, validate it like an uploaded
-// one and publish the tile directory.
 // Tile directory (and, for weighted images, the values directory) to HBM.
 fmx_status upload_dirs(fmx_ctx *ctx, fmx_spm *s)
 {

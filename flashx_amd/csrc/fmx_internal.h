@@ -327,9 +327,9 @@ fmx_status gather_order_lists(fmx_ctx *ctx, const fmx_spm *src, uint64_t ncols, 
 fmx_status decode_lists(fmx_ctx *ctx, const fmx_spm *src, uint32_t *rows, uint32_t *cols, void *vals,
                         uint32_t *uses);
 // The split items among the n device items of an image built on the device:
-// their ranges' ends move out of tile headers (binary) or back to a tile
-// start (weighted), and dir_begin, carry and the rotation fields are filled
-// in (image_dev.hip).  Sets the flag in ctx->pinned if an item is
+// their ranges' ends move out of tile headers (binary) or to their share of
+// a tile's entries (weighted), and dir_begin, carry, before (weighted) and the
+// rotation fields are filled in (image_dev.hip).  Sets the flag in ctx->pinned if an item is
 // inconsistent; on ctx->stream, not synchronised.
 fmx_status plan_cuts(fmx_ctx *ctx, const fmx_spm *s, Item *items, uint32_t n);
 fmx_status finish_streamed(fmx_ctx *ctx, fmx_spm *s, uint64_t chunk_bytes, bool whole_file);
@@ -354,8 +354,7 @@ constexpr uint32_t kSpmmRoundFirst = 1u << 31;
 
 // Launches the SpMM kernel over plan items [item_begin, item_end) with the
 // image at img (absolute u16 word w of the image is img[w]) and, if reduce,
-// the in-order reduction of the plan's split bands.
-// the kernels' part of the FMX_SPMM_* flags (FMX_SPMM_SEQ, FMX_SPMM_Y_COLMAJOR).
+// the in-order reduction of the plan's split bands.  flags: the kernels' part of the FMX_SPMM_* flags (FMX_SPMM_SEQ, FMX_SPMM_Y_COLMAJOR).
 // Columns below nhot are read from Xhot (nhot x k, leading dimension k),
 // column c >= nhot from row c - nhot of X.
 fmx_status launch_spmm(fmx_ctx *ctx, const fmx_spm *spm, const Plan *plan,

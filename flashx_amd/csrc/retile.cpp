@@ -188,12 +188,18 @@ void retile_image(const fmx_spm *s, uint32_t h2, std::vector<uint8_t> &img, std:
 // Tile height of the work image (0: none); FMX_WORK_ROWS overrides it (0
 // turns the work image off).  Taller tiles than 64 rows are re-cut to 32: a
 // 32-row band of 16 FP32 columns and its queue leave room in LDS for as many
-// waves as the registers do, a 64-row one for 13 of those 20.  64 against 32
+// waves as the kernel is compiled for, a 64-row one for 13 of those 20.  64 against 32
 // rows: four NMF sweeps of rank 20 over 260,000 vertices 1.53 / 1.32 ms, a
 // training step at 131,072 vertices (k = 64) 0.88 / 0.80 ms, scale 16 FP64
 // k = 8 22 / 20 us, 700,001 x 10 FP32 106 / 106; one column, which pays for
 // every tile header, is slower (a PageRank sweep of 2^20 vertices 109 / 117
-// us).  16 rows lose 10% at k = 10 and 23% at k = 1.  A 64-row image stays as
+// us).  Rows of 64 FP32 columns gain most (R-MAT scales 18, 20, 21: 141 / 93,
+// 571 / 380, 1229 / 839 us); in plain order at scale 20 and above rows of up
+// to 64 bytes lose up to 13% (FP64 k = 8 163 / 185 us), which the gather order,
+// in 64-row tiles, mostly takes over there.  A streamed matrix pays for the
+// headers on the host link (k = 32, scale 18 281 / 274 us, scale 20 1146 / 1284)
+// and is re-cut to the same height all the same: an FP64 row's sum depends on
+// the height, and streamed products are the resident ones bit for bit.  16 rows lose 10% at k = 10 and 23% at k = 1.  A 64-row image stays as
 // it is.
 uint32_t work_rows_for(const fmx_spm *s)
 {
