@@ -59,6 +59,7 @@ struct SpmmArgs {
     const double *rscale;  // floating-point data: Y row r is scaled by rscale[r] (or null)
     int ycol;              // Y column-major: element (r, j) at Y[j * ldy + r]
     int round_first;       // a scaled row's sum is rounded to T before it is scaled
+    int low_bands;         // bands are lower than tiles: entries outside an item's band are met
     const void *Xhot;      // gather-order images: rows of columns < nhot (leading dimension k)
     uint64_t nhot;         // columns c >= nhot are row c - nhot of X
     const void *Xcold;     // narrow forms: X - nhot rows, so that row c of it is column c >= nhot
@@ -182,6 +183,7 @@ template <typename T, int K>
 struct Row {
     static constexpr int E = row_elems<T, K>();
     uint32_t g, nzp, colb, off[E];
+    bool on = true;  // the lane has a share
     __device__ __forceinline__ Row(int k, int lane)
     {
         if constexpr (K > 0) {
@@ -198,7 +200,7 @@ struct Row {
             g = lane / L;
             const uint32_t q = lane - g * L;
             const uint32_t col0 = min(q * E, (uint32_t)k - E), skip = q * E - col0;
-            const bool on = g < nzp;
+            on = g < nzp;
 #pragma unroll
             for (uint32_t i = 0; i < (uint32_t)E; i++) off[i] = !on || i < skip ? E * L : (i - skip) * L + q;
             if (!on) g = 0;
@@ -466,18 +468,46 @@ __device__ __forceinline__ void fill_queue(const Queue<NARROW> &q, uint32_t *qva
     wave_sync();
 }
 
-// Adds a batch to the band, run by run; scale(pp, i, x) is entry pp's element
-// i in the accumulator's type (times its value).
+// Whether lanes without a share of a batch are kept from adding: at runtime
+// widths, which can leave 31 of 64 lanes over, and where many entries go side
+// by side.  Elsewhere the mask costs more than it saves (FP32 k = 64, few
+// non-zeros: 3%).
+template <typename T, int K>
+constexpr bool stays_out()
+{
+    if constexpr (K > 0) return Lanes<T, K>::NZP >= 16;
+    else return true;
+}
+
+// Adds a batch to the band, run by run; elem(pp, i) is entry pp's element i
+// in the accumulator's type (times its value).  Lane groups without an entry
+// (`some` is false, in a chunk's last batch) and lanes without a share of a row
+// stay out, and single adds (!RUNS) of entries outside the band are left out
+// where there are any: all of those go to one row, whose adds the LDS takes
+// one after the other (2^20 evenly picked columns, 4 edges a vertex, FP64 k = 1
+// in 32-row tiles: 151 us with them, 52 without).
 template <typename T, int K, typename A, bool RUNS, typename F>
-__device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, const Row<T, K> &row, const uint32_t *rr, F elem)
+__device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, const Row<T, K> &row, const uint32_t *rr,
+                                                 bool some, bool low_bands, uint32_t dump, F elem)
 {
     constexpr int E = row_elems<T, K>();
+    if (stays_out<T, K>() && (!some || !row.on)) return;
     if constexpr (!RUNS) {
+        if (low_bands) {
 #pragma unroll
-        for (int pp = 0; pp < kP; pp++) {
-            A *dst = band + __umul24(rr[pp], S);
+            for (int pp = 0; pp < kP; pp++) {
+                if (rr[pp] == dump) continue;
+                A *dst = band + __umul24(rr[pp], S);
 #pragma unroll
-            for (int i = 0; i < E; i++) lds_add(dst + row.off[i], elem(pp, i));
+                for (int i = 0; i < E; i++) lds_add(dst + row.off[i], elem(pp, i));
+            }
+        } else {
+#pragma unroll
+            for (int pp = 0; pp < kP; pp++) {
+                A *dst = band + __umul24(rr[pp], S);
+#pragma unroll
+                for (int i = 0; i < E; i++) lds_add(dst + row.off[i], elem(pp, i));
+            }
         }
     } else {
         A acc[E];
@@ -517,14 +547,16 @@ __device__ __forceinline__ void accumulate_batch(A *band, uint32_t S, const Row<
 // inside a group is chained in registers, which is the same sequence of
 // roundings.
 template <typename T, int K>
-__device__ __forceinline__ void accumulate_batch_seq(T *band, uint32_t S, int lane, const Vec<T, Lanes<T, K>::E> *v,
-                                                     const uint32_t *rr)
+__device__ __forceinline__ void accumulate_batch_seq(T *band, uint32_t S, int lane, uint32_t entries,
+                                                     const Vec<T, Lanes<T, K>::E> *v, const uint32_t *rr)
 {
 #pragma clang fp contract(off)
     using C = Lanes<T, K>;
     const int q = lane % C::L;
     const int g = lane / C::L;
-    for (int gg = 0; gg < C::NZP; gg++) {
+    // (the groups with entries, where there may be many without)
+    const int groups = C::NZP >= 32 && entries < C::NZP * kP ? (int)(entries + kP - 1) / kP : C::NZP;
+    for (int gg = 0; gg < groups; gg++) {
         if (g == gg) {
             T acc[C::E];
             uint32_t cur = rr[0];
@@ -586,7 +618,7 @@ __device__ __forceinline__ void drain_generic(const SpmmArgs &a, A *band, uint32
             q.get(e, gc, qr);
             v[pp] = (A)*xrow<T, false, NARROW>(a, gc, j * sizeof(T));
             if constexpr (!std::is_void<V>::value) v[pp] *= (A)load_value<V>(vimg + qval[e]);
-            dst[pp] = f < tot ? qr * S + j : 0xFFFFFFFFu;
+            dst[pp] = f < tot && qr != a.hs ? qr * S + j : 0xFFFFFFFFu;
         }
 #pragma unroll
         for (int pp = 0; pp < kP; pp++)
@@ -872,6 +904,7 @@ __device__ __forceinline__ void spmm_body(const SpmmArgs &a)
                     fetch_next();
                     fetched = true;
                 }
+                const bool some = base + row.g * kP < qn;
                 if constexpr (SEQ) {
                     if constexpr (W) {
                         // products rounded in T, then added in order
@@ -881,9 +914,9 @@ __device__ __forceinline__ void spmm_body(const SpmmArgs &a)
 #pragma unroll
                             for (int i = 0; i < E; i++) v[pp].v[i] = v[pp].v[i] * (T)vals[pp];
                     }
-                    accumulate_batch_seq<T, K>(band, S, lane, v, rr);
+                    accumulate_batch_seq<T, K>(band, S, lane, qn - base, v, rr);
                 } else if constexpr (W) {
-                    accumulate_batch<T, K, A, true>(band, S, row, rr,
+                    accumulate_batch<T, K, A, true>(band, S, row, rr, some, a.low_bands, st.ic.dump,
                                                     [&](int pp, int i) { return (A)v[pp].v[i] * (A)vals[pp]; });
                 } else {
                     // 8-byte data: each entry adds straight into the band.
@@ -891,7 +924,7 @@ __device__ __forceinline__ void spmm_body(const SpmmArgs &a)
                     // per tile on R-MAT) and their divergent branches cost
                     // more than that for E <= 2 (FP64 k = 16: 1.17 ms
                     // against 1.34 ms with run sums)
-                    accumulate_batch<T, K, A, sizeof(T) != 8>(band, S, row, rr,
+                    accumulate_batch<T, K, A, sizeof(T) != 8>(band, S, row, rr, some, a.low_bands, st.ic.dump,
                                                               [&](int pp, int i) { return (A)v[pp].v[i]; });
                 }
             }
@@ -1108,6 +1141,7 @@ fmx_status launch_t(fmx_ctx *ctx, const fmx_spm *spm, const Plan *plan, int k,
     a.rscale = rscale;
     a.ycol = (flags & FMX_SPMM_Y_COLMAJOR) ? 1 : 0;
     a.round_first = (flags & kSpmmRoundFirst) ? 1 : 0;
+    a.low_bands = plan->hs < spm->H;
     a.Xhot = Xhot;
     a.nhot = Xhot ? nhot : 0;
     // 16-byte vector gathers need aligned rows; otherwise the runtime-width path.

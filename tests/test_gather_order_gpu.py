@@ -147,3 +147,21 @@ def test_gather_order_where_columns_are_skewed(fmx, monkeypatch, graph, n, weigh
     Z = torch.empty_like(X)
     spm.multiply_async(X, Z)
     assert torch.equal(Y, Z)
+
+
+@pytest.mark.parametrize("dt", ["int64", "float64"])
+def test_one_column_below_its_alignment(fmx, orc, rmat16, forced, dt):
+    """One column of 8-byte elements that starts between two of them: the
+    one-column form takes it as it takes an aligned one."""
+    import torch
+    src, dst = rmat16
+    img = orc.build_2d(src, dst, n=1 << 16, log2h=6, log2w=15)
+    spm = fmx.SparseMatrix.upload(img.data, img.offs)
+    X = np.random.default_rng(4).integers(-9, 10, (img.n, 1)).astype(dt)
+    raw = torch.zeros(8 * img.n + 4, dtype=torch.uint8, device="cuda")
+    raw[4:].copy_(torch.from_numpy(X.view(np.uint8).reshape(-1)))
+    Y = torch.empty((img.n, 1), dtype=getattr(torch, dt), device="cuda")
+    ctx = spm.ctx
+    ctx.check(fmx.lib().fmx_spmm(ctx.handle, spm.handle, fmx.dtype_code(Y.dtype), 1, raw.data_ptr() + 4, 1,
+                                 Y.data_ptr(), 1, ctx.stream_ptr()), "fmx_spmm")
+    assert np.array_equal(Y.cpu().numpy(), orc.spmm(img, X))

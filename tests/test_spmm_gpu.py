@@ -594,3 +594,36 @@ def test_threads_own_streams_have_their_own_scratch(fmx, monkeypatch):
     assert all(f >= least for f in free), free
     for y, (_, _, want) in zip(Y, pair):
         assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("lh", [5, 6, 15])
+@pytest.mark.parametrize("dt", ["int64", "float64"])
+def test_few_entries_a_chunk_cost_8_byte_types_no_more(fmx, lh, dt):
+    """One column on a sparse graph, whose chunks of 512 words hold far fewer
+    entries than a batch has places: 8-byte elements, which are added one by
+    one, take at most 1.6 times as long as 4-byte ones (twice the bytes of X
+    and Y beside the same image; adding the empty places too took 2 to 3.4
+    times as long)."""
+    import torch
+    n = 1 << 20
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9)
+    src, dst = (torch.randint(0, n, (4 * n,), device="cuda", generator=g, dtype=torch.int32) for _ in range(2))
+    spm = fmx.SparseMatrix.build(src, dst, n=n, log2_h=lh)
+
+    def us(dtype):
+        X = torch.randint(-9, 10, (n, 1), device="cuda", generator=g).to(dtype)
+        Y = torch.empty_like(X)
+        best = 1e9
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                spm.multiply_async(X, Y)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 50)
+        return best
+
+    narrow, wide = us(torch.float32), us(getattr(torch, dt))
+    assert wide <= 1.6 * narrow, (wide, narrow)
