@@ -821,44 +821,52 @@ static int value_prim(fmx_dtype dt)
     }
 }
 
-// Whether an SpMM with X rows of rb bytes runs on the matrix's gather-order
-// image.  Never for rows of a full 128-byte line, which gain nothing from
-// lying next to another hot row.  Otherwise by the number of columns (the
-// narrower the rows, the more of them a line of the hot block serves, and
-// copying the hot rows has to be worth while) and by the share of them that is
-// hot.  Plain / gather-order image, us, FP32, re-cut default tiles:
-// R-MAT, 4 and 24 edges a vertex, a fifth of the columns hot, binary:
-//   4-byte rows   370,001 columns 19 / 16 and 42 / 35, 2^20 44 / 33 and 126 / 100
-//   16-byte rows  370,001 31 / 25 and 56 / 52, 2^20 81 / 54 and 186 / 133
-//   32-byte rows  370,001 25 / 26 and 58 / 58, 2^19 33 / 31 and 81 / 76
-//   40-byte rows  2^19 36 / 39 and 98 / 95, 741,001 49 / 49 and 152 / 131
-//   64-byte rows  741,001 44 / 49 and 124 / 129, 2^20 62 / 64 and 192 / 184
-//   96-byte rows  2^20 100 / 109 and 327 / 307, 1,500,001 152 / 151 and 512 / 457
-// and weighted, which has more tiles to step through:
-//   16-byte rows  230,001 27 / 25 and 65 / 54, 2^19 57 / 45 and 146 / 102
-//   32-byte rows  2^18 24 / 26 and 60 / 61, 370,001 33 / 32 and 82 / 75
-//   64-byte rows  2^18 25 / 32 and 65 / 71, 2^19 44 / 50 and 126 / 118,
-//                 741,001 60 / 64 and 179 / 165, 2^20 85 / 85 and 258 / 237
-//   96-byte rows  2^18 37 / 46 and 99 / 109, 741,001 94 / 101 and 270 / 271,
-//                 1,500,001 194 / 192 and 622 / 595
+// Whether an SpMM with rows of k elements of es bytes runs on the matrix's
+// gather-order image.  Never for rows of a full 128-byte line, which gain
+// nothing from lying next to another hot row.  Otherwise by the number of
+// columns (the narrower the rows, the more of them a line of the hot block
+// serves, and copying the hot rows has to be worth while) and by the share of
+// them that is hot.  Plain / gather-order image, us, re-cut default tiles,
+// R-MAT with 4 and 24 edges a vertex, a fifth of the columns hot.  Binary,
+// 4-byte elements:
+//   k = 1   370,001 columns 18 / 16 and 42 / 35, 2^20 42 / 33 and 125 / 100
+//   k = 4   370,001 21 / 21 and 51 / 50, 2^20 50 / 41 and 159 / 127
+//   k = 8   370,001 22 / 25 and 55 / 57, 2^19 28 / 30 and 77 / 74
+//   k = 10  2^19 34 / 38 and 96 / 94, 741,001 46 / 48 and 148 / 130
+//   k = 16  741,001 43 / 49 and 122 / 128, 2^20 60 / 64 and 190 / 183
+//   k = 24  2^20 97 / 107 and 318 / 300, 1,500,001 146 / 149 and 508 / 453
+// 8-byte elements, whose adds one by one weigh more than the lines:
+//   k = 1   370,001 17 / 17 and 44 / 49, 2^19 23 / 22 and 65 / 66
+//   k = 4   741,001 39 / 41 and 136 / 156, 2^20 53 / 53 and 197 / 216,
+//           1,500,001 78 / 70 and 306 / 302
+//   k = 8   2^20 60 / 63 and 213 / 234, 1,500,001 86 / 85 and 333 / 330
+// Weighted, which has more tiles to step through, 4-byte elements:
+//   k = 4   230,001 20 / 21 and 51 / 48, 2^19 38 / 34 and 108 / 91
+//   k = 8   2^18 23 / 24 and 59 / 59, 370,001 29 / 30 and 79 / 73
+//   k = 16  2^19 43 / 49 and 122 / 118, 741,001 58 / 63 and 174 / 164
+//   k = 24  741,001 93 / 101 and 264 / 269, 2^20 130 / 137 and 392 / 390
+// (64-row tiles, 4 and 16 edges: k = 16 2^18 27 / 31 and 62 / 58, 2^19 47 / 49
+// and 105 / 92) and 8-byte ones (4 and 16 edges):
+//   k = 1   230,001 21 / 19 and 45 / 35;  k = 8  24 / 28 and 50 / 50
 // Columns picked evenly (4 and 16 edges, 85% and 91% of them hot), where
-// gathers get no denser and only rows of at most 16 bytes still gain, from
-// the taller tiles, when there are many:
-//   4-byte rows   2^19 18 / 25 and 44 / 54, 2^20 48 / 43 and 105 / 114
-//   16-byte rows  2^19 34 / 43 and 80 / 84, 2^20 105 / 80 and 234 / 237
-//   64-byte rows  2^20 95 / 117 and 312 / 334, 2^21 198 / 238 and 659 / 709
-// and with 62% and 75% hot:
-//   16-byte rows  2^19 33 / 40 and 65 / 68, 2^20 103 / 71 and 182 / 152
-//   32-byte rows  2^20 77 / 69 and 207 / 191
-//   64-byte rows  2^20 77 / 89 and 237 / 232, 2^21 170 / 183 and 536 / 522.
+// gathers get no denser and only the tiles, if they are taller, help one
+// 4-byte column of a very sparse matrix:
+//   k = 1   2^19 18 / 25, 2^20 46 / 43 and 105 / 115 (a ring of 4: 27 / 21)
+//   k = 4   2^19 29 / 35, 2^20 69 / 76 and 228 / 231
+//   k = 16  2^20 95 / 117 and 312 / 334
+// and with 75% hot, 16 edges:
+//   k = 4   2^19 61 / 64, 2^20 179 / 148;  k = 16  2^20 237 / 232.
 // (FMX_HOT_MIN_BYTES, read at every call, puts an X-size threshold instead.)
-static bool gather_order_pays(const fmx_spm *s, uint64_t rb)
+static bool gather_order_pays(const fmx_spm *s, int k, int es)
 {
+    const uint64_t rb = (uint64_t)k * es;
     if (rb >= 128) return false;
     if (const char *hm = getenv("FMX_HOT_MIN_BYTES")) return s->ncols * rb > strtoull(hm, nullptr, 10);
-    uint64_t least = s->esz ? std::max<uint64_t>(11500 * rb, 200000) : std::max<uint64_t>(16384 * rb, 300000);
+    uint64_t least;
+    if (s->esz) least = es == 8 || rb <= 16 ? 200000 : s->work ? 11500 * rb : 300000;
+    else least = std::max<uint64_t>(16384 * rb, es == 4 ? 300000 : k == 1 ? 500000 : 1050000);
     if (8 * s->nhot > 5 * s->ncols) {
-        if (rb > 16 && 5 * s->nhot > 4 * s->ncols) return false;
+        if (5 * s->nhot > 4 * s->ncols && (rb > 4 || !s->work || s->nnz >= 6 * s->ncols)) return false;
         least += least * 3 / 4;
     }
     return s->ncols > least;
@@ -899,7 +907,7 @@ fmx_status spmm_exec(fmx_ctx *ctx, const fmx_spm *cspm, fmx_dtype dtype, int k, 
     // tiles are taller than a band
     const fmx_spm *orig = spm;
     GraphScratch &graphs = spm->graphs;
-    const bool hot = !seq && spm->fast && gather_order_pays(spm, (uint64_t)k * es);
+    const bool hot = !seq && spm->fast && gather_order_pays(spm, k, es);
     if (hot) spm = spm->fast.get();
     else if (spm->work) spm = spm->work.get();
     Plan *plan = nullptr;

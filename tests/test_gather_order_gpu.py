@@ -109,8 +109,9 @@ def test_gather_order_restages_x_rows_only(fmx, orc, rmat16, forced, n, k, col):
 
 @pytest.mark.parametrize("graph,n,weighted,k,hot", [
     ("even", 1 << 21, False, 16, False), ("even", 1 << 20, True, 16, False), ("even", 1 << 19, False, 4, False),
-    ("even", 1 << 20, False, 4, True), ("ring", 1 << 20, False, 10, False), ("rmat", 1 << 21, False, 16, True),
-    ("rmat", 1 << 20, True, 16, True), ("rmat", 1 << 18, True, 16, False), ("rmat", 1 << 21, True, 4, True)])
+    ("even", 1 << 20, False, 4, False), ("even", 1 << 20, False, 1, True), ("ring", 1 << 20, False, 10, False),
+    ("rmat", 1 << 21, False, 16, True), ("rmat", 1 << 20, True, 16, True), ("rmat", 1 << 18, True, 16, False),
+    ("rmat", 1 << 21, True, 4, True)])
 def test_gather_order_where_columns_are_skewed(fmx, monkeypatch, graph, n, weighted, k, hot):
     """Which image a multiply runs on, told by the hot block that the first
     call of a context allocates: the gather order where a small share of the
@@ -165,3 +166,23 @@ def test_one_column_below_its_alignment(fmx, orc, rmat16, forced, dt):
     ctx.check(fmx.lib().fmx_spmm(ctx.handle, spm.handle, fmx.dtype_code(Y.dtype), 1, raw.data_ptr() + 4, 1,
                                  Y.data_ptr(), 1, ctx.stream_ptr()), "fmx_spmm")
     assert np.array_equal(Y.cpu().numpy(), orc.spmm(img, X))
+
+
+def test_gather_order_from_more_columns_of_8_byte_elements(fmx, monkeypatch):
+    """FP64 rows of two and more elements take the gather order from 1,050,000
+    columns, one element from 500,000 (told as above)."""
+    import torch
+    monkeypatch.delenv("FMX_HOT_MIN_BYTES", raising=False)
+    for n, k, hot in ((1 << 20, 4, False), (1 << 21, 4, True), (1 << 21, 1, True), (1 << 20, 7, False)):
+        ctx = fmx.Context()
+        src, dst = fmx.rmat_edges((n - 1).bit_length(), 4 * n, 7)
+        spm = fmx.SparseMatrix.build(src, dst, n=n, log2_h=15, ctx=ctx)
+        block = spm.info.hot_columns * k * 8
+        X = torch.ones((n, k), device="cuda", dtype=torch.float64)
+        Y = torch.empty_like(X)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        spm.multiply_async(X, Y)
+        torch.cuda.synchronize()
+        taken = free - torch.cuda.mem_get_info()[0]
+        assert taken >= block > 2 << 20 if hot else taken < block, (n, k, taken, block)
